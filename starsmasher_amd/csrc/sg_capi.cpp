@@ -46,6 +46,8 @@ struct sg_context {
     int64_t cap_psipart = 0;
     unsigned char *nearflag = nullptr;
     int64_t cap_flag = 0;
+    unsigned char *sym = nullptr;       // tables of the unordered-pair pass
+    int64_t cap_sym = 0;
     // [4]: chunk visits, near chunk visits, wide chunk visits (FP64-formed
     // differences in the far loop), pairs evaluated in FP64 (FP32C pass)
     unsigned long long *stats = nullptr;
@@ -226,7 +228,40 @@ int auto_jsplit(int niblocks, int wg, int ntiles, int64_t ni)
     return (int)std::max<int64_t>(1, std::min(want, cap));
 }
 
-EvalPlan plan_eval(int n, int ni, int wg, int ipl, int jsplit_cfg, int precision, bool psi)
+// Byte offsets in the buffer of a sym plan's tables.
+struct SymLayout {
+    int64_t boxes, bits, seg, bytes;
+};
+static SymLayout sym_layout(int nchunks)
+{
+    SymLayout l{};
+    l.bits = (int64_t)nchunks * 2 * sizeof(float4);
+    l.seg = l.bits + (int64_t)nchunks * ((nchunks + 63) / 64) * 8;
+    l.bytes = l.seg + ((int64_t)nchunks + 2) * 4;
+    return l;
+}
+
+// The whole-set FP32C pass evaluates each unordered far pair once.  Up to
+// SYM_MAX_SB superblocks make the work items (8,256 pairs of them at 128, 16
+// rounds of the workgroups that fit at once) and the partial-sum slabs (32 B
+// per particle each).  A workgroup has as many waves as its superblock has
+// column groups of four chunks, up to four.
+static void plan_sym(EvalPlan &p, int n)
+{
+    const int nchunks = (int)(p.padded / TC);
+    const int want = (nchunks + SYM_MAX_SB - 1) / SYM_MAX_SB;
+    p.waves = want > 8 ? 4 : (want > 4 ? 2 : 1);
+    const int step = 4 * p.waves;   // a column group: four chunks per wave
+    p.sb = (want + step - 1) / step * step;
+    p.nsb = (nchunks + p.sb - 1) / p.sb;
+    p.jsplit = p.nsb + 1;
+    p.part_elems = (int64_t)p.jsplit * 4 * n + ((int64_t)SYM_SEGS + nchunks) * 4 * TC;
+    p.sym_bytes = sym_layout(nchunks).bytes;
+    p.sym = true;
+}
+
+EvalPlan plan_eval(int n, int ni, int wg, int ipl, int jsplit_cfg, int precision, bool psi,
+                   bool allow_sym)
 {
     EvalPlan p{};
     p.padded = ((int64_t)n + TJ - 1) / TJ * TJ;
@@ -250,6 +285,9 @@ EvalPlan plan_eval(int n, int ni, int wg, int ipl, int jsplit_cfg, int precision
     const bool flagged = psi || precision != SG_PREC_FP32C;
     p.flag_elems = flagged ? p.ngroups * p.ntiles : 1;
     p.psipart_elems = psi ? (int64_t)p.jsplit * ni : 0;
+    if (allow_sym && precision == SG_PREC_FP32C && !psi && ni == n && n >= SYM_MIN_N && n <= SYM_MAX_N &&
+        ipl == 1 && jsplit_cfg == 0 && (wg == 0 || wg == (ni <= AUTO_SMALL_NI ? 128 : 256)))
+        plan_sym(p, n);
     return p;
 }
 
@@ -314,6 +352,38 @@ hipError_t enqueue_eval(const EvalPlan &p, const EvalBuffers &bufs, int n, int i
     }
     SG_ENQ(launch_fill_zero_int((int *)bufs.stats, 2 * STAT_WORDS, s));
 
+    if (p.sym) {
+        SymArgs y{};
+        y.p = a.j;
+        y.chunks = b.chunks;
+        y.bbox = b.bbox;
+        y.n = n;
+        y.nchunks = (int)(p.padded / TC);
+        y.words = (y.nchunks + 63) / 64;
+        y.sb = p.sb;
+        y.nsb = p.nsb;
+        y.waves = p.waves;
+        const SymLayout l = sym_layout(y.nchunks);
+        y.boxes = (float4 *)(bufs.sym + l.boxes);
+        y.sym = (uint64_t *)(bufs.sym + l.bits);
+        y.seg = (int *)(bufs.sym + l.seg);
+        y.segsum = bufs.partial + (int64_t)p.jsplit * 4 * n;
+        y.ax = ax;
+        y.ay = ay;
+        y.az = az;
+        y.pot = pot;
+        y.nkernel = nkernel;
+        y.partial = bufs.partial;
+        y.stats = bufs.stats;
+        SG_ENQ(launch_sym_classify(y, s));
+        if (ev) SG_ENQ(hipEventRecord(ev[1], s));
+        SG_ENQ(launch_sym(y, s));
+        SG_ENQ(launch_sym_rest(y, s));
+        if (ev) SG_ENQ(hipEventRecord(ev[2], s));
+        SG_ENQ(launch_sym_reduce(y, s));
+        if (ev) SG_ENQ(hipEventRecord(ev[3], s));
+        return hipSuccess;
+    }
     if (ev) SG_ENQ(hipEventRecord(ev[1], s));
     SG_ENQ(launch_pair_far(precision, a, p.wg, s));
     if (ev) SG_ENQ(hipEventRecord(ev[2], s));
@@ -411,7 +481,7 @@ int sg_destroy(sg_context *c)
                     c->scot[0], c->scot[1], c->scot[2], c->scot[3],
                     c->vin[0], c->vin[1], c->vin[2], c->vin[3],
                     c->vout[0], c->vout[1], c->vout[2], c->vout[3], c->vout[4], c->psipart,
-                    c->psi_out, c->epot_work};
+                    c->psi_out, c->epot_work, c->sym};
     if (c->gexec) (void)hipGraphExecDestroy(c->gexec);
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
@@ -474,8 +544,20 @@ int compute_device_impl(sg_context *c, int n, int ibeg, int ni, const double *x,
     c->last_shape[0] = 0;   // set again by a single-set pair pass
     if (ni == 0) return SG_OK;
 
-    const sg::EvalPlan p = sg::plan_eval(n, ni, c->wg[precision], c->ipl[precision],
-                                         c->jsplit[precision], precision, psi != nullptr);
+    auto plan = [&](bool allow_sym) {
+        return sg::plan_eval(n, ni, c->wg[precision], c->ipl[precision], c->jsplit[precision],
+                             precision, psi != nullptr, allow_sym);
+    };
+    sg::EvalPlan p = plan(true);
+    if (p.sym) {
+        // the slabs of the unordered-pair pass are its price: where the device
+        // cannot hold them the ordered pass runs
+        if (grow(&c->partial, &c->cap_part, p.part_elems) != SG_OK ||
+            grow(&c->sym, &c->cap_sym, p.sym_bytes) != SG_OK) {
+            (void)hipGetLastError();
+            p = plan(false);
+        }
+    }
     if (psi && p.psipart_elems > INT32_MAX / 2) return SG_ERR_ARG;
     int rc = ensure_capacity(c, n, p.padded, ni);
     if (rc != SG_OK) return rc;
@@ -483,7 +565,8 @@ int compute_device_impl(sg_context *c, int n, int ibeg, int ni, const double *x,
     if ((rc = grow(&c->nearflag, &c->cap_flag, p.flag_elems)) != SG_OK) return rc;
     if (psi && (rc = grow(&c->psipart, &c->cap_psipart, p.psipart_elems)) != SG_OK) return rc;
     const sg::EvalBuffers bufs{c->pb,       c->sort_tmp, c->sort_tmp_bytes, c->partial,
-                               c->nearflag, c->stats,    c->psipart,        false};
+                               c->nearflag, c->stats,    c->psipart,        false,
+                               c->sym};
     const hipEvent_t ev[4] = {c->ev_p0, c->ev_k0, c->ev_kf, c->ev_k1};
     HIP_TRY(sg::enqueue_eval(p, bufs, n, ibeg, ni, x, y, z, m, range2, nkernel, precision, ax, ay,
                              az, pot, psi, c->stream, ev));

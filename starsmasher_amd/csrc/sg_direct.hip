@@ -263,7 +263,25 @@ struct NearSlice {
     uint32_t list[NLIST];    // (tile - t0) << 4 | chunk mask
 };
 
-// Stages chunk c of tile t in the wave's slice and evaluates it.  Each pair
+// Stages one particle per lane in the wave's slice: its position relative to
+// the origin, mass and signed H.  Returns the lanes that hold particles (not
+// massless padding).
+__device__ __forceinline__ uint64_t near_stage(NearSlice &sl, double rx, double ry, double rz,
+                                               double mj, double hs)
+{
+    const int lane = threadIdx.x & 63;
+    const float mh[2] = {(float)mj, (float)(hs * hs)};
+    const uint64_t real = __ballot(mj > 0.0);
+    wave_lds_sync();
+    sl.p[lane] = make_double4(rx, ry, rz, __builtin_bit_cast(double, mh));
+    sl.hs[lane] = hs;
+    sl.hinv[lane] = 1.0 / fabs(hs);
+    sl.m[lane] = mj;
+    wave_lds_sync();
+    return real;
+}
+
+// Evaluates the chunk staged in the slice (particles j0c ..).  Each pair
 // difference is formed in FP64 and rounded once to FP32 (two ops per axis;
 // near pairs are close, where the hi+lo difference would lose the low bits
 // of the i position whenever |x_i - O| < |x_j - O|, an error that does not
@@ -275,28 +293,12 @@ struct NearSlice {
 // exactly one of the two, so a borderline FP32 decision costs only
 // rounding).  Wave-local: no block barrier.
 template <int IPL, int NK>
-__device__ __forceinline__ void near_chunk_slice(
-    NearSlice &sl, const SortedSet &J, int t, int c, double Ox, double Oy, double Oz,
-    const double (&xr)[IPL], const double (&yr)[IPL], const double (&zr)[IPL],
-    const double (&Hi)[IPL], const double (&invHi)[IPL], const double (&hi2)[IPL],
-    const int (&idi)[IPL], double (&ax)[IPL], double (&ay)[IPL], double (&az)[IPL],
-    double (&ap)[IPL], unsigned (&nfp64)[IPL])
+__device__ __forceinline__ void near_chunk_eval(
+    NearSlice &sl, uint64_t real, const SortedSet &J, int64_t j0c, const double (&xr)[IPL],
+    const double (&yr)[IPL], const double (&zr)[IPL], const double (&Hi)[IPL],
+    const double (&invHi)[IPL], const double (&hi2)[IPL], const int (&idi)[IPL], double (&ax)[IPL],
+    double (&ay)[IPL], double (&az)[IPL], double (&ap)[IPL], unsigned (&nfp64)[IPL])
 {
-    const int lane = threadIdx.x & 63;
-    uint64_t real;   // wave-uniform: j that are particles (not massless padding)
-    {
-        const int64_t j = (int64_t)t * TJ + c * TC + lane;
-        const double rx = J.x[j] - Ox, ry = J.y[j] - Oy, rz = J.z[j] - Oz, mj = J.m[j];
-        const double hs = J.Hs[j];
-        const float mh[2] = {(float)mj, (float)(hs * hs)};
-        real = __ballot(mj > 0.0);
-        wave_lds_sync();
-        sl.p[lane] = make_double4(rx, ry, rz, __builtin_bit_cast(double, mh));
-        sl.hs[lane] = hs;
-        sl.hinv[lane] = 1.0 / fabs(hs);
-        sl.m[lane] = mj;
-        wave_lds_sync();
-    }
     float hi2f[IPL];
 #pragma unroll
     for (int k = 0; k < IPL; ++k) hi2f[k] = (float)hi2[k];
@@ -370,11 +372,27 @@ __device__ __forceinline__ void near_chunk_slice(
             const double ddx = p.x - xr[k], ddy = p.y - yr[k], ddz = p.z - zr[k];
             // the self pair only matters at r = 0: the index is read then
             const bool same = ddx == 0.0 && ddy == 0.0 && ddz == 0.0 &&
-                              J.idx[(int64_t)t * TJ + c * TC + jj] == idi[k];
+                              J.idx[j0c + jj] == idi[k];
             near_pair<true, NK>(ddx, ddy, ddz, Hi[k], invHi[k], hi2[k], ha, hinv, ha * ha, mj,
                                 hs > 0.0, same, ax[k], ay[k], az[k], ap[k]);
         }
     }
+}
+
+// Stages chunk c of tile t and evaluates it.
+template <int IPL, int NK>
+__device__ __forceinline__ void near_chunk_slice(
+    NearSlice &sl, const SortedSet &J, int t, int c, double Ox, double Oy, double Oz,
+    const double (&xr)[IPL], const double (&yr)[IPL], const double (&zr)[IPL],
+    const double (&Hi)[IPL], const double (&invHi)[IPL], const double (&hi2)[IPL],
+    const int (&idi)[IPL], double (&ax)[IPL], double (&ay)[IPL], double (&az)[IPL],
+    double (&ap)[IPL], unsigned (&nfp64)[IPL])
+{
+    const int lane = threadIdx.x & 63;
+    const int64_t j = (int64_t)t * TJ + c * TC + lane;
+    const uint64_t real = near_stage(sl, J.x[j] - Ox, J.y[j] - Oy, J.z[j] - Oz, J.m[j], J.Hs[j]);
+    near_chunk_eval<IPL, NK>(sl, real, J, (int64_t)t * TJ + c * TC, xr, yr, zr, Hi, invHi, hi2, idi,
+                             ax, ay, az, ap, nfp64);
 }
 
 // FUSED (the forward FP32C pass): the chunks a wave cannot classify as far
@@ -927,6 +945,161 @@ __global__ __launch_bounds__(64 * NEAR_WAVES) void k_near_psi(PairArgs a)
     near_group<1, FAST, NK, true>(a.i, a.j, g, lds, s_red);
 }
 
+// ------------------------------------------- ordered rest of a whole-set pass
+// The unset bits of one row of SymArgs::sym from the k-th on, in order.
+struct RestBits {
+    const uint64_t *row;
+    int nchunks, words, wb, src;
+    uint64_t rest, any, bits;   // rest: per lane; the others wave-uniform
+
+    __device__ __forceinline__ void block()
+    {
+        const int k = wb + (threadIdx.x & 63);
+        rest = 0;
+        if (k < words) {
+            const int left = nchunks - k * 64;
+            rest = ~row[k] & (left >= 64 ? ~0ull : (1ull << left) - 1ull);
+        }
+        any = __ballot(rest != 0);
+    }
+    __device__ __forceinline__ bool word()
+    {
+        while (!any) {
+            wb += 64;
+            if (wb >= words) return false;
+            block();
+        }
+        src = __builtin_ctzll(any);
+        any &= any - 1;
+        bits = (uint64_t)(unsigned)__builtin_amdgcn_readlane((int)(rest & 0xffffffffu), src) |
+               (uint64_t)(unsigned)__builtin_amdgcn_readlane((int)(rest >> 32), src) << 32;
+        return true;
+    }
+    __device__ __forceinline__ void start(int skip)
+    {
+        wb = 0;
+        bits = 0;
+        block();
+        while (word()) {
+            const int c = __builtin_popcountll(bits);
+            if (c > skip) break;
+            skip -= c;
+        }
+        for (; skip > 0; --skip) bits &= bits - 1;
+    }
+    // The next column chunk (the caller knows how many are left).
+    __device__ __forceinline__ int next()
+    {
+        if (!bits) word();
+        const int c = (wb + src) * 64 + __builtin_ctzll(bits);
+        bits &= bits - 1;
+        return c;
+    }
+};
+
+// The (row chunk, column chunk) visits that k_sym leaves (bits unset in
+// a.sym): near chunks and those too close to the row chunk for hi-only
+// differences.  One wave per segment of a row's visits, so that the rows that
+// meet thousands of chunks (those of the largest H, and those that straddle a
+// jump of the curve) do not outlast the rest.  The next chunk's particles are
+// loaded while the current one is evaluated.
+template <int NK>
+__global__ __launch_bounds__(64) void k_sym_rest(SymArgs a)
+{
+    __shared__ NearSlice sl;
+    const int lane = threadIdx.x;
+    const int g = (int)blockIdx.x;
+    if (g >= a.seg[a.nchunks]) return;
+    int ci = 0;   // the last row whose first segment is not after g
+    for (int hi = a.nchunks - 1; ci < hi;) {
+        const int mid = (ci + hi + 1) / 2;
+        if (a.seg[mid] <= g) ci = mid;
+        else hi = mid - 1;
+    }
+    ci = uniform_i(ci);
+    const int len = uniform_i(a.seg[a.nchunks + 1]);
+    const int k0 = uniform_i(g - a.seg[ci]) * len;
+    const SortedSet &P = a.p;
+    const int64_t gbase = (int64_t)ci * TC;
+    const int64_t io = min(gbase + TC / 2, a.n - 1);
+    const double Ox = P.x[io], Oy = P.y[io], Oz = P.z[io];
+    const bool valid = gbase + lane < a.n;
+    const int64_t ii[1] = {valid ? gbase + lane : a.n - 1};
+    const double xr[1] = {P.x[ii[0]] - Ox}, yr[1] = {P.y[ii[0]] - Oy}, zr[1] = {P.z[ii[0]] - Oz};
+    double Hi[1], invHi[1], hi2[1];
+    int idi[1];
+    near_i_state<1>(P, ii, Hi, invHi, hi2, idi);
+    const float px = (float)xr[0], py = (float)yr[0], pz = (float)zr[0], ph = (float)Hi[0];
+    double ax[1] = {0.0}, ay[1] = {0.0}, az[1] = {0.0}, ap[1] = {0.0};
+    unsigned nfp64[1] = {0}, visits = 0, nearv = 0;
+
+    RestBits it;
+    it.row = a.sym + (int64_t)ci * a.words;
+    it.nchunks = a.nchunks;
+    it.words = a.words;
+    int left = 0;   // visits of this segment
+    {
+        // the row's last segment is the short one
+        int total = 0;
+        for (int wb = 0; wb < a.words; wb += 64) {
+            const int k = wb + lane;
+            if (k < a.words) total += __builtin_popcountll(it.row[k]);
+        }
+        for (int o = 32; o > 0; o >>= 1) total += __shfl_xor(total, o, 64);
+        left = min(len, a.nchunks - uniform_i(total) - k0);
+    }
+    it.start(k0);
+    int cj = it.next();
+    double jx = P.x[(int64_t)cj * TC + lane], jy = P.y[(int64_t)cj * TC + lane],
+           jz = P.z[(int64_t)cj * TC + lane], jm = P.m[(int64_t)cj * TC + lane],
+           jh = P.Hs[(int64_t)cj * TC + lane];
+    for (;;) {
+        const TileMeta &cm = a.chunks[cj];
+        const float gx = fmaxf(0.0f, fmaxf((float)(cm.lo[0] - Ox) - px, px - (float)(cm.hi[0] - Ox)));
+        const float gy = fmaxf(0.0f, fmaxf((float)(cm.lo[1] - Oy) - py, py - (float)(cm.hi[1] - Oy)));
+        const float gz = fmaxf(0.0f, fmaxf((float)(cm.lo[2] - Oz) - pz, pz - (float)(cm.hi[2] - Oz)));
+        const float hm = fmaxf(ph, (float)cm.maxH);
+        const bool lane_near = !(fmaf(gx, gx, fmaf(gy, gy, gz * gz)) > hm * hm * (1.0f + FAR_MARGIN));
+        const bool is_near = __ballot(lane_near) != 0;
+        const uint64_t real = near_stage(sl, jx - Ox, jy - Oy, jz - Oz, jm, jh);
+        const int64_t j0c = (int64_t)cj * TC;
+        ++visits;
+        if (--left > 0) {
+            cj = it.next();
+            const int64_t j = (int64_t)cj * TC + lane;
+            jx = P.x[j];
+            jy = P.y[j];
+            jz = P.z[j];
+            jm = P.m[j];
+            jh = P.Hs[j];
+        }
+        if (is_near) {
+            ++nearv;
+            near_chunk_eval<1, NK>(sl, real, P, j0c, xr, yr, zr, Hi, invHi, hi2, idi, ax, ay, az, ap,
+                                   nfp64);
+        } else {
+            const float none[1] = {0.0f};
+            far_chunk_fp32<1, true>(nullptr, sl.p, none, none, none, xr, yr, zr, ax, ay, az, ap);
+        }
+        if (left <= 0) break;
+    }
+    double *s = a.segsum + (int64_t)g * 4 * TC + lane;
+    s[0] = ax[0];
+    s[TC] = ay[0];
+    s[2 * TC] = az[0];
+    s[3 * TC] = ap[0];
+    if (a.stats) {
+        const unsigned long long fw = wave_sum_count(valid ? nfp64[0] : 0u);
+        if (lane == 0) {
+            unsigned long long *st = stat_copy(a.stats);
+            atomicAdd(&st[0], (unsigned long long)visits);
+            atomicAdd(&st[1], (unsigned long long)nearv);
+            atomicAdd(&st[2], (unsigned long long)(visits - nearv));
+            atomicAdd(&st[3], fw);
+        }
+    }
+}
+
 // ------------------------------------------------- grad-h term on its own
 // psi_i = -(2/H_i^2) sum_{j: r <= H_i} m_j (P(q_i) + q_i^2 A(q_i)) of the
 // gas particles of the i-set, without the accelerations: one wave per
@@ -1230,6 +1403,19 @@ hipError_t launch_psi_only(const PairArgs &a, hipStream_t s)
     case 0: hipLaunchKernelGGL((k_psi_only<0>), grid, block, 0, s, a); break;
     case 1: hipLaunchKernelGGL((k_psi_only<1>), grid, block, 0, s, a); break;
     case 2: hipLaunchKernelGGL((k_psi_only<2>), grid, block, 0, s, a); break;
+    default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
+}
+
+hipError_t launch_sym_rest(const SymArgs &a, hipStream_t s)
+{
+    // as many waves as there can be segments; those past the last one end at once
+    const dim3 grid((unsigned)(SYM_SEGS + a.nchunks)), block(64);
+    switch (a.nkernel) {
+    case 0: hipLaunchKernelGGL((k_sym_rest<0>), grid, block, 0, s, a); break;
+    case 1: hipLaunchKernelGGL((k_sym_rest<1>), grid, block, 0, s, a); break;
+    case 2: hipLaunchKernelGGL((k_sym_rest<2>), grid, block, 0, s, a); break;
     default: return hipErrorInvalidValue;
     }
     return hipGetLastError();

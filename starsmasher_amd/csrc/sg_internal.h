@@ -69,6 +69,35 @@ struct PairArgs {
     double *psipart;              // [jsplit][ni] its partial sums (with psi)
 };
 
+// The far pairs of a whole set, each unordered pair once (sg_sym.hip), and
+// the ordered rest (sg_direct.hip).  Superblocks are sb consecutive chunks;
+// slab b < nsb of a particle's partial sums belongs to the superblock pair
+// with b, slab nsb to the columns of its own superblock.  The rest of a row
+// chunk is cut into segments with partial sums of their own: at most SYM_SEGS
+// + nchunks of them, of SYM_SEG_MIN chunk visits or more.
+constexpr int SYM_SEGS = 32768, SYM_SEG_MIN = 8;
+struct SymArgs {
+    SortedSet p;
+    const TileMeta *chunks;
+    const double *bbox;      // PrepBuffers::bbox
+    float4 *boxes;           // [nchunks][2]: FP32 chunk boxes
+    uint64_t *sym;           // [nchunks][words]: bit set = chunk pair in k_sym
+    int *seg;                // [nchunks + 2]: first segment of each row, their number, length
+    int64_t n;               // real particles
+    int nchunks, words;      // padded / TC, (nchunks + 63) / 64
+    int sb, nsb;             // chunks per superblock, superblocks
+    int waves;               // waves per workgroup of k_sym (1, 2, 4)
+    int nkernel;
+    double *partial;         // [nsb + 1][4][n], sorted order
+    double *segsum;          // [SYM_SEGS + nchunks][4][TC]
+    double *ax, *ay, *az, *pot;   // outputs, input order
+    unsigned long long *stats;
+};
+hipError_t launch_sym_classify(const SymArgs &a, hipStream_t s);
+hipError_t launch_sym(const SymArgs &a, hipStream_t s);
+hipError_t launch_sym_rest(const SymArgs &a, hipStream_t s);   // sg_direct.hip
+hipError_t launch_sym_reduce(const SymArgs &a, hipStream_t s);
+
 // A batch of independent particle sets laid out back to back in one padded
 // sorted array; each set starts at a tile boundary.  A set of more than
 // BATCH_JTILES tiles has its j range cut into jsplit strided partitions
@@ -149,7 +178,7 @@ struct PrepBuffers {
     // scratch
     double *red;          // [nred_blocks * 8] reduction partials
     int nred_blocks;
-    double *bbox;         // [8]: lo xyz, hi xyz, (unused)
+    double *bbox;         // [8]: lo xyz, hi xyz, length scale, mass scale
     int *err;             // [1]: validation bit flags
     uint64_t *keys_in, *keys_out;
     int *vals_in, *vals_out;
@@ -222,14 +251,27 @@ struct EvalPlan {
     int64_t part_elems;    // doubles of j-partition partial sums: jsplit * 4 * ni
     int64_t flag_elems;    // near-flag bytes (FP64 and grad-h passes; else 1)
     int64_t psipart_elems; // grad-h partial sums: jsplit * ni (with psi; else 0)
+    // each unordered far pair once (sg_sym.hip): jsplit counts its slabs
+    bool sym;
+    int sb, nsb, waves;
+    int64_t sym_bytes;     // chunk boxes, chunk-pair bits, segment table
 };
 int auto_jsplit(int niblocks, int wg, int ntiles, int64_t ni);
 // i-ranges up to this many particles take workgroups of 128 when the
 // configured workgroup size is 0 (automatic), larger ones 256
 constexpr int AUTO_SMALL_NI = 65536;
+// Whole-set FP32C passes of these sizes evaluate each unordered far pair once
+// (sg_sym.hip).  Pair kernels of one Plummer sphere, ordered against
+// unordered, same card: 33,333 particles 0.74 against 0.80 ms, 50,001 1.42
+// against 1.26, 65,536 2.18 against 1.73, 131,072 7.35 against 5.38; a giant
+// star of 1,048,576 320 against 218 ms.  The upper limit keeps the chunk-pair
+// bits (N^2 / 32,768 bytes) at 512 MB and the slabs at 17 GB; where the device
+// cannot hold them the ordered pass runs.
+constexpr int SYM_MIN_N = 40960, SYM_MAX_N = 1 << 22, SYM_MAX_SB = 128;
 // the HIP error that sg_status_string(SG_ERR_HIP) describes
 void record_hip_error(hipError_t e);
-EvalPlan plan_eval(int n, int ni, int wg, int ipl, int jsplit_cfg, int precision, bool psi);
+EvalPlan plan_eval(int n, int ni, int wg, int ipl, int jsplit_cfg, int precision, bool psi,
+                   bool allow_sym);
 
 // The device memory one evaluation works in.
 struct EvalBuffers {
@@ -241,6 +283,7 @@ struct EvalBuffers {
     unsigned long long *stats;   // [STAT_WORDS]
     double *psipart;             // with psi only
     bool merge_sort;             // sort with merge_sort_pairs (same order, no memset)
+    unsigned char *sym;          // [sym_bytes] (sym plans only)
 };
 
 // Enqueues validation, sort, gather, tile boxes, the pair kernels and the

@@ -49,6 +49,18 @@ __device__ inline void block_minmax6(double v[6])
     }
 }
 
+// Block-wide maximum; result valid in thread 0.
+__device__ inline double block_max(double v)
+{
+    __shared__ double sh[RB / 64];
+    v = warp_max(v);
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
+    __syncthreads();
+    if (threadIdx.x == 0)
+        for (int w = 1; w < RB / 64; ++w) v = fmax(v, sh[w]);
+    return v;
+}
+
 __global__ __launch_bounds__(RB) void k_fill_zero_int(int *p, int n)
 {
     const int t = blockIdx.x * RB + threadIdx.x;
@@ -63,6 +75,7 @@ __global__ __launch_bounds__(RB) void k_validate_bbox(const double *__restrict__
                                                       double *__restrict__ red, int *err)
 {
     double v[6] = {INFINITY, INFINITY, INFINITY, -INFINITY, -INFINITY, -INFINITY};
+    double mmax = 0.0;
     int flags = 0;
     for (int64_t k = blockIdx.x * (int64_t)RB + threadIdx.x; k < n; k += (int64_t)gridDim.x * RB) {
         const double px = x[k], py = y[k], pz = z[k], pm = m[k], pr = r2[k];
@@ -70,26 +83,44 @@ __global__ __launch_bounds__(RB) void k_validate_bbox(const double *__restrict__
             flags |= ERR_NONFINITE;
         if (!(pm > 0.0)) flags |= ERR_MASS;
         if (pr == 0.0) flags |= ERR_RANGE2;
+        mmax = fmax(mmax, pm);
         v[0] = fmin(v[0], px); v[1] = fmin(v[1], py); v[2] = fmin(v[2], pz);
         v[3] = fmax(v[3], px); v[4] = fmax(v[4], py); v[5] = fmax(v[5], pz);
     }
     if (flags) atomicOr(err, flags);
     block_minmax6(v);
-    if (threadIdx.x == 0)
+    mmax = block_max(mmax);
+    if (threadIdx.x == 0) {
         for (int c = 0; c < 6; ++c) red[blockIdx.x * 8 + c] = v[c];
+        red[blockIdx.x * 8 + 6] = mmax;
+    }
 }
 
+// The power of two that brings v to [1, 2) (1 where v has none).
+__device__ inline double unit_scale(double v)
+{
+    return v > 0.0 && isfinite(v) ? ldexp(1.0, -ilogb(v)) : 1.0;
+}
+
+// bbox: lo xyz, hi xyz, and the scales that bring the set's extent and its
+// largest mass to order one (sg_sym.hip).
 __global__ __launch_bounds__(RB) void k_bbox_final(const double *__restrict__ red, int nblocks,
                                                    double *__restrict__ bbox)
 {
     double v[6] = {INFINITY, INFINITY, INFINITY, -INFINITY, -INFINITY, -INFINITY};
+    double mmax = 0.0;
     for (int b = threadIdx.x; b < nblocks; b += RB) {
         for (int c = 0; c < 3; ++c) v[c] = fmin(v[c], red[b * 8 + c]);
         for (int c = 3; c < 6; ++c) v[c] = fmax(v[c], red[b * 8 + c]);
+        mmax = fmax(mmax, red[b * 8 + 6]);
     }
     block_minmax6(v);
-    if (threadIdx.x == 0)
+    mmax = block_max(mmax);
+    if (threadIdx.x == 0) {
         for (int c = 0; c < 6; ++c) bbox[c] = v[c];
+        bbox[6] = unit_scale(fmax(fmax(v[3] - v[0], v[4] - v[1]), v[5] - v[2]));
+        bbox[7] = unit_scale(mmax);
+    }
 }
 
 // Gravitational potential energy, the diagnostic of output.f:232-252:

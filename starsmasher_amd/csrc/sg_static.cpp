@@ -142,7 +142,7 @@ extern "C" int sg_compute_device_static(int n, int ibeg, int ni, const double *x
     int rc = scratch_address(device, &base);
     if (rc != SG_OK) return rc;
 
-    const sg::EvalPlan p = sg::plan_eval(n, ni, 0, IPL, 0, precision, false);
+    const sg::EvalPlan p = sg::plan_eval(n, ni, 0, IPL, 0, precision, false, false);
     size_t sort_bytes = 0;
     hipError_t e = sg::merge_sort_pairs_temp_bytes(n, &sort_bytes);
     if (e != hipSuccess) {

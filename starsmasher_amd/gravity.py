@@ -129,29 +129,59 @@ def hip_runtimes() -> list:
     return sorted(paths)
 
 
+class _DlInfo(C.Structure):
+    """struct dl_phdr_info up to the load counters (glibc's <link.h>)."""
+    _fields_ = [("addr", C.c_void_p), ("name", C.c_char_p), ("phdr", C.c_void_p),
+                ("phnum", C.c_uint16), ("adds", C.c_ulonglong), ("subs", C.c_ulonglong)]
+
+
+_dl_counts = [0, 0]
+
+
+@C.CFUNCTYPE(C.c_int, C.POINTER(_DlInfo), C.c_size_t, C.c_void_p)
+def _dl_first(info, size, _):
+    _dl_counts[0], _dl_counts[1] = info.contents.adds, info.contents.subs
+    return 1   # the counters are the same in every entry
+
+
+_dl_iterate_phdr = C.CDLL(None).dl_iterate_phdr
+_one_runtime_at = None   # the load counters when a single HIP runtime was last seen
+
+
 def _check_shared_runtime(name):
     """Device pointers and streams of torch are only meaningful to the library
     when both use one HIP runtime.  torch wheels bundle their own
     libamdhip64, and a pointer or stream of one runtime is not valid in the
     other, so a second runtime in the process makes torch tensors unusable
-    here (allocate through starsmasher_amd.hipmem instead)."""
+    here (allocate through starsmasher_amd.hipmem instead).
+
+    Reading the process's maps takes 0.5 ms with torch loaded, so a verdict
+    stands until a shared object is loaded or unloaded (the dynamic linker's
+    own counters, 2 us)."""
+    global _one_runtime_at
     _lib.load()
+    _dl_iterate_phdr(_dl_first, None)
+    at = tuple(_dl_counts)
+    if at == _one_runtime_at:
+        return
     rts = hip_runtimes()
     if len(rts) != 1:
         raise TypeError(f"{name}: torch tensors cannot be passed: this process maps "
                         f"{len(rts)} HIP runtimes ({', '.join(rts)}), and device pointers "
                         "and streams of one are invalid in another; allocate with "
                         "starsmasher_amd.hipmem.DeviceArray")
+    _one_runtime_at = at
 
 
 def _is_torch(t) -> bool:
     return type(t).__module__.startswith("torch")
 
 
-def _dev_ptr(t, name, n=None):
+def _dev_ptr(t, name, n=None, shared=False):
     """Device pointer of a :class:`starsmasher_amd.hipmem.DeviceArray`, a raw
     integer address, or a torch tensor (float64, contiguous, on a GPU; only
-    accepted when torch and the library share one HIP runtime)."""
+    accepted when torch and the library share one HIP runtime; `shared`: the
+    caller has checked that)."""
     if isinstance(t, int):
         return t
     if hasattr(t, "ptr") and hasattr(t, "size"):
@@ -164,12 +194,23 @@ def _dev_ptr(t, name, n=None):
         raise TypeError(f"{name}: pass an integer device address or a torch tensor") from e
     if not isinstance(t, torch.Tensor):
         raise TypeError(f"{name} must be a torch tensor on the GPU or a device address")
-    _check_shared_runtime(name)
+    if not shared:
+        _check_shared_runtime(name)
     if t.device.type != "cuda" or t.dtype != torch.float64 or not t.is_contiguous():
         raise TypeError(f"{name} must be a contiguous float64 tensor on a GPU")
     if n is not None and t.numel() < n:
         raise ValueError(f"{name} has {t.numel()} entries, needs {n}")
     return t.data_ptr()
+
+
+def _dev_ptrs(arrays):
+    """Device pointers of (array, name, length) triples, the HIP runtime
+    checked once for all of them."""
+    ptrs, shared = [], False
+    for t, name, n in arrays:
+        ptrs.append(_dev_ptr(t, name, n, shared))
+        shared = shared or _is_torch(t)
+    return ptrs, shared
 
 
 class Gravity:
@@ -292,22 +333,22 @@ class Gravity:
         """Enqueue a device-resident adjoint (addresses or device arrays of
         length n); call ``synchronize``."""
         n = int(n)
-        ptrs = [_dev_ptr(a, nm, n) for a, nm in ((x, "x"), (y, "y"), (z, "z"), (m, "m"),
-                                                  (range2, "range2"), (wx, "wx"), (wy, "wy"),
-                                                  (wz, "wz"), (u, "u"), (gx, "gx"), (gy, "gy"),
-                                                  (gz, "gz"), (gm, "gm"), (gH, "gH"))]
+        ptrs, shared = _dev_ptrs([(a, nm, n) for a, nm in (
+            (x, "x"), (y, "y"), (z, "z"), (m, "m"), (range2, "range2"), (wx, "wx"), (wy, "wy"),
+            (wz, "wz"), (u, "u"), (gx, "gx"), (gy, "gy"), (gz, "gz"), (gm, "gm"), (gH, "gH"))])
         vp = [C.c_void_p(p) for p in ptrs]
-        self._stream_for(x)
+        self._stream_for(x, shared)
         st = self._L.sg_vjp_device(self._h, n, *vp[:5], int(nkernel), int(precision), *vp[5:])
         check(st, "sg_vjp_device")
 
-    def _stream_for(self, t):
+    def _stream_for(self, t, shared=False):
         """Enqueue on the caller's current torch stream when `t` is a torch
         tensor (ordered after the work that produced it), else on the
         context's own stream, so a torch call's stream does not linger into
         later calls on device arrays."""
         if _is_torch(t):
-            _check_shared_runtime("stream")
+            if not shared:
+                _check_shared_runtime("stream")
             import torch
             self.set_stream(torch.cuda.current_stream(t.device).cuda_stream)
         else:
@@ -319,13 +360,13 @@ class Gravity:
         torch tensors when torch shares the library's HIP runtime)."""
         n = int(n)
         ni = n - ibeg if ni is None else int(ni)
-        ins = [_dev_ptr(a, nm, n) for a, nm in ((x, "x"), (y, "y"), (z, "z"), (m, "m"),
-                                                 (range2, "range2"))]
-        outs = [_dev_ptr(a, nm, ni) for a, nm in ((ax, "ax"), (ay, "ay"), (az, "az"), (pot, "pot"))]
-        self._stream_for(x)
-        st = self._L.sg_compute_device(self._h, n, int(ibeg), ni, *[C.c_void_p(p) for p in ins],
-                                       int(nkernel), int(precision),
-                                       *[C.c_void_p(p) for p in outs])
+        ptrs, shared = _dev_ptrs(
+            [(a, nm, n) for a, nm in ((x, "x"), (y, "y"), (z, "z"), (m, "m"), (range2, "range2"))] +
+            [(a, nm, ni) for a, nm in ((ax, "ax"), (ay, "ay"), (az, "az"), (pot, "pot"))])
+        self._stream_for(x, shared)
+        vp = [C.c_void_p(p) for p in ptrs]
+        st = self._L.sg_compute_device(self._h, n, int(ibeg), ni, *vp[:5], int(nkernel),
+                                       int(precision), *vp[5:])
         check(st, "sg_compute_device")
 
     # ------------------------------------------------------------ batch
@@ -345,15 +386,14 @@ class Gravity:
         offsets[s]..offsets[s+1]-1 of the device arrays."""
         off = np.ascontiguousarray(offsets, dtype=np.int64)
         ntot = int(off[-1])
-        ins = [_dev_ptr(a, nm, ntot) for a, nm in ((x, "x"), (y, "y"), (z, "z"), (m, "m"),
-                                                    (range2, "range2"))]
-        outs = [_dev_ptr(a, nm, ntot) for a, nm in ((ax, "ax"), (ay, "ay"), (az, "az"),
-                                                     (pot, "pot"))]
-        self._stream_for(x)
+        ptrs, shared = _dev_ptrs([(a, nm, ntot) for a, nm in (
+            (x, "x"), (y, "y"), (z, "z"), (m, "m"), (range2, "range2"),
+            (ax, "ax"), (ay, "ay"), (az, "az"), (pot, "pot"))])
+        self._stream_for(x, shared)
+        vp = [C.c_void_p(p) for p in ptrs]
         st = self._L.sg_compute_batch_device(
             self._h, off.size - 1, off.ctypes.data_as(C.POINTER(C.c_longlong)),
-            *[C.c_void_p(p) for p in ins], int(nkernel), int(precision), int(bool(use_graph)),
-            *[C.c_void_p(p) for p in outs])
+            *vp[:5], int(nkernel), int(precision), int(bool(use_graph)), *vp[5:])
         check(st, "sg_compute_batch_device")
 
     def compute_batch(self, sets, nkernel=0, precision=SG_PREC_FP32C, use_graph=False):

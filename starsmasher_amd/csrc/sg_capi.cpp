@@ -285,9 +285,19 @@ EvalPlan plan_eval(int n, int ni, int wg, int ipl, int jsplit_cfg, int precision
     const bool flagged = psi || precision != SG_PREC_FP32C;
     p.flag_elems = flagged ? p.ngroups * p.ntiles : 1;
     p.psipart_elems = psi ? (int64_t)p.jsplit * ni : 0;
-    if (allow_sym && precision == SG_PREC_FP32C && !psi && ni == n && n >= SYM_MIN_N && n <= SYM_MAX_N &&
-        ipl == 1 && jsplit_cfg == 0 && (wg == 0 || wg == (ni <= AUTO_SMALL_NI ? 128 : 256)))
-        plan_sym(p, n);
+    // the automatic shape, or asked for by its workgroup size
+    const bool automatic = precision == SG_PREC_FP32C && !psi && ipl == 1 && jsplit_cfg == 0 &&
+                           (wg == 0 || wg == (ni <= AUTO_SMALL_NI ? 128 : 256));
+    if (automatic && ni <= WAVE_MAX_NI) {
+        const int64_t nic = (ni + TC - 1) / TC, nchunks = (int64_t)p.ntiles * CHUNKS;
+        // n > SG_STATIC_MAX_N: no static scratch to fit (2^20 i-partitions)
+        const int64_t waves = n > SG_STATIC_MAX_N ? 2 * WAVE_COUNT : WAVE_COUNT;
+        p.wave = true;
+        p.jsub = nic * nchunks <= WAVE_COUNT / 2 ? 4 : 1;
+        p.jsplit = p.jsub * (int)std::max<int64_t>(1, std::min(waves / (nic * p.jsub), nchunks));
+        p.part_elems = (int64_t)p.jsplit * 4 * ni;
+    }
+    if (allow_sym && automatic && ni == n && n >= SYM_MIN_N && n <= SYM_MAX_N) plan_sym(p, n);
     return p;
 }
 
@@ -339,6 +349,8 @@ hipError_t enqueue_eval(const EvalPlan &p, const EvalBuffers &bufs, int n, int i
     a.niblocks = p.niblocks;
     a.ngroups = p.ngroups;
     a.jsplit = p.jsplit;
+    a.wave = p.wave;
+    a.jsub = p.jsub;
     a.ax = ax;
     a.ay = ay;
     a.az = az;

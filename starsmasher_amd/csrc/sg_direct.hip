@@ -945,6 +945,369 @@ __global__ __launch_bounds__(64 * NEAR_WAVES) void k_near_psi(PairArgs a)
     near_group<1, FAST, NK, true>(a.i, a.j, g, lds, s_red);
 }
 
+// ------------------------------------------------- one wave, one column chunk
+// The kernels below evaluate chunk visits wave by wave: 64 i, one per lane,
+// against the 64 j staged in the wave's slice.  Their pair loops run in
+// groups of PG pairs whose v_rsq_f32 are issued together at raised wave
+// priority: a v_rsq_f32 issues alone, and at equal priority the wave that is
+// first past its own runs ahead and the two waves of a SIMD no longer issue
+// their other FP32 instructions together (sg_sym.hip).
+constexpr int PG = 4;
+
+// LDS of a wave: the staged chunk, and the softened pairs of a visit dealt
+// evenly over the lanes.
+constexpr int NSOFT = 1024;   // listed pairs; a visit with more has enough on every lane
+struct WaveLds {
+    NearSlice sl;
+    uint16_t list[NSOFT];     // i lane << 6 | j
+    double res[4][64];        // sums of one pair per lane
+};
+
+__device__ __forceinline__ void rsq_group(const float (&r2)[PG], float (&ri)[PG])
+{
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_setprio(3);
+#pragma unroll
+    for (int u = 0; u < PG; ++u) ri[u] = __builtin_amdgcn_rsqf(r2[u]);
+    __builtin_amdgcn_s_setprio(0);
+    __builtin_amdgcn_sched_barrier(0);
+}
+
+// FP32 sums of one fold.
+struct Fold4 {
+    float x = 0.0f, y = 0.0f, z = 0.0f, p = 0.0f;
+    __device__ __forceinline__ void add(float ri, float m, float dx, float dy, float dz)
+    {
+        const float mr = m * ri, mr3 = mr * ri * ri;
+        x = fmaf(mr3, dx, x);
+        y = fmaf(mr3, dy, y);
+        z = fmaf(mr3, dz, z);
+        p += mr;
+    }
+    __device__ __forceinline__ void to(double (&acc)[4]) const
+    {
+        acc[0] += (double)x;
+        acc[1] += (double)y;
+        acc[2] += (double)z;
+        acc[3] -= (double)p;
+    }
+};
+
+enum Visit { VISIT_FAR, VISIT_WIDE, VISIT_NEAR };
+
+// How the chunk with box and largest H cm is evaluated by a wave with one
+// particle per lane at (px, py, pz) relative to O (distance^2 rho2 from it)
+// and support ph: near when some lane's pairs may be softened, else wide when
+// a lane is too close, relative to its distance from O, for differences of
+// positions rounded relative to O.
+__device__ __forceinline__ Visit classify_visit(const TileMeta &cm, double Ox, double Oy, double Oz,
+                                                float px, float py, float pz, float ph, float rho2)
+{
+    const float gx = fmaxf(0.0f, fmaxf((float)(cm.lo[0] - Ox) - px, px - (float)(cm.hi[0] - Ox)));
+    const float gy = fmaxf(0.0f, fmaxf((float)(cm.lo[1] - Oy) - py, py - (float)(cm.hi[1] - Oy)));
+    const float gz = fmaxf(0.0f, fmaxf((float)(cm.lo[2] - Oz) - pz, pz - (float)(cm.hi[2] - Oz)));
+    const float d2 = fmaf(gx, gx, fmaf(gy, gy, gz * gz));
+    const float hm = fmaxf(ph, (float)cm.maxH);
+    if (__ballot(!(d2 > hm * hm * (1.0f + FAR_MARGIN)))) return VISIT_NEAR;
+    if (__ballot(!(d2 > WIDE_K * WIDE_K * rho2 * (1.0f + FAR_MARGIN)))) return VISIT_WIDE;
+    return VISIT_FAR;
+}
+
+// One side of a softened pair without a branch: the polynomials, or the
+// Newtonian terms beyond H.  q = 0 (r = 0, with ri passed as 0) gives the
+// r -> 0 limit.
+template <int NK>
+__device__ __forceinline__ void side_select(double r, double ri, double r2, double H, double invH,
+                                            double &gacc, double &gpot)
+{
+    const double q = r * invH, q2 = q * q;
+    double A, P;
+    if (NK == 0) {
+        // both branches of the cubic spline (poly_AP), the right one kept
+        const double iq = H * ri, iq3 = iq * iq * iq;
+        const double Ai = 10.666666666667 + q2 * (32.0 * q - 38.4);
+        const double Pi = -2.8 + q2 * (5.333333333333 + q2 * (6.4 * q - 9.6));
+        const double Ao = 21.333333333333 + q * (-48.0 + q * (38.4 - 10.666666666667 * q)) -
+                          0.066666666667 * iq3;
+        const double Po = -3.2 + 0.066666666667 * iq +
+                          q2 * (10.666666666667 + q * (-16.0 + q * (9.6 - 2.133333333333 * q)));
+        const bool in = q < 0.5;
+        A = in ? Ai : Ao;
+        P = in ? Pi : Po;
+    } else {
+        poly_AP(NK, q, 0.0, A, P);
+    }
+    const bool soft = r2 <= H * H;
+    gacc += soft ? A * invH * invH * invH : ri * ri * ri;
+    gpot += soft ? P * invH : -ri;
+}
+
+// near_pair for a pair that is (or within rounding of being) softened, with
+// no branch: dealt over the lanes such pairs take different ones, and a wave
+// would walk them all.  dead: the self pair of a point particle.
+template <int NK>
+__device__ __forceinline__ void soft_pair(double dx, double dy, double dz, double Hi, double invHi,
+                                          double Hj, double invHj, double mj, bool dead,
+                                          double (&f)[4])
+{
+    const double r2 = fma(dx, dx, fma(dy, dy, dz * dz));
+    const bool apart = r2 > 0.0;
+    const double ri = apart ? rsqrt64<true>(apart ? r2 : 1.0) : 0.0;
+    const double r = r2 * ri;
+    double gacc = 0.0, gpot = 0.0;
+    side_select<NK>(r, ri, r2, Hi, invHi, gacc, gpot);
+    side_select<NK>(r, ri, r2, Hj, invHj, gacc, gpot);
+    const double hm = dead ? 0.0 : 0.5 * mj;
+    const double g = hm * gacc;
+    f[0] = g * dx;
+    f[1] = g * dy;
+    f[2] = g * dz;
+    f[3] = hm * gpot;
+}
+
+// The visits below cover j = jb .. je - 1 of the staged chunk (multiples of
+// PG).  Near: differences formed in FP64 and rounded once, the FP32 body for every
+// pair (r^-1 = 0 for those that may be softened, r^2 < max(H_i^2, H_j^2) in
+// FP32, r = 0 included), and those in FP64.  A lane has few of them and the
+// busiest several times the mean, and one costs some 300 dependent FP64
+// operations, so they are dealt over all lanes, 64 at a time, and each lane
+// collects the sums of its own.
+template <int NK>
+__device__ __forceinline__ void visit_near(WaveLds &lds, uint64_t real, const SortedSet &J,
+                                           int64_t j0c, int jb, int je, double xr, double yr, double zr, double Hi,
+                                           double invHi, double hi2, int idi, double (&acc)[4],
+                                           unsigned &nfp64)
+{
+    const NearSlice &sl = lds.sl;
+    const float hi2f = (float)hi2;
+    uint64_t mine = 0;   // bit 63 - jj: the lane's pair with jj is softened
+#pragma unroll 1
+    for (int f = jb; f < je; f += FOLD) {
+        const int fe = min(f + FOLD, je);
+        Fold4 sum;
+        uint32_t list = 0;
+#pragma unroll 1
+        for (int j0 = f; j0 < fe; j0 += PG) {
+            float dx[PG], dy[PG], dz[PG], m[PG], r2[PG], ri[PG];
+#pragma unroll
+            for (int u = 0; u < PG; ++u) {
+                const double4 p = sl.p[j0 + u];
+                const float2 mh = __builtin_bit_cast(float2, p.w);   // m_j, H_j^2
+                dx[u] = (float)(p.x - xr);
+                dy[u] = (float)(p.y - yr);
+                dz[u] = (float)(p.z - zr);
+                m[u] = mh.x;
+                const float q = fmaf(dx[u], dx[u], fmaf(dy[u], dy[u], dz[u] * dz[u]));
+                const bool soft = q < fmaxf(hi2f, mh.y);
+                r2[u] = soft ? INFINITY : q;
+                list = list + list + (soft ? 1u : 0u);
+            }
+            rsq_group(r2, ri);
+#pragma unroll
+            for (int u = 0; u < PG; ++u) sum.add(ri[u], m[u], dx[u], dy[u], dz[u]);
+        }
+        sum.to(acc);
+        mine |= (uint64_t)list << (TC - fe);
+    }
+    // the counter covers pairs of particles, not padding
+    nfp64 += (unsigned)__builtin_popcountll(mine & __brevll(real));
+    // lane's first place in the list, and the list's length, from the bits of
+    // the counts
+    const unsigned count = (unsigned)__builtin_popcountll(mine);
+    unsigned at = 0, total = 0;
+#pragma unroll
+    for (int b = 0; b < 7; ++b) {
+        const uint64_t m = __ballot((count >> b) & 1u);
+        at += __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u))
+              << b;
+        total += (unsigned)__builtin_popcountll(m) << b;
+    }
+    if (total > (unsigned)NSOFT) {
+        while (mine) {
+            const int jj = __builtin_clzll(mine);
+            mine &= ~(0x8000000000000000ull >> jj);
+            const double4 p = sl.p[jj];
+            const double hs = sl.hs[jj];
+            const double dx = p.x - xr, dy = p.y - yr, dz = p.z - zr;
+            // the self pair only matters at r = 0: the index is read then
+            const bool dead = dx == 0.0 && dy == 0.0 && dz == 0.0 && hs < 0.0 && J.idx[j0c + jj] == idi;
+            double f[4];
+            soft_pair<NK>(dx, dy, dz, Hi, invHi, fabs(hs), sl.hinv[jj], sl.m[jj], dead, f);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) acc[k] += f[k];
+        }
+        return;
+    }
+    const int lane = threadIdx.x & 63;
+    for (unsigned k = at; mine; ++k) {
+        const int jj = __builtin_clzll(mine);
+        mine &= ~(0x8000000000000000ull >> jj);
+        lds.list[k] = (uint16_t)(lane << 6 | jj);
+    }
+    for (unsigned b0 = 0; b0 < total; b0 += 64) {
+        wave_lds_sync();
+        const unsigned e = min(b0 + (unsigned)lane, total - 1);   // lanes past the end repeat the last
+        const int il = lds.list[e] >> 6, jj = lds.list[e] & 63;
+        const double4 p = sl.p[jj];
+        const double hs = sl.hs[jj];
+        const double H = __shfl(Hi, il, 64), invH = __shfl(invHi, il, 64);
+        const int id = __shfl(idi, il, 64);
+        const double dx = p.x - __shfl(xr, il, 64), dy = p.y - __shfl(yr, il, 64),
+                     dz = p.z - __shfl(zr, il, 64);
+        const bool dead = dx == 0.0 && dy == 0.0 && dz == 0.0 && hs < 0.0 && J.idx[j0c + jj] == id;
+        double f[4];
+        soft_pair<NK>(dx, dy, dz, H, invH, fabs(hs), sl.hinv[jj], sl.m[jj], dead, f);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) lds.res[k][lane] = f[k];
+        wave_lds_sync();
+        // each lane adds its own pairs, in the list's order
+        const unsigned hi = min(at + count, b0 + 64);
+        for (unsigned k = max(at, b0); k < hi; ++k) {
+#pragma unroll
+            for (int c = 0; c < 4; ++c) acc[c] += lds.res[c][k - b0];
+        }
+    }
+}
+
+// Wide: as near, with every pair Newtonian.
+__device__ __forceinline__ void visit_wide(const NearSlice &sl, int jb, int je, double xr, double yr,
+                                           double zr, double (&acc)[4])
+{
+#pragma unroll 1
+    for (int f = jb; f < je; f += FOLD) {
+        const int fe = min(f + FOLD, je);
+        Fold4 sum;
+#pragma unroll 2
+        for (int j0 = f; j0 < fe; j0 += PG) {
+            float dx[PG], dy[PG], dz[PG], m[PG], r2[PG], ri[PG];
+#pragma unroll
+            for (int u = 0; u < PG; ++u) {
+                const double4 p = sl.p[j0 + u];
+                dx[u] = (float)(p.x - xr);
+                dy[u] = (float)(p.y - yr);
+                dz[u] = (float)(p.z - zr);
+                m[u] = __builtin_bit_cast(float2, p.w).x;
+                r2[u] = fmaf(dx[u], dx[u], fmaf(dy[u], dy[u], dz[u] * dz[u]));
+            }
+            rsq_group(r2, ri);
+#pragma unroll
+            for (int u = 0; u < PG; ++u) sum.add(ri[u], m[u], dx[u], dy[u], dz[u]);
+        }
+        sum.to(acc);
+    }
+}
+
+// Far: differences of FP32 positions relative to O.
+__device__ __forceinline__ void visit_far(const float4 *s_hi, int jb, int je, float xh, float yh,
+                                          float zh, double (&acc)[4])
+{
+#pragma unroll 1
+    for (int f = jb; f < je; f += FOLD) {
+        const int fe = min(f + FOLD, je);
+        Fold4 sum;
+#pragma unroll 2
+        for (int j0 = f; j0 < fe; j0 += PG) {
+            float dx[PG], dy[PG], dz[PG], m[PG], r2[PG], ri[PG];
+#pragma unroll
+            for (int u = 0; u < PG; ++u) {
+                const float4 p = s_hi[j0 + u];
+                dx[u] = p.x - xh;
+                dy[u] = p.y - yh;
+                dz[u] = p.z - zh;
+                m[u] = p.w;
+                r2[u] = fmaf(dx[u], dx[u], fmaf(dy[u], dy[u], dz[u] * dz[u]));
+            }
+            rsq_group(r2, ri);
+#pragma unroll
+            for (int u = 0; u < PG; ++u) sum.add(ri[u], m[u], dx[u], dy[u], dz[u]);
+        }
+        sum.to(acc);
+    }
+}
+
+// ------------------------------------------------------ wave-sized work items
+// The forward FP32C pass of small i-ranges: one wave per 64 i and j partition
+// (strided chunks, or parts of them), so that a few thousand particles still
+// make thousands of waves and a wave's near chunks are few.  The next chunk's
+// particles are loaded while the current one is evaluated.
+template <int NK>
+__global__ __launch_bounds__(64) void k_pair_wave(PairArgs a)
+{
+    __shared__ WaveLds lds;
+    NearSlice &sl = lds.sl;
+    const int lane = threadIdx.x;
+    const unsigned nic = (unsigned)((a.ni + TC - 1) / TC);
+    const int ci = (int)(blockIdx.x % nic), jp = (int)(blockIdx.x / nic);
+    const int nchunks = a.ntiles * CHUNKS;
+    const int64_t gbase = (int64_t)ci * TC;
+    const int64_t io = min(gbase + TC / 2, a.ni - 1);
+    const double Ox = a.i.x[io], Oy = a.i.y[io], Oz = a.i.z[io];
+    const bool valid = gbase + lane < a.ni;
+    const int64_t ii[1] = {valid ? gbase + lane : a.ni - 1};
+    const double xr = a.i.x[ii[0]] - Ox, yr = a.i.y[ii[0]] - Oy, zr = a.i.z[ii[0]] - Oz;
+    double Hi[1], invHi[1], hi2[1];
+    int idi[1];
+    near_i_state<1>(a.i, ii, Hi, invHi, hi2, idi);
+    const float px = (float)xr, py = (float)yr, pz = (float)zr, ph = (float)Hi[0];
+    const float rho2 = fmaf(px, px, fmaf(py, py, pz * pz));
+    double acc[4] = {0.0, 0.0, 0.0, 0.0};
+    unsigned nfp64 = 0, visits = 0, nearv = 0, widev = 0;
+    // partition jp: part jp % jsub of every (jsplit / jsub)-th chunk
+    const int stride = a.jsplit / a.jsub, first = jp / a.jsub;
+    const int jb = jp % a.jsub * (TC / a.jsub), je = jb + TC / a.jsub;
+    int64_t j = (int64_t)first * TC + lane;
+    double jx = a.j.x[j], jy = a.j.y[j], jz = a.j.z[j], jm = a.j.m[j], jh = a.j.Hs[j];
+    for (int cj = first; cj < nchunks; cj += stride) {
+        const Visit v = classify_visit(a.chunks[cj], Ox, Oy, Oz, px, py, pz, ph, rho2);
+        const double rx = jx - Ox, ry = jy - Oy, rz = jz - Oz;
+        uint64_t real = 0;
+        if (v == VISIT_FAR) {
+            wave_lds_sync();
+            reinterpret_cast<float4 *>(sl.p)[lane] =
+                make_float4((float)rx, (float)ry, (float)rz, (float)jm);
+            wave_lds_sync();
+        } else {
+            real = near_stage(sl, rx, ry, rz, jm, jh);
+        }
+        const int64_t j0c = (int64_t)cj * TC;
+        if (cj + stride < nchunks) {
+            j = j0c + (int64_t)stride * TC + lane;
+            jx = a.j.x[j];
+            jy = a.j.y[j];
+            jz = a.j.z[j];
+            jm = a.j.m[j];
+            jh = a.j.Hs[j];
+        }
+        ++visits;
+        if (v == VISIT_NEAR) {
+            ++nearv;
+            visit_near<NK>(lds, real, a.j, j0c, jb, je, xr, yr, zr, Hi[0], invHi[0], hi2[0], idi[0], acc, nfp64);
+        } else if (v == VISIT_WIDE) {
+            ++widev;
+            visit_wide(sl, jb, je, xr, yr, zr, acc);
+        } else {
+            visit_far(reinterpret_cast<const float4 *>(sl.p), jb, je, px, py, pz, acc);
+        }
+    }
+    if (valid) {
+        double *part = a.partial + (int64_t)jp * 4 * a.ni + ii[0];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) part[k * a.ni] = acc[k];
+    }
+    if (a.stats) {
+        const unsigned long long fw = wave_sum_count(valid ? nfp64 : 0u);
+        if (lane == 0) {
+            unsigned long long *st = stat_copy(a.stats);
+            if (jb == 0) {   // a divided chunk is one visit
+                atomicAdd(&st[0], (unsigned long long)visits);
+                atomicAdd(&st[1], (unsigned long long)nearv);
+                atomicAdd(&st[2], (unsigned long long)widev);
+            }
+            atomicAdd(&st[3], fw);
+        }
+    }
+}
+
 // ------------------------------------------- ordered rest of a whole-set pass
 // The unset bits of one row of SymArgs::sym from the k-th on, in order.
 struct RestBits {
@@ -1006,7 +1369,8 @@ struct RestBits {
 template <int NK>
 __global__ __launch_bounds__(64) void k_sym_rest(SymArgs a)
 {
-    __shared__ NearSlice sl;
+    __shared__ WaveLds lds;
+    NearSlice &sl = lds.sl;
     const int lane = threadIdx.x;
     const int g = (int)blockIdx.x;
     if (g >= a.seg[a.nchunks]) return;
@@ -1025,13 +1389,14 @@ __global__ __launch_bounds__(64) void k_sym_rest(SymArgs a)
     const double Ox = P.x[io], Oy = P.y[io], Oz = P.z[io];
     const bool valid = gbase + lane < a.n;
     const int64_t ii[1] = {valid ? gbase + lane : a.n - 1};
-    const double xr[1] = {P.x[ii[0]] - Ox}, yr[1] = {P.y[ii[0]] - Oy}, zr[1] = {P.z[ii[0]] - Oz};
+    const double xr = P.x[ii[0]] - Ox, yr = P.y[ii[0]] - Oy, zr = P.z[ii[0]] - Oz;
     double Hi[1], invHi[1], hi2[1];
     int idi[1];
     near_i_state<1>(P, ii, Hi, invHi, hi2, idi);
-    const float px = (float)xr[0], py = (float)yr[0], pz = (float)zr[0], ph = (float)Hi[0];
-    double ax[1] = {0.0}, ay[1] = {0.0}, az[1] = {0.0}, ap[1] = {0.0};
-    unsigned nfp64[1] = {0}, visits = 0, nearv = 0;
+    const float px = (float)xr, py = (float)yr, pz = (float)zr, ph = (float)Hi[0];
+    const float rho2 = fmaf(px, px, fmaf(py, py, pz * pz));
+    double acc[4] = {0.0, 0.0, 0.0, 0.0};
+    unsigned nfp64 = 0, visits = 0, nearv = 0, widev = 0;
 
     RestBits it;
     it.row = a.sym + (int64_t)ci * a.words;
@@ -1054,14 +1419,17 @@ __global__ __launch_bounds__(64) void k_sym_rest(SymArgs a)
            jz = P.z[(int64_t)cj * TC + lane], jm = P.m[(int64_t)cj * TC + lane],
            jh = P.Hs[(int64_t)cj * TC + lane];
     for (;;) {
-        const TileMeta &cm = a.chunks[cj];
-        const float gx = fmaxf(0.0f, fmaxf((float)(cm.lo[0] - Ox) - px, px - (float)(cm.hi[0] - Ox)));
-        const float gy = fmaxf(0.0f, fmaxf((float)(cm.lo[1] - Oy) - py, py - (float)(cm.hi[1] - Oy)));
-        const float gz = fmaxf(0.0f, fmaxf((float)(cm.lo[2] - Oz) - pz, pz - (float)(cm.hi[2] - Oz)));
-        const float hm = fmaxf(ph, (float)cm.maxH);
-        const bool lane_near = !(fmaf(gx, gx, fmaf(gy, gy, gz * gz)) > hm * hm * (1.0f + FAR_MARGIN));
-        const bool is_near = __ballot(lane_near) != 0;
-        const uint64_t real = near_stage(sl, jx - Ox, jy - Oy, jz - Oz, jm, jh);
+        const Visit v = classify_visit(a.chunks[cj], Ox, Oy, Oz, px, py, pz, ph, rho2);
+        const double rx = jx - Ox, ry = jy - Oy, rz = jz - Oz;
+        uint64_t real = 0;
+        if (v == VISIT_FAR) {
+            wave_lds_sync();
+            reinterpret_cast<float4 *>(sl.p)[lane] =
+                make_float4((float)rx, (float)ry, (float)rz, (float)jm);
+            wave_lds_sync();
+        } else {
+            real = near_stage(sl, rx, ry, rz, jm, jh);
+        }
         const int64_t j0c = (int64_t)cj * TC;
         ++visits;
         if (--left > 0) {
@@ -1073,28 +1441,27 @@ __global__ __launch_bounds__(64) void k_sym_rest(SymArgs a)
             jm = P.m[j];
             jh = P.Hs[j];
         }
-        if (is_near) {
+        if (v == VISIT_NEAR) {
             ++nearv;
-            near_chunk_eval<1, NK>(sl, real, P, j0c, xr, yr, zr, Hi, invHi, hi2, idi, ax, ay, az, ap,
-                                   nfp64);
+            visit_near<NK>(lds, real, P, j0c, 0, TC, xr, yr, zr, Hi[0], invHi[0], hi2[0], idi[0], acc, nfp64);
+        } else if (v == VISIT_WIDE) {
+            ++widev;
+            visit_wide(sl, 0, TC, xr, yr, zr, acc);
         } else {
-            const float none[1] = {0.0f};
-            far_chunk_fp32<1, true>(nullptr, sl.p, none, none, none, xr, yr, zr, ax, ay, az, ap);
+            visit_far(reinterpret_cast<const float4 *>(sl.p), 0, TC, px, py, pz, acc);
         }
         if (left <= 0) break;
     }
     double *s = a.segsum + (int64_t)g * 4 * TC + lane;
-    s[0] = ax[0];
-    s[TC] = ay[0];
-    s[2 * TC] = az[0];
-    s[3 * TC] = ap[0];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) s[k * TC] = acc[k];
     if (a.stats) {
-        const unsigned long long fw = wave_sum_count(valid ? nfp64[0] : 0u);
+        const unsigned long long fw = wave_sum_count(valid ? nfp64 : 0u);
         if (lane == 0) {
             unsigned long long *st = stat_copy(a.stats);
             atomicAdd(&st[0], (unsigned long long)visits);
             atomicAdd(&st[1], (unsigned long long)nearv);
-            atomicAdd(&st[2], (unsigned long long)(visits - nearv));
+            atomicAdd(&st[2], (unsigned long long)widev);
             atomicAdd(&st[3], fw);
         }
     }
@@ -1158,26 +1525,21 @@ __global__ __launch_bounds__(256) void k_psi_only(PairArgs a)
     a.psi[o] = Hs > 0.0 ? -2.0 * invHi * invHi * ps : 0.0;
 }
 
-// Fixed-order FP64 sum of the j-partition partials, scattered to input order.
+// Fixed-order FP64 sum of the j-partition partials, scattered to input order:
+// one thread per particle and sum (blockIdx.y: ax, ay, az, pot, psi), eight
+// partitions' loads in flight.
 __global__ __launch_bounds__(256) void k_reduce_partials(PairArgs a)
 {
     const int64_t i = blockIdx.x * (int64_t)256 + threadIdx.x;
+    const int c = blockIdx.y;
     if (i >= a.ni) return;
-    double s[4] = {0.0, 0.0, 0.0, 0.0};
-    for (int jp = 0; jp < a.jsplit; ++jp) {
-        const double *p = a.partial + (int64_t)jp * 4 * a.ni;
-        for (int c = 0; c < 4; ++c) s[c] += p[c * a.ni + i];
-    }
-    const int64_t o = (int64_t)a.i.idx[i] - a.ibeg;
-    a.ax[o] = s[0];
-    a.ay[o] = s[1];
-    a.az[o] = s[2];
-    a.pot[o] = s[3];
-    if (a.psi) {
-        double p = 0.0;
-        for (int jp = 0; jp < a.jsplit; ++jp) p += a.psipart[(int64_t)jp * a.ni + i];
-        a.psi[o] = p;
-    }
+    const int64_t step = c < 4 ? 4 * a.ni : a.ni;
+    const double *p = c < 4 ? a.partial + c * a.ni + i : a.psipart + i;
+    double s = 0.0;
+#pragma unroll 8
+    for (int jp = 0; jp < a.jsplit; ++jp) s += p[jp * step];
+    double *out = c == 0 ? a.ax : (c == 1 ? a.ay : (c == 2 ? a.az : (c == 3 ? a.pot : a.psi)));
+    out[(int64_t)a.i.idx[i] - a.ibeg] = s;
 }
 
 // ============================================================= batch kernels
@@ -1329,6 +1691,16 @@ hipError_t launch_pair_far(int precision, const PairArgs &a, int wg, hipStream_t
         }
         return hipGetLastError();
     }
+    if (precision == 0 && a.wave) {
+        const dim3 grid((unsigned)((a.ni + TC - 1) / TC) * (unsigned)a.jsplit), block(64);
+        switch (a.nkernel) {
+        case 0: hipLaunchKernelGGL((k_pair_wave<0>), grid, block, 0, s, a); break;
+        case 1: hipLaunchKernelGGL((k_pair_wave<1>), grid, block, 0, s, a); break;
+        case 2: hipLaunchKernelGGL((k_pair_wave<2>), grid, block, 0, s, a); break;
+        default: return hipErrorInvalidValue;
+        }
+        return hipGetLastError();
+    }
     if (precision == 0) {
         if (wg == 64 && a.ipl == 1) return far_fused_launch<64, 1>(a, s);
         if (wg == 64 && a.ipl == 2) return far_fused_launch<64, 2>(a, s);
@@ -1424,7 +1796,8 @@ hipError_t launch_sym_rest(const SymArgs &a, hipStream_t s)
 hipError_t launch_reduce_partials(const PairArgs &a, hipStream_t s)
 {
     if (a.ni <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_reduce_partials, dim3((unsigned)((a.ni + 255) / 256)), dim3(256), 0, s, a);
+    hipLaunchKernelGGL(k_reduce_partials, dim3((unsigned)((a.ni + 255) / 256), a.psi ? 5 : 4),
+                       dim3(256), 0, s, a);
     return hipGetLastError();
 }
 

@@ -60,6 +60,8 @@ struct PairArgs {
     int niblocks;            // i-blocks
     int ipl;                 // i-particles per lane of the far kernel (groups of 64*ipl)
     int64_t ngroups;         // i-groups (waves of the far kernel)
+    bool wave;               // FP32C: one wave per 64 i and j partition (k_pair_wave)
+    int jsub;                // with wave: parts each j chunk is divided into (1, 2, 4)
     double *ax, *ay, *az, *pot;   // final outputs, input order, length ni
     double *partial;              // [jsplit][4][ni] sorted-order partial sums
     unsigned char *nearflag;      // [ngroups][ntiles]: bit c set = chunk c of the tile may
@@ -253,6 +255,8 @@ struct EvalPlan {
     int64_t psipart_elems; // grad-h partial sums: jsplit * ni (with psi; else 0)
     // each unordered far pair once (sg_sym.hip): jsplit counts its slabs
     bool sym;
+    bool wave;             // one wave per 64 i and j partition (k_pair_wave)
+    int jsub;
     int sb, nsb, waves;
     int64_t sym_bytes;     // chunk boxes, chunk-pair bits, segment table
 };
@@ -260,14 +264,23 @@ int auto_jsplit(int niblocks, int wg, int ntiles, int64_t ni);
 // i-ranges up to this many particles take workgroups of 128 when the
 // configured workgroup size is 0 (automatic), larger ones 256
 constexpr int AUTO_SMALL_NI = 65536;
+// i-ranges of up to WAVE_MAX_NI particles run k_pair_wave, about WAVE_COUNT
+// waves of it (twice that for n above the static entry point's limit); with
+// fewer than half as many (64 i, 64 j) visits each is divided in four.  Pair
+// kernel, block kernel against this one, same card: 1,974 particles 0.355
+// against 0.030 ms, 4,944 0.261 against 0.053, 16,384 0.305 against 0.183,
+// 33,333 0.747 against 0.516, 32,771 of 262,144 3.74 against 2.89; with 4,096
+// waves 16,384 take 0.232, with 8,192 0.223.  Whole sets of 131,072 and more
+// are faster in blocks of 256 (262,144: 23.0 against 23.9 ms).
+constexpr int WAVE_MAX_NI = 49151, WAVE_COUNT = 16384;
 // Whole-set FP32C passes of these sizes evaluate each unordered far pair once
-// (sg_sym.hip).  Pair kernels of one Plummer sphere, ordered against
-// unordered, same card: 33,333 particles 0.74 against 0.80 ms, 50,001 1.42
-// against 1.26, 65,536 2.18 against 1.73, 131,072 7.35 against 5.38; a giant
-// star of 1,048,576 320 against 218 ms.  The upper limit keeps the chunk-pair
-// bits (N^2 / 32,768 bytes) at 512 MB and the slabs at 17 GB; where the device
-// cannot hold them the ordered pass runs.
-constexpr int SYM_MIN_N = 40960, SYM_MAX_N = 1 << 22, SYM_MAX_SB = 128;
+// (sg_sym.hip).  Pair kernels of one Plummer sphere, one wave per 64 i against
+// unordered, same card: 33,333 particles 0.52 against 0.71 ms, 50,001 1.21
+// against 1.10, 65,536 1.86 against 1.50, 131,072 (two stars) 6.15 against
+// 4.96; a giant star of 1,048,576 takes 210 ms, 320 in blocks of 256.  The
+// upper limit keeps the chunk-pair bits (N^2 / 32,768 bytes) at 512 MB and the
+// slabs at 17 GB; where the device cannot hold them the ordered pass runs.
+constexpr int SYM_MIN_N = 49152, SYM_MAX_N = 1 << 22, SYM_MAX_SB = 128;
 // the HIP error that sg_status_string(SG_ERR_HIP) describes
 void record_hip_error(hipError_t e);
 EvalPlan plan_eval(int n, int ni, int wg, int ipl, int jsplit_cfg, int precision, bool psi,

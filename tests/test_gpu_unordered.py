@@ -1,7 +1,7 @@
 """The whole-set FP32C pass that evaluates each unordered far pair once
 (sg_sym.hip), against the oracle and against the ordered pass.
 
-A context takes it at its automatic configuration from 40,960 particles on;
+A context takes it at its automatic configuration from 49,152 particles on;
 an explicit j-split asks for the ordered pass.  Bounds: the library's stated
 FP32C errors (1e-5 on the acceleration, 1e-6 on the potential, as in the other
 parity tests); both passes round each pair to FP32 and sum at most 32 pairs in
@@ -39,12 +39,12 @@ def _set(kind, n):
     return d
 
 
-# 40,960 is the smallest set of the pass and 40,959 the largest before it;
-# 40,961 and 65,537 end in a chunk of one particle, 69,889 and 131,073 leave
-# a superblock of one tile behind whole ones; up to 32,768 / 65,536 / more
-# particles a workgroup has one / two / four waves
+# 49,152 is the smallest set of the pass and 49,151 the largest before it;
+# 49,153 and 65,537 end in a chunk of one particle, 69,889 and 131,073 leave
+# a superblock of one tile behind whole ones; up to 65,536 particles a
+# workgroup has two waves, then four
 @pytest.mark.parametrize("kind,n,nk", [
-    ("plummer", 40959, 0), ("plummer", 40960, 0), ("two", 40961, 1), ("giant", 50000, 2),
+    ("plummer", 49151, 0), ("plummer", 49152, 0), ("two", 49153, 1), ("giant", 50000, 2),
     ("bigH", 65537, 0), ("twins", 69889, 1), ("two", 100003, 2), ("giant", 131073, 0),
 ])
 def test_against_oracle_and_ordered_pass(grav, kind, n, nk):
@@ -57,7 +57,7 @@ def test_against_oracle_and_ordered_pass(grav, kind, n, nk):
         np.testing.assert_array_equal(a, b)     # fixed order of every sum
     chunks = -(-n // 256) * 4
     assert 0 < nearv + widev < visits and fp64 >= n - (d["range2"] < 0).sum()
-    if n >= 40960:
+    if n >= 49152:
         assert visits == chunks ** 2            # every chunk pair, each order once
     old = grav.get_config(SG_PREC_FP32C)
     grav.set_config(SG_PREC_FP32C, 256, 1, 7)
@@ -83,7 +83,7 @@ def test_against_oracle_and_ordered_pass(grav, kind, n, nk):
 def test_particles_on_a_line(grav):
     """All chunks of a set on one axis: boxes of zero width, no far chunk
     rejected by two of the three axes."""
-    n = 45000
+    n = 50000
     rng = np.random.default_rng(8)
     x = np.sort(rng.uniform(-50.0, 50.0, n))
     z = np.zeros(n)
@@ -103,7 +103,7 @@ def test_units(grav, length, mass):
     """The same set in other units (metres and kilograms of a wide system, and
     the reverse): r^-3 by itself leaves the FP32 range, the result scales
     exactly up to FP32 rounding of the scaled inputs."""
-    d = _set("plummer", 45000)
+    d = _set("plummer", 50000)
     base = grav.compute(d["x"], d["y"], d["z"], d["m"], d["range2"])
     res = grav.compute(d["x"] * length, d["y"] * length, d["z"] * length, d["m"] * mass,
                        d["range2"] * length ** 2)

@@ -301,6 +301,27 @@ EvalPlan plan_eval(int n, int ni, int wg, int ipl, int jsplit_cfg, int precision
     return p;
 }
 
+// The preparation of a whole set: validation, curve order, gather into the
+// sorted j arrays, tile and chunk boxes, zeroed statistics.
+static hipError_t enqueue_prep(PrepBuffers &b, void *sort_tmp, size_t sort_bytes, bool merge_sort,
+                               int n, int64_t padded, const double *x, const double *y,
+                               const double *z, const double *m, const double *range2,
+                               unsigned long long *stats, hipStream_t s)
+{
+    hipError_t e;
+    if (n <= SMALL_PREP_N) {
+        e = launch_prep_small(x, y, z, m, range2, n, b, stats, s);
+    } else {
+        auto sort = merge_sort ? merge_sort_pairs : sort_pairs;
+        if ((e = launch_validate_bbox(x, y, z, m, range2, n, b, s)) == hipSuccess &&
+            (e = launch_morton(x, y, z, 0, n, b, s)) == hipSuccess &&
+            (e = sort(sort_tmp, sort_bytes, b.keys_in, b.keys_out, b.vals_in, b.vals_out, n, s)) ==
+                hipSuccess)
+            e = launch_fill_zero_int((int *)stats, 2 * STAT_WORDS, s);
+    }
+    return e == hipSuccess ? launch_gather_tiles(x, y, z, m, range2, n, padded, b, s) : e;
+}
+
 hipError_t enqueue_eval(const EvalPlan &p, const EvalBuffers &bufs, int n, int ibeg, int ni,
                         const double *x, const double *y, const double *z, const double *m,
                         const double *range2, int nkernel, int precision, double *ax, double *ay,
@@ -314,17 +335,8 @@ hipError_t enqueue_eval(const EvalPlan &p, const EvalBuffers &bufs, int n, int i
     } while (0)
     PrepBuffers b = bufs.pb;
     if (ev) SG_ENQ(hipEventRecord(ev[0], s));
-    // 1-2: validate + bbox, Morton keys of all n
-    SG_ENQ(launch_validate_bbox(x, y, z, m, range2, n, b, s));
-    SG_ENQ(launch_morton(x, y, z, 0, n, b, s));
-    // 3: sort
-    auto sort = bufs.merge_sort ? merge_sort_pairs : sort_pairs;
-    SG_ENQ(sort(bufs.sort_tmp, bufs.sort_tmp_bytes, b.keys_in, b.keys_out, b.vals_in, b.vals_out,
-                n, s));
-    // 4-5: gather sorted j arrays, tile metadata
-    SG_ENQ(launch_gather(x, y, z, m, range2, b.vals_out, n, p.padded, b.sx, b.sy, b.sz, b.sm,
-                         b.sH, b.sidx, s));
-    SG_ENQ(launch_tile_meta(b.sx, b.sy, b.sz, b.sH, p.ntiles, b.tiles, b.chunks, s));
+    SG_ENQ(enqueue_prep(b, bufs.sort_tmp, bufs.sort_tmp_bytes, bufs.merge_sort, n, p.padded, x, y, z,
+                        m, range2, bufs.stats, s));
 
     PairArgs a{};
     a.j = SortedSet{b.sx, b.sy, b.sz, b.sm, b.sH, b.sidx, n, p.padded};
@@ -332,6 +344,7 @@ hipError_t enqueue_eval(const EvalPlan &p, const EvalBuffers &bufs, int n, int i
         a.i = a.j;
     } else {
         // the i-range gets its own curve order
+        auto sort = bufs.merge_sort ? merge_sort_pairs : sort_pairs;
         SG_ENQ(launch_morton(x, y, z, ibeg, ni, b, s));
         SG_ENQ(sort(bufs.sort_tmp, bufs.sort_tmp_bytes, b.keys_in, b.keys_out, b.vals_in,
                     b.vals_out, ni, s));
@@ -362,8 +375,6 @@ hipError_t enqueue_eval(const EvalPlan &p, const EvalBuffers &bufs, int n, int i
         a.psi = psi;
         a.psipart = bufs.psipart;
     }
-    SG_ENQ(launch_fill_zero_int((int *)bufs.stats, 2 * STAT_WORDS, s));
-
     if (p.sym) {
         SymArgs y{};
         y.p = a.j;
@@ -619,14 +630,11 @@ int sg_psi_device(sg_context *c, int n, int ibeg, int ni, const double *x, const
     hipStream_t s = c->stream;
     sg::PrepBuffers &b = c->pb;
     HIP_TRY(hipEventRecord(c->ev_p0, s));
-    HIP_TRY(sg::launch_validate_bbox(x, y, z, m, range2, n, b, s));
-    HIP_TRY(sg::launch_morton(x, y, z, 0, n, b, s));
-    HIP_TRY(sg::sort_pairs(c->sort_tmp, c->sort_tmp_bytes, b.keys_in, b.keys_out, b.vals_in,
-                           b.vals_out, n, s));
-    HIP_TRY(sg::launch_gather(x, y, z, m, range2, b.vals_out, n, padded, b.sx, b.sy, b.sz, b.sm,
-                              b.sH, b.sidx, s));
+    // the psi-only pass classifies no chunks: its statistics read zero
+    // rather than the previous evaluation's counts
+    HIP_TRY(sg::enqueue_prep(b, c->sort_tmp, c->sort_tmp_bytes, false, n, padded, x, y, z, m, range2,
+                             c->stats, s));
     const int ntiles = (int)(padded / TJ);
-    HIP_TRY(sg::launch_tile_meta(b.sx, b.sy, b.sz, b.sH, ntiles, b.tiles, b.chunks, s));
     sg::PairArgs a{};
     a.j = sg::SortedSet{b.sx, b.sy, b.sz, b.sm, b.sH, b.sidx, n, padded};
     if (ibeg == 0 && ni == n) {
@@ -649,9 +657,6 @@ int sg_psi_device(sg_context *c, int n, int ibeg, int ni, const double *x, const
     a.jsplit = 1;
     a.ngroups = (ni + 63) / 64;
     a.psi = psi;
-    // the psi-only pass classifies no chunks: its statistics read zero
-    // rather than the previous evaluation's counts
-    HIP_TRY(sg::launch_fill_zero_int((int *)c->stats, 2 * sg::STAT_WORDS, s));
     HIP_TRY(hipEventRecord(c->ev_k0, s));
     HIP_TRY(hipEventRecord(c->ev_kf, s));
     HIP_TRY(sg::launch_psi_only(a, s));
@@ -1057,14 +1062,9 @@ int sg_vjp_device(sg_context *c, int n, const double *x, const double *y, const 
     hipStream_t s = c->stream;
     sg::PrepBuffers &b = c->pb;
     HIP_TRY(hipEventRecord(c->ev_p0, s));
-    HIP_TRY(sg::launch_validate_bbox(x, y, z, m, range2, n, b, s));
-    HIP_TRY(sg::launch_morton(x, y, z, 0, n, b, s));
-    HIP_TRY(sg::sort_pairs(c->sort_tmp, c->sort_tmp_bytes, b.keys_in, b.keys_out, b.vals_in,
-                           b.vals_out, n, s));
-    HIP_TRY(sg::launch_gather(x, y, z, m, range2, b.vals_out, n, padded, b.sx, b.sy, b.sz, b.sm,
-                              b.sH, b.sidx, s));
+    HIP_TRY(sg::enqueue_prep(b, c->sort_tmp, c->sort_tmp_bytes, false, n, padded, x, y, z, m, range2,
+                             c->stats, s));
     const int ntiles = (int)(padded / TJ);
-    HIP_TRY(sg::launch_tile_meta(b.sx, b.sy, b.sz, b.sH, ntiles, b.tiles, b.chunks, s));
     HIP_TRY(sg::launch_gather_cot(wx, wy, wz, u, b.vals_out, n, padded, c->scot[0], c->scot[1],
                                   c->scot[2], c->scot[3], b, s));
 
@@ -1093,7 +1093,6 @@ int sg_vjp_device(sg_context *c, int n, const double *x, const double *y, const 
     if ((rc = grow(&c->nearflag, &c->cap_flag, a.ngroups * ntiles)) != SG_OK) return rc;
     a.nearflag = c->nearflag;
     a.stats = c->stats;
-    HIP_TRY(sg::launch_fill_zero_int((int *)c->stats, 2 * sg::STAT_WORDS, s));
 
     HIP_TRY(hipEventRecord(c->ev_k0, s));
     HIP_TRY(sg::launch_adj_far(precision, a, wg, s));

@@ -1526,20 +1526,27 @@ __global__ __launch_bounds__(256) void k_psi_only(PairArgs a)
 }
 
 // Fixed-order FP64 sum of the j-partition partials, scattered to input order:
-// one thread per particle and sum (blockIdx.y: ax, ay, az, pot, psi), eight
-// partitions' loads in flight.
+// a block takes 64 particles of one sum (blockIdx.y: ax, ay, az, pot, psi),
+// each of its waves a quarter of the partitions, eight loads in flight.
 __global__ __launch_bounds__(256) void k_reduce_partials(PairArgs a)
 {
-    const int64_t i = blockIdx.x * (int64_t)256 + threadIdx.x;
+    __shared__ double s_sum[4][64];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int64_t i = blockIdx.x * (int64_t)64 + lane;
     const int c = blockIdx.y;
-    if (i >= a.ni) return;
     const int64_t step = c < 4 ? 4 * a.ni : a.ni;
-    const double *p = c < 4 ? a.partial + c * a.ni + i : a.psipart + i;
     double s = 0.0;
+    if (i < a.ni) {
+        const double *p = c < 4 ? a.partial + c * a.ni + i : a.psipart + i;
+        const int end = a.jsplit * (w + 1) / 4;
 #pragma unroll 8
-    for (int jp = 0; jp < a.jsplit; ++jp) s += p[jp * step];
+        for (int jp = a.jsplit * w / 4; jp < end; ++jp) s += p[jp * step];
+    }
+    s_sum[w][lane] = s;
+    __syncthreads();
+    if (w != 0 || i >= a.ni) return;
     double *out = c == 0 ? a.ax : (c == 1 ? a.ay : (c == 2 ? a.az : (c == 3 ? a.pot : a.psi)));
-    out[(int64_t)a.i.idx[i] - a.ibeg] = s;
+    out[(int64_t)a.i.idx[i] - a.ibeg] = s + s_sum[1][lane] + s_sum[2][lane] + s_sum[3][lane];
 }
 
 // ============================================================= batch kernels
@@ -1796,7 +1803,7 @@ hipError_t launch_sym_rest(const SymArgs &a, hipStream_t s)
 hipError_t launch_reduce_partials(const PairArgs &a, hipStream_t s)
 {
     if (a.ni <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_reduce_partials, dim3((unsigned)((a.ni + 255) / 256), a.psi ? 5 : 4),
+    hipLaunchKernelGGL(k_reduce_partials, dim3((unsigned)((a.ni + 63) / 64), a.psi ? 5 : 4),
                        dim3(256), 0, s, a);
     return hipGetLastError();
 }

@@ -214,6 +214,16 @@ hipError_t launch_gather_cot(const double *wx, const double *wy, const double *w
 hipError_t launch_tile_meta(const double *sx, const double *sy, const double *sz,
                             const double *sH, int ntiles, TileMeta *tiles, TileMeta *chunks,
                             hipStream_t s);
+// Sets of up to SMALL_PREP_N particles: validation, box, curve order (in
+// b.vals_out) and zeroed statistics in one launch.
+constexpr int SMALL_PREP_N = 8192;
+hipError_t launch_prep_small(const double *x, const double *y, const double *z, const double *m,
+                             const double *r2, int n, const PrepBuffers &b,
+                             unsigned long long *stats, hipStream_t s);
+// The sorted, padded j set and its tile and chunk boxes from b.vals_out.
+hipError_t launch_gather_tiles(const double *x, const double *y, const double *z, const double *m,
+                               const double *r2, int count, int64_t padded, const PrepBuffers &b,
+                               hipStream_t s);
 hipError_t launch_fill_zero_int(int *p, int n, hipStream_t s);
 // 1/2 sum m pot in FP64 into work[nwork - 1] (work holds nwork doubles)
 hipError_t launch_potential_energy(const double *m, const double *pot, int n, double *work,

@@ -251,18 +251,14 @@ __global__ __launch_bounds__(RB) void k_gather_cot(const double *__restrict__ wx
     if (!(isfinite(a) && isfinite(b) && isfinite(c) && isfinite(d))) atomicOr(err, (int)ERR_NONFINITE);
 }
 
-__global__ __launch_bounds__(TJ) void k_tile_meta(const double *__restrict__ sx,
-                                                  const double *__restrict__ sy,
-                                                  const double *__restrict__ sz,
-                                                  const double *__restrict__ sH,
-                                                  TileMeta *__restrict__ tiles,
-                                                  TileMeta *__restrict__ chunks)
+// Boxes and largest H of one tile and its chunks from one particle per
+// thread.
+__device__ inline void tile_boxes(double px, double py, double pz, double h, TileMeta *tile,
+                                  TileMeta *chunks)
 {
     static_assert(TJ == RB, "one thread per tile particle");
     static_assert(TC == 64 && CHUNKS * TC == TJ, "one wave per chunk");
-    const int64_t k = (int64_t)blockIdx.x * TJ + threadIdx.x;
-    double v[6] = {sx[k], sy[k], sz[k], sx[k], sy[k], sz[k]};
-    double h = fabs(sH[k]);
+    double v[6] = {px, py, pz, px, py, pz};
     // chunk box: one wave per TC particles
     double c[6];
     for (int q = 0; q < 3; ++q) c[q] = warp_min(v[q]);
@@ -276,9 +272,9 @@ __global__ __launch_bounds__(TJ) void k_tile_meta(const double *__restrict__ sx,
         }
         t.maxH = h;
         t.pad = 0.0;
-        chunks[(int64_t)blockIdx.x * CHUNKS + (threadIdx.x >> 6)] = t;
+        chunks[threadIdx.x >> 6] = t;
     }
-    block_minmax6(v);
+    block_minmax6(c);
     __shared__ double shH[TJ / 64];
     if ((threadIdx.x & 63) == 0) shH[threadIdx.x >> 6] = h;
     __syncthreads();
@@ -286,12 +282,158 @@ __global__ __launch_bounds__(TJ) void k_tile_meta(const double *__restrict__ sx,
         for (int w = 1; w < TJ / 64; ++w) h = fmax(h, shH[w]);
         TileMeta t;
         for (int q = 0; q < 3; ++q) {
-            t.lo[q] = v[q];
-            t.hi[q] = v[3 + q];
+            t.lo[q] = c[q];
+            t.hi[q] = c[3 + q];
         }
         t.maxH = h;
         t.pad = 0.0;
-        tiles[blockIdx.x] = t;
+        *tile = t;
+    }
+}
+
+__global__ __launch_bounds__(TJ) void k_tile_meta(const double *__restrict__ sx,
+                                                  const double *__restrict__ sy,
+                                                  const double *__restrict__ sz,
+                                                  const double *__restrict__ sH,
+                                                  TileMeta *__restrict__ tiles,
+                                                  TileMeta *__restrict__ chunks)
+{
+    const int64_t k = (int64_t)blockIdx.x * TJ + threadIdx.x;
+    tile_boxes(sx[k], sy[k], sz[k], fabs(sH[k]), tiles + blockIdx.x,
+               chunks + (int64_t)blockIdx.x * CHUNKS);
+}
+
+// k_gather of the padded j set and k_tile_meta in one pass, a tile per block.
+__global__ __launch_bounds__(TJ) void k_gather_tiles(
+    const double *__restrict__ x, const double *__restrict__ y, const double *__restrict__ z,
+    const double *__restrict__ m, const double *__restrict__ r2, const int *__restrict__ perm,
+    int count, double *__restrict__ ox, double *__restrict__ oy, double *__restrict__ oz,
+    double *__restrict__ om, double *__restrict__ oH, int *__restrict__ oidx,
+    TileMeta *__restrict__ tiles, TileMeta *__restrict__ chunks)
+{
+    const int64_t k = (int64_t)blockIdx.x * TJ + threadIdx.x;
+    const bool real = k < count;
+    const int src = perm[real ? k : count - 1];
+    const double rr = r2[src], px = x[src], py = y[src], pz = z[src];
+    const double H = sqrt(rr > 0.0 ? rr : -rr);
+    ox[k] = px;
+    oy[k] = py;
+    oz[k] = pz;
+    om[k] = real ? m[src] : 0.0;
+    oH[k] = (real && rr > 0.0) ? H : -H;   // padding carries no self potential
+    oidx[k] = real ? src : -1;
+    tile_boxes(px, py, pz, H, tiles + blockIdx.x, chunks + (int64_t)blockIdx.x * CHUNKS);
+}
+
+// Everything before the gather for a small set, in one launch: validation,
+// box, curve order and the zeroing of the statistics.  A call on a few
+// thousand particles is a chain of launches of some 4 us each; this replaces
+// eight to eleven of them.  Each workgroup ranks SRANK particles: it computes
+// the box and every key itself (a few us of reads from L2; one word per
+// particle, the upper 51 bits of the key above the particle's index, so 17
+// bits per axis order the curve and no two are equal), its half-waves count
+// the smaller keys of a part of the set each, and the counts' sum is the
+// particle's place: 256 compares a lane at 8,192 particles.  A bitonic sort in
+// one workgroup took 89 us there and 30 us at 1,974.
+constexpr int SB = 1024;   // threads
+constexpr int SW = SB / 64;
+constexpr int SBITS = 13;  // index bits
+constexpr int SRANK = 32;
+constexpr int SPARTS = SB / SRANK;
+constexpr int SITEMS = SMALL_PREP_N / SB;   // particles a thread reads
+static_assert(SMALL_PREP_N == 1 << SBITS, "index fits its bits");
+
+__global__ __launch_bounds__(SB) void k_prep_small(const double *__restrict__ x,
+                                                   const double *__restrict__ y,
+                                                   const double *__restrict__ z,
+                                                   const double *__restrict__ m,
+                                                   const double *__restrict__ r2, int n, int seg,
+                                                   double *__restrict__ bbox, int *__restrict__ err,
+                                                   unsigned long long *__restrict__ stats,
+                                                   int *__restrict__ order)
+{
+    // SPARTS * seg keys (64 KB at most); first the waves' boxes and flags, last
+    // the counts
+    extern __shared__ uint64_t s_key[];
+    double(*s_box)[8] = reinterpret_cast<double(*)[8]>(s_key);
+    int(*s_count)[SRANK] = reinterpret_cast<int(*)[SRANK]>(s_key);
+    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+    if (blockIdx.x == 0)
+        for (int k = t; k < STAT_WORDS; k += SB) stats[k] = 0;
+    double v[7] = {INFINITY, INFINITY, INFINITY, -INFINITY, -INFINITY, -INFINITY, 0.0};
+    int flags = 0;
+    double px[SITEMS], py[SITEMS], pz[SITEMS];
+#pragma unroll
+    for (int q = 0; q < SITEMS; ++q) {   // all loads in flight; past the end the last particle
+        const int k = min(t + q * SB, n - 1);
+        px[q] = x[k];
+        py[q] = y[k];
+        pz[q] = z[k];
+    }
+#pragma unroll
+    for (int q = 0; q < SITEMS; ++q) {
+        v[0] = fmin(v[0], px[q]); v[1] = fmin(v[1], py[q]); v[2] = fmin(v[2], pz[q]);
+        v[3] = fmax(v[3], px[q]); v[4] = fmax(v[4], py[q]); v[5] = fmax(v[5], pz[q]);
+        if (blockIdx.x == 0) {
+            const int k = min(t + q * SB, n - 1);
+            const double pm = m[k], pr = r2[k];
+            if (!(isfinite(px[q]) && isfinite(py[q]) && isfinite(pz[q]) && isfinite(pm) && isfinite(pr)))
+                flags |= ERR_NONFINITE;
+            if (!(pm > 0.0)) flags |= ERR_MASS;
+            if (pr == 0.0) flags |= ERR_RANGE2;
+            v[6] = fmax(v[6], pm);
+        }
+    }
+    for (int c = 0; c < 3; ++c) v[c] = warp_min(v[c]);
+    for (int c = 3; c < 7; ++c) v[c] = warp_max(v[c]);
+    int seen = 0;   // of the wave
+    for (int bit = 1; bit <= ERR_NONFINITE; bit <<= 1)
+        if (__ballot(flags & bit)) seen |= bit;
+    if (lane == 0) {
+        for (int c = 0; c < 7; ++c) s_box[w][c] = v[c];
+        s_box[w][7] = seen;
+    }
+    __syncthreads();
+    for (int ww = 0; ww < SW; ++ww) {
+        for (int c = 0; c < 3; ++c) v[c] = fmin(v[c], s_box[ww][c]);
+        for (int c = 3; c < 7; ++c) v[c] = fmax(v[c], s_box[ww][c]);
+        seen |= (int)s_box[ww][7];
+    }
+    __syncthreads();
+    const double ext = fmax(fmax(v[3] - v[0], v[4] - v[1]), v[5] - v[2]);
+    if (blockIdx.x == 0 && t == 0) {
+        for (int c = 0; c < 6; ++c) bbox[c] = v[c];
+        bbox[6] = unit_scale(ext);
+        bbox[7] = unit_scale(v[6]);
+        *err = seen;
+    }
+    const double scale = ext > 0.0 ? 2097151.0 / ext : 0.0;
+#pragma unroll
+    for (int q = 0; q < SITEMS; ++q) {
+        const int k = t + q * SB;
+        uint64_t key = ~0ull;
+        if (k < n) {
+            key = (spread3(quant21(px[q], v[0], scale)) << 2) |
+                  (spread3(quant21(py[q], v[1], scale)) << 1) | spread3(quant21(pz[q], v[2], scale));
+            key = key >> (SBITS - 1) << SBITS | (uint64_t)k;
+        }
+        if (k < SPARTS * seg) s_key[k] = key;
+    }
+    __syncthreads();
+    const int part = t / SRANK, slot = t % SRANK;
+    const int i = blockIdx.x * SRANK + slot;
+    const uint64_t mine = s_key[min(i, n - 1)];
+    int count = 0;
+    const uint64_t *key = s_key + part * seg;
+#pragma unroll 8
+    for (int k = 0; k < seg; ++k) count += key[k] < mine ? 1 : 0;
+    __syncthreads();
+    s_count[part][slot] = count;
+    __syncthreads();
+    if (t < SRANK && i < n) {
+        int at = 0;
+        for (int q = 0; q < SPARTS; ++q) at += s_count[q][t];
+        order[at] = i;
     }
 }
 
@@ -397,6 +539,29 @@ hipError_t launch_potential_energy(const double *m, const double *pot, int n, do
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(k_epot_final, dim3(1), dim3(RB), 0, s, work, nb, work + nwork - 1);
+    return hipGetLastError();
+}
+
+hipError_t launch_prep_small(const double *x, const double *y, const double *z, const double *m,
+                             const double *r2, int n, const PrepBuffers &b,
+                             unsigned long long *stats, hipStream_t s)
+{
+    if (n < 1 || n > SMALL_PREP_N) return hipErrorInvalidValue;
+    // keys per part: whole groups of eight, and room for the counts
+    const int seg = std::max(16, ((n + SPARTS - 1) / SPARTS + 7) / 8 * 8);
+    hipLaunchKernelGGL(k_prep_small, dim3((unsigned)((n + SRANK - 1) / SRANK)), dim3(SB),
+                       sizeof(uint64_t) * (size_t)SPARTS * seg, s, x, y, z, m, r2, n, seg, b.bbox,
+                       b.err, stats, b.vals_out);
+    return hipGetLastError();
+}
+
+hipError_t launch_gather_tiles(const double *x, const double *y, const double *z, const double *m,
+                               const double *r2, int count, int64_t padded, const PrepBuffers &b,
+                               hipStream_t s)
+{
+    if (padded <= 0) return hipSuccess;
+    hipLaunchKernelGGL(k_gather_tiles, dim3((unsigned)(padded / TJ)), dim3(TJ), 0, s, x, y, z, m, r2,
+                       b.vals_out, count, b.sx, b.sy, b.sz, b.sm, b.sH, b.sidx, b.tiles, b.chunks);
     return hipGetLastError();
 }
 

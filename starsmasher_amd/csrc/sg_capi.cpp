@@ -654,9 +654,12 @@ int sg_psi_device(sg_context *c, int n, int ibeg, int ni, const double *x, const
     a.nkernel = nkernel;
     a.ntiles = ntiles;
     a.ipl = 1;
-    a.jsplit = 1;
     a.ngroups = (ni + 63) / 64;
+    // parts of a group's chunks, for some 8,192 waves
+    a.jsplit = (int)std::max<int64_t>(1, std::min<int64_t>(16, 8192 / a.ngroups));
     a.psi = psi;
+    if ((rc = grow(&c->psipart, &c->cap_psipart, (int64_t)a.jsplit * ni)) != SG_OK) return rc;
+    a.psipart = c->psipart;
     HIP_TRY(hipEventRecord(c->ev_k0, s));
     HIP_TRY(hipEventRecord(c->ev_kf, s));
     HIP_TRY(sg::launch_psi_only(a, s));

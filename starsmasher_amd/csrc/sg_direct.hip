@@ -1013,6 +1013,22 @@ __device__ __forceinline__ Visit classify_visit(const TileMeta &cm, double Ox, d
     return VISIT_FAR;
 }
 
+// A(q) and P(q) of the cubic spline (poly_AP) without a branch: both pieces,
+// the right one kept.
+__device__ __forceinline__ void cubic_AP(double q, double invq, double &A, double &P)
+{
+    const double q2 = q * q, iq3 = invq * invq * invq;
+    const double Ai = 10.666666666667 + q2 * (32.0 * q - 38.4);
+    const double Pi = -2.8 + q2 * (5.333333333333 + q2 * (6.4 * q - 9.6));
+    const double Ao = 21.333333333333 + q * (-48.0 + q * (38.4 - 10.666666666667 * q)) -
+                      0.066666666667 * iq3;
+    const double Po = -3.2 + 0.066666666667 * invq +
+                      q2 * (10.666666666667 + q * (-16.0 + q * (9.6 - 2.133333333333 * q)));
+    const bool in = q < 0.5;
+    A = in ? Ai : Ao;
+    P = in ? Pi : Po;
+}
+
 // One side of a softened pair without a branch: the polynomials, or the
 // Newtonian terms beyond H.  q = 0 (r = 0, with ri passed as 0) gives the
 // r -> 0 limit.
@@ -1020,23 +1036,10 @@ template <int NK>
 __device__ __forceinline__ void side_select(double r, double ri, double r2, double H, double invH,
                                             double &gacc, double &gpot)
 {
-    const double q = r * invH, q2 = q * q;
+    const double q = r * invH;
     double A, P;
-    if (NK == 0) {
-        // both branches of the cubic spline (poly_AP), the right one kept
-        const double iq = H * ri, iq3 = iq * iq * iq;
-        const double Ai = 10.666666666667 + q2 * (32.0 * q - 38.4);
-        const double Pi = -2.8 + q2 * (5.333333333333 + q2 * (6.4 * q - 9.6));
-        const double Ao = 21.333333333333 + q * (-48.0 + q * (38.4 - 10.666666666667 * q)) -
-                          0.066666666667 * iq3;
-        const double Po = -3.2 + 0.066666666667 * iq +
-                          q2 * (10.666666666667 + q * (-16.0 + q * (9.6 - 2.133333333333 * q)));
-        const bool in = q < 0.5;
-        A = in ? Ai : Ao;
-        P = in ? Pi : Po;
-    } else {
-        poly_AP(NK, q, 0.0, A, P);
-    }
+    if (NK == 0) cubic_AP(q, H * ri, A, P);
+    else poly_AP(NK, q, 0.0, A, P);
     const bool soft = r2 <= H * H;
     gacc += soft ? A * invH * invH * invH : ri * ri * ri;
     gpot += soft ? P * invH : -ri;
@@ -1469,24 +1472,98 @@ __global__ __launch_bounds__(64) void k_sym_rest(SymArgs a)
 
 // ------------------------------------------------- grad-h term on its own
 // psi_i = -(2/H_i^2) sum_{j: r <= H_i} m_j (P(q_i) + q_i^2 A(q_i)) of the
-// gas particles of the i-set, without the accelerations: one wave per
-// 64-particle i-group tests every tile and chunk against the group's box
-// (r <= H_i needs only the wave's largest H) and sums the chunks it cannot
-// rule out, staged through its own LDS slice.  FP64 throughout.
+// gas particles of the i-set, without the accelerations.  One wave per
+// 64-particle i-group and part: its lanes test 64 tiles at a time against the
+// group's box (r <= H_i needs only the wave's largest H), the parts deal the
+// chunks that cannot be ruled out among themselves, and the pairs within H_i
+// of a chunk are listed and dealt over the lanes (as in visit_near), since a
+// lane has about one in a chunk.  FP64 throughout.  65,536 particles: 0.4 ms;
+// with one wave a group testing tile after tile and every pair's polynomial
+// under its own branch 5.0 ms.
+struct PsiLds {
+    double4 p[TC];
+    uint16_t list[NSOFT];
+    double res[64];
+};
+
 template <int NK>
-__global__ __launch_bounds__(256) void k_psi_only(PairArgs a)
+__device__ __forceinline__ double psi_pair(double dx, double dy, double dz, double H, double invH,
+                                           double mj)
 {
-    __shared__ double4 s_p[4][TC];
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int64_t gi = (int64_t)blockIdx.x * 4 + w;
-    if (gi >= a.ngroups) return;   // whole wave; no block barrier below
-    const int64_t gbase = gi * 64;
+    const double r2 = fma(dx, dx, fma(dy, dy, dz * dz));
+    const bool apart = r2 > 0.0;
+    const double ri = apart ? rsqrt_pos64(apart ? r2 : 1.0) : 0.0;
+    const double r = r2 * ri, q = r * invH;
+    double A, P;
+    if (NK == 0) cubic_AP(q, H * ri, A, P);
+    else poly_AP(NK, q, 0.0, A, P);
+    return mj * fma(q * q, A, P);
+}
+
+template <int NK>
+__device__ __forceinline__ void psi_visit(PsiLds &lds, double xr, double yr, double zr, double Hi,
+                                          double invHi, double hi2, double &ps)
+{
+    const int lane = threadIdx.x & 63;
+    uint64_t mine = 0;   // bit jj: the pair with jj is within H_i
+#pragma unroll 4
+    for (int jj = 0; jj < TC; ++jj) {
+        const double4 p = lds.p[jj];
+        const double dx = p.x - xr, dy = p.y - yr, dz = p.z - zr;
+        const bool in = fma(dx, dx, fma(dy, dy, dz * dz)) <= hi2;
+        mine |= (uint64_t)(in ? 1u : 0u) << jj;
+    }
+    const unsigned count = (unsigned)__builtin_popcountll(mine);
+    unsigned at = 0, total = 0;
+#pragma unroll
+    for (int b = 0; b < 7; ++b) {
+        const uint64_t m = __ballot((count >> b) & 1u);
+        at += __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u))
+              << b;
+        total += (unsigned)__builtin_popcountll(m) << b;
+    }
+    if (total > (unsigned)NSOFT) {
+        while (mine) {
+            const int jj = __builtin_ctzll(mine);
+            mine &= mine - 1;
+            const double4 p = lds.p[jj];
+            ps += psi_pair<NK>(p.x - xr, p.y - yr, p.z - zr, Hi, invHi, p.w);
+        }
+        return;
+    }
+    for (unsigned k = at; mine; ++k) {
+        const int jj = __builtin_ctzll(mine);
+        mine &= mine - 1;
+        lds.list[k] = (uint16_t)(lane << 6 | jj);
+    }
+    for (unsigned b0 = 0; b0 < total; b0 += 64) {
+        wave_lds_sync();
+        const unsigned e = min(b0 + (unsigned)lane, total - 1);
+        const int il = lds.list[e] >> 6, jj = lds.list[e] & 63;
+        const double4 p = lds.p[jj];
+        lds.res[lane] = psi_pair<NK>(p.x - __shfl(xr, il, 64), p.y - __shfl(yr, il, 64),
+                                     p.z - __shfl(zr, il, 64), __shfl(Hi, il, 64),
+                                     __shfl(invHi, il, 64), p.w);
+        wave_lds_sync();
+        const unsigned hi = min(at + count, b0 + 64);
+        for (unsigned k = max(at, b0); k < hi; ++k) ps += lds.res[k - b0];
+    }
+}
+
+template <int NK>
+__global__ __launch_bounds__(64) void k_psi_only(PairArgs a)
+{
+    __shared__ PsiLds lds;
+    const int lane = threadIdx.x;
+    const unsigned ng = (unsigned)a.ngroups;
+    const int64_t gbase = (int64_t)(blockIdx.x % ng) * 64;
+    const int part = (int)(blockIdx.x / ng);
     const int64_t io = min(gbase + 32, a.ni - 1);
     const double Ox = a.i.x[io], Oy = a.i.y[io], Oz = a.i.z[io];
     const bool valid = gbase + lane < a.ni;
     const int64_t i = valid ? gbase + lane : a.ni - 1;
     const double xr = a.i.x[i] - Ox, yr = a.i.y[i] - Oy, zr = a.i.z[i] - Oz;
-    const double Hs = a.i.Hs[i], Hi = fabs(Hs), invHi = 1.0 / Hi, hi2 = Hi * Hi;
+    const double Hi = fabs(a.i.Hs[i]), invHi = 1.0 / Hi, hi2 = Hi * Hi;
     float bl[3] = {(float)xr, (float)yr, (float)zr}, bh[3] = {bl[0], bl[1], bl[2]};
     for (int c = 0; c < 3; ++c) {
         bl[c] = wave_min(bl[c]);
@@ -1496,33 +1573,50 @@ __global__ __launch_bounds__(256) void k_psi_only(PairArgs a)
     // H_i (with the far test's margin) holds no contributing pair
     const float hmax = wave_max((float)Hi);
     const float lim2 = hmax * hmax * (1.0f + FAR_MARGIN);
+    const float px = (float)xr, py = (float)yr, pz = (float)zr;
+    const float reach2 = (float)hi2 * (1.0f + FAR_MARGIN);
     double ps = 0.0;
-    for (int t = 0; t < a.ntiles; ++t) {
-        if (uniform_i(box_dist2(a.tiles[t], Ox, Oy, Oz, bl, bh) <= lim2) == 0) continue;
-        for (int c = 0; c < CHUNKS; ++c) {
-            const TileMeta &cm = a.chunks[(int64_t)t * CHUNKS + c];
-            if (uniform_i(box_dist2(cm, Ox, Oy, Oz, bl, bh) <= lim2) == 0) continue;
-            const int64_t j = (int64_t)t * TJ + c * TC + lane;
-            wave_lds_sync();
-            s_p[w][lane] = make_double4(a.j.x[j] - Ox, a.j.y[j] - Oy, a.j.z[j] - Oz, a.j.m[j]);
-            wave_lds_sync();
-#pragma unroll 2
-            for (int jj = 0; jj < TC; ++jj) {
-                const double4 p = s_p[w][jj];
-                const double dx = p.x - xr, dy = p.y - yr, dz = p.z - zr;
-                const double r2 = fma(dx, dx, fma(dy, dy, dz * dz));
-                if (r2 <= hi2) {
-                    const double r = sqrt(r2), q = r * invHi;
-                    double A, P;
-                    poly_AP(NK, q, q > 0.0 ? 1.0 / q : 0.0, A, P);
-                    ps = fma(p.w, fma(q * q, A, P), ps);
-                }
+    int cnt = 0;   // wave-uniform: chunks met so far, modulo the parts
+    for (int tb = 0; tb < a.ntiles; tb += 64) {
+        const int tl = min(tb + lane, a.ntiles - 1);
+        uint64_t tiles = __ballot(tb + lane < a.ntiles &&
+                                  box_dist2(a.tiles[tl], Ox, Oy, Oz, bl, bh) <= lim2);
+        for (; tiles; tiles &= tiles - 1) {
+            const int64_t c0 = (int64_t)(tb + __builtin_ctzll(tiles)) * CHUNKS;
+            unsigned bits = (unsigned)__ballot(
+                lane < CHUNKS && box_dist2(a.chunks[c0 + (lane & (CHUNKS - 1))], Ox, Oy, Oz, bl, bh) <= lim2);
+            for (; bits; bits &= bits - 1) {
+                // the group's box and largest H pass many chunks that no lane's
+                // own particle reaches
+                const TileMeta &cm = a.chunks[c0 + __builtin_ctz(bits)];
+                const float gx = fmaxf(0.0f, fmaxf((float)(cm.lo[0] - Ox) - px, px - (float)(cm.hi[0] - Ox)));
+                const float gy = fmaxf(0.0f, fmaxf((float)(cm.lo[1] - Oy) - py, py - (float)(cm.hi[1] - Oy)));
+                const float gz = fmaxf(0.0f, fmaxf((float)(cm.lo[2] - Oz) - pz, pz - (float)(cm.hi[2] - Oz)));
+                if (!__ballot(fmaf(gx, gx, fmaf(gy, gy, gz * gz)) <= reach2)) continue;
+                const int at = cnt;
+                cnt = cnt + 1 == a.jsplit ? 0 : cnt + 1;
+                if (at != part) continue;
+                const int64_t j = (c0 + __builtin_ctz(bits)) * TC + lane;
+                wave_lds_sync();
+                lds.p[lane] = make_double4(a.j.x[j] - Ox, a.j.y[j] - Oy, a.j.z[j] - Oz, a.j.m[j]);
+                wave_lds_sync();
+                psi_visit<NK>(lds, xr, yr, zr, Hi, invHi, hi2, ps);
             }
         }
     }
-    if (!valid) return;
-    const int64_t o = (int64_t)a.i.idx[i] - a.ibeg;
-    a.psi[o] = Hs > 0.0 ? -2.0 * invHi * invHi * ps : 0.0;
+    if (valid) a.psipart[(int64_t)part * a.ni + i] = ps;
+}
+
+// Fixed-order sum of the parts, scattered to input order (0 for point
+// particles).
+__global__ __launch_bounds__(256) void k_psi_reduce(PairArgs a)
+{
+    const int64_t i = blockIdx.x * (int64_t)256 + threadIdx.x;
+    if (i >= a.ni) return;
+    double ps = 0.0;
+    for (int p = 0; p < a.jsplit; ++p) ps += a.psipart[(int64_t)p * a.ni + i];
+    const double Hs = a.i.Hs[i];
+    a.psi[(int64_t)a.i.idx[i] - a.ibeg] = Hs > 0.0 ? -2.0 / (Hs * Hs) * ps : 0.0;
 }
 
 // Fixed-order FP64 sum of the j-partition partials, scattered to input order:
@@ -1777,13 +1871,16 @@ bool pair_config_supported(int precision, int wg, int ipl)
 hipError_t launch_psi_only(const PairArgs &a, hipStream_t s)
 {
     if (a.ni <= 0) return hipSuccess;
-    const dim3 grid((unsigned)((a.ngroups + 3) / 4)), block(256);
+    const dim3 grid((unsigned)a.ngroups * (unsigned)a.jsplit), block(64);
     switch (a.nkernel) {
     case 0: hipLaunchKernelGGL((k_psi_only<0>), grid, block, 0, s, a); break;
     case 1: hipLaunchKernelGGL((k_psi_only<1>), grid, block, 0, s, a); break;
     case 2: hipLaunchKernelGGL((k_psi_only<2>), grid, block, 0, s, a); break;
     default: return hipErrorInvalidValue;
     }
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(k_psi_reduce, dim3((unsigned)((a.ni + 255) / 256)), dim3(256), 0, s, a);
     return hipGetLastError();
 }
 

@@ -166,7 +166,8 @@ bool adj_config_supported(int wg);
 hipError_t launch_pair_far(int precision, const PairArgs &a, int wg, hipStream_t s);
 hipError_t launch_pair_near(int precision, const PairArgs &a, hipStream_t s);
 hipError_t launch_reduce_partials(const PairArgs &a, hipStream_t s);
-// Grad-h term alone (a.psi, no accelerations): groups of 64 i, a.ngroups of them.
+// Grad-h term alone (a.psi, no accelerations): groups of 64 i, a.ngroups of
+// them, each in a.jsplit parts (a.psipart: [jsplit][ni]).
 hipError_t launch_psi_only(const PairArgs &a, hipStream_t s);
 bool pair_config_supported(int precision, int wg, int ipl);
 // Batch: queue reset, persistent far kernel on nwg workgroups, near kernel,

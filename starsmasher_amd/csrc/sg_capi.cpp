@@ -286,7 +286,7 @@ EvalPlan plan_eval(int n, int ni, int wg, int ipl, int jsplit_cfg, int precision
     p.flag_elems = flagged ? p.ngroups * p.ntiles : 1;
     p.psipart_elems = psi ? (int64_t)p.jsplit * ni : 0;
     // the automatic shape, or asked for by its workgroup size
-    const bool automatic = precision == SG_PREC_FP32C && !psi && ipl == 1 && jsplit_cfg == 0 &&
+    const bool automatic = precision == SG_PREC_FP32C && p.ipl == 1 && jsplit_cfg == 0 &&
                            (wg == 0 || wg == (ni <= AUTO_SMALL_NI ? 128 : 256));
     if (automatic && ni <= WAVE_MAX_NI) {
         const int64_t nic = (ni + TC - 1) / TC, nchunks = (int64_t)p.ntiles * CHUNKS;
@@ -296,8 +296,10 @@ EvalPlan plan_eval(int n, int ni, int wg, int ipl, int jsplit_cfg, int precision
         p.jsub = nic * nchunks <= WAVE_COUNT / 2 ? 4 : 1;
         p.jsplit = p.jsub * (int)std::max<int64_t>(1, std::min(waves / (nic * p.jsub), nchunks));
         p.part_elems = (int64_t)p.jsplit * 4 * ni;
+        p.flag_elems = 1;
+        p.psipart_elems = psi ? (int64_t)p.jsplit * ni : 0;
     }
-    if (allow_sym && automatic && ni == n && n >= SYM_MIN_N && n <= SYM_MAX_N) plan_sym(p, n);
+    if (allow_sym && automatic && !psi && ni == n && n >= SYM_MIN_N && n <= SYM_MAX_N) plan_sym(p, n);
     return p;
 }
 

@@ -180,4 +180,79 @@ __device__ __forceinline__ void wave_lds_sync()
     __builtin_amdgcn_wave_barrier();
 }
 
+// The unset bits of one row of SymArgs::sym from the k-th on, in order.
+struct RestBits {
+    const uint64_t *row;
+    int nchunks, words, wb, src;
+    uint64_t rest, any, bits;   // rest: per lane; the others wave-uniform
+
+    __device__ __forceinline__ void block()
+    {
+        const int k = wb + (threadIdx.x & 63);
+        rest = 0;
+        if (k < words) {
+            const int left = nchunks - k * 64;
+            rest = ~row[k] & (left >= 64 ? ~0ull : (1ull << left) - 1ull);
+        }
+        any = __ballot(rest != 0);
+    }
+    __device__ __forceinline__ bool word()
+    {
+        while (!any) {
+            wb += 64;
+            if (wb >= words) return false;
+            block();
+        }
+        src = __builtin_ctzll(any);
+        any &= any - 1;
+        bits = (uint64_t)(unsigned)__builtin_amdgcn_readlane((int)(rest & 0xffffffffu), src) |
+               (uint64_t)(unsigned)__builtin_amdgcn_readlane((int)(rest >> 32), src) << 32;
+        return true;
+    }
+    __device__ __forceinline__ void start(int skip)
+    {
+        wb = 0;
+        bits = 0;
+        block();
+        while (word()) {
+            const int c = __builtin_popcountll(bits);
+            if (c > skip) break;
+            skip -= c;
+        }
+        for (; skip > 0; --skip) bits &= bits - 1;
+    }
+    // The next column chunk (the caller knows how many are left).
+    __device__ __forceinline__ int next()
+    {
+        if (!bits) word();
+        const int c = (wb + src) * 64 + __builtin_ctzll(bits);
+        bits &= bits - 1;
+        return c;
+    }
+};
+
+// Row chunk of segment g (seg: SymArgs::seg, the first segment of each row).
+__device__ __forceinline__ int segment_row(const int *seg, int nchunks, int g)
+{
+    int ci = 0;   // the last row whose first segment is not after g
+    for (int hi = nchunks - 1; ci < hi;) {
+        const int mid = (ci + hi + 1) / 2;
+        if (seg[mid] <= g) ci = mid;
+        else hi = mid - 1;
+    }
+    return uniform_i(ci);
+}
+
+// Number of unset bits of a row.
+__device__ __forceinline__ int rest_total(const uint64_t *row, int nchunks, int words)
+{
+    int total = 0;
+    for (int wb = 0; wb < words; wb += 64) {
+        const int k = wb + (threadIdx.x & 63);
+        if (k < words) total += __builtin_popcountll(row[k]);
+    }
+    for (int o = 32; o > 0; o >>= 1) total += __shfl_xor(total, o, 64);
+    return nchunks - uniform_i(total);
+}
+
 }  // namespace sg

@@ -960,7 +960,7 @@ constexpr int NSOFT = 1024;   // listed pairs; a visit with more has enough on e
 struct WaveLds {
     NearSlice sl;
     uint16_t list[NSOFT];     // i lane << 6 | j
-    double res[4][64];        // sums of one pair per lane
+    double res[5][64];        // sums of one pair per lane (ax, ay, az, pot, psi)
 };
 
 __device__ __forceinline__ void rsq_group(const float (&r2)[PG], float (&ri)[PG])
@@ -984,7 +984,8 @@ struct Fold4 {
         z = fmaf(mr3, dz, z);
         p += mr;
     }
-    __device__ __forceinline__ void to(double (&acc)[4]) const
+    template <int N>
+    __device__ __forceinline__ void to(double (&acc)[N]) const
     {
         acc[0] += (double)x;
         acc[1] += (double)y;
@@ -1034,7 +1035,7 @@ __device__ __forceinline__ void cubic_AP(double q, double invq, double &A, doubl
 // r -> 0 limit.
 template <int NK>
 __device__ __forceinline__ void side_select(double r, double ri, double r2, double H, double invH,
-                                            double &gacc, double &gpot)
+                                            double &gacc, double &gpot, double *ps = nullptr)
 {
     const double q = r * invH;
     double A, P;
@@ -1043,22 +1044,24 @@ __device__ __forceinline__ void side_select(double r, double ri, double r2, doub
     const bool soft = r2 <= H * H;
     gacc += soft ? A * invH * invH * invH : ri * ri * ri;
     gpot += soft ? P * invH : -ri;
+    if (ps) *ps = soft ? fma(q * q, A, P) : 0.0;
 }
 
 // near_pair for a pair that is (or within rounding of being) softened, with
 // no branch: dealt over the lanes such pairs take different ones, and a wave
-// would walk them all.  dead: the self pair of a point particle.
-template <int NK>
+// would walk them all.  dead: the self pair of a point particle.  With PSI
+// f[4] is m_j (P(q_i) + q_i^2 A(q_i)) where r <= H_i, as in near_pair.
+template <int NK, bool PSI>
 __device__ __forceinline__ void soft_pair(double dx, double dy, double dz, double Hi, double invHi,
                                           double Hj, double invHj, double mj, bool dead,
-                                          double (&f)[4])
+                                          double (&f)[PSI ? 5 : 4])
 {
     const double r2 = fma(dx, dx, fma(dy, dy, dz * dz));
     const bool apart = r2 > 0.0;
     const double ri = apart ? rsqrt64<true>(apart ? r2 : 1.0) : 0.0;
     const double r = r2 * ri;
-    double gacc = 0.0, gpot = 0.0;
-    side_select<NK>(r, ri, r2, Hi, invHi, gacc, gpot);
+    double gacc = 0.0, gpot = 0.0, ps = 0.0;
+    side_select<NK>(r, ri, r2, Hi, invHi, gacc, gpot, PSI ? &ps : nullptr);
     side_select<NK>(r, ri, r2, Hj, invHj, gacc, gpot);
     const double hm = dead ? 0.0 : 0.5 * mj;
     const double g = hm * gacc;
@@ -1066,6 +1069,7 @@ __device__ __forceinline__ void soft_pair(double dx, double dy, double dz, doubl
     f[1] = g * dy;
     f[2] = g * dz;
     f[3] = hm * gpot;
+    if (PSI) f[PSI ? 4 : 0] = mj * ps;
 }
 
 // The visits below cover j = jb .. je - 1 of the staged chunk (multiples of
@@ -1074,13 +1078,15 @@ __device__ __forceinline__ void soft_pair(double dx, double dy, double dz, doubl
 // FP32, r = 0 included), and those in FP64.  A lane has few of them and the
 // busiest several times the mean, and one costs some 300 dependent FP64
 // operations, so they are dealt over all lanes, 64 at a time, and each lane
-// collects the sums of its own.
-template <int NK>
+// collects the sums of its own.  PSI also forms the grad-h sum (acc[4]).
+template <int NK, bool PSI>
 __device__ __forceinline__ void visit_near(WaveLds &lds, uint64_t real, const SortedSet &J,
                                            int64_t j0c, int jb, int je, double xr, double yr, double zr, double Hi,
-                                           double invHi, double hi2, int idi, double (&acc)[4],
+                                           double invHi, double hi2, int idi,
+                                           double (&acc)[PSI ? 5 : 4],
                                            unsigned &nfp64)
 {
+    constexpr int NS = PSI ? 5 : 4;
     const NearSlice &sl = lds.sl;
     const float hi2f = (float)hi2;
     uint64_t mine = 0;   // bit 63 - jj: the lane's pair with jj is softened
@@ -1134,10 +1140,10 @@ __device__ __forceinline__ void visit_near(WaveLds &lds, uint64_t real, const So
             const double dx = p.x - xr, dy = p.y - yr, dz = p.z - zr;
             // the self pair only matters at r = 0: the index is read then
             const bool dead = dx == 0.0 && dy == 0.0 && dz == 0.0 && hs < 0.0 && J.idx[j0c + jj] == idi;
-            double f[4];
-            soft_pair<NK>(dx, dy, dz, Hi, invHi, fabs(hs), sl.hinv[jj], sl.m[jj], dead, f);
+            double f[NS];
+            soft_pair<NK, PSI>(dx, dy, dz, Hi, invHi, fabs(hs), sl.hinv[jj], sl.m[jj], dead, f);
 #pragma unroll
-            for (int k = 0; k < 4; ++k) acc[k] += f[k];
+            for (int k = 0; k < NS; ++k) acc[k] += f[k];
         }
         return;
     }
@@ -1158,23 +1164,24 @@ __device__ __forceinline__ void visit_near(WaveLds &lds, uint64_t real, const So
         const double dx = p.x - __shfl(xr, il, 64), dy = p.y - __shfl(yr, il, 64),
                      dz = p.z - __shfl(zr, il, 64);
         const bool dead = dx == 0.0 && dy == 0.0 && dz == 0.0 && hs < 0.0 && J.idx[j0c + jj] == id;
-        double f[4];
-        soft_pair<NK>(dx, dy, dz, H, invH, fabs(hs), sl.hinv[jj], sl.m[jj], dead, f);
+        double f[NS];
+        soft_pair<NK, PSI>(dx, dy, dz, H, invH, fabs(hs), sl.hinv[jj], sl.m[jj], dead, f);
 #pragma unroll
-        for (int k = 0; k < 4; ++k) lds.res[k][lane] = f[k];
+        for (int k = 0; k < NS; ++k) lds.res[k][lane] = f[k];
         wave_lds_sync();
         // each lane adds its own pairs, in the list's order
         const unsigned hi = min(at + count, b0 + 64);
         for (unsigned k = max(at, b0); k < hi; ++k) {
 #pragma unroll
-            for (int c = 0; c < 4; ++c) acc[c] += lds.res[c][k - b0];
+            for (int c = 0; c < NS; ++c) acc[c] += lds.res[c][k - b0];
         }
     }
 }
 
 // Wide: as near, with every pair Newtonian.
+template <int N>
 __device__ __forceinline__ void visit_wide(const NearSlice &sl, int jb, int je, double xr, double yr,
-                                           double zr, double (&acc)[4])
+                                           double zr, double (&acc)[N])
 {
 #pragma unroll 1
     for (int f = jb; f < je; f += FOLD) {
@@ -1201,8 +1208,9 @@ __device__ __forceinline__ void visit_wide(const NearSlice &sl, int jb, int je, 
 }
 
 // Far: differences of FP32 positions relative to O.
+template <int N>
 __device__ __forceinline__ void visit_far(const float4 *s_hi, int jb, int je, float xh, float yh,
-                                          float zh, double (&acc)[4])
+                                          float zh, double (&acc)[N])
 {
 #pragma unroll 1
     for (int f = jb; f < je; f += FOLD) {
@@ -1233,7 +1241,7 @@ __device__ __forceinline__ void visit_far(const float4 *s_hi, int jb, int je, fl
 // (strided chunks, or parts of them), so that a few thousand particles still
 // make thousands of waves and a wave's near chunks are few.  The next chunk's
 // particles are loaded while the current one is evaluated.
-template <int NK>
+template <int NK, bool PSI>
 __global__ __launch_bounds__(64) void k_pair_wave(PairArgs a)
 {
     __shared__ WaveLds lds;
@@ -1253,7 +1261,7 @@ __global__ __launch_bounds__(64) void k_pair_wave(PairArgs a)
     near_i_state<1>(a.i, ii, Hi, invHi, hi2, idi);
     const float px = (float)xr, py = (float)yr, pz = (float)zr, ph = (float)Hi[0];
     const float rho2 = fmaf(px, px, fmaf(py, py, pz * pz));
-    double acc[4] = {0.0, 0.0, 0.0, 0.0};
+    double acc[PSI ? 5 : 4] = {};
     unsigned nfp64 = 0, visits = 0, nearv = 0, widev = 0;
     // partition jp: part jp % jsub of every (jsplit / jsub)-th chunk
     const int stride = a.jsplit / a.jsub, first = jp / a.jsub;
@@ -1284,7 +1292,7 @@ __global__ __launch_bounds__(64) void k_pair_wave(PairArgs a)
         ++visits;
         if (v == VISIT_NEAR) {
             ++nearv;
-            visit_near<NK>(lds, real, a.j, j0c, jb, je, xr, yr, zr, Hi[0], invHi[0], hi2[0], idi[0], acc, nfp64);
+            visit_near<NK, PSI>(lds, real, a.j, j0c, jb, je, xr, yr, zr, Hi[0], invHi[0], hi2[0], idi[0], acc, nfp64);
         } else if (v == VISIT_WIDE) {
             ++widev;
             visit_wide(sl, jb, je, xr, yr, zr, acc);
@@ -1296,6 +1304,10 @@ __global__ __launch_bounds__(64) void k_pair_wave(PairArgs a)
         double *part = a.partial + (int64_t)jp * 4 * a.ni + ii[0];
 #pragma unroll
         for (int k = 0; k < 4; ++k) part[k * a.ni] = acc[k];
+        // point particles (negative H) carry no psi (advance.f90:750-753)
+        if (PSI)
+            a.psipart[(int64_t)jp * a.ni + ii[0]] =
+                a.i.Hs[ii[0]] > 0.0 ? -2.0 * invHi[0] * invHi[0] * acc[PSI ? 4 : 0] : 0.0;
     }
     if (a.stats) {
         const unsigned long long fw = wave_sum_count(valid ? nfp64 : 0u);
@@ -1312,57 +1324,6 @@ __global__ __launch_bounds__(64) void k_pair_wave(PairArgs a)
 }
 
 // ------------------------------------------- ordered rest of a whole-set pass
-// The unset bits of one row of SymArgs::sym from the k-th on, in order.
-struct RestBits {
-    const uint64_t *row;
-    int nchunks, words, wb, src;
-    uint64_t rest, any, bits;   // rest: per lane; the others wave-uniform
-
-    __device__ __forceinline__ void block()
-    {
-        const int k = wb + (threadIdx.x & 63);
-        rest = 0;
-        if (k < words) {
-            const int left = nchunks - k * 64;
-            rest = ~row[k] & (left >= 64 ? ~0ull : (1ull << left) - 1ull);
-        }
-        any = __ballot(rest != 0);
-    }
-    __device__ __forceinline__ bool word()
-    {
-        while (!any) {
-            wb += 64;
-            if (wb >= words) return false;
-            block();
-        }
-        src = __builtin_ctzll(any);
-        any &= any - 1;
-        bits = (uint64_t)(unsigned)__builtin_amdgcn_readlane((int)(rest & 0xffffffffu), src) |
-               (uint64_t)(unsigned)__builtin_amdgcn_readlane((int)(rest >> 32), src) << 32;
-        return true;
-    }
-    __device__ __forceinline__ void start(int skip)
-    {
-        wb = 0;
-        bits = 0;
-        block();
-        while (word()) {
-            const int c = __builtin_popcountll(bits);
-            if (c > skip) break;
-            skip -= c;
-        }
-        for (; skip > 0; --skip) bits &= bits - 1;
-    }
-    // The next column chunk (the caller knows how many are left).
-    __device__ __forceinline__ int next()
-    {
-        if (!bits) word();
-        const int c = (wb + src) * 64 + __builtin_ctzll(bits);
-        bits &= bits - 1;
-        return c;
-    }
-};
-
 // The (row chunk, column chunk) visits that k_sym leaves (bits unset in
 // a.sym): near chunks and those too close to the row chunk for hi-only
 // differences.  One wave per segment of a row's visits, so that the rows that
@@ -1377,13 +1338,7 @@ __global__ __launch_bounds__(64) void k_sym_rest(SymArgs a)
     const int lane = threadIdx.x;
     const int g = (int)blockIdx.x;
     if (g >= a.seg[a.nchunks]) return;
-    int ci = 0;   // the last row whose first segment is not after g
-    for (int hi = a.nchunks - 1; ci < hi;) {
-        const int mid = (ci + hi + 1) / 2;
-        if (a.seg[mid] <= g) ci = mid;
-        else hi = mid - 1;
-    }
-    ci = uniform_i(ci);
+    const int ci = segment_row(a.seg, a.nchunks, g);
     const int len = uniform_i(a.seg[a.nchunks + 1]);
     const int k0 = uniform_i(g - a.seg[ci]) * len;
     const SortedSet &P = a.p;
@@ -1405,17 +1360,8 @@ __global__ __launch_bounds__(64) void k_sym_rest(SymArgs a)
     it.row = a.sym + (int64_t)ci * a.words;
     it.nchunks = a.nchunks;
     it.words = a.words;
-    int left = 0;   // visits of this segment
-    {
-        // the row's last segment is the short one
-        int total = 0;
-        for (int wb = 0; wb < a.words; wb += 64) {
-            const int k = wb + lane;
-            if (k < a.words) total += __builtin_popcountll(it.row[k]);
-        }
-        for (int o = 32; o > 0; o >>= 1) total += __shfl_xor(total, o, 64);
-        left = min(len, a.nchunks - uniform_i(total) - k0);
-    }
+    // visits of this segment: a row's last one is the short one
+    int left = min(len, rest_total(it.row, a.nchunks, a.words) - k0);
     it.start(k0);
     int cj = it.next();
     double jx = P.x[(int64_t)cj * TC + lane], jy = P.y[(int64_t)cj * TC + lane],
@@ -1446,7 +1392,7 @@ __global__ __launch_bounds__(64) void k_sym_rest(SymArgs a)
         }
         if (v == VISIT_NEAR) {
             ++nearv;
-            visit_near<NK>(lds, real, P, j0c, 0, TC, xr, yr, zr, Hi[0], invHi[0], hi2[0], idi[0], acc, nfp64);
+            visit_near<NK, false>(lds, real, P, j0c, 0, TC, xr, yr, zr, Hi[0], invHi[0], hi2[0], idi[0], acc, nfp64);
         } else if (v == VISIT_WIDE) {
             ++widev;
             visit_wide(sl, 0, TC, xr, yr, zr, acc);
@@ -1777,11 +1723,26 @@ static hipError_t far_fused_launch(const PairArgs &a, hipStream_t s)
     return hipGetLastError();
 }
 
-// FP32C: the fused far kernel (no near kernel follows), or, with the grad-h
-// term, the split far kernel with one i per lane.  FP64: the far kernel.
+template <bool PSI>
+static hipError_t wave_launch(const PairArgs &a, hipStream_t s)
+{
+    const dim3 grid((unsigned)((a.ni + TC - 1) / TC) * (unsigned)a.jsplit), block(64);
+    switch (a.nkernel) {
+    case 0: hipLaunchKernelGGL((k_pair_wave<0, PSI>), grid, block, 0, s, a); break;
+    case 1: hipLaunchKernelGGL((k_pair_wave<1, PSI>), grid, block, 0, s, a); break;
+    case 2: hipLaunchKernelGGL((k_pair_wave<2, PSI>), grid, block, 0, s, a); break;
+    default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
+}
+
+// FP32C: one wave per 64 i and j partition (a.wave), else the fused far kernel
+// (no near kernel follows either), or, with the grad-h term, the split far
+// kernel with one i per lane.  FP64: the far kernel.
 hipError_t launch_pair_far(int precision, const PairArgs &a, int wg, hipStream_t s)
 {
     if (a.ni <= 0) return hipSuccess;
+    if (precision == 0 && a.wave) return a.psi ? wave_launch<true>(a, s) : wave_launch<false>(a, s);
     if (precision == 0 && a.psi) {
         if (a.ipl != 1) return hipErrorInvalidConfiguration;
         switch (wg) {
@@ -1789,16 +1750,6 @@ hipError_t launch_pair_far(int precision, const PairArgs &a, int wg, hipStream_t
         case 128: hipLaunchKernelGGL((k_far_fp32c_split<128>), grid_of(a), dim3(128), 0, s, a); break;
         case 256: hipLaunchKernelGGL((k_far_fp32c_split<256>), grid_of(a), dim3(256), 0, s, a); break;
         default: return hipErrorInvalidConfiguration;
-        }
-        return hipGetLastError();
-    }
-    if (precision == 0 && a.wave) {
-        const dim3 grid((unsigned)((a.ni + TC - 1) / TC) * (unsigned)a.jsplit), block(64);
-        switch (a.nkernel) {
-        case 0: hipLaunchKernelGGL((k_pair_wave<0>), grid, block, 0, s, a); break;
-        case 1: hipLaunchKernelGGL((k_pair_wave<1>), grid, block, 0, s, a); break;
-        case 2: hipLaunchKernelGGL((k_pair_wave<2>), grid, block, 0, s, a); break;
-        default: return hipErrorInvalidValue;
         }
         return hipGetLastError();
     }
@@ -1843,6 +1794,7 @@ hipError_t launch_pair_near(int precision, const PairArgs &a, hipStream_t s)
 {
     if (a.ni <= 0) return hipSuccess;
     if (a.nkernel < 0 || a.nkernel > 2) return hipErrorInvalidValue;
+    if (precision == 0 && a.wave) return hipSuccess;   // its waves take the near chunks
     const dim3 grid((unsigned)(a.ngroups * a.jsplit)), block(64 * NEAR_WAVES);
     if (a.psi) {
         if (a.ipl != 1) return hipErrorInvalidConfiguration;

@@ -543,22 +543,361 @@ __global__ __launch_bounds__(64 * ANEAR_WAVES) void k_adj_near(AdjArgs a)
     part[4 * a.n + i] += g[8];
 }
 
-// Fixed-order FP64 sum over the j-partitions, scattered to input order.
+// ------------------------------------------------- one wave, one column chunk
+// LDS of a wave: the staged chunk, and its pairs in FP64 dealt evenly over the
+// lanes.
+constexpr int ANLIST = 1024;   // listed pairs; a visit with more has enough on every lane
+struct AdjWaveLds {
+    double4 p[ACHUNK];   // x, y, z relative to the origin; m
+    double4 w[ACHUNK];   // wx, wy, wz, u
+    double2 h[ACHUNK];   // signed H, original index
+    float4 wf[ACHUNK];   // wx, wy, wz, u in FP32
+    float2 mf[ACHUNK];   // m, H^2 in FP32
+    uint16_t list[ANLIST];   // i lane << 6 | j
+    double res[9][64];       // sums of one pair per lane
+};
+
+// adj_side without a branch: the polynomials, or the Newtonian terms beyond H
+// (ri = 0 at r = 0 gives the r -> 0 limit).
+template <int NK>
+__device__ __forceinline__ void adj_side_select(double r, double ri, double r2, double H,
+                                                double invH, Side &s)
+{
+    const double q = r * invH, iq = H * ri;
+    double A, P, Aq;
+    if (NK == 0) {
+        cubic_AP(q, iq, A, P);
+        const double iq2 = iq * iq;
+        const double in = 96.0 * q - 76.8;
+        const double out = (-48.0 + q * (76.8 - 32.000000000001 * q) + 0.200000000001 * iq2 * iq2) * iq;
+        Aq = q < 0.5 ? in : out;
+    } else {
+        poly_AP(NK, q, iq, A, P);
+        Aq = poly_Aq(NK, q, iq);
+    }
+    const bool soft = r2 <= H * H;
+    const double iH2 = invH * invH, iH3 = iH2 * invH, ri2 = ri * ri, ri3 = ri2 * ri;
+    s.F = soft ? A * iH3 : ri3;
+    s.P = soft ? P * invH : -ri;
+    s.Fr = soft ? Aq * iH3 * iH2 : -3.0 * ri3 * ri2;
+    s.FH = soft ? -fma(q * q, Aq, 3.0 * A) * iH2 * iH2 : 0.0;
+    s.PH = soft ? -fma(q * q, A, P) * iH2 : 0.0;
+}
+
+// adj_pair64 with no branch, for pairs dealt over the lanes.  The self pair
+// (same) keeps its potential terms only, none for a point particle.
+template <int NK>
+__device__ __forceinline__ void adj_pair_select(double dx, double dy, double dz, double Hk,
+                                                double invHk, double mk, double wkx, double wky,
+                                                double wkz, double uk, double Hl, double ml,
+                                                double wlx, double wly, double wlz, double ul,
+                                                bool same, bool gas, Acc9 &g)
+{
+    const double r2 = fma(dx, dx, fma(dy, dy, dz * dz));
+    const bool apart = r2 > 0.0;
+    const double ri = apart ? rsqrt64<true>(apart ? r2 : 1.0) : 0.0;
+    const double r = r2 * ri;
+    Side sk, sl;
+    adj_side_select<NK>(r, ri, r2, Hk, invHk, sk);
+    adj_side_select<NK>(r, ri, r2, Hl, 1.0 / Hl, sl);
+    const double half = same && !gas ? 0.0 : 0.5;
+    const double F = same ? 0.0 : half * (sk.F + sl.F);
+    const double P = half * (sk.P + sl.P), Fr = half * (sk.Fr + sl.Fr);
+    const double wkdr = fma(wkx, dx, fma(wky, dy, wkz * dz));
+    const double wldr = fma(wlx, dx, fma(wly, dy, wlz * dz));
+    const double t = fma(ml, wkdr, -mk * wldr);
+    const double s = fma(ml, uk, mk * ul);
+    const double c = -fma(Fr, t, F * s);
+    g[0] = F * wlx;
+    g[1] = F * wly;
+    g[2] = F * wlz;
+    g[3] = F * ml;
+    g[4] = c * dx;
+    g[5] = c * dy;
+    g[6] = c * dz;
+    g[7] = fma(ul, P, -F * wldr);
+    g[8] = half * fma(sk.FH, t, sk.PH * s);
+}
+
+// The i side of a lane.
+struct AdjLane {
+    double x, y, z, m, wx, wy, wz, u, H, invH;
+    bool gas;
+    int id;
+    Lane32 q;      // FP32 (positions unused)
+    float px, py, pz, ph;
+};
+
+__device__ __forceinline__ void adj_lane(const SortedSet &P, const double *wx, const double *wy,
+                                         const double *wz, const double *u, int64_t i, double Ox,
+                                         double Oy, double Oz, AdjLane &l)
+{
+    l.x = P.x[i] - Ox;
+    l.y = P.y[i] - Oy;
+    l.z = P.z[i] - Oz;
+    l.m = P.m[i];
+    l.wx = wx[i];
+    l.wy = wy[i];
+    l.wz = wz[i];
+    l.u = u[i];
+    const double Hs = P.Hs[i];
+    l.H = fabs(Hs);
+    l.invH = 1.0 / l.H;
+    l.gas = Hs > 0.0;
+    l.id = P.idx[i];
+    l.q.xh = l.q.yh = l.q.zh = l.q.xl = l.q.yl = l.q.zl = 0.0f;
+    l.q.m = (float)l.m;
+    l.q.wx = (float)l.wx;
+    l.q.wy = (float)l.wy;
+    l.q.wz = (float)l.wz;
+    l.q.u = (float)l.u;
+    l.q.h2 = (float)(l.H * l.H);
+    l.px = (float)l.x;
+    l.py = (float)l.y;
+    l.pz = (float)l.z;
+    l.ph = (float)l.H;
+}
+
+// Whether some lane's pairs with the chunk of box and largest H cm may be
+// softened.
+__device__ __forceinline__ bool adj_chunk_near(const TileMeta &cm, double Ox, double Oy, double Oz,
+                                               const AdjLane &l)
+{
+    const float gx = fmaxf(0.0f, fmaxf((float)(cm.lo[0] - Ox) - l.px, l.px - (float)(cm.hi[0] - Ox)));
+    const float gy = fmaxf(0.0f, fmaxf((float)(cm.lo[1] - Oy) - l.py, l.py - (float)(cm.hi[1] - Oy)));
+    const float gz = fmaxf(0.0f, fmaxf((float)(cm.lo[2] - Oz) - l.pz, l.pz - (float)(cm.hi[2] - Oz)));
+    const float hm = fmaxf(l.ph, (float)cm.maxH);
+    return __ballot(!(fmaf(gx, gx, fmaf(gy, gy, gz * gz)) > hm * hm * (1.0f + FAR_MARGIN))) != 0;
+}
+
+__device__ __forceinline__ void adj_stage(AdjWaveLds &lds, double rx, double ry, double rz, double m,
+                                          double hs, int idx, double wx, double wy, double wz, double u)
+{
+    const int lane = threadIdx.x & 63;
+    wave_lds_sync();
+    lds.p[lane] = make_double4(rx, ry, rz, m);
+    lds.w[lane] = make_double4(wx, wy, wz, u);
+    lds.h[lane] = make_double2(hs, (double)idx);
+    lds.wf[lane] = make_float4((float)wx, (float)wy, (float)wz, (float)u);
+    lds.mf[lane] = make_float2((float)m, (float)(hs * hs));
+    wave_lds_sync();
+}
+
+// The staged chunk: Newtonian pairs in FP32 on FP64-formed differences, four
+// at a time (their v_rsq_f32 together at raised wave priority, sg_sym.hip);
+// NEAR: softened, self and coincident pairs and those within the margin of a
+// support in FP64, dealt over the lanes 64 at a time (a lane has few, the
+// busiest several times the mean), each lane collecting the sums of its own.
+template <int NK, bool NEAR>
+__device__ __forceinline__ void adj_visit(AdjWaveLds &lds, const AdjLane &l, Acc9 &g)
+{
+    constexpr int PG = 4;
+    uint64_t own = 0;
+#pragma unroll 1
+    for (int f0 = 0; f0 < ACHUNK; f0 += AFOLD) {
+        float f[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 1
+        for (int j0 = f0; j0 < f0 + AFOLD; j0 += PG) {
+            float dx[PG], dy[PG], dz[PG], m[PG], r2[PG], ri[PG];
+#pragma unroll
+            for (int k = 0; k < PG; ++k) {
+                const double4 p = lds.p[j0 + k];
+                const float2 mh = lds.mf[j0 + k];
+                dx[k] = (float)(p.x - l.x);
+                dy[k] = (float)(p.y - l.y);
+                dz[k] = (float)(p.z - l.z);
+                m[k] = mh.x;
+                const float q = fmaf(dx[k], dx[k], fmaf(dy[k], dy[k], dz[k] * dz[k]));
+                const bool newton = !NEAR || q > fmaxf(l.q.h2, mh.y) * (1.0f + FAR_MARGIN);
+                r2[k] = newton ? q : INFINITY;
+                if (NEAR) own |= (uint64_t)(newton ? 0u : 1u) << (j0 + k);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            __builtin_amdgcn_s_setprio(3);
+#pragma unroll
+            for (int k = 0; k < PG; ++k) ri[k] = __builtin_amdgcn_rsqf(r2[k]);
+            __builtin_amdgcn_s_setprio(0);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int k = 0; k < PG; ++k)
+                adj_newton_fp32(dx[k], dy[k], dz[k], ri[k], m[k], lds.wf[j0 + k], l.q, f);
+        }
+#pragma unroll
+        for (int c = 0; c < 7; ++c) g[c] += (double)f[c];
+        g[7] -= (double)f[7];
+    }
+    if (!NEAR) return;
+    const int lane = threadIdx.x & 63;
+    const unsigned count = (unsigned)__builtin_popcountll(own);
+    unsigned at, total;
+    list_places(count, at, total);
+    if (total > (unsigned)ANLIST) {
+        while (own) {
+            const int jj = __builtin_ctzll(own);
+            own &= own - 1;
+            const double4 p = lds.p[jj], c = lds.w[jj];
+            const double2 h = lds.h[jj];
+            Acc9 f;
+            adj_pair_select<NK>(p.x - l.x, p.y - l.y, p.z - l.z, l.H, l.invH, l.m, l.wx, l.wy, l.wz,
+                                l.u, fabs(h.x), p.w, c.x, c.y, c.z, c.w, (int)h.y == l.id, l.gas, f);
+            for (int k = 0; k < 9; ++k) g[k] += f[k];
+        }
+        return;
+    }
+    for (unsigned k = at; own; ++k) {
+        const int jj = __builtin_ctzll(own);
+        own &= own - 1;
+        lds.list[k] = (uint16_t)(lane << 6 | jj);
+    }
+    for (unsigned b0 = 0; b0 < total; b0 += 64) {
+        wave_lds_sync();
+        const unsigned e = min(b0 + (unsigned)lane, total - 1);   // lanes past the end repeat the last
+        const int il = lds.list[e] >> 6, jj = lds.list[e] & 63;
+        const double4 p = lds.p[jj], c = lds.w[jj];
+        const double2 h = lds.h[jj];
+        Acc9 f;
+        adj_pair_select<NK>(p.x - __shfl(l.x, il, 64), p.y - __shfl(l.y, il, 64),
+                            p.z - __shfl(l.z, il, 64), __shfl(l.H, il, 64), __shfl(l.invH, il, 64),
+                            __shfl(l.m, il, 64), __shfl(l.wx, il, 64), __shfl(l.wy, il, 64),
+                            __shfl(l.wz, il, 64), __shfl(l.u, il, 64), fabs(h.x), p.w, c.x, c.y, c.z,
+                            c.w, (int)h.y == __shfl(l.id, il, 64), h.x > 0.0, f);
+#pragma unroll
+        for (int k = 0; k < 9; ++k) lds.res[k][lane] = f[k];
+        wave_lds_sync();
+        const unsigned hi = min(at + count, b0 + 64);
+        for (unsigned k = max(at, b0); k < hi; ++k) {
+#pragma unroll
+            for (int v = 0; v < 9; ++v) g[v] += lds.res[v][k - b0];
+        }
+    }
+}
+
+// The visits that k_adj_sym leaves, one wave per segment (k_sym_rest's).  Three
+// waves a SIMD (168 VGPRs, 30 spilled outside the pair loops) instead of the two
+// the compiler takes: 2.27 -> 2.12 ms at 131,072 particles, and 0.41 -> 0.37 ms
+// for k_adj_wave at 16,384.
+template <int NK>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3)))
+void k_adj_rest(AdjSymArgs a)
+{
+    __shared__ AdjWaveLds lds;
+    const SymArgs &y = a.y;
+    const SortedSet &P = y.p;
+    const int lane = threadIdx.x;
+    const int s = (int)blockIdx.x;
+    if (s >= y.seg[y.nchunks]) return;
+    const int ci = segment_row(y.seg, y.nchunks, s);
+    const int len = uniform_i(y.seg[y.nchunks + 1]);
+    const int k0 = uniform_i(s - y.seg[ci]) * len;
+    const int64_t gbase = (int64_t)ci * TC;
+    const int64_t io = min(gbase + TC / 2, y.n - 1);
+    const double Ox = P.x[io], Oy = P.y[io], Oz = P.z[io];
+    AdjLane l;
+    adj_lane(P, a.wx, a.wy, a.wz, a.u, min(gbase + lane, y.n - 1), Ox, Oy, Oz, l);
+    Acc9 g = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+    RestBits it;
+    it.row = y.sym + (int64_t)ci * y.words;
+    it.nchunks = y.nchunks;
+    it.words = y.words;
+    int left = min(len, rest_total(it.row, y.nchunks, y.words) - k0);
+    unsigned visits = 0, nearv = 0;
+    it.start(k0);
+    for (; left > 0; --left) {
+        const int cj = it.next();
+        const int64_t j = (int64_t)cj * TC + lane;
+        const bool near = adj_chunk_near(y.chunks[cj], Ox, Oy, Oz, l);
+        adj_stage(lds, P.x[j] - Ox, P.y[j] - Oy, P.z[j] - Oz, P.m[j], P.Hs[j], P.idx[j], a.wx[j],
+                  a.wy[j], a.wz[j], a.u[j]);
+        ++visits;
+        if (near) {
+            ++nearv;
+            adj_visit<NK, true>(lds, l, g);
+        } else {
+            adj_visit<NK, false>(lds, l, g);
+        }
+    }
+    double *out = y.segsum + (int64_t)s * 5 * TC + lane;
+    out[0] = l.m * g[0] - l.wx * g[3] + g[4];
+    out[TC] = l.m * g[1] - l.wy * g[3] + g[5];
+    out[2 * TC] = l.m * g[2] - l.wz * g[3] + g[6];
+    out[3 * TC] = g[7];
+    out[4 * TC] = g[8];
+    if (y.stats && lane == 0) {
+        unsigned long long *st = stat_copy(y.stats);
+        atomicAdd(&st[0], (unsigned long long)visits);
+        atomicAdd(&st[1], (unsigned long long)nearv);
+    }
+}
+
+// Small sets: one wave per 64 i and j partition (every jsplit-th chunk).
+template <int NK>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3)))
+void k_adj_wave(AdjArgs a)
+{
+    __shared__ AdjWaveLds lds;
+    const SortedSet &P = a.p;
+    const int lane = threadIdx.x;
+    const unsigned nic = (unsigned)((a.n + TC - 1) / TC);
+    const int ci = (int)(blockIdx.x % nic), jp = (int)(blockIdx.x / nic);
+    const int nchunks = a.ntiles * CHUNKS;
+    const int64_t gbase = (int64_t)ci * TC;
+    const int64_t io = min(gbase + TC / 2, a.n - 1);
+    const double Ox = P.x[io], Oy = P.y[io], Oz = P.z[io];
+    const bool valid = gbase + lane < a.n;
+    const int64_t i = valid ? gbase + lane : a.n - 1;
+    AdjLane l;
+    adj_lane(P, a.wx, a.wy, a.wz, a.u, i, Ox, Oy, Oz, l);
+    Acc9 g = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+    unsigned visits = 0, nearv = 0;
+    for (int cj = jp; cj < nchunks; cj += a.jsplit) {
+        const int64_t j = (int64_t)cj * TC + lane;
+        const bool near = adj_chunk_near(a.chunks[cj], Ox, Oy, Oz, l);
+        adj_stage(lds, P.x[j] - Ox, P.y[j] - Oy, P.z[j] - Oz, P.m[j], P.Hs[j], P.idx[j], a.wx[j],
+                  a.wy[j], a.wz[j], a.u[j]);
+        ++visits;
+        if (near) {
+            ++nearv;
+            adj_visit<NK, true>(lds, l, g);
+        } else {
+            adj_visit<NK, false>(lds, l, g);
+        }
+    }
+    if (valid) {
+        double *part = a.partial + (int64_t)jp * 5 * a.n;
+        part[i] = l.m * g[0] - l.wx * g[3] + g[4];
+        part[a.n + i] = l.m * g[1] - l.wy * g[3] + g[5];
+        part[2 * a.n + i] = l.m * g[2] - l.wz * g[3] + g[6];
+        part[3 * a.n + i] = g[7];
+        part[4 * a.n + i] = g[8];
+    }
+    if (a.stats && lane == 0) {
+        unsigned long long *st = stat_copy(a.stats);
+        atomicAdd(&st[0], (unsigned long long)visits);
+        atomicAdd(&st[1], (unsigned long long)nearv);
+    }
+}
+
+// Fixed-order FP64 sum over the j-partitions, scattered to input order: a block
+// takes 64 particles of one gradient (blockIdx.y), each of its waves a quarter
+// of the partitions.
 __global__ __launch_bounds__(256) void k_adj_reduce(AdjArgs a)
 {
-    const int64_t i = blockIdx.x * (int64_t)256 + threadIdx.x;
-    if (i >= a.n) return;
-    double s[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-    for (int jp = 0; jp < a.jsplit; ++jp) {
-        const double *p = a.partial + (int64_t)jp * 5 * a.n;
-        for (int c = 0; c < 5; ++c) s[c] += p[c * a.n + i];
+    __shared__ double s_sum[4][64];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int64_t i = blockIdx.x * (int64_t)64 + lane;
+    const int c = blockIdx.y;
+    double s = 0.0;
+    if (i < a.n) {
+        const double *p = a.partial + c * a.n + i;
+        const int end = a.jsplit * (w + 1) / 4;
+#pragma unroll 8
+        for (int jp = a.jsplit * w / 4; jp < end; ++jp) s += p[(int64_t)jp * 5 * a.n];
     }
-    const int o = a.p.idx[i];
-    a.gx[o] = s[0];
-    a.gy[o] = s[1];
-    a.gz[o] = s[2];
-    a.gm[o] = s[3];
-    a.gH[o] = s[4];
+    s_sum[w][lane] = s;
+    __syncthreads();
+    if (w != 0 || i >= a.n) return;
+    double *out = c == 0 ? a.gx : (c == 1 ? a.gy : (c == 2 ? a.gz : (c == 3 ? a.gm : a.gH)));
+    out[a.p.idx[i]] = s + s_sum[1][lane] + s_sum[2][lane] + s_sum[3][lane];
 }
 
 }  // namespace
@@ -617,10 +956,35 @@ hipError_t launch_adj_near(int precision, const AdjArgs &a, hipStream_t s)
     return hipGetLastError();
 }
 
+hipError_t launch_adj_sym_rest(const AdjSymArgs &a, hipStream_t s)
+{
+    // as many waves as there can be segments; those past the last one end at once
+    const dim3 grid((unsigned)(SYM_SEGS + a.y.nchunks)), block(64);
+    switch (a.y.nkernel) {
+    case 0: hipLaunchKernelGGL((k_adj_rest<0>), grid, block, 0, s, a); break;
+    case 1: hipLaunchKernelGGL((k_adj_rest<1>), grid, block, 0, s, a); break;
+    case 2: hipLaunchKernelGGL((k_adj_rest<2>), grid, block, 0, s, a); break;
+    default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
+}
+
+hipError_t launch_adj_wave(const AdjArgs &a, hipStream_t s)
+{
+    const dim3 grid((unsigned)((a.n + TC - 1) / TC) * (unsigned)a.jsplit), block(64);
+    switch (a.nkernel) {
+    case 0: hipLaunchKernelGGL((k_adj_wave<0>), grid, block, 0, s, a); break;
+    case 1: hipLaunchKernelGGL((k_adj_wave<1>), grid, block, 0, s, a); break;
+    case 2: hipLaunchKernelGGL((k_adj_wave<2>), grid, block, 0, s, a); break;
+    default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
+}
+
 hipError_t launch_adj_reduce(const AdjArgs &a, hipStream_t s)
 {
     if (a.n <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_adj_reduce, dim3((unsigned)((a.n + 255) / 256)), dim3(256), 0, s, a);
+    hipLaunchKernelGGL(k_adj_reduce, dim3((unsigned)((a.n + 63) / 64), 5), dim3(256), 0, s, a);
     return hipGetLastError();
 }
 

@@ -260,6 +260,31 @@ static void plan_sym(EvalPlan &p, int n)
     p.sym = true;
 }
 
+static SymArgs sym_args(const EvalPlan &p, int n, int nchunks, const PrepBuffers &b,
+                        unsigned char *tables, double *partial, double *segsum, int nkernel,
+                        unsigned long long *stats)
+{
+    const SymLayout l = sym_layout(nchunks);
+    SymArgs y{};
+    y.p = SortedSet{b.sx, b.sy, b.sz, b.sm, b.sH, b.sidx, n, p.padded};
+    y.chunks = b.chunks;
+    y.bbox = b.bbox;
+    y.boxes = (float4 *)(tables + l.boxes);
+    y.sym = (uint64_t *)(tables + l.bits);
+    y.seg = (int *)(tables + l.seg);
+    y.n = n;
+    y.nchunks = nchunks;
+    y.words = (nchunks + 63) / 64;
+    y.sb = p.sb;
+    y.nsb = p.nsb;
+    y.waves = p.waves;
+    y.nkernel = nkernel;
+    y.partial = partial;
+    y.segsum = segsum;
+    y.stats = stats;
+    return y;
+}
+
 EvalPlan plan_eval(int n, int ni, int wg, int ipl, int jsplit_cfg, int precision, bool psi,
                    bool allow_sym)
 {
@@ -378,28 +403,12 @@ hipError_t enqueue_eval(const EvalPlan &p, const EvalBuffers &bufs, int n, int i
         a.psipart = bufs.psipart;
     }
     if (p.sym) {
-        SymArgs y{};
-        y.p = a.j;
-        y.chunks = b.chunks;
-        y.bbox = b.bbox;
-        y.n = n;
-        y.nchunks = (int)(p.padded / TC);
-        y.words = (y.nchunks + 63) / 64;
-        y.sb = p.sb;
-        y.nsb = p.nsb;
-        y.waves = p.waves;
-        const SymLayout l = sym_layout(y.nchunks);
-        y.boxes = (float4 *)(bufs.sym + l.boxes);
-        y.sym = (uint64_t *)(bufs.sym + l.bits);
-        y.seg = (int *)(bufs.sym + l.seg);
-        y.segsum = bufs.partial + (int64_t)p.jsplit * 4 * n;
+        SymArgs y = sym_args(p, n, (int)(p.padded / TC), b, bufs.sym, bufs.partial,
+                             bufs.partial + (int64_t)p.jsplit * 4 * n, nkernel, bufs.stats);
         y.ax = ax;
         y.ay = ay;
         y.az = az;
         y.pot = pot;
-        y.nkernel = nkernel;
-        y.partial = bufs.partial;
-        y.stats = bufs.stats;
         SG_ENQ(launch_sym_classify(y, s));
         if (ev) SG_ENQ(hipEventRecord(ev[1], s));
         SG_ENQ(launch_sym(y, s));
@@ -1084,25 +1093,70 @@ int sg_vjp_device(sg_context *c, int n, const double *x, const double *y, const 
     a.n = n;
     a.nkernel = nkernel;
     a.ntiles = ntiles;
-    const int wg = sg::adj_config_supported(c->wg[precision]) ? c->wg[precision] : 256;
-    a.niblocks = (int)((n + (int64_t)wg - 1) / wg);
-    a.ngroups = (int64_t)a.niblocks * (wg / 64);
-    a.jsplit = sg::auto_jsplit(a.niblocks, wg, ntiles, n);
     a.gx = gx;
     a.gy = gy;
     a.gz = gz;
     a.gm = gm;
     a.gH = gH;
+    a.stats = c->stats;
+    // the FP32C pass: sets of ADJ_SYM_MIN_N particles on take each unordered far
+    // pair once, where the device holds its slabs; smaller ones one wave per 64 i
+    if (precision == SG_PREC_FP32C && n >= sg::ADJ_SYM_MIN_N && n <= sg::SYM_MAX_N) {
+        sg::EvalPlan p{};
+        p.padded = padded;
+        sg::plan_sym(p, n);
+        p.waves = 4;
+        p.sb = (p.sb + 7) / 8 * 8;   // whole column groups of k_adj_sym
+        const int nchunks = (int)(padded / sg::TC);
+        p.nsb = (nchunks + p.sb - 1) / p.sb;
+        const int64_t slabs = (int64_t)(p.nsb + 1) * 4 * n;
+        if (grow(&c->partial, &c->cap_part,
+                 slabs + ((int64_t)sg::SYM_SEGS + nchunks) * 5 * sg::TC) == SG_OK &&
+            grow(&c->sym, &c->cap_sym, p.sym_bytes) == SG_OK) {
+            sg::AdjSymArgs q{};
+            q.y = sg::sym_args(p, n, nchunks, b, c->sym, c->partial, c->partial + slabs, nkernel,
+                               c->stats);
+            q.wx = a.wx;
+            q.wy = a.wy;
+            q.wz = a.wz;
+            q.u = a.u;
+            q.gx = gx;
+            q.gy = gy;
+            q.gz = gz;
+            q.gm = gm;
+            q.gH = gH;
+            HIP_TRY(sg::launch_sym_classify(q.y, s));
+            HIP_TRY(hipEventRecord(c->ev_k0, s));
+            HIP_TRY(sg::launch_adj_sym(q, s));
+            HIP_TRY(hipEventRecord(c->ev_kf, s));
+            HIP_TRY(sg::launch_adj_sym_rest(q, s));
+            HIP_TRY(sg::launch_adj_sym_reduce(q, s));
+            HIP_TRY(hipEventRecord(c->ev_k1, s));
+            c->launched = true;
+            return SG_OK;
+        }
+        (void)hipGetLastError();
+    }
+    const bool wave = precision == SG_PREC_FP32C && n < sg::ADJ_SYM_MIN_N;
+    const int wg = sg::adj_config_supported(c->wg[precision]) ? c->wg[precision] : 256;
+    a.niblocks = (int)((n + (int64_t)wg - 1) / wg);
+    a.ngroups = (int64_t)a.niblocks * (wg / 64);
+    if (wave) {
+        const int64_t nic = (n + sg::TC - 1) / sg::TC;
+        a.jsplit = (int)std::max<int64_t>(
+            1, std::min<int64_t>(sg::WAVE_COUNT / nic, (int64_t)ntiles * sg::CHUNKS));
+    } else {
+        a.jsplit = sg::auto_jsplit(a.niblocks, wg, ntiles, n);
+    }
     if ((rc = grow(&c->partial, &c->cap_part, (int64_t)a.jsplit * 5 * n)) != SG_OK) return rc;
     a.partial = c->partial;
-    if ((rc = grow(&c->nearflag, &c->cap_flag, a.ngroups * ntiles)) != SG_OK) return rc;
+    if (!wave && (rc = grow(&c->nearflag, &c->cap_flag, a.ngroups * ntiles)) != SG_OK) return rc;
     a.nearflag = c->nearflag;
-    a.stats = c->stats;
 
     HIP_TRY(hipEventRecord(c->ev_k0, s));
-    HIP_TRY(sg::launch_adj_far(precision, a, wg, s));
+    HIP_TRY(wave ? sg::launch_adj_wave(a, s) : sg::launch_adj_far(precision, a, wg, s));
     HIP_TRY(hipEventRecord(c->ev_kf, s));
-    HIP_TRY(sg::launch_adj_near(precision, a, s));
+    if (!wave) HIP_TRY(sg::launch_adj_near(precision, a, s));
     HIP_TRY(sg::launch_adj_reduce(a, s));
     HIP_TRY(hipEventRecord(c->ev_k1, s));
     c->launched = true;

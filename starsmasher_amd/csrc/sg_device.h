@@ -144,6 +144,22 @@ __device__ __forceinline__ void poly_AP(int nk, double q, double invq, double &A
     }
 }
 
+// A(q) and P(q) of the cubic spline (poly_AP) without a branch: both pieces,
+// the right one kept.
+__device__ __forceinline__ void cubic_AP(double q, double invq, double &A, double &P)
+{
+    const double q2 = q * q, iq3 = invq * invq * invq;
+    const double Ai = 10.666666666667 + q2 * (32.0 * q - 38.4);
+    const double Pi = -2.8 + q2 * (5.333333333333 + q2 * (6.4 * q - 9.6));
+    const double Ao = 21.333333333333 + q * (-48.0 + q * (38.4 - 10.666666666667 * q)) -
+                      0.066666666667 * iq3;
+    const double Po = -3.2 + 0.066666666667 * invq +
+                      q2 * (10.666666666667 + q * (-16.0 + q * (9.6 - 2.133333333333 * q)));
+    const bool in = q < 0.5;
+    A = in ? Ai : Ao;
+    P = in ? Pi : Po;
+}
+
 __device__ __forceinline__ double self_coeff(int nk)
 {
     return nk == 0 ? 1.4 : (nk == 1 ? 1.9140625 : 1.71875);
@@ -171,6 +187,20 @@ __device__ __forceinline__ double rsqrt_pos64(double x)
     const double y = __builtin_amdgcn_rsq(x);
     const double e = fma((-x) * y, y, 1.0);
     return fma(y * e, fma(e, 0.375, 0.5), y);
+}
+
+// Where the lane's `count` (at most 64) entries begin in a wave-wide list in
+// lane order, and the list's length, from the bits of the counts.
+__device__ __forceinline__ void list_places(unsigned count, unsigned &at, unsigned &total)
+{
+    at = total = 0;
+#pragma unroll
+    for (int b = 0; b < 7; ++b) {
+        const uint64_t m = __ballot((count >> b) & 1u);
+        at += __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u))
+              << b;
+        total += (unsigned)__builtin_popcountll(m) << b;
+    }
 }
 
 // Orders the LDS writes of one wave before its reads (and the reverse).

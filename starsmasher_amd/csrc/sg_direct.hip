@@ -1014,22 +1014,6 @@ __device__ __forceinline__ Visit classify_visit(const TileMeta &cm, double Ox, d
     return VISIT_FAR;
 }
 
-// A(q) and P(q) of the cubic spline (poly_AP) without a branch: both pieces,
-// the right one kept.
-__device__ __forceinline__ void cubic_AP(double q, double invq, double &A, double &P)
-{
-    const double q2 = q * q, iq3 = invq * invq * invq;
-    const double Ai = 10.666666666667 + q2 * (32.0 * q - 38.4);
-    const double Pi = -2.8 + q2 * (5.333333333333 + q2 * (6.4 * q - 9.6));
-    const double Ao = 21.333333333333 + q * (-48.0 + q * (38.4 - 10.666666666667 * q)) -
-                      0.066666666667 * iq3;
-    const double Po = -3.2 + 0.066666666667 * invq +
-                      q2 * (10.666666666667 + q * (-16.0 + q * (9.6 - 2.133333333333 * q)));
-    const bool in = q < 0.5;
-    A = in ? Ai : Ao;
-    P = in ? Pi : Po;
-}
-
 // One side of a softened pair without a branch: the polynomials, or the
 // Newtonian terms beyond H.  q = 0 (r = 0, with ri passed as 0) gives the
 // r -> 0 limit.
@@ -1120,17 +1104,9 @@ __device__ __forceinline__ void visit_near(WaveLds &lds, uint64_t real, const So
     }
     // the counter covers pairs of particles, not padding
     nfp64 += (unsigned)__builtin_popcountll(mine & __brevll(real));
-    // lane's first place in the list, and the list's length, from the bits of
-    // the counts
     const unsigned count = (unsigned)__builtin_popcountll(mine);
-    unsigned at = 0, total = 0;
-#pragma unroll
-    for (int b = 0; b < 7; ++b) {
-        const uint64_t m = __ballot((count >> b) & 1u);
-        at += __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u))
-              << b;
-        total += (unsigned)__builtin_popcountll(m) << b;
-    }
+    unsigned at, total;
+    list_places(count, at, total);
     if (total > (unsigned)NSOFT) {
         while (mine) {
             const int jj = __builtin_clzll(mine);
@@ -1460,14 +1436,8 @@ __device__ __forceinline__ void psi_visit(PsiLds &lds, double xr, double yr, dou
         mine |= (uint64_t)(in ? 1u : 0u) << jj;
     }
     const unsigned count = (unsigned)__builtin_popcountll(mine);
-    unsigned at = 0, total = 0;
-#pragma unroll
-    for (int b = 0; b < 7; ++b) {
-        const uint64_t m = __ballot((count >> b) & 1u);
-        at += __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u))
-              << b;
-        total += (unsigned)__builtin_popcountll(m) << b;
-    }
+    unsigned at, total;
+    list_places(count, at, total);
     if (total > (unsigned)NSOFT) {
         while (mine) {
             const int jj = __builtin_ctzll(mine);

@@ -155,10 +155,24 @@ struct AdjArgs {
     unsigned long long *stats;          // [STAT_WORDS] statistics copies
 };
 
+// The adjoint with each unordered far pair once (sg_adjsym.hip) and the
+// ordered rest (sg_adjoint.hip): tables and items as in SymArgs, whose slabs
+// hold gx, gy, gz, gm and whose segments gx, gy, gz, gm, gH.
+struct AdjSymArgs {
+    SymArgs y;
+    const double *wx, *wy, *wz, *u;     // sorted-order cotangents
+    double *gx, *gy, *gz, *gm, *gH;     // outputs, input order
+};
+hipError_t launch_adj_sym(const AdjSymArgs &a, hipStream_t s);
+hipError_t launch_adj_sym_rest(const AdjSymArgs &a, hipStream_t s);
+hipError_t launch_adj_sym_reduce(const AdjSymArgs &a, hipStream_t s);
+
 // Adjoint launchers (sg_adjoint.hip): far, near, reduce in stream order.
 hipError_t launch_adj_far(int precision, const AdjArgs &a, int wg, hipStream_t s);
 hipError_t launch_adj_near(int precision, const AdjArgs &a, hipStream_t s);
 hipError_t launch_adj_reduce(const AdjArgs &a, hipStream_t s);
+// FP32C pass of small sets: a.jsplit partitions of strided chunks, then reduce.
+hipError_t launch_adj_wave(const AdjArgs &a, hipStream_t s);
 bool adj_config_supported(int wg);
 
 // Launchers (sg_direct.hip).  Return hipError_t of the launch.
@@ -292,6 +306,12 @@ constexpr int WAVE_MAX_NI = 49151, WAVE_COUNT = 16384;
 // upper limit keeps the chunk-pair bits (N^2 / 32,768 bytes) at 512 MB and the
 // slabs at 17 GB; where the device cannot hold them the ordered pass runs.
 constexpr int SYM_MIN_N = 49152, SYM_MAX_N = 1 << 22, SYM_MAX_SB = 128;
+// FP32C adjoints from this size on evaluate each unordered far pair once
+// (sg_adjsym.hip), smaller ones run one wave per 64 i and j partition.  Whole
+// calls, flagged near chunks (the pass before both) / waves / unordered, same
+// card: 2,000 particles 0.253 / 0.128 ms, 16,384 0.69 / 0.48 / 0.65, 33,333
+// 1.52 / 1.26 / 1.16, 50,001 2.88 / 2.73 / 2.34, 131,072 13.3 / 15.7 / 9.3.
+constexpr int ADJ_SYM_MIN_N = 32768;
 // the HIP error that sg_status_string(SG_ERR_HIP) describes
 void record_hip_error(hipError_t e);
 EvalPlan plan_eval(int n, int ni, int wg, int ipl, int jsplit_cfg, int precision, bool psi,

@@ -785,9 +785,9 @@ void k_adj_rest(AdjSymArgs a)
     const SortedSet &P = y.p;
     const int lane = threadIdx.x;
     const int s = (int)blockIdx.x;
-    if (s >= y.seg[y.nchunks]) return;
+    if (s >= y.segtot[0]) return;
     const int ci = segment_row(y.seg, y.nchunks, s);
-    const int len = uniform_i(y.seg[y.nchunks + 1]);
+    const int len = uniform_i(y.segtot[1]);
     const int k0 = uniform_i(s - y.seg[ci]) * len;
     const int64_t gbase = (int64_t)ci * TC;
     const int64_t io = min(gbase + TC / 2, y.n - 1);

@@ -81,6 +81,10 @@ struct sg_context {
         int wg = 0, ipl = 0;
         int64_t padded = 0, ngroups = 0, nflags = 0, nparts = 0;
         int nitems = 0;
+        // the unordered-pair form (FP32C at the default shape)
+        int sym_items = 0, sym_chunks = 0;
+        int64_t sym_slabs = 0, sym_words = 0;
+        bool sym_fits = false;
     } plan;
     int64_t *d_offsets = nullptr;
     int64_t cap_offsets = 0;
@@ -89,9 +93,18 @@ struct sg_context {
     int2 *d_items = nullptr;
     int64_t cap_items = 0;
     unsigned *d_counter = nullptr;
+    sg::SymSet *d_symsets = nullptr;
+    int64_t cap_symsets = 0;
+    int2 *d_symitems = nullptr;
+    int64_t cap_symitems = 0;
+    double *d_setbox = nullptr;
+    int64_t cap_setbox = 0;
+    int *d_setof = nullptr;
+    int64_t cap_setof = 0;
     // captured compute of the last batch call (replayed when nothing changed)
     hipGraphExec_t gexec = nullptr;
     sg::BatchArgs g_args{};
+    sg::SymArgs g_sym{};
     int g_key[5] = {-1, -1, -1, -1, -1};   // precision, nkernel, wg, ipl, nwg
     hipStream_t g_stream = nullptr;
 };
@@ -232,14 +245,15 @@ int auto_jsplit(int niblocks, int wg, int ntiles, int64_t ni)
 struct SymLayout {
     int64_t boxes, bits, seg, bytes;
 };
-static SymLayout sym_layout(int nchunks)
+static SymLayout sym_layout(int nchunks, int64_t words)
 {
     SymLayout l{};
     l.bits = (int64_t)nchunks * 2 * sizeof(float4);
-    l.seg = l.bits + (int64_t)nchunks * ((nchunks + 63) / 64) * 8;
-    l.bytes = l.seg + ((int64_t)nchunks + 2) * 4;
+    l.seg = l.bits + words * 8;
+    l.bytes = l.seg + ((int64_t)nchunks + 3) * 4;
     return l;
 }
+static int64_t sym_words(int nchunks) { return (int64_t)nchunks * ((nchunks + 63) / 64); }
 
 // The whole-set FP32C pass evaluates each unordered far pair once.  Up to
 // SYM_MAX_SB superblocks make the work items (8,256 pairs of them at 128, 16
@@ -256,7 +270,7 @@ static void plan_sym(EvalPlan &p, int n)
     p.nsb = (nchunks + p.sb - 1) / p.sb;
     p.jsplit = p.nsb + 1;
     p.part_elems = (int64_t)p.jsplit * 4 * n + ((int64_t)SYM_SEGS + nchunks) * 4 * TC;
-    p.sym_bytes = sym_layout(nchunks).bytes;
+    p.sym_bytes = sym_layout(nchunks, sym_words(nchunks)).bytes;
     p.sym = true;
 }
 
@@ -264,7 +278,7 @@ static SymArgs sym_args(const EvalPlan &p, int n, int nchunks, const PrepBuffers
                         unsigned char *tables, double *partial, double *segsum, int nkernel,
                         unsigned long long *stats)
 {
-    const SymLayout l = sym_layout(nchunks);
+    const SymLayout l = sym_layout(nchunks, sym_words(nchunks));
     SymArgs y{};
     y.p = SortedSet{b.sx, b.sy, b.sz, b.sm, b.sH, b.sidx, n, p.padded};
     y.chunks = b.chunks;
@@ -272,6 +286,7 @@ static SymArgs sym_args(const EvalPlan &p, int n, int nchunks, const PrepBuffers
     y.boxes = (float4 *)(tables + l.boxes);
     y.sym = (uint64_t *)(tables + l.bits);
     y.seg = (int *)(tables + l.seg);
+    y.segtot = y.seg + nchunks + 1;
     y.n = n;
     y.nchunks = nchunks;
     y.words = (nchunks + 63) / 64;
@@ -515,7 +530,7 @@ int sg_destroy(sg_context *c)
                     c->scot[0], c->scot[1], c->scot[2], c->scot[3],
                     c->vin[0], c->vin[1], c->vin[2], c->vin[3],
                     c->vout[0], c->vout[1], c->vout[2], c->vout[3], c->vout[4], c->psipart,
-                    c->psi_out, c->epot_work, c->sym};
+                    c->psi_out, c->epot_work, c->sym, c->d_symsets, c->d_symitems, c->d_setof, c->d_setbox};
     if (c->gexec) (void)hipGraphExecDestroy(c->gexec);
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
@@ -737,6 +752,64 @@ int sg_get_batch_config(sg_context *c, int precision, int *wg, int *ipl)
 
 namespace {
 
+// The batch's tables of the unordered-pair pass.  One superblock size for all
+// sets, a multiple of the 16 chunks of a workgroup's column group and such that
+// the batch makes at least some 8,192 full items (16 rounds of the workgroups
+// that fit at once) where it is large enough; items of the largest sets first.
+int build_sym_plan(sg_context *c, const std::vector<sg::BatchSet> &sets)
+{
+    auto &P = c->plan;
+    const int nsets = (int)sets.size();
+    std::vector<sg::SymSet> ss(nsets);
+    std::vector<int> setof((size_t)(P.padded / sg::TC));
+    double pairs = 0.0;   // unordered chunk pairs of the batch
+    double nsum = 0.0, nsq = 0.0;
+    P.sym_fits = true;
+    for (const sg::BatchSet &b : sets) {
+        const double nc = (double)b.ntiles * sg::CHUNKS;
+        pairs += 0.5 * nc * nc;
+        nsum += (double)b.n;
+        nsq += (double)b.n * (double)b.n;
+        if (b.n > sg::SYM_MAX_N) P.sym_fits = false;
+    }
+    if (nsq < sg::BATCH_SYM_MEAN * nsum) P.sym_fits = false;
+    if (!P.sym_fits) return SG_OK;
+    const int sb = 16 * std::max(1, (int)std::ceil(std::sqrt(pairs / 8192.0) / 16.0));
+    P.sym_words = P.sym_slabs = 0;
+    for (int k = 0; k < nsets; ++k) {
+        sg::SymSet &q = ss[k];
+        q.pofs = sets[k].pofs;
+        q.n = sets[k].n;
+        q.chunk0 = (int)(sets[k].pofs / sg::TC);
+        q.nchunks = sets[k].ntiles * sg::CHUNKS;
+        q.words = (q.nchunks + 63) / 64;
+        q.sb = sb;
+        q.nsb = (q.nchunks + sb - 1) / sb;
+        q.bitsofs = P.sym_words;
+        q.slabofs = P.sym_slabs;
+        P.sym_words += sg::sym_words(q.nchunks);
+        P.sym_slabs += (int64_t)(q.nsb + 1) * 4 * q.n;
+        std::fill_n(setof.begin() + q.chunk0, q.nchunks, k);
+    }
+    std::vector<int> order(nsets);
+    for (int k = 0; k < nsets; ++k) order[k] = k;
+    std::stable_sort(order.begin(), order.end(), [&](int u, int v) { return ss[u].n > ss[v].n; });
+    std::vector<int2> items;
+    for (int k : order)
+        for (int t = 0; t < ss[k].nsb * (ss[k].nsb + 1) / 2; ++t) items.push_back(make_int2(k, t));
+    P.sym_items = (int)items.size();
+    P.sym_chunks = (int)setof.size();
+    int rc;
+    if ((rc = grow(&c->d_symsets, &c->cap_symsets, nsets)) != SG_OK) return rc;
+    if ((rc = grow(&c->d_symitems, &c->cap_symitems, (int64_t)items.size())) != SG_OK) return rc;
+    if ((rc = grow(&c->d_setof, &c->cap_setof, (int64_t)setof.size())) != SG_OK) return rc;
+    if ((rc = grow(&c->d_setbox, &c->cap_setbox, (int64_t)nsets * 8)) != SG_OK) return rc;
+    HIP_TRY(hipMemcpy(c->d_symsets, ss.data(), sizeof(sg::SymSet) * nsets, hipMemcpyHostToDevice));
+    HIP_TRY(hipMemcpy(c->d_symitems, items.data(), sizeof(int2) * items.size(), hipMemcpyHostToDevice));
+    HIP_TRY(hipMemcpy(c->d_setof, setof.data(), sizeof(int) * setof.size(), hipMemcpyHostToDevice));
+    return SG_OK;
+}
+
 // Host part of a batch plan: per-set layout, near-flag and partial-sum
 // offsets and the work items, longest first.  An item is one i-block of a
 // set against one j partition; sets of more than BATCH_JTILES tiles are cut
@@ -796,7 +869,7 @@ int build_plan(sg_context *c, int nsets, const long long *offsets, int wg, int i
     HIP_TRY(hipMemcpy(c->d_sets, sets.data(), sizeof(sg::BatchSet) * nsets, hipMemcpyHostToDevice));
     HIP_TRY(hipMemcpy(c->d_items, items.data(), sizeof(int2) * items.size(),
                       hipMemcpyHostToDevice));
-    return SG_OK;
+    return wg == 256 && ipl == 1 ? build_sym_plan(c, sets) : SG_OK;
 }
 
 }  // namespace
@@ -829,8 +902,20 @@ int sg_compute_batch_device(sg_context *c, int nsets, const long long *offsets, 
         if ((rc = build_plan(c, nsets, offsets, wg, ipl)) != SG_OK) return rc;
     }
     if ((rc = ensure_capacity(c, ntot, P.padded, 1)) != SG_OK) return rc;
-    if ((rc = grow(&c->partial, &c->cap_part, P.nparts)) != SG_OK) return rc;
-    if ((rc = grow(&c->nearflag, &c->cap_flag, std::max<int64_t>(P.nflags, 1))) != SG_OK) return rc;
+    // FP32C at the default shape: each unordered far pair once, where the device
+    // holds its slabs
+    bool sym = precision == SG_PREC_FP32C && wg == 256 && ipl == 1 && P.sym_fits;
+    const sg::SymLayout layout = sg::sym_layout(P.sym_chunks, P.sym_words);
+    if (sym && (grow(&c->partial, &c->cap_part,
+                     P.sym_slabs + ((int64_t)sg::SYM_SEGS + P.sym_chunks) * 4 * sg::TC) != SG_OK ||
+                grow(&c->sym, &c->cap_sym, layout.bytes) != SG_OK)) {
+        (void)hipGetLastError();
+        sym = false;
+    }
+    if (!sym) {
+        if ((rc = grow(&c->partial, &c->cap_part, P.nparts)) != SG_OK) return rc;
+        if ((rc = grow(&c->nearflag, &c->cap_flag, std::max<int64_t>(P.nflags, 1))) != SG_OK) return rc;
+    }
 
     hipStream_t s = c->stream;
     sg::PrepBuffers &b = c->pb;
@@ -865,22 +950,59 @@ int sg_compute_batch_device(sg_context *c, int nsets, const long long *offsets, 
     a.az = az;
     a.pot = pot;
     a.stats = c->stats;
-    const int nwg = sg::batch_resident_workgroups(precision, nkernel, wg, ipl, c->device);
+    const int nwg = sym ? 1 : sg::batch_resident_workgroups(precision, nkernel, wg, ipl, c->device);
     if (nwg <= 0) return SG_ERR_CONFIG;
+    sg::SymArgs u;
+    std::memset((void *)&u, 0, sizeof(y));   // compared as bytes below
+    if (sym) {
+        u.p = a.j;
+        u.chunks = b.chunks;
+        u.bbox = c->d_setbox;
+        u.boxes = (float4 *)(c->sym + layout.boxes);
+        u.sym = (uint64_t *)(c->sym + layout.bits);
+        u.seg = (int *)(c->sym + layout.seg);
+        u.segtot = u.seg + P.sym_chunks + 1;
+        u.n = ntot;
+        u.nchunks = P.sym_chunks;
+        u.waves = 4;
+        u.nkernel = nkernel;
+        u.partial = c->partial;
+        u.segsum = c->partial + P.sym_slabs;
+        u.ax = ax;
+        u.ay = ay;
+        u.az = az;
+        u.pot = pot;
+        u.stats = c->stats;
+        u.sets = c->d_symsets;
+        u.items = c->d_symitems;
+        u.setof = c->d_setof;
+        u.nitems = P.sym_items;
+    }
+    // kernels only, so that they can be captured
+    auto compute = [&]() -> hipError_t {
+        hipError_t e = sg::launch_fill_zero_int((int *)c->stats, 2 * sg::STAT_WORDS, s);
+        if (e != hipSuccess) return e;
+        if (!sym) return sg::launch_batch(precision, a, wg, ipl, nwg, s);
+        if ((e = sg::launch_set_boxes(u, nsets, c->d_setbox, s)) != hipSuccess) return e;
+        if ((e = sg::launch_sym_classify(u, s)) != hipSuccess) return e;
+        if ((e = sg::launch_sym(u, s)) != hipSuccess) return e;
+        if ((e = sg::launch_sym_rest(u, s)) != hipSuccess) return e;
+        return sg::launch_sym_reduce(u, s);
+    };
 
     HIP_TRY(hipEventRecord(c->ev_k0, s));
     if (use_graph) {
         const int key[5] = {precision, nkernel, wg, ipl, nwg};
         const bool reuse = c->gexec && c->g_stream == s &&
                            std::memcmp(&c->g_args, &a, sizeof(a)) == 0 &&
+                           std::memcmp((const void *)&c->g_sym, (const void *)&u, sizeof(u)) == 0 &&
                            std::memcmp(c->g_key, key, sizeof(key)) == 0;
         if (!reuse) {
             if (c->gexec) HIP_TRY(hipGraphExecDestroy(c->gexec));
             c->gexec = nullptr;
             hipGraph_t graph = nullptr;
             HIP_TRY(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-            HIP_TRY(sg::launch_fill_zero_int((int *)c->stats, 2 * sg::STAT_WORDS, s));
-            const hipError_t le = sg::launch_batch(precision, a, wg, ipl, nwg, s);
+            const hipError_t le = compute();
             const hipError_t ee = hipStreamEndCapture(s, &graph);
             HIP_TRY(le);
             HIP_TRY(ee);
@@ -888,13 +1010,13 @@ int sg_compute_batch_device(sg_context *c, int nsets, const long long *offsets, 
             (void)hipGraphDestroy(graph);
             HIP_TRY(ie);
             c->g_args = a;
+            std::memcpy((void *)&c->g_sym, (const void *)&u, sizeof(u));
             std::memcpy(c->g_key, key, sizeof(key));
             c->g_stream = s;
         }
         HIP_TRY(hipGraphLaunch(c->gexec, s));
     } else {
-        HIP_TRY(sg::launch_fill_zero_int((int *)c->stats, 2 * sg::STAT_WORDS, s));
-        HIP_TRY(sg::launch_batch(precision, a, wg, ipl, nwg, s));
+        HIP_TRY(compute());
     }
     HIP_TRY(hipEventRecord(c->ev_kf, s));
     HIP_TRY(hipEventRecord(c->ev_k1, s));

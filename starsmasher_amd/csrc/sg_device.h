@@ -210,6 +210,30 @@ __device__ __forceinline__ void wave_lds_sync()
     __builtin_amdgcn_wave_barrier();
 }
 
+// The arguments of one set of a batch.
+__device__ __forceinline__ SymArgs sym_view(SymArgs a, int set)
+{
+    const SymSet s = a.sets[uniform_i(set)];
+    a.p.x += s.pofs;
+    a.p.y += s.pofs;
+    a.p.z += s.pofs;
+    a.p.m += s.pofs;
+    a.p.Hs += s.pofs;
+    a.p.idx += s.pofs;
+    a.bbox += 8 * (int64_t)set;
+    a.chunks += s.chunk0;
+    a.boxes += 2 * (int64_t)s.chunk0;
+    a.sym += s.bitsofs;
+    a.seg += s.chunk0;
+    a.partial += s.slabofs;
+    a.n = s.n;
+    a.nchunks = s.nchunks;
+    a.words = s.words;
+    a.sb = s.sb;
+    a.nsb = s.nsb;
+    return a;
+}
+
 // The unset bits of one row of SymArgs::sym from the k-th on, in order.
 struct RestBits {
     const uint64_t *row;

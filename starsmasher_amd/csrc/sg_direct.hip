@@ -1313,10 +1313,15 @@ __global__ __launch_bounds__(64) void k_sym_rest(SymArgs a)
     NearSlice &sl = lds.sl;
     const int lane = threadIdx.x;
     const int g = (int)blockIdx.x;
-    if (g >= a.seg[a.nchunks]) return;
-    const int ci = segment_row(a.seg, a.nchunks, g);
-    const int len = uniform_i(a.seg[a.nchunks + 1]);
+    if (g >= a.segtot[0]) return;
+    int ci = segment_row(a.seg, a.nchunks, g);
+    const int len = uniform_i(a.segtot[1]);
     const int k0 = uniform_i(g - a.seg[ci]) * len;
+    if (a.sets) {
+        const int set = a.setof[ci];
+        ci -= uniform_i(a.sets[set].chunk0);
+        a = sym_view(a, set);
+    }
     const SortedSet &P = a.p;
     const int64_t gbase = (int64_t)ci * TC;
     const int64_t io = min(gbase + TC / 2, a.n - 1);

@@ -78,13 +78,20 @@ struct PairArgs {
 // chunk is cut into segments with partial sums of their own: at most SYM_SEGS
 // + nchunks of them, of SYM_SEG_MIN chunk visits or more.
 constexpr int SYM_SEGS = 32768, SYM_SEG_MIN = 8;
+// A set of a batch: where its particles, chunks, bits and slabs begin in the
+// batch's arrays.  Segments are numbered over the whole batch.
+struct SymSet {
+    int64_t pofs, n, bitsofs, slabofs;
+    int chunk0, nchunks, words, sb, nsb;
+};
 struct SymArgs {
     SortedSet p;
     const TileMeta *chunks;
-    const double *bbox;      // PrepBuffers::bbox
+    const double *bbox;      // PrepBuffers::bbox (of each set of a batch)
     float4 *boxes;           // [nchunks][2]: FP32 chunk boxes
     uint64_t *sym;           // [nchunks][words]: bit set = chunk pair in k_sym
-    int *seg;                // [nchunks + 2]: first segment of each row, their number, length
+    int *seg;                // [nchunks + 1]: first segment of each row, and their number
+    int *segtot;             // their number and length
     int64_t n;               // real particles
     int nchunks, words;      // padded / TC, (nchunks + 63) / 64
     int sb, nsb;             // chunks per superblock, superblocks
@@ -94,7 +101,15 @@ struct SymArgs {
     double *segsum;          // [SYM_SEGS + nchunks][4][TC]
     double *ax, *ay, *az, *pot;   // outputs, input order
     unsigned long long *stats;
+    // a batch: its sets, the work items (set, superblock pair) and each chunk's
+    // set; nchunks and n then span the batch (null: one set)
+    const SymSet *sets;
+    const int2 *items;
+    const int *setof;
+    int nitems;
 };
+// The box and scales of every set of a batch, from its chunks.
+hipError_t launch_set_boxes(const SymArgs &a, int nsets, double *boxes, hipStream_t s);
 hipError_t launch_sym_classify(const SymArgs &a, hipStream_t s);
 hipError_t launch_sym(const SymArgs &a, hipStream_t s);
 hipError_t launch_sym_rest(const SymArgs &a, hipStream_t s);   // sg_direct.hip
@@ -306,6 +321,14 @@ constexpr int WAVE_MAX_NI = 49151, WAVE_COUNT = 16384;
 // upper limit keeps the chunk-pair bits (N^2 / 32,768 bytes) at 512 MB and the
 // slabs at 17 GB; where the device cannot hold them the ordered pass runs.
 constexpr int SYM_MIN_N = 49152, SYM_MAX_N = 1 << 22, SYM_MAX_SB = 128;
+// FP32C batches at the default shape do so too, unless the average particle's
+// set is smaller than this (nearly all of its chunk pairs are then near, and
+// the one kernel of the ordered pass is shorter than five).  Ordered against
+// unordered, kernels, same card: 1,000 sets of 100 0.205 against 0.314 ms, 200
+// of 500 0.168 against 0.111, 64 of 4,096 1.06 against 0.69, 8 of 2,048 to
+// 131,072 3.77 against 2.53, 64 of these 43.8 against 33.2, four of 200,000
+// 48.5 against 35.2.
+constexpr double BATCH_SYM_MEAN = 256.0;
 // FP32C adjoints from this size on evaluate each unordered far pair once
 // (sg_adjsym.hip), smaller ones run one wave per 64 i and j partition.  Whole
 // calls, flagged near chunks (the pass before both) / waves / unordered, same

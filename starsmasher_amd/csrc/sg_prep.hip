@@ -502,9 +502,40 @@ __global__ __launch_bounds__(RB) void k_gather_batch(
     oidx[slot] = real ? src : -1;
 }
 
+// Box and scales (as bbox) of each set of a batch; one workgroup per set.
+__global__ __launch_bounds__(RB) void k_set_boxes(SymArgs a, double *__restrict__ boxes)
+{
+    const SymSet st = a.sets[blockIdx.x];
+    double v[6] = {INFINITY, INFINITY, INFINITY, -INFINITY, -INFINITY, -INFINITY};
+    double mmax = 0.0;
+    for (int c = threadIdx.x; c < st.nchunks; c += RB) {
+        const TileMeta &t = a.chunks[st.chunk0 + c];
+        for (int q = 0; q < 3; ++q) {
+            v[q] = fmin(v[q], t.lo[q]);
+            v[3 + q] = fmax(v[3 + q], t.hi[q]);
+        }
+    }
+#pragma unroll 4
+    for (int64_t k = threadIdx.x; k < st.n; k += RB) mmax = fmax(mmax, a.p.m[st.pofs + k]);
+    block_minmax6(v);
+    mmax = block_max(mmax);
+    if (threadIdx.x == 0) {
+        double *o = boxes + 8 * (int64_t)blockIdx.x;
+        for (int c = 0; c < 6; ++c) o[c] = v[c];
+        o[6] = unit_scale(fmax(fmax(v[3] - v[0], v[4] - v[1]), v[5] - v[2]));
+        o[7] = unit_scale(mmax);
+    }
+}
+
 inline int nblocks_for(int64_t n) { return (int)((n + RB - 1) / RB); }
 
 }  // namespace
+
+hipError_t launch_set_boxes(const SymArgs &a, int nsets, double *boxes, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_set_boxes, dim3((unsigned)nsets), dim3(RB), 0, s, a, boxes);
+    return hipGetLastError();
+}
 
 hipError_t launch_morton_batch(const double *x, const double *y, const double *z, int n,
                                const int64_t *offsets, int nsets, const PrepBuffers &b,

@@ -49,6 +49,7 @@ __global__ __launch_bounds__(256) void k_sym_boxes(SymArgs a)
     const int c = blockIdx.x * 256 + threadIdx.x;
     if (c >= a.nchunks) return;
     const TileMeta m = a.chunks[c];
+    if (a.sets) a.bbox += 8 * (int64_t)a.setof[c];
     float lo[3], hi[3], rho2 = 0.0f;
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
@@ -67,11 +68,17 @@ __global__ __launch_bounds__(256) void k_sym_boxes(SymArgs a)
 // chunk index, the row in k_sym, for both (ci, cj) and (cj, ci), so the bit
 // matrix is symmetric.
 constexpr int CROWS = 4;
+static_assert(CHUNKS % CROWS == 0, "a tile's chunks are whole groups of rows");
 __global__ __launch_bounds__(256) void k_sym_classify(SymArgs a)
 {
     const int lane = threadIdx.x & 63;
-    const int r0 = uniform_i((int)(blockIdx.x * 4 + (threadIdx.x >> 6)) * CROWS);
+    int r0 = uniform_i((int)(blockIdx.x * 4 + (threadIdx.x >> 6)) * CROWS);
     if (r0 >= a.nchunks) return;
+    if (a.sets) {   // sets begin at a tile, so CROWS rows share one
+        const int set = a.setof[r0];
+        r0 -= uniform_i(a.sets[set].chunk0);
+        a = sym_view(a, set);
+    }
     float4 rl[CROWS], rh[CROWS];
     int rest[CROWS];
 #pragma unroll
@@ -144,7 +151,8 @@ __global__ __launch_bounds__(1024) void k_sym_segments(SymArgs a)
     }
     if (t == 1023) {
         a.seg[a.nchunks] = at;
-        a.seg[a.nchunks + 1] = len;
+        a.segtot[0] = at;
+        a.segtot[1] = len;
     }
 }
 
@@ -257,8 +265,13 @@ void k_sym(SymArgs a)
     const int lane = threadIdx.x & 63;
     const int w = uniform_i(threadIdx.x >> 6);
     const int p = lane >> 4, q = lane & 15;
-    int bi, bj;
-    sym_item((int)blockIdx.x, a.nsb, bi, bj);
+    int bi, bj, item = (int)blockIdx.x;
+    if (a.sets) {
+        const int2 it = a.items[item];
+        a = sym_view(a, it.x);
+        item = uniform_i(it.y);
+    }
+    sym_item(item, a.nsb, bi, bj);
     const int ci0 = bi * a.sb, ci1 = min(ci0 + a.sb, a.nchunks);
     const int cj0 = bj * a.sb, cj1 = min(cj0 + a.sb, a.nchunks);
     const bool diag = bi == bj;
@@ -408,7 +421,12 @@ void k_sym(SymArgs a)
 // scattered to input order.
 __global__ __launch_bounds__(256) void k_sym_reduce(SymArgs a)
 {
-    const int64_t i = blockIdx.x * (int64_t)256 + threadIdx.x;
+    int64_t i = blockIdx.x * (int64_t)256 + threadIdx.x;
+    if (a.sets) {   // a block is a tile, of one set
+        const int set = a.setof[blockIdx.x * (int64_t)CHUNKS];
+        a = sym_view(a, set);
+        i -= a.sets[set].pofs;
+    }
     if (i >= a.n) return;
     double s[4] = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll 4
@@ -439,7 +457,8 @@ __global__ __launch_bounds__(256) void k_sym_reduce(SymArgs a)
 
 hipError_t launch_sym_reduce(const SymArgs &a, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_sym_reduce, dim3((unsigned)((a.n + 255) / 256)), dim3(256), 0, s, a);
+    const int64_t slots = a.sets ? (int64_t)a.nchunks * TC : a.n;
+    hipLaunchKernelGGL(k_sym_reduce, dim3((unsigned)((slots + 255) / 256)), dim3(256), 0, s, a);
     return hipGetLastError();
 }
 
@@ -458,7 +477,7 @@ hipError_t launch_sym_classify(const SymArgs &a, hipStream_t s)
 
 hipError_t launch_sym(const SymArgs &a, hipStream_t s)
 {
-    const dim3 grid((unsigned)(a.nsb * (a.nsb + 1) / 2));
+    const dim3 grid((unsigned)(a.sets ? a.nitems : a.nsb * (a.nsb + 1) / 2));
     switch (a.waves) {
     case 1: hipLaunchKernelGGL((k_sym<1>), grid, dim3(64), 0, s, a); break;
     case 2: hipLaunchKernelGGL((k_sym<2>), grid, dim3(128), 0, s, a); break;

@@ -953,7 +953,7 @@ int sg_compute_batch_device(sg_context *c, int nsets, const long long *offsets, 
     const int nwg = sym ? 1 : sg::batch_resident_workgroups(precision, nkernel, wg, ipl, c->device);
     if (nwg <= 0) return SG_ERR_CONFIG;
     sg::SymArgs u;
-    std::memset((void *)&u, 0, sizeof(y));   // compared as bytes below
+    std::memset((void *)&u, 0, sizeof(u));   // compared as bytes below
     if (sym) {
         u.p = a.j;
         u.chunks = b.chunks;

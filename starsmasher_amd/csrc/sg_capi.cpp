@@ -255,23 +255,26 @@ static SymLayout sym_layout(int nchunks, int64_t words)
 }
 static int64_t sym_words(int nchunks) { return (int64_t)nchunks * ((nchunks + 63) / 64); }
 
-// The whole-set FP32C pass evaluates each unordered far pair once.  Up to
+// The whole-set pass evaluates each unordered far pair once.  Up to
 // SYM_MAX_SB superblocks make the work items (8,256 pairs of them at 128, 16
 // rounds of the workgroups that fit at once) and the partial-sum slabs (32 B
 // per particle each).  A workgroup has as many waves as its superblock has
-// column groups of four chunks, up to four.
-static void plan_sym(EvalPlan &p, int n)
+// column groups of four chunks, up to four; in FP64 always four, of two chunks
+// each.
+static void plan_sym(EvalPlan &p, int n, bool fp64)
 {
     const int nchunks = (int)(p.padded / TC);
     const int want = (nchunks + SYM_MAX_SB - 1) / SYM_MAX_SB;
-    p.waves = want > 8 ? 4 : (want > 4 ? 2 : 1);
-    const int step = 4 * p.waves;   // a column group: four chunks per wave
+    p.waves = fp64 || want > 8 ? 4 : (want > 4 ? 2 : 1);
+    const int step = fp64 ? SYM64_STEP : 4 * p.waves;   // a column group
     p.sb = (want + step - 1) / step * step;
     p.nsb = (nchunks + p.sb - 1) / p.sb;
     p.jsplit = p.nsb + 1;
     p.part_elems = (int64_t)p.jsplit * 4 * n + ((int64_t)SYM_SEGS + nchunks) * 4 * TC;
+    p.flag_elems = 1;
     p.sym_bytes = sym_layout(nchunks, sym_words(nchunks)).bytes;
     p.sym = true;
+    p.fp64 = fp64;
 }
 
 static SymArgs sym_args(const EvalPlan &p, int n, int nchunks, const PrepBuffers &b,
@@ -293,6 +296,7 @@ static SymArgs sym_args(const EvalPlan &p, int n, int nchunks, const PrepBuffers
     y.sb = p.sb;
     y.nsb = p.nsb;
     y.waves = p.waves;
+    y.fp64 = p.fp64;
     y.nkernel = nkernel;
     y.partial = partial;
     y.segsum = segsum;
@@ -326,9 +330,10 @@ EvalPlan plan_eval(int n, int ni, int wg, int ipl, int jsplit_cfg, int precision
     p.flag_elems = flagged ? p.ngroups * p.ntiles : 1;
     p.psipart_elems = psi ? (int64_t)p.jsplit * ni : 0;
     // the automatic shape, or asked for by its workgroup size
-    const bool automatic = precision == SG_PREC_FP32C && p.ipl == 1 && jsplit_cfg == 0 &&
-                           (wg == 0 || wg == (ni <= AUTO_SMALL_NI ? 128 : 256));
-    if (automatic && ni <= WAVE_MAX_NI) {
+    const bool automatic =
+        p.ipl == 1 && jsplit_cfg == 0 && (wg == 0 || wg == (ni <= AUTO_SMALL_NI ? 128 : 256));
+    const bool fp64 = precision != SG_PREC_FP32C;
+    if (automatic && !fp64 && ni <= WAVE_MAX_NI) {
         const int64_t nic = (ni + TC - 1) / TC, nchunks = (int64_t)p.ntiles * CHUNKS;
         // n > SG_STATIC_MAX_N: no static scratch to fit (2^20 i-partitions)
         const int64_t waves = n > SG_STATIC_MAX_N ? 2 * WAVE_COUNT : WAVE_COUNT;
@@ -339,7 +344,9 @@ EvalPlan plan_eval(int n, int ni, int wg, int ipl, int jsplit_cfg, int precision
         p.flag_elems = 1;
         p.psipart_elems = psi ? (int64_t)p.jsplit * ni : 0;
     }
-    if (allow_sym && automatic && !psi && ni == n && n >= SYM_MIN_N && n <= SYM_MAX_N) plan_sym(p, n);
+    if (allow_sym && automatic && !psi && ni == n && n >= (fp64 ? SYM64_MIN_N : SYM_MIN_N) &&
+        n <= SYM_MAX_N)
+        plan_sym(p, n, fp64);
     return p;
 }
 
@@ -426,7 +433,7 @@ hipError_t enqueue_eval(const EvalPlan &p, const EvalBuffers &bufs, int n, int i
         y.pot = pot;
         SG_ENQ(launch_sym_classify(y, s));
         if (ev) SG_ENQ(hipEventRecord(ev[1], s));
-        SG_ENQ(launch_sym(y, s));
+        SG_ENQ(p.fp64 ? launch_sym64(y, s) : launch_sym(y, s));
         SG_ENQ(launch_sym_rest(y, s));
         if (ev) SG_ENQ(hipEventRecord(ev[2], s));
         SG_ENQ(launch_sym_reduce(y, s));
@@ -1226,7 +1233,7 @@ int sg_vjp_device(sg_context *c, int n, const double *x, const double *y, const 
     if (precision == SG_PREC_FP32C && n >= sg::ADJ_SYM_MIN_N && n <= sg::SYM_MAX_N) {
         sg::EvalPlan p{};
         p.padded = padded;
-        sg::plan_sym(p, n);
+        sg::plan_sym(p, n, false);
         p.waves = 4;
         p.sb = (p.sb + 7) / 8 * 8;   // whole column groups of k_adj_sym
         const int nchunks = (int)(padded / sg::TC);

@@ -1035,14 +1035,14 @@ __device__ __forceinline__ void side_select(double r, double ri, double r2, doub
 // no branch: dealt over the lanes such pairs take different ones, and a wave
 // would walk them all.  dead: the self pair of a point particle.  With PSI
 // f[4] is m_j (P(q_i) + q_i^2 A(q_i)) where r <= H_i, as in near_pair.
-template <int NK, bool PSI>
+template <int NK, bool PSI, bool FAST>
 __device__ __forceinline__ void soft_pair(double dx, double dy, double dz, double Hi, double invHi,
                                           double Hj, double invHj, double mj, bool dead,
                                           double (&f)[PSI ? 5 : 4])
 {
     const double r2 = fma(dx, dx, fma(dy, dy, dz * dz));
     const bool apart = r2 > 0.0;
-    const double ri = apart ? rsqrt64<true>(apart ? r2 : 1.0) : 0.0;
+    const double ri = apart ? rsqrt64<FAST>(apart ? r2 : 1.0) : 0.0;
     const double r = r2 * ri;
     double gacc = 0.0, gpot = 0.0, ps = 0.0;
     side_select<NK>(r, ri, r2, Hi, invHi, gacc, gpot, PSI ? &ps : nullptr);
@@ -1056,13 +1056,73 @@ __device__ __forceinline__ void soft_pair(double dx, double dy, double dz, doubl
     if (PSI) f[PSI ? 4 : 0] = mj * ps;
 }
 
+// The pairs that visit_near and visit_near64 leave: bit 63 - jj of `mine` is the
+// lane's softened pair with jj of the staged chunk.  A lane has few of them and
+// the busiest several times the mean, and one costs some 300 dependent FP64
+// operations, so they are dealt over all lanes, 64 at a time, and each lane
+// collects the sums of its own.
+template <int NK, bool PSI, bool FAST>
+__device__ __forceinline__ void visit_soft(WaveLds &lds, uint64_t mine, const SortedSet &J,
+                                           int64_t j0c, double xr, double yr, double zr, double Hi,
+                                           double invHi, int idi, double (&acc)[PSI ? 5 : 4])
+{
+    constexpr int NS = PSI ? 5 : 4;
+    const NearSlice &sl = lds.sl;
+    const unsigned count = (unsigned)__builtin_popcountll(mine);
+    unsigned at, total;
+    list_places(count, at, total);
+    if (total > (unsigned)NSOFT) {
+        while (mine) {
+            const int jj = __builtin_clzll(mine);
+            mine &= ~(0x8000000000000000ull >> jj);
+            const double4 p = sl.p[jj];
+            const double hs = sl.hs[jj];
+            const double dx = p.x - xr, dy = p.y - yr, dz = p.z - zr;
+            // the self pair only matters at r = 0: the index is read then
+            const bool dead = dx == 0.0 && dy == 0.0 && dz == 0.0 && hs < 0.0 && J.idx[j0c + jj] == idi;
+            double f[NS];
+            soft_pair<NK, PSI, FAST>(dx, dy, dz, Hi, invHi, fabs(hs), sl.hinv[jj], sl.m[jj], dead, f);
+#pragma unroll
+            for (int k = 0; k < NS; ++k) acc[k] += f[k];
+        }
+        return;
+    }
+    const int lane = threadIdx.x & 63;
+    for (unsigned k = at; mine; ++k) {
+        const int jj = __builtin_clzll(mine);
+        mine &= ~(0x8000000000000000ull >> jj);
+        lds.list[k] = (uint16_t)(lane << 6 | jj);
+    }
+    for (unsigned b0 = 0; b0 < total; b0 += 64) {
+        wave_lds_sync();
+        const unsigned e = min(b0 + (unsigned)lane, total - 1);   // lanes past the end repeat the last
+        const int il = lds.list[e] >> 6, jj = lds.list[e] & 63;
+        const double4 p = sl.p[jj];
+        const double hs = sl.hs[jj];
+        const double H = __shfl(Hi, il, 64), invH = __shfl(invHi, il, 64);
+        const int id = __shfl(idi, il, 64);
+        const double dx = p.x - __shfl(xr, il, 64), dy = p.y - __shfl(yr, il, 64),
+                     dz = p.z - __shfl(zr, il, 64);
+        const bool dead = dx == 0.0 && dy == 0.0 && dz == 0.0 && hs < 0.0 && J.idx[j0c + jj] == id;
+        double f[NS];
+        soft_pair<NK, PSI, FAST>(dx, dy, dz, H, invH, fabs(hs), sl.hinv[jj], sl.m[jj], dead, f);
+#pragma unroll
+        for (int k = 0; k < NS; ++k) lds.res[k][lane] = f[k];
+        wave_lds_sync();
+        // each lane adds its own pairs, in the list's order
+        const unsigned hi = min(at + count, b0 + 64);
+        for (unsigned k = max(at, b0); k < hi; ++k) {
+#pragma unroll
+            for (int c = 0; c < NS; ++c) acc[c] += lds.res[c][k - b0];
+        }
+    }
+}
+
 // The visits below cover j = jb .. je - 1 of the staged chunk (multiples of
 // PG).  Near: differences formed in FP64 and rounded once, the FP32 body for every
 // pair (r^-1 = 0 for those that may be softened, r^2 < max(H_i^2, H_j^2) in
-// FP32, r = 0 included), and those in FP64.  A lane has few of them and the
-// busiest several times the mean, and one costs some 300 dependent FP64
-// operations, so they are dealt over all lanes, 64 at a time, and each lane
-// collects the sums of its own.  PSI also forms the grad-h sum (acc[4]).
+// FP32, r = 0 included), and those in FP64 (visit_soft).  PSI also forms the
+// grad-h sum (acc[4]).
 template <int NK, bool PSI>
 __device__ __forceinline__ void visit_near(WaveLds &lds, uint64_t real, const SortedSet &J,
                                            int64_t j0c, int jb, int je, double xr, double yr, double zr, double Hi,
@@ -1070,7 +1130,6 @@ __device__ __forceinline__ void visit_near(WaveLds &lds, uint64_t real, const So
                                            double (&acc)[PSI ? 5 : 4],
                                            unsigned &nfp64)
 {
-    constexpr int NS = PSI ? 5 : 4;
     const NearSlice &sl = lds.sl;
     const float hi2f = (float)hi2;
     uint64_t mine = 0;   // bit 63 - jj: the lane's pair with jj is softened
@@ -1104,54 +1163,36 @@ __device__ __forceinline__ void visit_near(WaveLds &lds, uint64_t real, const So
     }
     // the counter covers pairs of particles, not padding
     nfp64 += (unsigned)__builtin_popcountll(mine & __brevll(real));
-    const unsigned count = (unsigned)__builtin_popcountll(mine);
-    unsigned at, total;
-    list_places(count, at, total);
-    if (total > (unsigned)NSOFT) {
-        while (mine) {
-            const int jj = __builtin_clzll(mine);
-            mine &= ~(0x8000000000000000ull >> jj);
-            const double4 p = sl.p[jj];
-            const double hs = sl.hs[jj];
-            const double dx = p.x - xr, dy = p.y - yr, dz = p.z - zr;
-            // the self pair only matters at r = 0: the index is read then
-            const bool dead = dx == 0.0 && dy == 0.0 && dz == 0.0 && hs < 0.0 && J.idx[j0c + jj] == idi;
-            double f[NS];
-            soft_pair<NK, PSI>(dx, dy, dz, Hi, invHi, fabs(hs), sl.hinv[jj], sl.m[jj], dead, f);
-#pragma unroll
-            for (int k = 0; k < NS; ++k) acc[k] += f[k];
+    visit_soft<NK, PSI, true>(lds, mine, J, j0c, xr, yr, zr, Hi, invHi, idi, acc);
+}
+
+// Near and far chunks of an FP64 pass.
+template <int NK, bool NEAR>
+__device__ __forceinline__ void visit64(WaveLds &lds, const SortedSet &J, int64_t j0c, double xr,
+                                        double yr, double zr, double Hi, double invHi, double hi2,
+                                        int idi, double (&acc)[4])
+{
+    const NearSlice &sl = lds.sl;
+    uint64_t mine = 0;
+#pragma unroll 4
+    for (int j = 0; j < TC; ++j) {
+        const double4 p = sl.p[j];
+        const double dx = p.x - xr, dy = p.y - yr, dz = p.z - zr;
+        double r2 = fma(dx, dx, fma(dy, dy, dz * dz)), m = sl.m[j];
+        if (NEAR) {
+            const bool soft = r2 < fmax(hi2, sl.hs[j] * sl.hs[j]);
+            r2 = soft ? 1.0 : r2;
+            m = soft ? 0.0 : m;
+            mine = mine + mine + (soft ? 1u : 0u);
         }
-        return;
+        const double ri = rsqrt_pos64(r2);
+        const double mr = m * ri, mr3 = mr * ri * ri;
+        acc[0] = fma(mr3, dx, acc[0]);
+        acc[1] = fma(mr3, dy, acc[1]);
+        acc[2] = fma(mr3, dz, acc[2]);
+        acc[3] -= mr;
     }
-    const int lane = threadIdx.x & 63;
-    for (unsigned k = at; mine; ++k) {
-        const int jj = __builtin_clzll(mine);
-        mine &= ~(0x8000000000000000ull >> jj);
-        lds.list[k] = (uint16_t)(lane << 6 | jj);
-    }
-    for (unsigned b0 = 0; b0 < total; b0 += 64) {
-        wave_lds_sync();
-        const unsigned e = min(b0 + (unsigned)lane, total - 1);   // lanes past the end repeat the last
-        const int il = lds.list[e] >> 6, jj = lds.list[e] & 63;
-        const double4 p = sl.p[jj];
-        const double hs = sl.hs[jj];
-        const double H = __shfl(Hi, il, 64), invH = __shfl(invHi, il, 64);
-        const int id = __shfl(idi, il, 64);
-        const double dx = p.x - __shfl(xr, il, 64), dy = p.y - __shfl(yr, il, 64),
-                     dz = p.z - __shfl(zr, il, 64);
-        const bool dead = dx == 0.0 && dy == 0.0 && dz == 0.0 && hs < 0.0 && J.idx[j0c + jj] == id;
-        double f[NS];
-        soft_pair<NK, PSI>(dx, dy, dz, H, invH, fabs(hs), sl.hinv[jj], sl.m[jj], dead, f);
-#pragma unroll
-        for (int k = 0; k < NS; ++k) lds.res[k][lane] = f[k];
-        wave_lds_sync();
-        // each lane adds its own pairs, in the list's order
-        const unsigned hi = min(at + count, b0 + 64);
-        for (unsigned k = max(at, b0); k < hi; ++k) {
-#pragma unroll
-            for (int c = 0; c < NS; ++c) acc[c] += lds.res[c][k - b0];
-        }
-    }
+    if (NEAR) visit_soft<NK, false, false>(lds, mine, J, j0c, xr, yr, zr, Hi, invHi, idi, acc);
 }
 
 // Wide: as near, with every pair Newtonian.
@@ -1306,7 +1347,7 @@ __global__ __launch_bounds__(64) void k_pair_wave(PairArgs a)
 // meet thousands of chunks (those of the largest H, and those that straddle a
 // jump of the curve) do not outlast the rest.  The next chunk's particles are
 // loaded while the current one is evaluated.
-template <int NK>
+template <int NK, bool FP64>
 __global__ __launch_bounds__(64) void k_sym_rest(SymArgs a)
 {
     __shared__ WaveLds lds;
@@ -1349,10 +1390,11 @@ __global__ __launch_bounds__(64) void k_sym_rest(SymArgs a)
            jz = P.z[(int64_t)cj * TC + lane], jm = P.m[(int64_t)cj * TC + lane],
            jh = P.Hs[(int64_t)cj * TC + lane];
     for (;;) {
-        const Visit v = classify_visit(a.chunks[cj], Ox, Oy, Oz, px, py, pz, ph, rho2);
+        const Visit v =
+            classify_visit(a.chunks[cj], Ox, Oy, Oz, px, py, pz, ph, FP64 ? 0.0f : rho2);
         const double rx = jx - Ox, ry = jy - Oy, rz = jz - Oz;
         uint64_t real = 0;
-        if (v == VISIT_FAR) {
+        if (!FP64 && v == VISIT_FAR) {
             wave_lds_sync();
             reinterpret_cast<float4 *>(sl.p)[lane] =
                 make_float4((float)rx, (float)ry, (float)rz, (float)jm);
@@ -1371,9 +1413,15 @@ __global__ __launch_bounds__(64) void k_sym_rest(SymArgs a)
             jm = P.m[j];
             jh = P.Hs[j];
         }
-        if (v == VISIT_NEAR) {
-            ++nearv;
-            visit_near<NK, false>(lds, real, P, j0c, 0, TC, xr, yr, zr, Hi[0], invHi[0], hi2[0], idi[0], acc, nfp64);
+        if (v == VISIT_NEAR) ++nearv;
+        if (FP64) {
+            if (v == VISIT_NEAR)
+                visit64<NK, true>(lds, P, j0c, xr, yr, zr, Hi[0], invHi[0], hi2[0], idi[0], acc);
+            else
+                visit64<NK, false>(lds, P, j0c, xr, yr, zr, Hi[0], invHi[0], hi2[0], idi[0], acc);
+        } else if (v == VISIT_NEAR) {
+            visit_near<NK, false>(lds, real, P, j0c, 0, TC, xr, yr, zr, Hi[0], invHi[0], hi2[0],
+                                  idi[0], acc, nfp64);
         } else if (v == VISIT_WIDE) {
             ++widev;
             visit_wide(sl, 0, TC, xr, yr, zr, acc);
@@ -1815,10 +1863,13 @@ hipError_t launch_sym_rest(const SymArgs &a, hipStream_t s)
 {
     // as many waves as there can be segments; those past the last one end at once
     const dim3 grid((unsigned)(SYM_SEGS + a.nchunks)), block(64);
-    switch (a.nkernel) {
-    case 0: hipLaunchKernelGGL((k_sym_rest<0>), grid, block, 0, s, a); break;
-    case 1: hipLaunchKernelGGL((k_sym_rest<1>), grid, block, 0, s, a); break;
-    case 2: hipLaunchKernelGGL((k_sym_rest<2>), grid, block, 0, s, a); break;
+    switch (a.nkernel + (a.fp64 ? 3 : 0)) {
+    case 0: hipLaunchKernelGGL((k_sym_rest<0, false>), grid, block, 0, s, a); break;
+    case 1: hipLaunchKernelGGL((k_sym_rest<1, false>), grid, block, 0, s, a); break;
+    case 2: hipLaunchKernelGGL((k_sym_rest<2, false>), grid, block, 0, s, a); break;
+    case 3: hipLaunchKernelGGL((k_sym_rest<0, true>), grid, block, 0, s, a); break;
+    case 4: hipLaunchKernelGGL((k_sym_rest<1, true>), grid, block, 0, s, a); break;
+    case 5: hipLaunchKernelGGL((k_sym_rest<2, true>), grid, block, 0, s, a); break;
     default: return hipErrorInvalidValue;
     }
     return hipGetLastError();

@@ -78,6 +78,7 @@ struct PairArgs {
 // chunk is cut into segments with partial sums of their own: at most SYM_SEGS
 // + nchunks of them, of SYM_SEG_MIN chunk visits or more.
 constexpr int SYM_SEGS = 32768, SYM_SEG_MIN = 8;
+constexpr int SYM64_STEP = 8;   // superblocks of k_sym64 are multiples of this
 // A set of a batch: where its particles, chunks, bits and slabs begin in the
 // batch's arrays.  Segments are numbered over the whole batch.
 struct SymSet {
@@ -101,6 +102,7 @@ struct SymArgs {
     double *segsum;          // [SYM_SEGS + nchunks][4][TC]
     double *ax, *ay, *az, *pot;   // outputs, input order
     unsigned long long *stats;
+    bool fp64;               // FP64 throughout (k_sym64): no scales, no wide chunks
     // a batch: its sets, the work items (set, superblock pair) and each chunk's
     // set; nchunks and n then span the batch (null: one set)
     const SymSet *sets;
@@ -112,6 +114,7 @@ struct SymArgs {
 hipError_t launch_set_boxes(const SymArgs &a, int nsets, double *boxes, hipStream_t s);
 hipError_t launch_sym_classify(const SymArgs &a, hipStream_t s);
 hipError_t launch_sym(const SymArgs &a, hipStream_t s);
+hipError_t launch_sym64(const SymArgs &a, hipStream_t s);
 hipError_t launch_sym_rest(const SymArgs &a, hipStream_t s);   // sg_direct.hip
 hipError_t launch_sym_reduce(const SymArgs &a, hipStream_t s);
 
@@ -294,7 +297,7 @@ struct EvalPlan {
     int64_t flag_elems;    // near-flag bytes (FP64 and grad-h passes; else 1)
     int64_t psipart_elems; // grad-h partial sums: jsplit * ni (with psi; else 0)
     // each unordered far pair once (sg_sym.hip): jsplit counts its slabs
-    bool sym;
+    bool sym, fp64;
     bool wave;             // one wave per 64 i and j partition (k_pair_wave)
     int jsub;
     int sb, nsb, waves;
@@ -321,6 +324,11 @@ constexpr int WAVE_MAX_NI = 49151, WAVE_COUNT = 16384;
 // upper limit keeps the chunk-pair bits (N^2 / 32,768 bytes) at 512 MB and the
 // slabs at 17 GB; where the device cannot hold them the ordered pass runs.
 constexpr int SYM_MIN_N = 49152, SYM_MAX_N = 1 << 22, SYM_MAX_SB = 128;
+// FP64 passes do so from this size on.  Preparation and pair kernels, ordered
+// against unordered, same card: 20,000 particles 0.62 against 0.63 ms, 24,576
+// 0.85 against 0.80, 32,768 1.26 / 1.09, 65,537 4.16 / 2.82, 131,072 14.0 / 9.3,
+// 262,144 49.4 / 34.9.
+constexpr int SYM64_MIN_N = 24576;
 // FP32C batches at the default shape do so too, unless the average particle's
 // set is smaller than this (nearly all of its chunk pairs are then near, and
 // the one kernel of the ordered pass is shorter than five).  Ordered against

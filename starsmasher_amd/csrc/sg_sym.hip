@@ -88,6 +88,7 @@ __global__ __launch_bounds__(256) void k_sym_classify(SymArgs a)
         rh[r] = a.boxes[2 * ci + 1];
         rest[r] = a.nchunks;
     }
+    const float wide = a.fp64 ? 0.0f : WIDE_K * WIDE_K;
     for (int w = 0; w < a.words; ++w) {
         const int cj = w * 64 + lane;
         const int cc = min(cj, a.nchunks - 1);
@@ -102,7 +103,7 @@ __global__ __launch_bounds__(256) void k_sym_classify(SymArgs a)
             const float hm = fmaxf(cl.w, rl[r].w);
             const float rho2 = cj < ci ? ch.w : rh[r].w;
             const bool ok = cj < a.nchunks && cj != ci &&
-                            d2 > fmaxf(hm * hm, WIDE_K * WIDE_K * rho2) * (1.0f + FAR_MARGIN);
+                            d2 > fmaxf(hm * hm, wide * rho2) * (1.0f + FAR_MARGIN);
             const uint64_t bits = __ballot(ok);
             rest[r] -= __builtin_popcountll(bits);
             if (ci < a.nchunks && lane == 0) a.sym[(int64_t)ci * a.words + w] = bits;
@@ -435,7 +436,7 @@ __global__ __launch_bounds__(256) void k_sym_reduce(SymArgs a)
         for (int k = 0; k < 4; ++k) s[k] += p[k * a.n];
     }
     // back to the caller's units: a has m / r^2, the potential m / r
-    const double len = a.bbox[6], unit = 1.0 / a.bbox[7];
+    const double len = a.fp64 ? 1.0 : a.bbox[6], unit = a.fp64 ? 1.0 : 1.0 / a.bbox[7];
     s[0] *= len * len * unit;
     s[1] *= len * len * unit;
     s[2] *= len * len * unit;

@@ -261,7 +261,7 @@ static int64_t sym_words(int nchunks) { return (int64_t)nchunks * ((nchunks + 63
 // per particle each).  A workgroup has as many waves as its superblock has
 // column groups of four chunks, up to four; in FP64 always four, of two chunks
 // each.
-static void plan_sym(EvalPlan &p, int n, bool fp64)
+static void plan_sym(EvalPlan &p, int n, bool fp64, bool psi)
 {
     const int nchunks = (int)(p.padded / TC);
     const int want = (nchunks + SYM_MAX_SB - 1) / SYM_MAX_SB;
@@ -270,7 +270,8 @@ static void plan_sym(EvalPlan &p, int n, bool fp64)
     p.sb = (want + step - 1) / step * step;
     p.nsb = (nchunks + p.sb - 1) / p.sb;
     p.jsplit = p.nsb + 1;
-    p.part_elems = (int64_t)p.jsplit * 4 * n + ((int64_t)SYM_SEGS + nchunks) * 4 * TC;
+    p.part_elems = (int64_t)p.jsplit * 4 * n + ((int64_t)SYM_SEGS + nchunks) * (psi ? 5 : 4) * TC;
+    p.psipart_elems = 0;
     p.flag_elems = 1;
     p.sym_bytes = sym_layout(nchunks, sym_words(nchunks)).bytes;
     p.sym = true;
@@ -344,9 +345,9 @@ EvalPlan plan_eval(int n, int ni, int wg, int ipl, int jsplit_cfg, int precision
         p.flag_elems = 1;
         p.psipart_elems = psi ? (int64_t)p.jsplit * ni : 0;
     }
-    if (allow_sym && automatic && !psi && ni == n && n >= (fp64 ? SYM64_MIN_N : SYM_MIN_N) &&
+    if (allow_sym && automatic && ni == n && n >= (fp64 ? SYM64_MIN_N : SYM_MIN_N) &&
         n <= SYM_MAX_N)
-        plan_sym(p, n, fp64);
+        plan_sym(p, n, fp64, psi);
     return p;
 }
 
@@ -431,6 +432,7 @@ hipError_t enqueue_eval(const EvalPlan &p, const EvalBuffers &bufs, int n, int i
         y.ay = ay;
         y.az = az;
         y.pot = pot;
+        y.psi = psi;
         SG_ENQ(launch_sym_classify(y, s));
         if (ev) SG_ENQ(hipEventRecord(ev[1], s));
         SG_ENQ(p.fp64 ? launch_sym64(y, s) : launch_sym(y, s));
@@ -1233,7 +1235,7 @@ int sg_vjp_device(sg_context *c, int n, const double *x, const double *y, const 
     if (precision == SG_PREC_FP32C && n >= sg::ADJ_SYM_MIN_N && n <= sg::SYM_MAX_N) {
         sg::EvalPlan p{};
         p.padded = padded;
-        sg::plan_sym(p, n, false);
+        sg::plan_sym(p, n, false, false);
         p.waves = 4;
         p.sb = (p.sb + 7) / 8 * 8;   // whole column groups of k_adj_sym
         const int nchunks = (int)(padded / sg::TC);

@@ -99,8 +99,9 @@ struct SymArgs {
     int waves;               // waves per workgroup of k_sym (1, 2, 4)
     int nkernel;
     double *partial;         // [nsb + 1][4][n], sorted order
-    double *segsum;          // [SYM_SEGS + nchunks][4][TC]
+    double *segsum;          // [SYM_SEGS + nchunks][4 (5 with psi)][TC]
     double *ax, *ay, *az, *pot;   // outputs, input order
+    double *psi;             // the grad-h term (null: not formed)
     unsigned long long *stats;
     bool fp64;               // FP64 throughout (k_sym64): no scales, no wide chunks
     // a batch: its sets, the work items (set, superblock pair) and each chunk's

@@ -441,13 +441,19 @@ __global__ __launch_bounds__(256) void k_sym_reduce(SymArgs a)
     s[1] *= len * len * unit;
     s[2] *= len * len * unit;
     s[3] *= len * unit;
-    const int c = (int)(i / TC);
+    const int c = (int)(i / TC), ns = a.psi ? 5 : 4;
     const int e = a.seg[c + 1];
+    double psi = 0.0;
     for (int g = a.seg[c]; g < e; ++g) {
-        const double *p = a.segsum + (int64_t)g * 4 * TC + (i & (TC - 1));
+        const double *p = a.segsum + (int64_t)g * ns * TC + (i & (TC - 1));
         for (int k = 0; k < 4; ++k) s[k] += p[k * TC];
+        if (a.psi) psi += p[4 * TC];
     }
     const int64_t o = a.p.idx[i];
+    if (a.psi) {
+        const double H = a.p.Hs[i];   // point particles carry no grad-h term
+        a.psi[o] = H > 0.0 ? -2.0 * psi / (H * H) : 0.0;
+    }
     a.ax[o] = s[0];
     a.ay[o] = s[1];
     a.az[o] = s[2];

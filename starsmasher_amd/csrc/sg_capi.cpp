@@ -305,6 +305,8 @@ static SymArgs sym_args(const EvalPlan &p, int n, int nchunks, const PrepBuffers
     return y;
 }
 
+static_assert(SYM_MIN_N > SG_STATIC_MAX_N && SYM64_MIN_N > SG_STATIC_MAX_N,
+              "the static entry point and a context run the same pass");
 EvalPlan plan_eval(int n, int ni, int wg, int ipl, int jsplit_cfg, int precision, bool psi,
                    bool allow_sym)
 {

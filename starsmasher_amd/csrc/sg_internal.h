@@ -325,11 +325,12 @@ constexpr int WAVE_MAX_NI = 49151, WAVE_COUNT = 16384;
 // upper limit keeps the chunk-pair bits (N^2 / 32,768 bytes) at 512 MB and the
 // slabs at 17 GB; where the device cannot hold them the ordered pass runs.
 constexpr int SYM_MIN_N = 49152, SYM_MAX_N = 1 << 22, SYM_MAX_SB = 128;
-// FP64 passes do so from this size on.  Preparation and pair kernels, ordered
-// against unordered, same card: 20,000 particles 0.62 against 0.63 ms, 24,576
-// 0.85 against 0.80, 32,768 1.26 / 1.09, 65,537 4.16 / 2.82, 131,072 14.0 / 9.3,
-// 262,144 49.4 / 34.9.
-constexpr int SYM64_MIN_N = 24576;
+// FP64 passes do so above the static entry point's limit, whose results are
+// those of a context bit for bit and whose scratch holds no slabs.  Preparation
+// and pair kernels, ordered against unordered, same card: 20,000 particles 0.62
+// against 0.63 ms, 24,576 0.85 / 0.80, 32,768 1.26 / 1.09, 65,537 4.16 / 2.82,
+// 131,072 14.0 / 9.3, 262,144 49.4 / 34.9.
+constexpr int SYM64_MIN_N = 32769;
 // FP32C batches at the default shape do so too, unless the average particle's
 // set is smaller than this (nearly all of its chunk pairs are then near, and
 // the one kernel of the ordered pass is shorter than five).  Ordered against

@@ -1,7 +1,7 @@
 """The whole-set FP64 pass that evaluates each unordered far pair once
 (sg_sym64.hip), against the oracle and against the ordered pass.
 
-A context takes it at its automatic configuration from 24,576 particles on; an
+A context takes it at its automatic configuration from 32,769 particles on; an
 explicit j-split asks for the ordered pass.  Bounds: the FP64 errors of the other
 parity tests (1e-11 on the acceleration, 1e-12 on the potential); the two passes
 differ by no more than twice that.
@@ -24,11 +24,11 @@ def grav():
     g.close()
 
 
-# 24,575 and 24,576: the two sides of the rule; 24,577 and 65,537 end in a chunk
+# 32,768 and 32,769: the two sides of the rule; 32,769 and 65,537 end in a chunk
 # of one particle; from 65,537 on a superblock has two column groups, from
 # 131,073 three; 69,889 leaves one tile behind whole superblocks
 @pytest.mark.parametrize("kind,n,nk", [
-    ("plummer", 24575, 0), ("plummer", 24576, 1), ("two", 24577, 2), ("bigH", 30011, 0),
+    ("plummer", 32768, 0), ("two", 32769, 1), ("plummer", 34000, 2), ("bigH", 40011, 0),
     ("giant", 65536, 0), ("twins", 65537, 1), ("two", 69889, 2), ("plummer", 131073, 0),
 ])
 def test_against_oracle_and_ordered_pass(grav, kind, n, nk):
@@ -41,7 +41,7 @@ def test_against_oracle_and_ordered_pass(grav, kind, n, nk):
         np.testing.assert_array_equal(a, b)     # fixed order of every sum
     chunks = -(-n // 256) * 4
     assert 0 < nearv < visits and widev == 0 and fp64 == 0
-    if n >= 24576:
+    if n >= 32769:
         assert visits == chunks * chunks
     rng = np.random.default_rng(1)
     rows = np.unique(np.concatenate([rng.choice(n, 200, replace=False), [0, n - 1]]))
@@ -61,7 +61,7 @@ def test_against_oracle_and_ordered_pass(grav, kind, n, nk):
 @pytest.mark.parametrize("length,mass", [(1e11, 1e33), (1e-60, 1e-30)])
 def test_units(grav, length, mass):
     """r^-3 of FP64 pairs in units far from one."""
-    d = ics.plummer(25000, seed=3)
+    d = ics.plummer(33000, seed=3)
     g = grav.compute(d["x"], d["y"], d["z"], d["m"], d["range2"], precision=SG_PREC_FP64)
     s = grav.compute(d["x"] * length, d["y"] * length, d["z"] * length, d["m"] * mass,
                      d["range2"] * length ** 2, precision=SG_PREC_FP64)

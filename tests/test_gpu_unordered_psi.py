@@ -28,7 +28,7 @@ def grav():
 @pytest.mark.parametrize("kind,n,nk,prec", [
     ("plummer", 49151, 0, SG_PREC_FP32C), ("giant", 49152, 0, SG_PREC_FP32C),
     ("twins", 65537, 1, SG_PREC_FP32C), ("bigH", 50001, 2, SG_PREC_FP32C),
-    ("plummer", 24575, 1, SG_PREC_FP64), ("bigH", 24576, 0, SG_PREC_FP64),
+    ("plummer", 32768, 1, SG_PREC_FP64), ("bigH", 32769, 0, SG_PREC_FP64),
     ("twins", 40001, 2, SG_PREC_FP64),
 ])
 def test_grad_h_term(grav, kind, n, nk, prec):

@@ -775,16 +775,14 @@ int build_sym_plan(sg_context *c, const std::vector<sg::BatchSet> &sets)
     std::vector<int> setof((size_t)(P.padded / sg::TC));
     double pairs = 0.0;   // unordered chunk pairs of the batch
     double nsum = 0.0, nsq = 0.0;
-    P.sym_fits = true;
     for (const sg::BatchSet &b : sets) {
         const double nc = (double)b.ntiles * sg::CHUNKS;
         pairs += 0.5 * nc * nc;
         nsum += (double)b.n;
         nsq += (double)b.n * (double)b.n;
-        if (b.n > sg::SYM_MAX_N) P.sym_fits = false;
+        if (b.n > sg::SYM_MAX_N) return SG_OK;
     }
-    if (nsq < sg::BATCH_SYM_MEAN * nsum) P.sym_fits = false;
-    if (!P.sym_fits) return SG_OK;
+    if (nsq < sg::BATCH_SYM_MEAN * nsum) return SG_OK;
     const int sb = 16 * std::max(1, (int)std::ceil(std::sqrt(pairs / 8192.0) / 16.0));
     P.sym_words = P.sym_slabs = 0;
     for (int k = 0; k < nsets; ++k) {
@@ -818,6 +816,7 @@ int build_sym_plan(sg_context *c, const std::vector<sg::BatchSet> &sets)
     HIP_TRY(hipMemcpy(c->d_symsets, ss.data(), sizeof(sg::SymSet) * nsets, hipMemcpyHostToDevice));
     HIP_TRY(hipMemcpy(c->d_symitems, items.data(), sizeof(int2) * items.size(), hipMemcpyHostToDevice));
     HIP_TRY(hipMemcpy(c->d_setof, setof.data(), sizeof(int) * setof.size(), hipMemcpyHostToDevice));
+    P.sym_fits = true;
     return SG_OK;
 }
 
@@ -834,6 +833,7 @@ int build_sym_plan(sg_context *c, const std::vector<sg::BatchSet> &sets)
 int build_plan(sg_context *c, int nsets, const long long *offsets, int wg, int ipl)
 {
     auto &P = c->plan;
+    P.sym_fits = false;
     P.offsets.assign(offsets, offsets + nsets + 1);
     P.wg = wg;
     P.ipl = ipl;
@@ -910,7 +910,10 @@ int sg_compute_batch_device(sg_context *c, int nsets, const long long *offsets, 
     int rc;
     if (!same_plan) {
         HIP_TRY(hipStreamSynchronize(c->stream));
-        if ((rc = build_plan(c, nsets, offsets, wg, ipl)) != SG_OK) return rc;
+        if ((rc = build_plan(c, nsets, offsets, wg, ipl)) != SG_OK) {
+            P.offsets.clear();   // half built: the next call starts over
+            return rc;
+        }
     }
     if ((rc = ensure_capacity(c, ntot, P.padded, 1)) != SG_OK) return rc;
     // FP32C at the default shape: each unordered far pair once, where the device

@@ -144,12 +144,18 @@ int sg_compute_host(sg_context *ctx, int n, int ibeg, int ni,
  * for i-ranges of up to 65,536 particles and 256 above; ipl: i-particles per
  * lane (1 or 2); jsplit: number of j-partitions per i-block (>= 1, partial
  * sums are reduced in FP64 in a fixed order); 0 (the default) selects it
- * from n. */
+ * from n.  With ipl 1, jsplit 0 and wg 0 (or the size 0 stands for) the pass
+ * itself is chosen from n: FP32C i-ranges of up to 49,151 particles run one
+ * wave per 64 i and j partition; whole sets from 49,152 particles on (FP64:
+ * from 32,769) up to 2^22 evaluate each unordered far pair once, where the
+ * device holds the partial sums of up to 128 superblocks (32 B per particle
+ * each).  Every other call runs the ordered tile kernel of the given shape. */
 int sg_set_config(sg_context *ctx, int precision, int wg, int ipl, int jsplit);
 int sg_get_config(sg_context *ctx, int precision, int *wg, int *ipl, int *jsplit);
 /* The tile shape the last single-set evaluation on the context ran with
  * (sg_compute_device and the calls built on it, the automatic choices
- * resolved); SG_ERR_STATE before one, or when the last call was of another
+ * resolved; jsplit counts the partial-sum slabs of the pass that ran);
+ * SG_ERR_STATE before one, or when the last call was of another
  * kind (batch, psi-only, vector-Jacobian product). */
 int sg_last_config(sg_context *ctx, int *wg, int *ipl, int *jsplit);
 
@@ -158,11 +164,14 @@ int sg_last_config(sg_context *ctx, int *wg, int *ipl, int *jsplit);
  * offsets[s] .. offsets[s+1]-1 of the device arrays (offsets: HOST array of
  * nsets+1 entries, offsets[0] = 0, every set non-empty); particles interact
  * only within their set.  Outputs (device, length offsets[nsets]) are in
- * input order.  All sets run in one persistent launch whose workgroups take
- * (set, i-block, j-partition) items from a queue, longest first (sets of
- * more than 16,384 particles split their j range into partitions whose FP64
- * partial sums are added in a fixed order).  With use_graph the
- * queue reset, far, near and scatter kernels are captured once in a HIP graph
+ * input order.  All sets share each launch.  The default shape
+ * evaluates each unordered far pair once (work items of the largest sets
+ * first); other shapes, batches whose average particle sits in a set of
+ * fewer than 256, and sets above 2^22 run in one persistent launch whose
+ * workgroups take (set, i-block, j-partition) items from a queue, longest
+ * first (sets of more than 16,384 particles split their j range into
+ * partitions).  Partial sums are added in FP64 in a fixed order.  With
+ * use_graph the kernels after the preparation are captured once in a HIP graph
  * and replayed while the plan, pointers and precision stay the same; the
  * preparation (validation, sort, gather) runs eagerly before the replay.
  * Asynchronous like sg_compute_device; sg_synchronize reports validation. */
@@ -177,11 +186,11 @@ int sg_set_batch_config(sg_context *ctx, int precision, int wg, int ipl);
 int sg_get_batch_config(sg_context *ctx, int precision, int *wg, int *ipl);
 
 /* HIP-event timings of the last completed evaluation, in milliseconds:
- * prep = validation, curve sort, gather and tile boxes; far = the pair
- * kernel (in the FP32C forward pass it also takes the near chunks, listed
- * per wave and run after its far loop); near = the separate near-field
- * kernel where there is one (FP64 pass, grad-h pass, adjoint) plus the
- * final reduction.  Any pointer may be NULL. */
+ * prep = validation, curve sort, gather, tile boxes and chunk pairs; far = the
+ * pair kernels (near chunks included, except where a separate near-field
+ * kernel takes them: FP64, grad-h and adjoint passes of the ordered tile
+ * kernels); near = that kernel, if any, plus the final reduction (and, in the
+ * adjoint, the visits left to its rest kernel).  Any pointer may be NULL. */
 int sg_last_timings(sg_context *ctx, float *prep_ms, float *far_ms, float *near_ms);
 
 /* Statistics of the last evaluation: number of (wave, 64-particle j-chunk)
@@ -213,7 +222,7 @@ int sg_last_precision_stats(sg_context *ctx, long long *visits, long long *near_
  * on the CPU; here it is exact and comes out of the near-field pass that
  * already visits every pair with r < H_i.  psi (length ni, input order)
  * is written with ax..pot; other semantics as sg_compute_device / _host
- * (the pass runs the near kernel with one i per lane). */
+ * (the pass runs with one i per lane). */
 int sg_compute_psi_device(sg_context *ctx, int n, int ibeg, int ni,
                           const double *x, const double *y, const double *z,
                           const double *m, const double *range2,
@@ -227,7 +236,7 @@ int sg_compute_psi_host(sg_context *ctx, int n, int ibeg, int ni,
 
 /* The grad-h term alone (no accelerations), FP64: psi over the i-range as
  * in sg_compute_psi_device, from a pass that visits only the 64-particle
- * j-chunks within the i-group's largest H.  Replaces the psi part of
+ * j-chunks within reach of a particle of the i-group.  Replaces the psi part of
  * advance.f90:716-737 (bonetsumwithphi) at a fraction of a gravity
  * evaluation's cost.  Device pointers, asynchronous. */
 int sg_psi_device(sg_context *ctx, int n, int ibeg, int ni,
@@ -253,8 +262,10 @@ int sg_psi_host(sg_context *ctx, int n, int ibeg, int ni,
  * Device pointers, asynchronous on the context stream like
  * sg_compute_device (sg_synchronize reports validation, including
  * non-finite cotangents as SG_ERR_NONFINITE); sg_last_timings covers it.
- * The tile shape is the forward far kernel's workgroup size for the
- * precision (one i per lane). */
+ * SG_PREC_FP32C runs one wave per 64 particles and partition for sets below
+ * 32,768 particles and each unordered far pair once from there on to 2^22
+ * (where the device holds the partial sums); otherwise, and in FP64, the
+ * workgroup size is that of the forward kernel for the precision. */
 int sg_vjp_device(sg_context *ctx, int n,
                   const double *x, const double *y, const double *z,
                   const double *m, const double *range2, int nkernel, int precision,

@@ -81,7 +81,7 @@ struct sg_context {
         int wg = 0, ipl = 0;
         int64_t padded = 0, ngroups = 0, nflags = 0, nparts = 0;
         int nitems = 0;
-        // the unordered-pair form (FP32C at the default shape)
+        // the unordered-pair form (the default shape)
         int sym_items = 0, sym_chunks = 0;
         int64_t sym_slabs = 0, sym_words = 0;
         bool sym_fits = false;
@@ -916,9 +916,9 @@ int sg_compute_batch_device(sg_context *c, int nsets, const long long *offsets, 
         }
     }
     if ((rc = ensure_capacity(c, ntot, P.padded, 1)) != SG_OK) return rc;
-    // FP32C at the default shape: each unordered far pair once, where the device
-    // holds its slabs
-    bool sym = precision == SG_PREC_FP32C && wg == 256 && ipl == 1 && P.sym_fits;
+    // the default shape: each unordered far pair once, where the device holds its
+    // slabs
+    bool sym = wg == 256 && ipl == 1 && P.sym_fits;
     const sg::SymLayout layout = sg::sym_layout(P.sym_chunks, P.sym_words);
     if (sym && (grow(&c->partial, &c->cap_part,
                      P.sym_slabs + ((int64_t)sg::SYM_SEGS + P.sym_chunks) * 4 * sg::TC) != SG_OK ||
@@ -979,6 +979,7 @@ int sg_compute_batch_device(sg_context *c, int nsets, const long long *offsets, 
         u.n = ntot;
         u.nchunks = P.sym_chunks;
         u.waves = 4;
+        u.fp64 = precision == SG_PREC_FP64;
         u.nkernel = nkernel;
         u.partial = c->partial;
         u.segsum = c->partial + P.sym_slabs;
@@ -999,7 +1000,7 @@ int sg_compute_batch_device(sg_context *c, int nsets, const long long *offsets, 
         if (!sym) return sg::launch_batch(precision, a, wg, ipl, nwg, s);
         if ((e = sg::launch_set_boxes(u, nsets, c->d_setbox, s)) != hipSuccess) return e;
         if ((e = sg::launch_sym_classify(u, s)) != hipSuccess) return e;
-        if ((e = sg::launch_sym(u, s)) != hipSuccess) return e;
+        if ((e = u.fp64 ? sg::launch_sym64(u, s) : sg::launch_sym(u, s)) != hipSuccess) return e;
         if ((e = sg::launch_sym_rest(u, s)) != hipSuccess) return e;
         return sg::launch_sym_reduce(u, s);
     };

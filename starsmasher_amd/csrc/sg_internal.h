@@ -331,13 +331,13 @@ constexpr int SYM_MIN_N = 49152, SYM_MAX_N = 1 << 22, SYM_MAX_SB = 128;
 // against 0.63 ms, 24,576 0.85 / 0.80, 32,768 1.26 / 1.09, 65,537 4.16 / 2.82,
 // 131,072 14.0 / 9.3, 262,144 49.4 / 34.9.
 constexpr int SYM64_MIN_N = 32769;
-// FP32C batches at the default shape do so too, unless the average particle's
-// set is smaller than this (nearly all of its chunk pairs are then near, and
-// the one kernel of the ordered pass is shorter than five).  Ordered against
-// unordered, kernels, same card: 1,000 sets of 100 0.205 against 0.314 ms, 200
-// of 500 0.168 against 0.111, 64 of 4,096 1.06 against 0.69, 8 of 2,048 to
-// 131,072 3.77 against 2.53, 64 of these 43.8 against 33.2, four of 200,000
-// 48.5 against 35.2.
+// Batches at the default shape do so too, unless the average particle's set is
+// smaller than this (nearly all of its chunk pairs are then near, and the one
+// kernel of the ordered pass is shorter than five).  Ordered against unordered,
+// kernels, same card, FP32C (FP64): 1,000 sets of 100 0.205 against 0.314 ms, 200
+// of 500 0.168 / 0.111 (0.176 / 0.148), 64 of 4,096 1.06 / 0.69 (1.54 / 1.10), 8
+// of 2,048 to 131,072 3.77 / 2.53 (6.53 / 4.77), 64 of these 43.8 / 33.2 (88.2 /
+// 67.9), four of 200,000 48.5 / 35.2 (102.7 / 74.7).
 constexpr double BATCH_SYM_MEAN = 256.0;
 // FP32C adjoints from this size on evaluate each unordered far pair once
 // (sg_adjsym.hip), smaller ones run one wave per 64 i and j partition.  Whole

@@ -120,8 +120,13 @@ void k_sym64(SymArgs a)
     const int lane = threadIdx.x & 63;
     const int w = uniform_i(threadIdx.x >> 6);
     const int p = lane >> 3, q = lane & 7;
-    int bi, bj;
-    sym_item((int)blockIdx.x, a.nsb, bi, bj);
+    int bi, bj, item = (int)blockIdx.x;
+    if (a.sets) {
+        const int2 it = a.items[item];
+        a = sym_view(a, it.x);
+        item = uniform_i(it.y);
+    }
+    sym_item(item, a.nsb, bi, bj);
     const int ci0 = bi * a.sb, ci1 = min(ci0 + a.sb, a.nchunks);
     const int cj0 = bj * a.sb, cj1 = min(cj0 + a.sb, a.nchunks);
     const bool diag = bi == bj;
@@ -253,8 +258,8 @@ void k_sym64(SymArgs a)
 
 hipError_t launch_sym64(const SymArgs &a, hipStream_t s)
 {
-    if (a.sb % (NW * JC) != 0) return hipErrorInvalidConfiguration;
-    const dim3 grid((unsigned)(a.nsb * (a.nsb + 1) / 2));
+    if (!a.sets && a.sb % (NW * JC) != 0) return hipErrorInvalidConfiguration;
+    const dim3 grid((unsigned)(a.sets ? a.nitems : a.nsb * (a.nsb + 1) / 2));
     hipLaunchKernelGGL(k_sym64, grid, dim3(64 * NW), 0, s, a);
     return hipGetLastError();
 }

@@ -1,17 +1,18 @@
-"""FP32C batches that evaluate each unordered far pair once (the default batch
-shape), against the oracle and against the ordered batch kernel, which other
+"""Batches that evaluate each unordered far pair once (the default batch shape,
+both precisions), against the oracle and against the ordered batch kernel, which other
 shapes still run.
 
 Bounds: the library's stated FP32C errors (1e-5 on the acceleration, 1e-6 on
 the potential); both passes round each pair to FP32 and sum at most 32 pairs in
-FP32, so they differ by no more than twice that.
+FP32, so they differ by no more than twice that.  FP64: 1e-11 and 1e-12, as in the
+other parity tests.
 """
 import numpy as np
 import pytest
 
 import oracle
 from conftest import rel_errors
-from starsmasher_amd import SG_PREC_FP32C, Gravity, ics
+from starsmasher_amd import SG_PREC_FP32C, SG_PREC_FP64, Gravity, ics
 
 pytestmark = pytest.mark.gpu
 
@@ -32,18 +33,19 @@ def _scaled(d, length, mass):
     return e
 
 
-def _check(grav, sets, nk):
-    eager = grav.compute_batch(sets, nkernel=nk)
+def _check(grav, sets, nk, prec=SG_PREC_FP32C):
+    amax, pmax = (1e-5, 1e-6) if prec == SG_PREC_FP32C else (1e-11, 1e-12)
+    eager = grav.compute_batch(sets, nkernel=nk, precision=prec)
     for _ in range(2):   # capture, then replay
-        for r, g in zip(eager, grav.compute_batch(sets, nkernel=nk, use_graph=True)):
+        for r, g in zip(eager, grav.compute_batch(sets, nkernel=nk, precision=prec, use_graph=True)):
             for a, b in zip(r, g):
                 np.testing.assert_array_equal(a, b)
-    old = grav.get_batch_config(SG_PREC_FP32C)
-    grav.set_batch_config(SG_PREC_FP32C, 128, 1)
+    old = grav.get_batch_config(prec)
+    grav.set_batch_config(prec, 128, 1)
     try:
-        ordered = grav.compute_batch(sets, nkernel=nk)
+        ordered = grav.compute_batch(sets, nkernel=nk, precision=prec)
     finally:
-        grav.set_batch_config(SG_PREC_FP32C, *old)
+        grav.set_batch_config(prec, *old)
     rng = np.random.default_rng(4)
     for k, (d, r, o) in enumerate(zip(sets, eager, ordered)):
         n = d["x"].size
@@ -51,9 +53,9 @@ def _check(grav, sets, nk):
         ref = oracle.direct(d["x"], d["y"], d["z"], d["m"], d["range2"], nkernel=nk, rows=rows)
         if n > 1:
             ea, ep = rel_errors(np.stack(r[:3], -1)[rows], r[3][rows], np.stack(ref[:3], -1), ref[3])
-            assert ea.max() <= 1e-5 and ep.max() <= 1e-6, (k, n, ea.max(), ep.max())
+            assert ea.max() <= amax and ep.max() <= pmax, (k, n, ea.max(), ep.max())
             ea, ep = rel_errors(np.stack(r[:3], -1), r[3], np.stack(o[:3], -1), o[3])
-            assert ea.max() <= 2e-5 and ep.max() <= 2e-6, (k, n, ea.max(), ep.max())
+            assert ea.max() <= 2 * amax and ep.max() <= 2 * pmax, (k, n, ea.max(), ep.max())
         else:
             np.testing.assert_allclose(r[3], ref[3], rtol=1e-12)
 
@@ -62,6 +64,7 @@ def _check(grav, sets, nk):
 # of a tile and one more, of a superblock (1,024) and one more, of more than
 # 64 chunks (two words of bits); the largest last, first and alone; 320 chunks
 # and superblocks of 32 in a batch of 40 x 20,480
+@pytest.mark.parametrize("prec", [SG_PREC_FP32C, SG_PREC_FP64])
 @pytest.mark.parametrize("sizes,nk", [
     ([255] * 5, 0), ([256] * 5, 1),
     ([1, 1024, 1025, 257, 1, 4097, 70001], 0),
@@ -69,8 +72,9 @@ def _check(grav, sets, nk):
     ([33333], 1),
     ([20480] * 39 + [20481], 0),
 ])
-def test_sizes(grav, sizes, nk):
-    _check(grav, [ics.plummer(int(n), seed=17 * k + n) for k, n in enumerate(sizes)], nk)
+def test_sizes(grav, sizes, nk, prec):
+    _check(grav, [ics.plummer(int(n), seed=17 * k + n) for k, n in enumerate(sizes)], nk,
+           prec)
 
 
 def test_each_set_in_its_own_units(grav):

@@ -5,7 +5,13 @@
 // 256-wide shared-memory tiles, every pair through the full three-way softened
 // branch, float-float (Fast2Sum) accumulation of every term.
 //
-// Design here (wave64, VALU-bound):
+// Whole sets and batches take their far pairs from sg_sym.hip / sg_sym64.hip;
+// here are the visits these leave (k_sym_rest), the wave-sized work items of
+// small i-ranges (k_pair_wave), the grad-h term alone (k_psi_only) and the
+// ordered tile kernels, which run for explicit tile shapes, large parts of a
+// set and small FP64 sets.
+//
+// Design of the ordered tile kernels (wave64, VALU-bound):
 //   * particles arrive sorted along a Morton curve (sg_prep.hip), so an
 //     i-group of 64*IPL consecutive particles (one wave) and a j-tile of TJ
 //     consecutive particles (four chunks of TC) are both spatially compact;

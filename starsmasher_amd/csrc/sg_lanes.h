@@ -1,5 +1,5 @@
 // sg_lanes.h -- register reductions over the lanes of a wave and the work item
-// order shared by the unordered-pair kernels (sg_sym.hip, sg_adjsym.hip).
+// order shared by the unordered-pair kernels (sg_sym.hip, sg_sym64.hip, sg_adjsym.hip).
 #pragma once
 
 #include "sg_internal.h"

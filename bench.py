@@ -42,6 +42,9 @@ sys.path.insert(0, ROOT)
 
 METRIC = ("G pair-interactions/s at N=1M: FP32+comp vs FP64 GPU, max rel acc err ≤1e-5")
 FLOPS_PER_PAIR = 19           # 3 dr + 5 r^2 + 1 rsqrt + 3 (r^-2, m r^-1, m r^-3) + 6 acc + 1 pot
+# a pair evaluated once for both sides: 3 dr + 5 r^2 + 1 rsqrt + 2 (r^-2, r^-3)
+# + 2 (m r^-3) + 12 acc + 4 pot
+FLOPS_PER_UNORDERED_PAIR = 29
 PEAK_FP32_TFLOPS = 157.3      # MI355X FP32 vector (AMD spec)
 PEAK_FP64_TFLOPS = 78.6
 TC = 64                       # j per chunk (the unit of the near / wide decisions)
@@ -486,9 +489,9 @@ def time_adjoint(g, n_adj, steps, log_fn):
 
 
 def profiled_traffic(wg, ipl):
-    """HBM bytes per launch of the far kernel for this tile shape, from the
-    committed rocprofv3 FETCH_SIZE + WRITE_SIZE summary (None if absent)."""
-    path = os.path.join(ROOT, "profiles", "k_far_fp32c_giant1m.md")
+    """HBM bytes per launch of the far-pair kernel at the default shape, from
+    the committed rocprofv3 FETCH_SIZE + WRITE_SIZE summary (None if absent)."""
+    path = os.path.join(ROOT, "profiles", "k_sym_giant1m.md")
     try:
         for ln in open(path):
             if ln.startswith("traffic_bytes_per_launch"):
@@ -610,10 +613,18 @@ def main():
     visits, nearv = r32["stats"][:2]
     near_frac = nearv / max(1, visits)
     padded = -(-n // 256) * 256
-    # the FP32C pass is one kernel over every (i, padded j) pair: far chunks
-    # and near chunks alike, each counted at the same 19 flops
+    # the pair kernels cover every (i, padded j) pair, far and near alike.  At
+    # the default shape a far pair is evaluated once for both sides: those
+    # flops are counted, not the ones of the two ordered pairs it replaces
     kernel_pairs = float(n) * padded
-    achieved = FLOPS_PER_PAIR * kernel_pairs / (r32["far_ms"] * 1e-3) / 1e12
+
+    def executed_flops(prec):
+        w, i, js = g.get_config(prec)
+        once = i == 1 and js == 0 and w in (0, 256) and 65536 < n <= 1 << 22
+        return once, kernel_pairs * (FLOPS_PER_UNORDERED_PAIR / 2 if once else FLOPS_PER_PAIR)
+
+    once, flops = executed_flops(SG_PREC_FP32C)
+    achieved = flops / (r32["far_ms"] * 1e-3) / 1e12
 
     acc = {}
     if r64 is not None:
@@ -651,8 +662,8 @@ def main():
         "roofline": {"bound": "valu", "achieved": round(achieved, 3), "peak": PEAK_FP32_TFLOPS,
                      "unit": "TFLOP/s", "frac": round(achieved / PEAK_FP32_TFLOPS, 4),
                      "traffic": (profiled_traffic(wg, ipl) if args.workload == "giant1m" else None),
-                     "kernel": "k_far_fp32c",
-                     "flops_per_pair": FLOPS_PER_PAIR,
+                     "kernel": "k_sym + k_sym_rest" if once else "k_far_fp32c",
+                     "flops_per_pair": flops / kernel_pairs,
                      "pairs_per_launch": kernel_pairs, "kernel_ms": round(r32["far_ms"], 3)},
         "phases_ms": {"prep": round(r32["prep_ms"], 3), "pair_kernel": round(r32["far_ms"], 3),
                       "reduce": round(r32["near_ms"], 3)},
@@ -670,8 +681,8 @@ def main():
     line.update(extra)
     if r64 is not None:
         v64 = pairs / (r64["ms_per_step"] * 1e-3) / 1e9
-        # the FP64 far kernel skips the near chunks (a separate kernel takes them)
-        a64 = FLOPS_PER_PAIR * kernel_pairs * (1.0 - near_frac) / (r64["far_ms"] * 1e-3) / 1e12
+        # far and near kernels together
+        a64 = executed_flops(SG_PREC_FP64)[1] / ((r64["far_ms"] + r64["near_ms"]) * 1e-3) / 1e12
         line["fp64_kernel"] = {"value": round(v64, 3), "unit": "Gpairs/s",
                                "ms_per_step": round(r64["ms_per_step"], 3),
                                "far_kernel_ms": round(r64["far_ms"], 3),

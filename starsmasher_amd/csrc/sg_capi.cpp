@@ -692,8 +692,9 @@ int sg_psi_device(sg_context *c, int n, int ibeg, int ni, const double *x, const
     a.ntiles = ntiles;
     a.ipl = 1;
     a.ngroups = (ni + 63) / 64;
-    // parts of a group's chunks, for some 8,192 waves
-    a.jsplit = (int)std::max<int64_t>(1, std::min<int64_t>(16, 8192 / a.ngroups));
+    // parts of a group's chunks, a power of two, for some PSI_WAVES waves
+    a.jsplit = 1;
+    while (a.jsplit < sg::PSI_MAX_PARTS && a.jsplit * a.ngroups < sg::PSI_WAVES) a.jsplit *= 2;
     a.psi = psi;
     if ((rc = grow(&c->psipart, &c->cap_psipart, (int64_t)a.jsplit * ni)) != SG_OK) return rc;
     a.psipart = c->psipart;

@@ -1458,15 +1458,19 @@ __global__ __launch_bounds__(64) void k_sym_rest(SymArgs a)
 // ------------------------------------------------- grad-h term on its own
 // psi_i = -(2/H_i^2) sum_{j: r <= H_i} m_j (P(q_i) + q_i^2 A(q_i)) of the
 // gas particles of the i-set, without the accelerations.  One wave per
-// 64-particle i-group and part: its lanes test 64 tiles at a time against the
-// group's box (r <= H_i needs only the wave's largest H), the parts deal the
-// chunks that cannot be ruled out among themselves, and the pairs within H_i
-// of a chunk are listed and dealt over the lanes (as in visit_near), since a
-// lane has about one in a chunk.  FP64 throughout.  65,536 particles: 0.4 ms;
-// with one wave a group testing tile after tile and every pair's polynomial
-// under its own branch 5.0 ms.
+// 64-particle i-group and part (every jsplit-th chunk): its lanes test 64 tiles
+// at a time against the group's box (r <= H_i needs only the wave's largest H),
+// then chunks, then each chunk against every lane's own reach.  The pairs of a
+// chunk that may be within H_i (an FP32 test with a margin for its rounding)
+// are listed and dealt over the lanes as in visit_soft, since a lane has about
+// one in a chunk, and decided and evaluated in FP64.  What bounds it are the
+// chunk tests of the groups whose box or largest H reaches most of the set, so
+// the parts share the tests and not only the visits.  65,536 particles: kernel
+// 0.50 ms with every part testing all chunks, whole call 0.88 -> 0.57 ms (0.80
+// from the FP32 test alone); 200,000 2.47 -> 1.49 ms.
 struct PsiLds {
     double4 p[TC];
+    float4 f[TC];             // the positions rounded to FP32
     uint16_t list[NSOFT];
     double res[64];
 };
@@ -1476,6 +1480,7 @@ __device__ __forceinline__ double psi_pair(double dx, double dy, double dz, doub
                                            double mj)
 {
     const double r2 = fma(dx, dx, fma(dy, dy, dz * dz));
+    if (r2 > H * H) return 0.0;   // listed by the FP32 test's margin
     const bool apart = r2 > 0.0;
     const double ri = apart ? rsqrt_pos64(apart ? r2 : 1.0) : 0.0;
     const double r = r2 * ri, q = r * invH;
@@ -1486,17 +1491,23 @@ __device__ __forceinline__ double psi_pair(double dx, double dy, double dz, doub
 }
 
 template <int NK>
-__device__ __forceinline__ void psi_visit(PsiLds &lds, double xr, double yr, double zr, double Hi,
-                                          double invHi, double hi2, double &ps)
+__device__ __forceinline__ void psi_visit(PsiLds &lds, double xr, double yr, double zr, float px,
+                                          float py, float pz, double Hi, double invHi, float cand2,
+                                          double &ps)
 {
     const int lane = threadIdx.x & 63;
-    uint64_t mine = 0;   // bit jj: the pair with jj is within H_i
-#pragma unroll 4
-    for (int jj = 0; jj < TC; ++jj) {
-        const double4 p = lds.p[jj];
-        const double dx = p.x - xr, dy = p.y - yr, dz = p.z - zr;
-        const bool in = fma(dx, dx, fma(dy, dy, dz * dz)) <= hi2;
-        mine |= (uint64_t)(in ? 1u : 0u) << jj;
+    uint64_t mine = 0;   // bit jj: the pair with jj may be within H_i
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        unsigned list = 0;
+#pragma unroll 8
+        for (int jj = 31; jj >= 0; --jj) {
+            const float4 p = lds.f[32 * h + jj];
+            const float dx = p.x - px, dy = p.y - py, dz = p.z - pz;
+            const bool in = fmaf(dx, dx, fmaf(dy, dy, dz * dz)) <= cand2;
+            list = list + list + (in ? 1u : 0u);
+        }
+        mine |= (uint64_t)list << (32 * h);
     }
     const unsigned count = (unsigned)__builtin_popcountll(mine);
     unsigned at, total;
@@ -1554,16 +1565,26 @@ __global__ __launch_bounds__(64) void k_psi_only(PairArgs a)
     const float lim2 = hmax * hmax * (1.0f + FAR_MARGIN);
     const float px = (float)xr, py = (float)yr, pz = (float)zr;
     const float reach2 = (float)hi2 * (1.0f + FAR_MARGIN);
+    // |x - O| of the lane's particle and of all j within its reach, largest axis
+    const float pmax = fmaxf(fabsf(px), fmaxf(fabsf(py), fabsf(pz)));
+    // r as FP32 sees it is off by at most sqrt(3) (2^-24 (2 pmax + r) + the
+    // subtraction's 2^-24 r) + 3 2^-24 r < 2^-22 (pmax + 2 r) for r <= H_i
+    const float cand = (float)Hi * (1.0f + 2.0e-6f) + 4.8e-7f * pmax;
+    const float cand2 = cand * cand;
     double ps = 0.0;
-    int cnt = 0;   // wave-uniform: chunks met so far, modulo the parts
+    // part p has every jsplit-th chunk (jsplit a power of two), of the tiles
+    // that hold one of them
+    const int other = a.jsplit - 1;
     for (int tb = 0; tb < a.ntiles; tb += 64) {
         const int tl = min(tb + lane, a.ntiles - 1);
         uint64_t tiles = __ballot(tb + lane < a.ntiles &&
+                                  ((tl * CHUNKS ^ part) & other & ~(CHUNKS - 1)) == 0 &&
                                   box_dist2(a.tiles[tl], Ox, Oy, Oz, bl, bh) <= lim2);
         for (; tiles; tiles &= tiles - 1) {
             const int64_t c0 = (int64_t)(tb + __builtin_ctzll(tiles)) * CHUNKS;
             unsigned bits = (unsigned)__ballot(
-                lane < CHUNKS && box_dist2(a.chunks[c0 + (lane & (CHUNKS - 1))], Ox, Oy, Oz, bl, bh) <= lim2);
+                lane < CHUNKS && ((lane ^ part) & other & (CHUNKS - 1)) == 0 &&
+                box_dist2(a.chunks[c0 + (lane & (CHUNKS - 1))], Ox, Oy, Oz, bl, bh) <= lim2);
             for (; bits; bits &= bits - 1) {
                 // the group's box and largest H pass many chunks that no lane's
                 // own particle reaches
@@ -1572,14 +1593,13 @@ __global__ __launch_bounds__(64) void k_psi_only(PairArgs a)
                 const float gy = fmaxf(0.0f, fmaxf((float)(cm.lo[1] - Oy) - py, py - (float)(cm.hi[1] - Oy)));
                 const float gz = fmaxf(0.0f, fmaxf((float)(cm.lo[2] - Oz) - pz, pz - (float)(cm.hi[2] - Oz)));
                 if (!__ballot(fmaf(gx, gx, fmaf(gy, gy, gz * gz)) <= reach2)) continue;
-                const int at = cnt;
-                cnt = cnt + 1 == a.jsplit ? 0 : cnt + 1;
-                if (at != part) continue;
                 const int64_t j = (c0 + __builtin_ctz(bits)) * TC + lane;
                 wave_lds_sync();
-                lds.p[lane] = make_double4(a.j.x[j] - Ox, a.j.y[j] - Oy, a.j.z[j] - Oz, a.j.m[j]);
+                const double jx = a.j.x[j] - Ox, jy = a.j.y[j] - Oy, jz = a.j.z[j] - Oz;
+                lds.p[lane] = make_double4(jx, jy, jz, a.j.m[j]);
+                lds.f[lane] = make_float4((float)jx, (float)jy, (float)jz, 0.0f);
                 wave_lds_sync();
-                psi_visit<NK>(lds, xr, yr, zr, Hi, invHi, hi2, ps);
+                psi_visit<NK>(lds, xr, yr, zr, px, py, pz, Hi, invHi, cand2, ps);
             }
         }
     }

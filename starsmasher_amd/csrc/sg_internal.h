@@ -325,6 +325,11 @@ constexpr int WAVE_MAX_NI = 49151, WAVE_COUNT = 16384;
 // upper limit keeps the chunk-pair bits (N^2 / 32,768 bytes) at 512 MB and the
 // slabs at 17 GB; where the device cannot hold them the ordered pass runs.
 constexpr int SYM_MIN_N = 49152, SYM_MAX_N = 1 << 22, SYM_MAX_SB = 128;
+// psi alone: the waves a launch aims at, and the most parts of a group's chunks.
+// Whole calls at 8,192 waves (16 parts at most) / 16,384 (16) / 32,768 (64) /
+// 65,536 (64), same card: 20,000 particles 0.47 / 0.47 / 0.39 / 0.39 ms, 65,536
+// 0.57 / 0.56 / 0.57 / 0.59, 200,000 1.75 / 1.54 / 1.49 / 1.52.
+constexpr int PSI_WAVES = 32768, PSI_MAX_PARTS = 64;
 // FP64 passes do so above the static entry point's limit, whose results are
 // those of a context bit for bit and whose scratch holds no slabs.  Preparation
 // and pair kernels, ordered against unordered, same card: 20,000 particles 0.62

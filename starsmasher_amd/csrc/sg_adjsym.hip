@@ -178,9 +178,8 @@ void k_adj_sym(AdjSymArgs a)
             // the wave whose turn it is fetches the next row chunk
             if (ci + 1 < ce && ((ci + 1) & (NW - 1)) == w) {
                 const int64_t i = (int64_t)(ci + 1) * TC + lane;
-                const TileMeta &m = y.chunks[ci + 1];
-                const double ox = 0.5 * (m.lo[0] + m.hi[0]), oy = 0.5 * (m.lo[1] + m.hi[1]),
-                             oz = 0.5 * (m.lo[2] + m.hi[2]);
+                double ox, oy, oz;
+                chunk_centre(y.chunks + ci + 1, ox, oy, oz);
                 const double mi = y.p.m[i] * unit, wx = a.wx[i], wy = a.wy[i], wz = a.wz[i];
                 const int nb = (ci + 1) & 1;
                 lds.xi[nb][lane] = make_float4((float)((y.p.x[i] - ox) * len),
@@ -199,14 +198,14 @@ void k_adj_sym(AdjSymArgs a)
             if (ci >= ci0) {
                 unsigned bits = 0;
                 if (cw < cj1)
-                    bits = (unsigned)(y.sym[(int64_t)ci * y.words + (cw >> 6)] >> (cw & 63)) & 0x3u;
+                    bits = (unsigned)(load_scalar(y.sym + (int64_t)ci * y.words + (cw >> 6)) >> (cw & 63)) &
+                           0x3u;
                 if (cw + JC > cj1) bits &= (1u << max(0, cj1 - cw)) - 1u;
                 if (diag) bits &= ci < cw ? 0x3u : (ci - cw >= JC ? 0u : 0x3u & (0x2u << (ci - cw)));
                 bits = (unsigned)uniform_i((int)bits);
                 if (bits) {
-                    const TileMeta &m = y.chunks[ci];
-                    const double cx = 0.5 * (m.lo[0] + m.hi[0]), cy = 0.5 * (m.lo[1] + m.hi[1]),
-                                 cz = 0.5 * (m.lo[2] + m.hi[2]);
+                    double cx, cy, cz;
+                    chunk_centre(y.chunks + ci, cx, cy, cz);
                     wave_lds_sync();
 #pragma unroll
                     for (int c = 0; c < JC; ++c) {

@@ -306,14 +306,11 @@ void k_sym(SymArgs a)
             double ox = 0.0, oy = 0.0, oz = 0.0;
             if (fetch) {
                 const int64_t i = (int64_t)(ci + 1) * TC + lane;
-                const TileMeta &m = a.chunks[ci + 1];
                 nx = a.p.x[i];
                 ny = a.p.y[i];
                 nz = a.p.z[i];
                 nm = a.p.m[i];
-                ox = 0.5 * (m.lo[0] + m.hi[0]);
-                oy = 0.5 * (m.lo[1] + m.hi[1]);
-                oz = 0.5 * (m.lo[2] + m.hi[2]);
+                chunk_centre(a.chunks + ci + 1, ox, oy, oz);
             }
             double old[4] = {0.0, 0.0, 0.0, 0.0};
             const int64_t irow = (int64_t)ci * TC + lane;
@@ -324,15 +321,15 @@ void k_sym(SymArgs a)
                 const int buf = ci & 1;
                 unsigned bits = 0;
                 if (cw < cj1)
-                    bits = (unsigned)(a.sym[(int64_t)ci * a.words + (cw >> 6)] >> (cw & 63)) & 0xfu;
+                    bits = (unsigned)(load_scalar(a.sym + (int64_t)ci * a.words + (cw >> 6)) >> (cw & 63)) &
+                           0xfu;
                 if (cw + JC > cj1) bits &= (1u << max(0, cj1 - cw)) - 1u;
                 if (diag) bits &= ci < cw ? 0xfu : (ci - cw >= JC ? 0u : 0xfu & (0xeu << (ci - cw)));
                 bits = (unsigned)uniform_i((int)bits);
                 float si[IA][4];
                 if (bits) {
-                    const TileMeta &m = a.chunks[ci];
-                    const double cx = 0.5 * (m.lo[0] + m.hi[0]), cy = 0.5 * (m.lo[1] + m.hi[1]),
-                                 cz = 0.5 * (m.lo[2] + m.hi[2]);
+                    double cx, cy, cz;
+                    chunk_centre(a.chunks + ci, cx, cy, cz);
                     wave_lds_sync();
 #pragma unroll
                     for (int c = 0; c < JC; ++c)

@@ -89,6 +89,11 @@ enum sg_precision {
 const char *sg_status_string(int status);
 int sg_last_status(void);         /* status of the last legacy-layer call */
 int sg_device_count(int *count);
+/* The dynamic linker's counts of shared objects loaded into and unloaded from
+ * the process so far (dl_iterate_phdr's dlpi_adds and dlpi_subs): what a caller
+ * found out about the loaded objects holds while both stand still.
+ * SG_ERR_STATE where the C library keeps no such counts. */
+int sg_loader_counts(unsigned long long *adds, unsigned long long *subs);
 
 typedef struct sg_context sg_context;
 

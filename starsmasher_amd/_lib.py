@@ -43,6 +43,7 @@ EXPORTS = (
     "sg_firsthalf", "sg_lasthalf", "sg_vjp_device", "sg_vjp_host", "sg_compute_psi_device",
     "sg_compute_psi_host", "sg_psi_device", "sg_psi_host", "sg_grav_psi", "sg_potential_energy",
     "sg_last_precision_stats", "sg_compute_device_static", "sg_last_config",
+    "sg_loader_counts",
 )
 
 
@@ -80,6 +81,7 @@ def load() -> C.CDLL:
     L.sg_status_string.restype = C.c_char_p
     L.sg_last_status.argtypes = []
     L.sg_device_count.argtypes = [_ip]
+    L.sg_loader_counts.argtypes = [C.POINTER(C.c_ulonglong)] * 2
     L.sg_create.argtypes = [C.c_int, C.POINTER(_vp)]
     L.sg_destroy.argtypes = [_vp]
     L.sg_compute_device.argtypes = [_vp, C.c_int, C.c_int, C.c_int] + [_vp] * 5 + [C.c_int, C.c_int] + [_vp] * 4
@@ -122,7 +124,7 @@ def load() -> C.CDLL:
                  "sg_firsthalf", "sg_lasthalf", "sg_vjp_device", "sg_vjp_host",
                  "sg_compute_psi_device", "sg_compute_psi_host", "sg_psi_device",
                  "sg_psi_host", "sg_grav_psi", "sg_potential_energy", "sg_last_precision_stats",
-                 "sg_compute_device_static", "sg_last_config"):
+                 "sg_compute_device_static", "sg_last_config", "sg_loader_counts"):
         getattr(L, name).restype = C.c_int
     _lib = L
     return L

@@ -13,8 +13,11 @@
 #include "sphgrav.h"
 #include "sg_internal.h"
 
+#include <link.h>
+
 #include <algorithm>
 #include <cmath>
+#include <cstddef>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -487,6 +490,29 @@ int sg_device_count(int *count)
     if (hipGetDeviceCount(&n) != hipSuccess) n = 0;
     *count = n;
     return n > 0 ? SG_OK : SG_ERR_NO_DEVICE;
+}
+
+// dl_iterate_phdr holds the linker's lock while it calls back, so the callback
+// is C and waits for nothing: in Python it would wait for the interpreter lock,
+// which a thread that loads an object may hold while it waits for the linker's.
+int sg_loader_counts(unsigned long long *adds, unsigned long long *subs)
+{
+    if (!adds || !subs) return SG_ERR_ARG;
+    unsigned long long out[3] = {0, 0, 0};   // adds, subs, whether they are kept
+    dl_iterate_phdr(
+        [](struct dl_phdr_info *info, size_t size, void *data) {
+            unsigned long long *o = (unsigned long long *)data;
+            if (size >= offsetof(struct dl_phdr_info, dlpi_subs) + sizeof(info->dlpi_subs)) {
+                o[0] = info->dlpi_adds;
+                o[1] = info->dlpi_subs;
+                o[2] = 1;
+            }
+            return 1;   // the counts are the same in every entry
+        },
+        out);
+    *adds = out[0];
+    *subs = out[1];
+    return out[2] ? SG_OK : SG_ERR_STATE;
 }
 
 int sg_create(int device, sg_context **out)

@@ -129,22 +129,6 @@ def hip_runtimes() -> list:
     return sorted(paths)
 
 
-class _DlInfo(C.Structure):
-    """struct dl_phdr_info up to the load counters (glibc's <link.h>)."""
-    _fields_ = [("addr", C.c_void_p), ("name", C.c_char_p), ("phdr", C.c_void_p),
-                ("phnum", C.c_uint16), ("adds", C.c_ulonglong), ("subs", C.c_ulonglong)]
-
-
-_dl_counts = [0, 0]
-
-
-@C.CFUNCTYPE(C.c_int, C.POINTER(_DlInfo), C.c_size_t, C.c_void_p)
-def _dl_first(info, size, _):
-    _dl_counts[0], _dl_counts[1] = info.contents.adds, info.contents.subs
-    return 1   # the counters are the same in every entry
-
-
-_dl_iterate_phdr = C.CDLL(None).dl_iterate_phdr
 _one_runtime_at = None   # the load counters when a single HIP runtime was last seen
 
 
@@ -159,10 +143,10 @@ def _check_shared_runtime(name):
     stands until a shared object is loaded or unloaded (the dynamic linker's
     own counters, 2 us)."""
     global _one_runtime_at
-    _lib.load()
-    _dl_iterate_phdr(_dl_first, None)
-    at = tuple(_dl_counts)
-    if at == _one_runtime_at:
+    adds, subs = C.c_ulonglong(), C.c_ulonglong()
+    counted = _lib.load().sg_loader_counts(C.byref(adds), C.byref(subs)) == _lib.SG_OK
+    at = (adds.value, subs.value)
+    if counted and at == _one_runtime_at:
         return
     rts = hip_runtimes()
     if len(rts) != 1:
@@ -170,7 +154,7 @@ def _check_shared_runtime(name):
                         f"{len(rts)} HIP runtimes ({', '.join(rts)}), and device pointers "
                         "and streams of one are invalid in another; allocate with "
                         "starsmasher_amd.hipmem.DeviceArray")
-    _one_runtime_at = at
+    _one_runtime_at = at if counted else None
 
 
 def _is_torch(t) -> bool:

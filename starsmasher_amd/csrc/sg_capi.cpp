@@ -145,73 +145,72 @@ int grow(T **p, int64_t *cap, int64_t need)
     return SG_OK;
 }
 
+// `count` arrays of one capacity.  The capacity reads 0 until all of them have
+// grown, so that a call after a failed allocation allocates them anew.
+template <typename T>
+int grow_all(T **p, int count, int64_t *cap, int64_t need)
+{
+    if (need <= *cap) return SG_OK;
+    *cap = 0;
+    for (int k = 0; k < count; ++k) {
+        int64_t none = 0;
+        const int rc = grow(&p[k], &none, need);
+        if (rc != SG_OK) return rc;
+    }
+    *cap = need;
+    return SG_OK;
+}
+
 // Capacity for n input particles (keys), `padded` sorted slots and ni
-// i-particles.
+// i-particles.  Each group's capacity reads 0 until all of it has grown.
 int ensure_capacity(sg_context *c, int64_t n, int64_t padded, int64_t ni)
 {
-    if (n > c->cap_n || !c->pb.keys_in) {
-        int64_t cap = 0;
-        const int64_t need = std::max<int64_t>(n, 1);
-        int rc;
-        if ((rc = grow(&c->pb.keys_in, &cap, need)) != SG_OK) return rc;
-        cap = 0;
-        if ((rc = grow(&c->pb.keys_out, &cap, need)) != SG_OK) return rc;
-        cap = 0;
-        if ((rc = grow(&c->pb.vals_in, &cap, need)) != SG_OK) return rc;
-        cap = 0;
-        if ((rc = grow(&c->pb.vals_out, &cap, need)) != SG_OK) return rc;
+    sg::PrepBuffers &b = c->pb;
+    int64_t none;   // of a buffer whose capacity is its group's
+    int rc;
+#define SG_GROW(p, need)                                               \
+    do {                                                               \
+        none = 0;                                                      \
+        if ((rc = grow(&(p), &none, (need))) != SG_OK) return rc;      \
+    } while (0)
+    if (n > c->cap_n) {
+        c->cap_n = 0;
+        SG_GROW(b.keys_in, n);
+        SG_GROW(b.keys_out, n);
+        SG_GROW(b.vals_in, n);
+        SG_GROW(b.vals_out, n);
         size_t bytes = 0;
-        HIP_TRY(sg::sort_pairs_temp_bytes((int)need, &bytes));
+        HIP_TRY(sg::sort_pairs_temp_bytes((int)n, &bytes));
         if (bytes > c->sort_tmp_bytes || !c->sort_tmp) {
             if (c->sort_tmp) HIP_TRY(hipFree(c->sort_tmp));
             c->sort_tmp = nullptr;
             HIP_TRY(hipMalloc(&c->sort_tmp, std::max<size_t>(bytes, 256)));
             c->sort_tmp_bytes = bytes;
         }
-        c->cap_n = need;
+        c->cap_n = n;
     }
-    if (!c->pb.red) {
-        c->pb.nred_blocks = 1024;
-        int64_t cap = 0;
-        int rc;
-        if ((rc = grow(&c->pb.red, &cap, (int64_t)c->pb.nred_blocks * 8)) != SG_OK) return rc;
-        cap = 0;
-        if ((rc = grow(&c->pb.bbox, &cap, 8)) != SG_OK) return rc;
-        cap = 0;
-        if ((rc = grow(&c->pb.err, &cap, 4)) != SG_OK) return rc;
-        cap = 0;
-        if ((rc = grow(&c->stats, &cap, sg::STAT_WORDS)) != SG_OK) return rc;
+    if (!c->stats) {   // the last of these
+        b.nred_blocks = 1024;
+        SG_GROW(b.red, (int64_t)b.nred_blocks * 8);
+        SG_GROW(b.bbox, 8);
+        SG_GROW(b.err, 4);
+        SG_GROW(c->stats, sg::STAT_WORDS);
     }
-    if (padded > c->cap_pad || !c->pb.sx) {
-        int64_t cap = 0;
-        int rc;
-        double **arrs[5] = {&c->pb.sx, &c->pb.sy, &c->pb.sz, &c->pb.sm, &c->pb.sH};
-        for (auto a : arrs) {
-            cap = 0;
-            if ((rc = grow(a, &cap, padded)) != SG_OK) return rc;
-        }
-        cap = 0;
-        if ((rc = grow(&c->pb.sidx, &cap, padded)) != SG_OK) return rc;
-        cap = 0;
-        if ((rc = grow(&c->pb.tiles, &cap, std::max<int64_t>(padded / TJ, 1))) != SG_OK) return rc;
-        cap = 0;
-        if ((rc = grow(&c->pb.chunks, &cap, std::max<int64_t>(padded / sg::TC, 1))) != SG_OK)
-            return rc;
+    if (padded > c->cap_pad) {
+        c->cap_pad = 0;
+        for (double **a : {&b.sx, &b.sy, &b.sz, &b.sm, &b.sH}) SG_GROW(*a, padded);
+        SG_GROW(b.sidx, padded);
+        SG_GROW(b.tiles, std::max<int64_t>(padded / TJ, 1));
+        SG_GROW(b.chunks, std::max<int64_t>(padded / sg::TC, 1));
         c->cap_pad = padded;
     }
-    if (ni > c->cap_ni || !c->pb.ix) {
-        int64_t cap = 0;
-        int rc;
-        const int64_t need = std::max<int64_t>(ni, 1);
-        double **arrs[5] = {&c->pb.ix, &c->pb.iy, &c->pb.iz, &c->pb.im, &c->pb.iH};
-        for (auto a : arrs) {
-            cap = 0;
-            if ((rc = grow(a, &cap, need)) != SG_OK) return rc;
-        }
-        cap = 0;
-        if ((rc = grow(&c->pb.iidx, &cap, need)) != SG_OK) return rc;
-        c->cap_ni = need;
+    if (ni > c->cap_ni) {
+        c->cap_ni = 0;
+        for (double **a : {&b.ix, &b.iy, &b.iz, &b.im, &b.iH}) SG_GROW(*a, ni);
+        SG_GROW(b.iidx, ni);
+        c->cap_ni = ni;
     }
+#undef SG_GROW
     return SG_OK;
 }
 
@@ -741,11 +740,7 @@ int sg_psi_host(sg_context *c, int n, int ibeg, int ni, const double *x, const d
     if (!x || !y || !z || !m || !range2 || (ni > 0 && !psi)) return SG_ERR_ARG;
     HIP_TRY(hipSetDevice(c->device));
     int rc;
-    for (int k = 0; k < 5; ++k) {
-        int64_t cap = c->cap_in;
-        if ((rc = grow(&c->in[k], &cap, n)) != SG_OK) return rc;
-    }
-    c->cap_in = std::max<int64_t>(c->cap_in, n);
+    if ((rc = grow_all(c->in, 5, &c->cap_in, n)) != SG_OK) return rc;
     if ((rc = grow(&c->psi_out, &c->cap_psi_out, std::max(ni, 1))) != SG_OK) return rc;
     const double *src[5] = {x, y, z, m, range2};
     for (int k = 0; k < 5; ++k)
@@ -1162,17 +1157,9 @@ int compute_host_impl(sg_context *c, int n, int ibeg, int ni, const double *x, c
     if (ni > 0 && (!ax || !ay || !az || !pot)) return SG_ERR_ARG;
     HIP_TRY(hipSetDevice(c->device));
     int rc;
-    for (int k = 0; k < 5; ++k) {
-        int64_t cap = c->cap_in;
-        if ((rc = grow(&c->in[k], &cap, n)) != SG_OK) return rc;
-    }
-    c->cap_in = std::max<int64_t>(c->cap_in, n);
-    for (int k = 0; k < 4; ++k) {
-        int64_t cap = c->cap_out;
-        if ((rc = grow(&c->out[k], &cap, std::max(ni, 1))) != SG_OK) return rc;
-    }
+    if ((rc = grow_all(c->in, 5, &c->cap_in, n)) != SG_OK) return rc;
+    if ((rc = grow_all(c->out, 4, &c->cap_out, std::max(ni, 1))) != SG_OK) return rc;
     if (psi && (rc = grow(&c->psi_out, &c->cap_psi_out, std::max(ni, 1))) != SG_OK) return rc;
-    c->cap_out = std::max<int64_t>(c->cap_out, std::max(ni, 1));
     const double *src[5] = {x, y, z, m, range2};
     for (int k = 0; k < 5; ++k)
         HIP_TRY(hipMemcpyAsync(c->in[k], src[k], sizeof(double) * (size_t)n, hipMemcpyHostToDevice,
@@ -1232,11 +1219,7 @@ int sg_vjp_device(sg_context *c, int n, const double *x, const double *y, const 
     const int64_t padded = ((int64_t)(n) + TJ - 1) / TJ * TJ;
     int rc = ensure_capacity(c, n, padded, 1);
     if (rc != SG_OK) return rc;
-    for (int k = 0; k < 4; ++k) {
-        int64_t cap = c->cap_cot;
-        if ((rc = grow(&c->scot[k], &cap, padded)) != SG_OK) return rc;
-    }
-    c->cap_cot = std::max<int64_t>(c->cap_cot, padded);
+    if ((rc = grow_all(c->scot, 4, &c->cap_cot, padded)) != SG_OK) return rc;
     hipStream_t s = c->stream;
     sg::PrepBuffers &b = c->pb;
     HIP_TRY(hipEventRecord(c->ev_p0, s));
@@ -1339,21 +1322,9 @@ int sg_vjp_host(sg_context *c, int n, const double *x, const double *y, const do
     if (!gx || !gy || !gz || !gm || !gH) return SG_ERR_ARG;
     HIP_TRY(hipSetDevice(c->device));
     int rc;
-    for (int k = 0; k < 5; ++k) {
-        int64_t cap = c->cap_in;
-        if ((rc = grow(&c->in[k], &cap, n)) != SG_OK) return rc;
-    }
-    c->cap_in = std::max<int64_t>(c->cap_in, n);
-    for (int k = 0; k < 4; ++k) {
-        int64_t cap = c->cap_vin;
-        if ((rc = grow(&c->vin[k], &cap, n)) != SG_OK) return rc;
-    }
-    c->cap_vin = std::max<int64_t>(c->cap_vin, n);
-    for (int k = 0; k < 5; ++k) {
-        int64_t cap = c->cap_vout;
-        if ((rc = grow(&c->vout[k], &cap, n)) != SG_OK) return rc;
-    }
-    c->cap_vout = std::max<int64_t>(c->cap_vout, n);
+    if ((rc = grow_all(c->in, 5, &c->cap_in, n)) != SG_OK) return rc;
+    if ((rc = grow_all(c->vin, 4, &c->cap_vin, n)) != SG_OK) return rc;
+    if ((rc = grow_all(c->vout, 5, &c->cap_vout, n)) != SG_OK) return rc;
     const double *src[5] = {x, y, z, m, range2};
     for (int k = 0; k < 5; ++k)
         HIP_TRY(hipMemcpyAsync(c->in[k], src[k], sizeof(double) * (size_t)n, hipMemcpyHostToDevice,
@@ -1485,16 +1456,8 @@ int sg_firsthalf(int n, int n_lower, int my_length, const double *x, const doubl
         L.pending = false;
     }
     const int ni = my_length;
-    for (int k = 0; k < 5; ++k) {
-        int64_t cap = c->cap_in;
-        if ((rc = grow(&c->in[k], &cap, n)) != SG_OK) return rc;
-    }
-    c->cap_in = std::max<int64_t>(c->cap_in, n);
-    for (int k = 0; k < 4; ++k) {
-        int64_t cap = c->cap_out;
-        if ((rc = grow(&c->out[k], &cap, std::max(ni, 1))) != SG_OK) return rc;
-    }
-    c->cap_out = std::max<int64_t>(c->cap_out, std::max(ni, 1));
+    if ((rc = grow_all(c->in, 5, &c->cap_in, n)) != SG_OK) return rc;
+    if ((rc = grow_all(c->out, 4, &c->cap_out, std::max(ni, 1))) != SG_OK) return rc;
     HIP_TRY(hipEventRecord(L.t0, c->stream));
     const double *src[5] = {x, y, z, m, range2};
     for (int k = 0; k < 5; ++k)

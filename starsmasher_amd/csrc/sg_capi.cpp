@@ -49,8 +49,10 @@ struct sg_context {
     int64_t cap_psipart = 0;
     unsigned char *nearflag = nullptr;
     int64_t cap_flag = 0;
-    unsigned char *sym = nullptr;       // tables of the unordered-pair pass
+    // tables, slabs and segment sums of the unordered-pair passes (sym_scratch)
+    unsigned char *sym = nullptr;
     int64_t cap_sym = 0;
+    int64_t sym_refused = INT64_MAX;    // the smallest size not to be had
     // [4]: chunk visits, near chunk visits, wide chunk visits (FP64-formed
     // differences in the far loop), pairs evaluated in FP64 (FP32C pass)
     unsigned long long *stats = nullptr;
@@ -132,29 +134,81 @@ hipError_t &last_hip_error()
     return e;
 }
 
+// Gives the unordered-pair passes' memory back; that size is not asked for again.
+int drop_sym(sg_context *c)
+{
+    c->sym_refused = std::min(c->sym_refused, c->cap_sym);
+    unsigned char *p = c->sym;
+    c->sym = nullptr;
+    c->cap_sym = 0;
+    HIP_TRY(hipFree(p));
+    return SG_OK;
+}
+
+// Memory a call cannot do without: where the device has no more, that of the
+// unordered-pair passes, which others can do without, is given back for it.
+int device_malloc(sg_context *c, void **p, size_t bytes)
+{
+    hipError_t e = hipMalloc(p, bytes);
+    if (e != hipSuccess && c->sym) {
+        (void)hipGetLastError();
+        const int rc = drop_sym(c);
+        if (rc != SG_OK) return rc;
+        e = hipMalloc(p, bytes);
+    }
+    if (e == hipSuccess) return SG_OK;
+    (void)hipGetLastError();   // reported here, not by the next launch
+    *p = nullptr;
+    last_hip_error() = e;
+    return SG_ERR_HIP;
+}
+
 template <typename T>
-int grow(T **p, int64_t *cap, int64_t need)
+int grow(sg_context *c, T **p, int64_t *cap, int64_t need)
 {
     if (need <= *cap && *p) return SG_OK;
     if (*p) HIP_TRY(hipFree(*p));
     *p = nullptr;
     *cap = 0;
     const int64_t n = std::max<int64_t>(need, 1);
-    HIP_TRY(hipMalloc((void **)p, sizeof(T) * (size_t)n));
+    const int rc = device_malloc(c, (void **)p, sizeof(T) * (size_t)n);
+    if (rc != SG_OK) return rc;
     *cap = n;
     return SG_OK;
+}
+
+// Memory of the passes that evaluate each unordered far pair once: tables,
+// slabs and segment sums in one allocation, taken when the call has all else it
+// needs.  False where it is not to be had; the call then runs the ordered pass.
+// A refused size is not asked for again, which would wait for the device in every
+// call.
+bool sym_scratch(sg_context *c, int64_t bytes)
+{
+    if (bytes <= c->cap_sym) return true;
+    if (bytes >= c->sym_refused) return false;
+    if (c->sym && hipFree(c->sym) != hipSuccess) (void)hipGetLastError();
+    c->sym = nullptr;
+    c->cap_sym = 0;
+    if (hipMalloc((void **)&c->sym, (size_t)bytes) != hipSuccess) {
+        (void)hipGetLastError();
+        c->sym = nullptr;
+        c->sym_refused = bytes;
+        return false;
+    }
+    c->cap_sym = bytes;
+    return true;
 }
 
 // `count` arrays of one capacity.  The capacity reads 0 until all of them have
 // grown, so that a call after a failed allocation allocates them anew.
 template <typename T>
-int grow_all(T **p, int count, int64_t *cap, int64_t need)
+int grow_all(sg_context *c, T **p, int count, int64_t *cap, int64_t need)
 {
     if (need <= *cap) return SG_OK;
     *cap = 0;
     for (int k = 0; k < count; ++k) {
         int64_t none = 0;
-        const int rc = grow(&p[k], &none, need);
+        const int rc = grow(c, &p[k], &none, need);
         if (rc != SG_OK) return rc;
     }
     *cap = need;
@@ -171,7 +225,7 @@ int ensure_capacity(sg_context *c, int64_t n, int64_t padded, int64_t ni)
 #define SG_GROW(p, need)                                               \
     do {                                                               \
         none = 0;                                                      \
-        if ((rc = grow(&(p), &none, (need))) != SG_OK) return rc;      \
+        if ((rc = grow(c, &(p), &none, (need))) != SG_OK) return rc;      \
     } while (0)
     if (n > c->cap_n) {
         c->cap_n = 0;
@@ -184,7 +238,7 @@ int ensure_capacity(sg_context *c, int64_t n, int64_t padded, int64_t ni)
         if (bytes > c->sort_tmp_bytes || !c->sort_tmp) {
             if (c->sort_tmp) HIP_TRY(hipFree(c->sort_tmp));
             c->sort_tmp = nullptr;
-            HIP_TRY(hipMalloc(&c->sort_tmp, std::max<size_t>(bytes, 256)));
+            if ((rc = device_malloc(c, &c->sort_tmp, std::max<size_t>(bytes, 256))) != SG_OK) return rc;
             c->sort_tmp_bytes = bytes;
         }
         c->cap_n = n;
@@ -243,16 +297,19 @@ int auto_jsplit(int niblocks, int wg, int ntiles, int64_t ni)
     return (int)std::max<int64_t>(1, std::min(want, cap));
 }
 
-// Byte offsets in the buffer of a sym plan's tables.
+// Byte offsets in the memory of a sym plan: `slabs` doubles of slabs, `sums`
+// per lane of a segment.
 struct SymLayout {
-    int64_t boxes, bits, seg, bytes;
+    int64_t boxes, bits, seg, slabs, segsum, bytes;
 };
-static SymLayout sym_layout(int nchunks, int64_t words)
+static SymLayout sym_layout(int nchunks, int64_t words, int64_t slabs, int sums)
 {
     SymLayout l{};
     l.bits = (int64_t)nchunks * 2 * sizeof(float4);
     l.seg = l.bits + words * 8;
-    l.bytes = l.seg + ((int64_t)nchunks + 3) * 4;
+    l.slabs = (l.seg + ((int64_t)nchunks + 3) * 4 + 255) / 256 * 256;
+    l.segsum = l.slabs + slabs * 8;
+    l.bytes = l.segsum + ((int64_t)SYM_SEGS + nchunks) * sums * TC * 8;
     return l;
 }
 static int64_t sym_words(int nchunks) { return (int64_t)nchunks * ((nchunks + 63) / 64); }
@@ -272,26 +329,24 @@ static void plan_sym(EvalPlan &p, int n, bool fp64, bool psi)
     p.sb = (want + step - 1) / step * step;
     p.nsb = (nchunks + p.sb - 1) / p.sb;
     p.jsplit = p.nsb + 1;
-    p.part_elems = (int64_t)p.jsplit * 4 * n + ((int64_t)SYM_SEGS + nchunks) * (psi ? 5 : 4) * TC;
-    p.psipart_elems = 0;
-    p.flag_elems = 1;
-    p.sym_bytes = sym_layout(nchunks, sym_words(nchunks)).bytes;
+    p.part_elems = p.psipart_elems = p.flag_elems = 0;
+    p.sums = psi ? 5 : 4;
+    p.sym_bytes = sym_layout(nchunks, sym_words(nchunks), (int64_t)p.jsplit * 4 * n, p.sums).bytes;
     p.sym = true;
     p.fp64 = fp64;
 }
 
 static SymArgs sym_args(const EvalPlan &p, int n, int nchunks, const PrepBuffers &b,
-                        unsigned char *tables, double *partial, double *segsum, int nkernel,
-                        unsigned long long *stats)
+                        unsigned char *mem, int nkernel, unsigned long long *stats)
 {
-    const SymLayout l = sym_layout(nchunks, sym_words(nchunks));
+    const SymLayout l = sym_layout(nchunks, sym_words(nchunks), (int64_t)p.jsplit * 4 * n, p.sums);
     SymArgs y{};
     y.p = SortedSet{b.sx, b.sy, b.sz, b.sm, b.sH, b.sidx, n, p.padded};
     y.chunks = b.chunks;
     y.bbox = b.bbox;
-    y.boxes = (float4 *)(tables + l.boxes);
-    y.sym = (uint64_t *)(tables + l.bits);
-    y.seg = (int *)(tables + l.seg);
+    y.boxes = (float4 *)(mem + l.boxes);
+    y.sym = (uint64_t *)(mem + l.bits);
+    y.seg = (int *)(mem + l.seg);
     y.segtot = y.seg + nchunks + 1;
     y.n = n;
     y.nchunks = nchunks;
@@ -301,8 +356,8 @@ static SymArgs sym_args(const EvalPlan &p, int n, int nchunks, const PrepBuffers
     y.waves = p.waves;
     y.fp64 = p.fp64;
     y.nkernel = nkernel;
-    y.partial = partial;
-    y.segsum = segsum;
+    y.partial = (double *)(mem + l.slabs);
+    y.segsum = (double *)(mem + l.segsum);
     y.stats = stats;
     return y;
 }
@@ -430,8 +485,7 @@ hipError_t enqueue_eval(const EvalPlan &p, const EvalBuffers &bufs, int n, int i
         a.psipart = bufs.psipart;
     }
     if (p.sym) {
-        SymArgs y = sym_args(p, n, (int)(p.padded / TC), b, bufs.sym, bufs.partial,
-                             bufs.partial + (int64_t)p.jsplit * 4 * n, nkernel, bufs.stats);
+        SymArgs y = sym_args(p, n, (int)(p.padded / TC), b, bufs.sym, nkernel, bufs.stats);
         y.ax = ax;
         y.ay = ay;
         y.az = az;
@@ -634,21 +688,15 @@ int compute_device_impl(sg_context *c, int n, int ibeg, int ni, const double *x,
                              precision, psi != nullptr, allow_sym);
     };
     sg::EvalPlan p = plan(true);
-    if (p.sym) {
-        // the slabs of the unordered-pair pass are its price: where the device
-        // cannot hold them the ordered pass runs
-        if (grow(&c->partial, &c->cap_part, p.part_elems) != SG_OK ||
-            grow(&c->sym, &c->cap_sym, p.sym_bytes) != SG_OK) {
-            (void)hipGetLastError();
-            p = plan(false);
-        }
-    }
-    if (psi && p.psipart_elems > INT32_MAX / 2) return SG_ERR_ARG;
     int rc = ensure_capacity(c, n, p.padded, ni);
     if (rc != SG_OK) return rc;
-    if ((rc = grow(&c->partial, &c->cap_part, p.part_elems)) != SG_OK) return rc;
-    if ((rc = grow(&c->nearflag, &c->cap_flag, p.flag_elems)) != SG_OK) return rc;
-    if (psi && (rc = grow(&c->psipart, &c->cap_psipart, p.psipart_elems)) != SG_OK) return rc;
+    if (p.sym && !sym_scratch(c, p.sym_bytes)) p = plan(false);
+    if (!p.sym) {
+        if (psi && p.psipart_elems > INT32_MAX / 2) return SG_ERR_ARG;
+        if ((rc = grow(c, &c->partial, &c->cap_part, p.part_elems)) != SG_OK) return rc;
+        if ((rc = grow(c, &c->nearflag, &c->cap_flag, p.flag_elems)) != SG_OK) return rc;
+        if (psi && (rc = grow(c, &c->psipart, &c->cap_psipart, p.psipart_elems)) != SG_OK) return rc;
+    }
     const sg::EvalBuffers bufs{c->pb,       c->sort_tmp, c->sort_tmp_bytes, c->partial,
                                c->nearflag, c->stats,    c->psipart,        false,
                                c->sym};
@@ -721,7 +769,7 @@ int sg_psi_device(sg_context *c, int n, int ibeg, int ni, const double *x, const
     a.jsplit = 1;
     while (a.jsplit < sg::PSI_MAX_PARTS && a.jsplit * a.ngroups < sg::PSI_WAVES) a.jsplit *= 2;
     a.psi = psi;
-    if ((rc = grow(&c->psipart, &c->cap_psipart, (int64_t)a.jsplit * ni)) != SG_OK) return rc;
+    if ((rc = grow(c, &c->psipart, &c->cap_psipart, (int64_t)a.jsplit * ni)) != SG_OK) return rc;
     a.psipart = c->psipart;
     HIP_TRY(hipEventRecord(c->ev_k0, s));
     HIP_TRY(hipEventRecord(c->ev_kf, s));
@@ -740,8 +788,8 @@ int sg_psi_host(sg_context *c, int n, int ibeg, int ni, const double *x, const d
     if (!x || !y || !z || !m || !range2 || (ni > 0 && !psi)) return SG_ERR_ARG;
     HIP_TRY(hipSetDevice(c->device));
     int rc;
-    if ((rc = grow_all(c->in, 5, &c->cap_in, n)) != SG_OK) return rc;
-    if ((rc = grow(&c->psi_out, &c->cap_psi_out, std::max(ni, 1))) != SG_OK) return rc;
+    if ((rc = grow_all(c, c->in, 5, &c->cap_in, n)) != SG_OK) return rc;
+    if ((rc = grow(c, &c->psi_out, &c->cap_psi_out, std::max(ni, 1))) != SG_OK) return rc;
     const double *src[5] = {x, y, z, m, range2};
     for (int k = 0; k < 5; ++k)
         HIP_TRY(hipMemcpyAsync(c->in[k], src[k], sizeof(double) * (size_t)n, hipMemcpyHostToDevice,
@@ -831,10 +879,10 @@ int build_sym_plan(sg_context *c, const std::vector<sg::BatchSet> &sets)
     P.sym_items = (int)items.size();
     P.sym_chunks = (int)setof.size();
     int rc;
-    if ((rc = grow(&c->d_symsets, &c->cap_symsets, nsets)) != SG_OK) return rc;
-    if ((rc = grow(&c->d_symitems, &c->cap_symitems, (int64_t)items.size())) != SG_OK) return rc;
-    if ((rc = grow(&c->d_setof, &c->cap_setof, (int64_t)setof.size())) != SG_OK) return rc;
-    if ((rc = grow(&c->d_setbox, &c->cap_setbox, (int64_t)nsets * 8)) != SG_OK) return rc;
+    if ((rc = grow(c, &c->d_symsets, &c->cap_symsets, nsets)) != SG_OK) return rc;
+    if ((rc = grow(c, &c->d_symitems, &c->cap_symitems, (int64_t)items.size())) != SG_OK) return rc;
+    if ((rc = grow(c, &c->d_setof, &c->cap_setof, (int64_t)setof.size())) != SG_OK) return rc;
+    if ((rc = grow(c, &c->d_setbox, &c->cap_setbox, (int64_t)nsets * 8)) != SG_OK) return rc;
     HIP_TRY(hipMemcpy(c->d_symsets, ss.data(), sizeof(sg::SymSet) * nsets, hipMemcpyHostToDevice));
     HIP_TRY(hipMemcpy(c->d_symitems, items.data(), sizeof(int2) * items.size(), hipMemcpyHostToDevice));
     HIP_TRY(hipMemcpy(c->d_setof, setof.data(), sizeof(int) * setof.size(), hipMemcpyHostToDevice));
@@ -893,10 +941,10 @@ int build_plan(sg_context *c, int nsets, const long long *offsets, int wg, int i
     P.nparts = partofs;
     P.nitems = (int)items.size();
     int rc;
-    if ((rc = grow(&c->d_offsets, &c->cap_offsets, nsets + 1)) != SG_OK) return rc;
-    if ((rc = grow(&c->d_sets, &c->cap_sets, nsets)) != SG_OK) return rc;
-    if ((rc = grow(&c->d_items, &c->cap_items, (int64_t)items.size())) != SG_OK) return rc;
-    if (!c->d_counter) HIP_TRY(hipMalloc((void **)&c->d_counter, 64));
+    if ((rc = grow(c, &c->d_offsets, &c->cap_offsets, nsets + 1)) != SG_OK) return rc;
+    if ((rc = grow(c, &c->d_sets, &c->cap_sets, nsets)) != SG_OK) return rc;
+    if ((rc = grow(c, &c->d_items, &c->cap_items, (int64_t)items.size())) != SG_OK) return rc;
+    if (!c->d_counter && (rc = device_malloc(c, (void **)&c->d_counter, 64)) != SG_OK) return rc;
     HIP_TRY(hipMemcpy(c->d_offsets, P.offsets.data(), sizeof(int64_t) * (nsets + 1),
                       hipMemcpyHostToDevice));
     HIP_TRY(hipMemcpy(c->d_sets, sets.data(), sizeof(sg::BatchSet) * nsets, hipMemcpyHostToDevice));
@@ -940,17 +988,11 @@ int sg_compute_batch_device(sg_context *c, int nsets, const long long *offsets, 
     if ((rc = ensure_capacity(c, ntot, P.padded, 1)) != SG_OK) return rc;
     // the default shape: each unordered far pair once, where the device holds its
     // slabs
-    bool sym = wg == 256 && ipl == 1 && P.sym_fits;
-    const sg::SymLayout layout = sg::sym_layout(P.sym_chunks, P.sym_words);
-    if (sym && (grow(&c->partial, &c->cap_part,
-                     P.sym_slabs + ((int64_t)sg::SYM_SEGS + P.sym_chunks) * 4 * sg::TC) != SG_OK ||
-                grow(&c->sym, &c->cap_sym, layout.bytes) != SG_OK)) {
-        (void)hipGetLastError();
-        sym = false;
-    }
+    const sg::SymLayout layout = sg::sym_layout(P.sym_chunks, P.sym_words, P.sym_slabs, 4);
+    const bool sym = wg == 256 && ipl == 1 && P.sym_fits && sym_scratch(c, layout.bytes);
     if (!sym) {
-        if ((rc = grow(&c->partial, &c->cap_part, P.nparts)) != SG_OK) return rc;
-        if ((rc = grow(&c->nearflag, &c->cap_flag, std::max<int64_t>(P.nflags, 1))) != SG_OK) return rc;
+        if ((rc = grow(c, &c->partial, &c->cap_part, P.nparts)) != SG_OK) return rc;
+        if ((rc = grow(c, &c->nearflag, &c->cap_flag, std::max<int64_t>(P.nflags, 1))) != SG_OK) return rc;
     }
 
     hipStream_t s = c->stream;
@@ -1003,8 +1045,8 @@ int sg_compute_batch_device(sg_context *c, int nsets, const long long *offsets, 
         u.waves = 4;
         u.fp64 = precision == SG_PREC_FP64;
         u.nkernel = nkernel;
-        u.partial = c->partial;
-        u.segsum = c->partial + P.sym_slabs;
+        u.partial = (double *)(c->sym + layout.slabs);
+        u.segsum = (double *)(c->sym + layout.segsum);
         u.ax = ax;
         u.ay = ay;
         u.az = az;
@@ -1082,7 +1124,7 @@ int sg_potential_energy(sg_context *c, int n, const double *m, const double *pot
     HIP_TRY(hipSetDevice(c->device));
     constexpr int NWORK = 1025;   // up to 1024 block sums, then the result
     int rc;
-    if ((rc = grow(&c->epot_work, &c->cap_epot, NWORK)) != SG_OK) return rc;
+    if ((rc = grow(c, &c->epot_work, &c->cap_epot, NWORK)) != SG_OK) return rc;
     HIP_TRY(sg::launch_potential_energy(m, pot, n, c->epot_work, NWORK, c->stream));
     HIP_TRY(hipMemcpyAsync(epot, c->epot_work + NWORK - 1, sizeof(double), hipMemcpyDeviceToHost,
                            c->stream));
@@ -1157,9 +1199,9 @@ int compute_host_impl(sg_context *c, int n, int ibeg, int ni, const double *x, c
     if (ni > 0 && (!ax || !ay || !az || !pot)) return SG_ERR_ARG;
     HIP_TRY(hipSetDevice(c->device));
     int rc;
-    if ((rc = grow_all(c->in, 5, &c->cap_in, n)) != SG_OK) return rc;
-    if ((rc = grow_all(c->out, 4, &c->cap_out, std::max(ni, 1))) != SG_OK) return rc;
-    if (psi && (rc = grow(&c->psi_out, &c->cap_psi_out, std::max(ni, 1))) != SG_OK) return rc;
+    if ((rc = grow_all(c, c->in, 5, &c->cap_in, n)) != SG_OK) return rc;
+    if ((rc = grow_all(c, c->out, 4, &c->cap_out, std::max(ni, 1))) != SG_OK) return rc;
+    if (psi && (rc = grow(c, &c->psi_out, &c->cap_psi_out, std::max(ni, 1))) != SG_OK) return rc;
     const double *src[5] = {x, y, z, m, range2};
     for (int k = 0; k < 5; ++k)
         HIP_TRY(hipMemcpyAsync(c->in[k], src[k], sizeof(double) * (size_t)n, hipMemcpyHostToDevice,
@@ -1219,7 +1261,7 @@ int sg_vjp_device(sg_context *c, int n, const double *x, const double *y, const 
     const int64_t padded = ((int64_t)(n) + TJ - 1) / TJ * TJ;
     int rc = ensure_capacity(c, n, padded, 1);
     if (rc != SG_OK) return rc;
-    if ((rc = grow_all(c->scot, 4, &c->cap_cot, padded)) != SG_OK) return rc;
+    if ((rc = grow_all(c, c->scot, 4, &c->cap_cot, padded)) != SG_OK) return rc;
     hipStream_t s = c->stream;
     sg::PrepBuffers &b = c->pb;
     HIP_TRY(hipEventRecord(c->ev_p0, s));
@@ -1256,13 +1298,12 @@ int sg_vjp_device(sg_context *c, int n, const double *x, const double *y, const 
         p.sb = (p.sb + 7) / 8 * 8;   // whole column groups of k_adj_sym
         const int nchunks = (int)(padded / sg::TC);
         p.nsb = (nchunks + p.sb - 1) / p.sb;
-        const int64_t slabs = (int64_t)(p.nsb + 1) * 4 * n;
-        if (grow(&c->partial, &c->cap_part,
-                 slabs + ((int64_t)sg::SYM_SEGS + nchunks) * 5 * sg::TC) == SG_OK &&
-            grow(&c->sym, &c->cap_sym, p.sym_bytes) == SG_OK) {
+        p.jsplit = p.nsb + 1;
+        p.sums = 5;
+        p.sym_bytes = sg::sym_layout(nchunks, sg::sym_words(nchunks), (int64_t)p.jsplit * 4 * n, p.sums).bytes;
+        if (sym_scratch(c, p.sym_bytes)) {
             sg::AdjSymArgs q{};
-            q.y = sg::sym_args(p, n, nchunks, b, c->sym, c->partial, c->partial + slabs, nkernel,
-                               c->stats);
+            q.y = sg::sym_args(p, n, nchunks, b, c->sym, nkernel, c->stats);
             q.wx = a.wx;
             q.wy = a.wy;
             q.wz = a.wz;
@@ -1282,7 +1323,6 @@ int sg_vjp_device(sg_context *c, int n, const double *x, const double *y, const 
             c->launched = true;
             return SG_OK;
         }
-        (void)hipGetLastError();
     }
     const bool wave = precision == SG_PREC_FP32C && n < sg::ADJ_SYM_MIN_N;
     const int wg = sg::adj_config_supported(c->wg[precision]) ? c->wg[precision] : 256;
@@ -1295,9 +1335,9 @@ int sg_vjp_device(sg_context *c, int n, const double *x, const double *y, const 
     } else {
         a.jsplit = sg::auto_jsplit(a.niblocks, wg, ntiles, n);
     }
-    if ((rc = grow(&c->partial, &c->cap_part, (int64_t)a.jsplit * 5 * n)) != SG_OK) return rc;
+    if ((rc = grow(c, &c->partial, &c->cap_part, (int64_t)a.jsplit * 5 * n)) != SG_OK) return rc;
     a.partial = c->partial;
-    if (!wave && (rc = grow(&c->nearflag, &c->cap_flag, a.ngroups * ntiles)) != SG_OK) return rc;
+    if (!wave && (rc = grow(c, &c->nearflag, &c->cap_flag, a.ngroups * ntiles)) != SG_OK) return rc;
     a.nearflag = c->nearflag;
 
     HIP_TRY(hipEventRecord(c->ev_k0, s));
@@ -1322,9 +1362,9 @@ int sg_vjp_host(sg_context *c, int n, const double *x, const double *y, const do
     if (!gx || !gy || !gz || !gm || !gH) return SG_ERR_ARG;
     HIP_TRY(hipSetDevice(c->device));
     int rc;
-    if ((rc = grow_all(c->in, 5, &c->cap_in, n)) != SG_OK) return rc;
-    if ((rc = grow_all(c->vin, 4, &c->cap_vin, n)) != SG_OK) return rc;
-    if ((rc = grow_all(c->vout, 5, &c->cap_vout, n)) != SG_OK) return rc;
+    if ((rc = grow_all(c, c->in, 5, &c->cap_in, n)) != SG_OK) return rc;
+    if ((rc = grow_all(c, c->vin, 4, &c->cap_vin, n)) != SG_OK) return rc;
+    if ((rc = grow_all(c, c->vout, 5, &c->cap_vout, n)) != SG_OK) return rc;
     const double *src[5] = {x, y, z, m, range2};
     for (int k = 0; k < 5; ++k)
         HIP_TRY(hipMemcpyAsync(c->in[k], src[k], sizeof(double) * (size_t)n, hipMemcpyHostToDevice,
@@ -1456,8 +1496,8 @@ int sg_firsthalf(int n, int n_lower, int my_length, const double *x, const doubl
         L.pending = false;
     }
     const int ni = my_length;
-    if ((rc = grow_all(c->in, 5, &c->cap_in, n)) != SG_OK) return rc;
-    if ((rc = grow_all(c->out, 4, &c->cap_out, std::max(ni, 1))) != SG_OK) return rc;
+    if ((rc = grow_all(c, c->in, 5, &c->cap_in, n)) != SG_OK) return rc;
+    if ((rc = grow_all(c, c->out, 4, &c->cap_out, std::max(ni, 1))) != SG_OK) return rc;
     HIP_TRY(hipEventRecord(L.t0, c->stream));
     const double *src[5] = {x, y, z, m, range2};
     for (int k = 0; k < 5; ++k)

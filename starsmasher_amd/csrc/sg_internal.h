@@ -302,7 +302,8 @@ struct EvalPlan {
     bool wave;             // one wave per 64 i and j partition (k_pair_wave)
     int jsub;
     int sb, nsb, waves;
-    int64_t sym_bytes;     // chunk boxes, chunk-pair bits, segment table
+    int sums;              // per lane of a segment
+    int64_t sym_bytes;     // tables, slabs and segment sums
 };
 int auto_jsplit(int niblocks, int wg, int ntiles, int64_t ni);
 // i-ranges up to this many particles take workgroups of 128 when the

@@ -112,3 +112,70 @@ def test_buffers_after_a_failed_allocation(ctx, call):
         ctx.state()
     else:
         raise AssertionError("every allocation failed")
+
+
+BIG = 1 << 20
+# what runs where the device holds the slabs of each unordered far pair once,
+# and where it does not
+UNORDERED = {
+    "compute": (lambda c: c.compute(BIG), "sym", "ordered"),
+    "fp64": (lambda c: c.compute(BIG, prec=1), "sym64", "ordered"),
+    "psi": (lambda c: c.compute(BIG, psi=True), "sym", "ordered"),
+    "vjp": (lambda c: c.vjp(BIG), "adj_sym", "adj_ordered256"),
+    "batch": (lambda c: c.batch([BIG // 2] * 4), "sym", "ordered_batch"),
+    "batch64": (lambda c: c.batch([BIG // 2] * 4, prec=1), "sym64", "ordered_batch"),
+}
+
+
+@pytest.mark.parametrize("call", sorted(UNORDERED))
+def test_a_refused_size_is_not_asked_for_again(ctx, call):
+    f, unordered, ordered = UNORDERED[call]
+    assert f(ctx) == OK and ctx.state() == [unordered]
+    full = ctx.used()
+    other = Context(ctx.L)
+    other.reset(budget=ctx.L.fake_used() + full // 2)
+    assert f(other) == OK and other.state() == [ordered]
+    graphs = ctx.L.fake_graphs()
+    for _ in range(3):   # no allocation, no wait, no other graph
+        other.reset(budget=ctx.L.fake_used())
+        assert f(other) == OK
+        assert other.state() == ([] if graphs else [ordered])
+        assert ctx.L.fake_mallocs() == ctx.L.fake_frees() == ctx.L.fake_graphs() == 0
+    # a smaller set's slabs fit
+    other.reset(budget=ctx.L.fake_used() + full // 2)
+    assert other.compute(100000) == OK and other.state() == ["sym"]
+    other.reset()
+    assert ctx.L.sg_destroy(other.h) == OK
+
+
+@pytest.mark.parametrize("call", sorted(UNORDERED))
+def test_whatever_fits_the_ordered_pass_runs(ctx, call):
+    """From the memory on that a call succeeds with, it succeeds with any more:
+    slabs are taken last and never from what the call needs."""
+    f, unordered, ordered = UNORDERED[call]
+    assert f(ctx) == OK
+    full = ctx.used()
+    seen = []
+    for percent in range(1, 111):
+        c = Context(ctx.L)
+        c.reset(budget=ctx.L.fake_used() + full * percent // 100)
+        seen.append((f(c), c.state()))
+        c.reset()
+        assert ctx.L.sg_destroy(c.h) == OK
+    status = [s for s, _ in seen]
+    first = status.index(OK)
+    assert status[first:] == [OK] * len(status[first:])
+    passes = [r for s, r in seen if s == OK]
+    assert passes[0] == [ordered] and passes[-1] == [unordered]
+    assert sorted(passes, key=lambda r: r == [unordered]) == passes
+
+
+def test_slabs_are_given_back_for_what_a_call_needs(ctx):
+    assert ctx.compute(BIG) == OK and ctx.state() == ["sym"]
+    held = ctx.used()
+    # one set too large for the pass, on a device with 200 MB left
+    ctx.reset(budget=ctx.L.fake_used() + (200 << 20))
+    assert ctx.compute((1 << 22) + 1) == OK and ctx.state() == ["ordered"]
+    assert ctx.used() < held
+    ctx.reset(budget=ctx.L.fake_used() + held)
+    assert ctx.compute(BIG) == OK and ctx.state() == ["ordered"]

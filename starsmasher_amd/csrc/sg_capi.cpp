@@ -845,8 +845,9 @@ int build_sym_plan(sg_context *c, const std::vector<sg::BatchSet> &sets)
     std::vector<int> setof((size_t)(P.padded / sg::TC));
     double pairs = 0.0;   // unordered chunk pairs of the batch
     double nsum = 0.0, nsq = 0.0;
+    auto chunks = [](int64_t n) { return (int)((n + sg::TC - 1) / sg::TC); };
     for (const sg::BatchSet &b : sets) {
-        const double nc = (double)b.ntiles * sg::CHUNKS;
+        const double nc = chunks(b.n);
         pairs += 0.5 * nc * nc;
         nsum += (double)b.n;
         nsq += (double)b.n * (double)b.n;
@@ -860,7 +861,7 @@ int build_sym_plan(sg_context *c, const std::vector<sg::BatchSet> &sets)
         q.pofs = sets[k].pofs;
         q.n = sets[k].n;
         q.chunk0 = (int)(sets[k].pofs / sg::TC);
-        q.nchunks = sets[k].ntiles * sg::CHUNKS;
+        q.nchunks = chunks(sets[k].n);   // those of padding only are left out
         q.words = (q.nchunks + 63) / 64;
         q.sb = sb;
         q.nsb = (q.nchunks + sb - 1) / sb;
@@ -868,7 +869,7 @@ int build_sym_plan(sg_context *c, const std::vector<sg::BatchSet> &sets)
         q.slabofs = P.sym_slabs;
         P.sym_words += sg::sym_words(q.nchunks);
         P.sym_slabs += (int64_t)(q.nsb + 1) * 4 * q.n;
-        std::fill_n(setof.begin() + q.chunk0, q.nchunks, k);
+        std::fill_n(setof.begin() + q.chunk0, sets[k].ntiles * sg::CHUNKS, k);
     }
     std::vector<int> order(nsets);
     for (int k = 0; k < nsets; ++k) order[k] = k;

@@ -110,8 +110,11 @@ __global__ __launch_bounds__(256) void k_sym_classify(SymArgs a)
         }
     }
 #pragma unroll
-    for (int r = 0; r < CROWS; ++r)
-        if (lane == 0 && r0 + r < a.nchunks) a.seg[r0 + r] = rest[r];
+    for (int r = 0; r < CROWS; ++r) {
+        if (lane != 0) continue;
+        if (r0 + r < a.nchunks) a.seg[r0 + r] = rest[r];
+        else if (a.sets) a.seg[r0 + r] = 0;   // the rest of the set's last tile: padding only
+    }
 }
 
 // Cuts each row's unset bits into segments of at most `len` visits, len chosen

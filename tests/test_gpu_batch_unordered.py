@@ -90,3 +90,15 @@ def test_changed_sizes_replan(grav):
     """The captured graph is not replayed for other offsets."""
     for sizes in ([3000, 5000], [5000, 3000], [8000], [3000, 5000]):
         _check(grav, [ics.plummer(n, seed=n) for n in sizes], 0)
+
+
+def _visits(grav, sizes, prec):
+    grav.compute_batch([ics.plummer(n, seed=n) for n in sizes], precision=prec)
+    return grav.last_tile_stats()[0]
+
+
+def test_chunks_of_padding_are_not_visited(grav):
+    """A set fills its last tile of 256 with padding; the visits are those of the
+    chunks with particles, each pair of them in both orders."""
+    sizes = [300, 700, 70, 513, 256, 3, 2500]
+    assert _visits(grav, sizes, SG_PREC_FP32C) == sum((-(-n // 64)) ** 2 for n in sizes)

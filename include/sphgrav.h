@@ -172,7 +172,7 @@ int sg_last_config(sg_context *ctx, int *wg, int *ipl, int *jsplit);
  * input order.  All sets share each launch.  The default shape
  * evaluates each unordered far pair once (work items of the largest sets
  * first); other shapes, batches whose average particle sits in a set of
- * fewer than 256, and sets above 2^22 run in one persistent launch whose
+ * fewer than 256 (FP64: 2,560), and sets above 2^22 run in one persistent launch whose
  * workgroups take (set, i-block, j-partition) items from a queue, longest
  * first (sets of more than 16,384 particles split their j range into
  * partitions).  Partial sums are added in FP64 in a fixed order.  With

@@ -90,6 +90,7 @@ struct sg_context {
         int sym_items = 0, sym_chunks = 0;
         int64_t sym_slabs = 0, sym_words = 0;
         bool sym_fits = false;
+        double mean = 0.0;   // size of the average particle's set
     } plan;
     int64_t *d_offsets = nullptr;
     int64_t cap_offsets = 0;
@@ -853,7 +854,8 @@ int build_sym_plan(sg_context *c, const std::vector<sg::BatchSet> &sets)
         nsq += (double)b.n * (double)b.n;
         if (b.n > sg::SYM_MAX_N) return SG_OK;
     }
-    if (nsq < sg::BATCH_SYM_MEAN * nsum) return SG_OK;
+    P.mean = nsq / nsum;
+    if (P.mean < sg::BATCH_SYM_MEAN) return SG_OK;
     const int sb = 16 * std::max(1, (int)std::ceil(std::sqrt(pairs / 8192.0) / 16.0));
     P.sym_words = P.sym_slabs = 0;
     for (int k = 0; k < nsets; ++k) {
@@ -990,7 +992,9 @@ int sg_compute_batch_device(sg_context *c, int nsets, const long long *offsets, 
     // the default shape: each unordered far pair once, where the device holds its
     // slabs
     const sg::SymLayout layout = sg::sym_layout(P.sym_chunks, P.sym_words, P.sym_slabs, 4);
-    const bool sym = wg == 256 && ipl == 1 && P.sym_fits && sym_scratch(c, layout.bytes);
+    const double least = precision == SG_PREC_FP64 ? sg::BATCH_SYM64_MEAN : sg::BATCH_SYM_MEAN;
+    const bool sym = wg == 256 && ipl == 1 && P.sym_fits && P.mean >= least &&
+                     sym_scratch(c, layout.bytes);
     if (!sym) {
         if ((rc = grow(c, &c->partial, &c->cap_part, P.nparts)) != SG_OK) return rc;
         if ((rc = grow(c, &c->nearflag, &c->cap_flag, std::max<int64_t>(P.nflags, 1))) != SG_OK) return rc;

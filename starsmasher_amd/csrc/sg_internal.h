@@ -338,13 +338,15 @@ constexpr int PSI_WAVES = 32768, PSI_MAX_PARTS = 64;
 // 131,072 14.0 / 9.3, 262,144 49.4 / 34.9.
 constexpr int SYM64_MIN_N = 32769;
 // Batches at the default shape do so too, unless the average particle's set is
-// smaller than this (nearly all of its chunk pairs are then near, and the one
-// kernel of the ordered pass is shorter than five).  Ordered against unordered,
-// kernels, same card, FP32C (FP64): 1,000 sets of 100 0.205 against 0.314 ms, 200
-// of 500 0.168 / 0.111 (0.176 / 0.148), 64 of 4,096 1.06 / 0.69 (1.54 / 1.10), 8
-// of 2,048 to 131,072 3.77 / 2.53 (6.53 / 4.77), 64 of these 43.8 / 33.2 (88.2 /
-// 67.9), four of 200,000 48.5 / 35.2 (102.7 / 74.7).
-constexpr double BATCH_SYM_MEAN = 256.0;
+// smaller than this: nearly all of its chunk pairs are then near, and the one
+// kernel of the ordered pass is shorter than five.  Whole calls, ordered against
+// unordered, same card.  FP32C: 1,000 sets of 100 0.205 against 0.314 ms (kernels),
+// 300 of 256 0.56 / 0.31, 300 of 1,024 1.51 / 0.98, 60 of 4,096 2.28 / 1.17, 20 of
+// 20,000 6.2 / 4.3.  FP64, whose near visits gain nothing: 60 of 300 0.27 / 0.27,
+// 60 of 1,024 0.315 / 0.425, 300 of 1,024 1.01 / 1.12, 16 of 2,048 0.35 / 0.39, 300
+// of 2,048 2.46 / 2.78, 16 of 3,000 0.55 / 0.48, 60 of 3,000 1.21 / 1.05, 60 of 4,096
+// 1.95 / 1.58, 60 of 8,192 5.3 / 4.6, 20 of 20,000 8.0 / 7.2.
+constexpr double BATCH_SYM_MEAN = 256.0, BATCH_SYM64_MEAN = 2560.0;
 // FP32C adjoints from this size on evaluate each unordered far pair once
 // (sg_adjsym.hip), smaller ones run one wave per 64 i and j partition.  Whole
 // calls, flagged near chunks (the pass before both) / waves / unordered, same

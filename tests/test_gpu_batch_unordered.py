@@ -102,3 +102,11 @@ def test_chunks_of_padding_are_not_visited(grav):
     chunks with particles, each pair of them in both orders."""
     sizes = [300, 700, 70, 513, 256, 3, 2500]
     assert _visits(grav, sizes, SG_PREC_FP32C) == sum((-(-n // 64)) ** 2 for n in sizes)
+
+
+def test_fp64_batches_of_small_sets_run_the_ordered_kernel(grav):
+    """The ordered kernel visits by tiles; in FP64 it is the shorter one up to a
+    mean set of 2,560."""
+    for n, unordered in ((300, False), (2449, False), (3001, True)):
+        assert (_visits(grav, [n] * 8, SG_PREC_FP64) == 8 * (-(-n // 64)) ** 2) == unordered
+        assert _visits(grav, [n] * 8, SG_PREC_FP32C) == 8 * (-(-n // 64)) ** 2

@@ -962,7 +962,7 @@ constexpr int PG = 4;
 
 // LDS of a wave: the staged chunk, and the softened pairs of a visit dealt
 // evenly over the lanes.
-constexpr int NSOFT = 1024;   // listed pairs; a visit with more has enough on every lane
+constexpr int NSOFT = 1024;   // listed pairs: a quarter of a visit's (visit_soft)
 struct WaveLds {
     NearSlice sl;
     uint16_t list[NSOFT];     // i lane << 6 | j
@@ -1062,37 +1062,60 @@ __device__ __forceinline__ void soft_pair(double dx, double dy, double dz, doubl
     if (PSI) f[PSI ? 4 : 0] = mj * ps;
 }
 
-// The pairs that visit_near and visit_near64 leave: bit 63 - jj of `mine` is the
+// The pairs that visit_near and visit64 leave: bit 63 - jj of `mine` is the
 // lane's softened pair with jj of the staged chunk.  A lane has few of them and
 // the busiest several times the mean, and one costs some 300 dependent FP64
 // operations, so they are dealt over all lanes, 64 at a time, and each lane
-// collects the sums of its own.
-template <int NK, bool PSI, bool FAST>
-__device__ __forceinline__ void visit_soft(WaveLds &lds, uint64_t mine, const SortedSet &J,
-                                           int64_t j0c, double xr, double yr, double zr, double Hi,
-                                           double invHi, int idi, double (&acc)[PSI ? 5 : 4])
+// collects the sums of its own.  A quarter of the visit's `npairs` pairs is dealt at
+// most: beyond it the busiest lane is near the mean and every lane walks its own
+// (4,096 particles with supports three times the usual, visits of 16 columns: 0.31
+// -> 0.15 ms).  DENSE, for FP64 and psi: `dense` tells whether more than half were
+// softened; the next near visit then lists all its pairs, without the body for the
+// others, a quarter of a softened pair's time.  65,537 particles in FP64 with
+// supports of ten and a hundred times the usual: 19.0 -> 14.6 and 19.8 -> 13.9 ms
+// (tile kernels 12.9 and 13.7).  Returns the lane's softened pairs, of particles.
+template <int NK, bool PSI, bool FAST, bool DENSE>
+__device__ __forceinline__ unsigned visit_soft(WaveLds &lds, uint64_t mine, uint64_t real,
+                                               const SortedSet &J, int64_t j0c, double xr, double yr,
+                                               double zr, double Hi, double invHi, double hi2, int idi,
+                                               double (&acc)[PSI ? 5 : 4], unsigned npairs, bool &dense)
 {
     constexpr int NS = PSI ? 5 : 4;
     const NearSlice &sl = lds.sl;
     const unsigned count = (unsigned)__builtin_popcountll(mine);
     unsigned at, total;
     list_places(count, at, total);
-    if (total > (unsigned)NSOFT) {
+    // softened pairs with particles, not padding
+    unsigned soft = (unsigned)__builtin_popcountll(mine & __brevll(real));
+    if (4 * total > npairs) {
+        if (DENSE) soft = 0;
         while (mine) {
             const int jj = __builtin_clzll(mine);
             mine &= ~(0x8000000000000000ull >> jj);
             const double4 p = sl.p[jj];
-            const double hs = sl.hs[jj];
+            const double hs = sl.hs[jj], Hj = fabs(hs), invHj = sl.hinv[jj], hj2 = Hj * Hj;
             const double dx = p.x - xr, dy = p.y - yr, dz = p.z - zr;
             // the self pair only matters at r = 0: the index is read then
-            const bool dead = dx == 0.0 && dy == 0.0 && dz == 0.0 && hs < 0.0 && J.idx[j0c + jj] == idi;
-            double f[NS];
-            soft_pair<NK, PSI, FAST>(dx, dy, dz, Hi, invHi, fabs(hs), sl.hinv[jj], sl.m[jj], dead, f);
+            const bool same = dx == 0.0 && dy == 0.0 && dz == 0.0 && J.idx[j0c + jj] == idi;
+            if (DENSE) {
+                near_pair<FAST, NK, PSI>(dx, dy, dz, Hi, invHi, hi2, Hj, invHj, hj2, sl.m[jj], hs > 0.0,
+                                         same, acc[0], acc[1], acc[2], acc[3], &acc[PSI ? 4 : 3]);
+                if (fma(dx, dx, fma(dy, dy, dz * dz)) < fmax(hi2, hj2))
+                    soft += (unsigned)(real >> jj & 1);
+            } else {
+                double f[NS];
+                soft_pair<NK, PSI, FAST>(dx, dy, dz, Hi, invHi, Hj, invHj, sl.m[jj], same && hs < 0.0, f);
 #pragma unroll
-            for (int k = 0; k < NS; ++k) acc[k] += f[k];
+                for (int k = 0; k < NS; ++k) acc[k] += f[k];
+            }
         }
-        return;
+        if (DENSE) {
+            list_places(soft, at, total);
+            dense = 2 * total > npairs;
+        }
+        return soft;
     }
+    dense = false;
     const int lane = threadIdx.x & 63;
     for (unsigned k = at; mine; ++k) {
         const int jj = __builtin_clzll(mine);
@@ -1122,6 +1145,7 @@ __device__ __forceinline__ void visit_soft(WaveLds &lds, uint64_t mine, const So
             for (int c = 0; c < NS; ++c) acc[c] += lds.res[c][k - b0];
         }
     }
+    return soft;
 }
 
 // The visits below cover j = jb .. je - 1 of the staged chunk (multiples of
@@ -1134,13 +1158,14 @@ __device__ __forceinline__ void visit_near(WaveLds &lds, uint64_t real, const So
                                            int64_t j0c, int jb, int je, double xr, double yr, double zr, double Hi,
                                            double invHi, double hi2, int idi,
                                            double (&acc)[PSI ? 5 : 4],
-                                           unsigned &nfp64)
+                                           unsigned &nfp64, bool &dense)
 {
     const NearSlice &sl = lds.sl;
     const float hi2f = (float)hi2;
     uint64_t mine = 0;   // bit 63 - jj: the lane's pair with jj is softened
+    if (PSI && dense) mine = (~0ull >> jb) & ~(je < TC ? ~0ull >> je : 0ull);
 #pragma unroll 1
-    for (int f = jb; f < je; f += FOLD) {
+    for (int f = PSI && dense ? je : jb; f < je; f += FOLD) {
         const int fe = min(f + FOLD, je);
         Fold4 sum;
         uint32_t list = 0;
@@ -1167,21 +1192,21 @@ __device__ __forceinline__ void visit_near(WaveLds &lds, uint64_t real, const So
         sum.to(acc);
         mine |= (uint64_t)list << (TC - fe);
     }
-    // the counter covers pairs of particles, not padding
-    nfp64 += (unsigned)__builtin_popcountll(mine & __brevll(real));
-    visit_soft<NK, PSI, true>(lds, mine, J, j0c, xr, yr, zr, Hi, invHi, idi, acc);
+    // without psi the FP32 body costs less than looking out for dense visits
+    nfp64 += visit_soft<NK, PSI, true, PSI>(lds, mine, real, J, j0c, xr, yr, zr, Hi, invHi, hi2, idi,
+                                            acc, 64 * (je - jb), dense);
 }
 
 // Near and far chunks of an FP64 pass.
 template <int NK, bool NEAR, bool PSI>
-__device__ __forceinline__ void visit64(WaveLds &lds, const SortedSet &J, int64_t j0c, double xr,
-                                        double yr, double zr, double Hi, double invHi, double hi2,
-                                        int idi, double (&acc)[PSI ? 5 : 4])
+__device__ __forceinline__ void visit64(WaveLds &lds, uint64_t real, const SortedSet &J, int64_t j0c,
+                                        double xr, double yr, double zr, double Hi, double invHi,
+                                        double hi2, int idi, double (&acc)[PSI ? 5 : 4], bool &dense)
 {
     const NearSlice &sl = lds.sl;
-    uint64_t mine = 0;
+    uint64_t mine = NEAR && dense ? ~0ull : 0;
 #pragma unroll 4
-    for (int j = 0; j < TC; ++j) {
+    for (int j = NEAR && dense ? TC : 0; j < TC; ++j) {
         const double4 p = sl.p[j];
         const double dx = p.x - xr, dy = p.y - yr, dz = p.z - zr;
         double r2 = fma(dx, dx, fma(dy, dy, dz * dz)), m = sl.m[j];
@@ -1198,7 +1223,9 @@ __device__ __forceinline__ void visit64(WaveLds &lds, const SortedSet &J, int64_
         acc[2] = fma(mr3, dz, acc[2]);
         acc[3] -= mr;
     }
-    if (NEAR) visit_soft<NK, PSI, false>(lds, mine, J, j0c, xr, yr, zr, Hi, invHi, idi, acc);
+    if (NEAR)
+        visit_soft<NK, PSI, false, true>(lds, mine, real, J, j0c, xr, yr, zr, Hi, invHi, hi2, idi, acc,
+                                         64 * TC, dense);
 }
 
 // Wide: as near, with every pair Newtonian.
@@ -1286,6 +1313,7 @@ __global__ __launch_bounds__(64) void k_pair_wave(PairArgs a)
     const float rho2 = fmaf(px, px, fmaf(py, py, pz * pz));
     double acc[PSI ? 5 : 4] = {};
     unsigned nfp64 = 0, visits = 0, nearv = 0, widev = 0;
+    bool dense = false;   // of the last near visit
     // partition jp: part jp % jsub of every (jsplit / jsub)-th chunk
     const int stride = a.jsplit / a.jsub, first = jp / a.jsub;
     const int jb = jp % a.jsub * (TC / a.jsub), je = jb + TC / a.jsub;
@@ -1315,7 +1343,7 @@ __global__ __launch_bounds__(64) void k_pair_wave(PairArgs a)
         ++visits;
         if (v == VISIT_NEAR) {
             ++nearv;
-            visit_near<NK, PSI>(lds, real, a.j, j0c, jb, je, xr, yr, zr, Hi[0], invHi[0], hi2[0], idi[0], acc, nfp64);
+            visit_near<NK, PSI>(lds, real, a.j, j0c, jb, je, xr, yr, zr, Hi[0], invHi[0], hi2[0], idi[0], acc, nfp64, dense);
         } else if (v == VISIT_WIDE) {
             ++widev;
             visit_wide(sl, jb, je, xr, yr, zr, acc);
@@ -1387,6 +1415,7 @@ __global__ __launch_bounds__(64) void k_sym_rest(SymArgs a)
     constexpr int NS = PSI ? 5 : 4;
     double acc[NS] = {};
     unsigned nfp64 = 0, visits = 0, nearv = 0, widev = 0;
+    bool dense = false;   // of the last near visit
 
     RestBits it;
     it.row = a.sym + (int64_t)ci * a.words;
@@ -1426,12 +1455,12 @@ __global__ __launch_bounds__(64) void k_sym_rest(SymArgs a)
         if (v == VISIT_NEAR) ++nearv;
         if (FP64) {
             if (v == VISIT_NEAR)
-                visit64<NK, true, PSI>(lds, P, j0c, xr, yr, zr, Hi[0], invHi[0], hi2[0], idi[0], acc);
+                visit64<NK, true, PSI>(lds, real, P, j0c, xr, yr, zr, Hi[0], invHi[0], hi2[0], idi[0], acc, dense);
             else
-                visit64<NK, false, PSI>(lds, P, j0c, xr, yr, zr, Hi[0], invHi[0], hi2[0], idi[0], acc);
+                visit64<NK, false, PSI>(lds, real, P, j0c, xr, yr, zr, Hi[0], invHi[0], hi2[0], idi[0], acc, dense);
         } else if (v == VISIT_NEAR) {
             visit_near<NK, PSI>(lds, real, P, j0c, 0, TC, xr, yr, zr, Hi[0], invHi[0], hi2[0],
-                                idi[0], acc, nfp64);
+                                idi[0], acc, nfp64, dense);
         } else if (v == VISIT_WIDE) {
             ++widev;
             visit_wide(sl, 0, TC, xr, yr, zr, acc);

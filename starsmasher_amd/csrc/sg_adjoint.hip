@@ -550,7 +550,7 @@ constexpr int ANLIST = 1024;   // listed pairs; a visit with more has enough on 
 struct AdjWaveLds {
     double4 p[ACHUNK];   // x, y, z relative to the origin; m
     double4 w[ACHUNK];   // wx, wy, wz, u
-    double2 h[ACHUNK];   // signed H, original index
+    double2 h[ACHUNK];   // signed H, 1 / H
     float4 wf[ACHUNK];   // wx, wy, wz, u in FP32
     float2 mf[ACHUNK];   // m, H^2 in FP32
     uint16_t list[ANLIST];   // i lane << 6 | j
@@ -589,7 +589,7 @@ __device__ __forceinline__ void adj_side_select(double r, double ri, double r2, 
 template <int NK>
 __device__ __forceinline__ void adj_pair_select(double dx, double dy, double dz, double Hk,
                                                 double invHk, double mk, double wkx, double wky,
-                                                double wkz, double uk, double Hl, double ml,
+                                                double wkz, double uk, double Hl, double invHl, double ml,
                                                 double wlx, double wly, double wlz, double ul,
                                                 bool same, bool gas, Acc9 &g)
 {
@@ -599,7 +599,7 @@ __device__ __forceinline__ void adj_pair_select(double dx, double dy, double dz,
     const double r = r2 * ri;
     Side sk, sl;
     adj_side_select<NK>(r, ri, r2, Hk, invHk, sk);
-    adj_side_select<NK>(r, ri, r2, Hl, 1.0 / Hl, sl);
+    adj_side_select<NK>(r, ri, r2, Hl, invHl, sl);
     const double half = same && !gas ? 0.0 : 0.5;
     const double F = same ? 0.0 : half * (sk.F + sl.F);
     const double P = half * (sk.P + sl.P), Fr = half * (sk.Fr + sl.Fr);
@@ -671,13 +671,13 @@ __device__ __forceinline__ bool adj_chunk_near(const TileMeta &cm, double Ox, do
 }
 
 __device__ __forceinline__ void adj_stage(AdjWaveLds &lds, double rx, double ry, double rz, double m,
-                                          double hs, int idx, double wx, double wy, double wz, double u)
+                                          double hs, double wx, double wy, double wz, double u)
 {
     const int lane = threadIdx.x & 63;
     wave_lds_sync();
     lds.p[lane] = make_double4(rx, ry, rz, m);
     lds.w[lane] = make_double4(wx, wy, wz, u);
-    lds.h[lane] = make_double2(hs, (double)idx);
+    lds.h[lane] = make_double2(hs, 1.0 / fabs(hs));
     lds.wf[lane] = make_float4((float)wx, (float)wy, (float)wz, (float)u);
     lds.mf[lane] = make_float2((float)m, (float)(hs * hs));
     wave_lds_sync();
@@ -688,13 +688,21 @@ __device__ __forceinline__ void adj_stage(AdjWaveLds &lds, double rx, double ry,
 // NEAR: softened, self and coincident pairs and those within the margin of a
 // support in FP64, dealt over the lanes 64 at a time (a lane has few, the
 // busiest several times the mean), each lane collecting the sums of its own.
+// Beyond a quarter of the visit's every lane walks its own; after a visit with more
+// than half of its pairs softened (`dense`) all pairs of the next near one are
+// taken in FP64, without the FP32 body.  One FP64 body for both ways: a second
+// instance spills 150 registers in its loop.  65,537 particles with supports of
+// one, three, ten and a hundred times the usual: 3.3, 10.7, 41.1 and 41.0 ms with
+// the FP32 body always and a division per pair, 3.2, 10.4, 32.5 and 32.5 ms so (tile
+// kernels 4.6, 9.9, 24.1 and 23.4, at two waves a SIMD without spills).
 template <int NK, bool NEAR>
-__device__ __forceinline__ void adj_visit(AdjWaveLds &lds, const AdjLane &l, Acc9 &g)
+__device__ __forceinline__ void adj_visit(AdjWaveLds &lds, const AdjLane &l, const int *idx, Acc9 &g,
+                                          bool &dense)
 {
     constexpr int PG = 4;
-    uint64_t own = 0;
+    uint64_t own = NEAR && dense ? ~0ull : 0;
 #pragma unroll 1
-    for (int f0 = 0; f0 < ACHUNK; f0 += AFOLD) {
+    for (int f0 = NEAR && dense ? ACHUNK : 0; f0 < ACHUNK; f0 += AFOLD) {
         float f[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll 1
         for (int j0 = f0; j0 < f0 + AFOLD; j0 += PG) {
@@ -729,38 +737,58 @@ __device__ __forceinline__ void adj_visit(AdjWaveLds &lds, const AdjLane &l, Acc
     if (!NEAR) return;
     const int lane = threadIdx.x & 63;
     const unsigned count = (unsigned)__builtin_popcountll(own);
-    unsigned at, total;
+    unsigned at, total, soft = 0;
     list_places(count, at, total);
-    if (total > (unsigned)ANLIST) {
-        while (own) {
+    const bool deal = total <= (unsigned)ANLIST;
+    if (deal)
+        for (unsigned k = at; own; ++k) {
             const int jj = __builtin_ctzll(own);
             own &= own - 1;
-            const double4 p = lds.p[jj], c = lds.w[jj];
-            const double2 h = lds.h[jj];
-            Acc9 f;
-            adj_pair_select<NK>(p.x - l.x, p.y - l.y, p.z - l.z, l.H, l.invH, l.m, l.wx, l.wy, l.wz,
-                                l.u, fabs(h.x), p.w, c.x, c.y, c.z, c.w, (int)h.y == l.id, l.gas, f);
-            for (int k = 0; k < 9; ++k) g[k] += f[k];
+            lds.list[k] = (uint16_t)(lane << 6 | jj);
         }
-        return;
-    }
-    for (unsigned k = at; own; ++k) {
-        const int jj = __builtin_ctzll(own);
-        own &= own - 1;
-        lds.list[k] = (uint16_t)(lane << 6 | jj);
-    }
-    for (unsigned b0 = 0; b0 < total; b0 += 64) {
-        wave_lds_sync();
-        const unsigned e = min(b0 + (unsigned)lane, total - 1);   // lanes past the end repeat the last
-        const int il = lds.list[e] >> 6, jj = lds.list[e] & 63;
+    // one body for both, which keeps its registers in check
+    for (unsigned b0 = 0;; b0 += 64) {
+        int il = lane, jj = 0, id = l.id;
+        double x = l.x, y = l.y, z = l.z, H = l.H, invH = l.invH, m = l.m;
+        double wx = l.wx, wy = l.wy, wz = l.wz, u = l.u;
+        const bool on = deal || own != 0;
+        if (deal) {
+            if (b0 >= total) break;
+            wave_lds_sync();
+            const unsigned e = min(b0 + (unsigned)lane, total - 1);   // lanes past the end repeat the last
+            il = lds.list[e] >> 6;
+            jj = lds.list[e] & 63;
+            x = __shfl(x, il, 64);
+            y = __shfl(y, il, 64);
+            z = __shfl(z, il, 64);
+            H = __shfl(H, il, 64);
+            invH = __shfl(invH, il, 64);
+            m = __shfl(m, il, 64);
+            wx = __shfl(wx, il, 64);
+            wy = __shfl(wy, il, 64);
+            wz = __shfl(wz, il, 64);
+            u = __shfl(u, il, 64);
+            id = __shfl(id, il, 64);
+        } else {
+            if (!__ballot(on)) break;
+            if (on) jj = __builtin_ctzll(own);
+            own &= own - 1;
+        }
         const double4 p = lds.p[jj], c = lds.w[jj];
         const double2 h = lds.h[jj];
+        const double dx = p.x - x, dy = p.y - y, dz = p.z - z, Hl = fabs(h.x);
+        // the self pair only matters at r = 0: the index is read then
+        const bool same = dx == 0.0 && dy == 0.0 && dz == 0.0 && idx[jj] == id;
         Acc9 f;
-        adj_pair_select<NK>(p.x - __shfl(l.x, il, 64), p.y - __shfl(l.y, il, 64),
-                            p.z - __shfl(l.z, il, 64), __shfl(l.H, il, 64), __shfl(l.invH, il, 64),
-                            __shfl(l.m, il, 64), __shfl(l.wx, il, 64), __shfl(l.wy, il, 64),
-                            __shfl(l.wz, il, 64), __shfl(l.u, il, 64), fabs(h.x), p.w, c.x, c.y, c.z,
-                            c.w, (int)h.y == __shfl(l.id, il, 64), h.x > 0.0, f);
+        adj_pair_select<NK>(dx, dy, dz, H, invH, m, wx, wy, wz, u, Hl, h.y, p.w, c.x, c.y, c.z, c.w,
+                            same, h.x > 0.0, f);
+        if (!deal) {
+#pragma unroll
+            for (int k = 0; k < 9; ++k) g[k] += on ? f[k] : 0.0;
+            const double hm = fmax(H, Hl);
+            soft += on && fma(dx, dx, fma(dy, dy, dz * dz)) < hm * hm ? 1u : 0u;
+            continue;
+        }
 #pragma unroll
         for (int k = 0; k < 9; ++k) lds.res[k][lane] = f[k];
         wave_lds_sync();
@@ -770,6 +798,8 @@ __device__ __forceinline__ void adj_visit(AdjWaveLds &lds, const AdjLane &l, Acc
             for (int v = 0; v < 9; ++v) g[v] += lds.res[v][k - b0];
         }
     }
+    list_places(soft, at, total);
+    dense = 2 * total > 64u * ACHUNK;
 }
 
 // The visits that k_adj_sym leaves, one wave per segment (k_sym_rest's).  Three
@@ -801,19 +831,20 @@ void k_adj_rest(AdjSymArgs a)
     it.words = y.words;
     int left = min(len, rest_total(it.row, y.nchunks, y.words) - k0);
     unsigned visits = 0, nearv = 0;
+    bool dense = false;
     it.start(k0);
     for (; left > 0; --left) {
         const int cj = it.next();
         const int64_t j = (int64_t)cj * TC + lane;
         const bool near = adj_chunk_near(y.chunks[cj], Ox, Oy, Oz, l);
-        adj_stage(lds, P.x[j] - Ox, P.y[j] - Oy, P.z[j] - Oz, P.m[j], P.Hs[j], P.idx[j], a.wx[j],
+        adj_stage(lds, P.x[j] - Ox, P.y[j] - Oy, P.z[j] - Oz, P.m[j], P.Hs[j], a.wx[j],
                   a.wy[j], a.wz[j], a.u[j]);
         ++visits;
         if (near) {
             ++nearv;
-            adj_visit<NK, true>(lds, l, g);
+            adj_visit<NK, true>(lds, l, P.idx + (int64_t)cj * TC, g, dense);
         } else {
-            adj_visit<NK, false>(lds, l, g);
+            adj_visit<NK, false>(lds, l, P.idx + (int64_t)cj * TC, g, dense);
         }
     }
     double *out = y.segsum + (int64_t)s * 5 * TC + lane;
@@ -849,17 +880,18 @@ void k_adj_wave(AdjArgs a)
     adj_lane(P, a.wx, a.wy, a.wz, a.u, i, Ox, Oy, Oz, l);
     Acc9 g = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
     unsigned visits = 0, nearv = 0;
+    bool dense = false;
     for (int cj = jp; cj < nchunks; cj += a.jsplit) {
         const int64_t j = (int64_t)cj * TC + lane;
         const bool near = adj_chunk_near(a.chunks[cj], Ox, Oy, Oz, l);
-        adj_stage(lds, P.x[j] - Ox, P.y[j] - Oy, P.z[j] - Oz, P.m[j], P.Hs[j], P.idx[j], a.wx[j],
+        adj_stage(lds, P.x[j] - Ox, P.y[j] - Oy, P.z[j] - Oz, P.m[j], P.Hs[j], a.wx[j],
                   a.wy[j], a.wz[j], a.u[j]);
         ++visits;
         if (near) {
             ++nearv;
-            adj_visit<NK, true>(lds, l, g);
+            adj_visit<NK, true>(lds, l, P.idx + (int64_t)cj * TC, g, dense);
         } else {
-            adj_visit<NK, false>(lds, l, g);
+            adj_visit<NK, false>(lds, l, P.idx + (int64_t)cj * TC, g, dense);
         }
     }
     if (valid) {

@@ -881,11 +881,12 @@ int build_sym_plan(sg_context *c, const std::vector<sg::BatchSet> &sets)
         for (int t = 0; t < ss[k].nsb * (ss[k].nsb + 1) / 2; ++t) items.push_back(make_int2(k, t));
     P.sym_items = (int)items.size();
     P.sym_chunks = (int)setof.size();
-    int rc;
-    if ((rc = grow(c, &c->d_symsets, &c->cap_symsets, nsets)) != SG_OK) return rc;
-    if ((rc = grow(c, &c->d_symitems, &c->cap_symitems, (int64_t)items.size())) != SG_OK) return rc;
-    if ((rc = grow(c, &c->d_setof, &c->cap_setof, (int64_t)setof.size())) != SG_OK) return rc;
-    if ((rc = grow(c, &c->d_setbox, &c->cap_setbox, (int64_t)nsets * 8)) != SG_OK) return rc;
+    // as optional as the slabs: without them the batch runs the ordered kernel
+    if (grow(c, &c->d_symsets, &c->cap_symsets, nsets) != SG_OK ||
+        grow(c, &c->d_symitems, &c->cap_symitems, (int64_t)items.size()) != SG_OK ||
+        grow(c, &c->d_setof, &c->cap_setof, (int64_t)setof.size()) != SG_OK ||
+        grow(c, &c->d_setbox, &c->cap_setbox, (int64_t)nsets * 8) != SG_OK)
+        return SG_OK;
     HIP_TRY(hipMemcpy(c->d_symsets, ss.data(), sizeof(sg::SymSet) * nsets, hipMemcpyHostToDevice));
     HIP_TRY(hipMemcpy(c->d_symitems, items.data(), sizeof(int2) * items.size(), hipMemcpyHostToDevice));
     HIP_TRY(hipMemcpy(c->d_setof, setof.data(), sizeof(int) * setof.size(), hipMemcpyHostToDevice));

@@ -179,3 +179,23 @@ def test_slabs_are_given_back_for_what_a_call_needs(ctx):
     assert ctx.used() < held
     ctx.reset(budget=ctx.L.fake_used() + held)
     assert ctx.compute(BIG) == OK and ctx.state() == ["ordered"]
+
+
+def test_a_batch_without_its_optional_tables(ctx):
+    """The tables of the unordered pass are as optional as its slabs: a batch that
+    cannot have one of these five allocations runs the ordered kernel."""
+    ran = []
+    for k in range(1, 100):
+        c = Context(ctx.L)
+        ctx.reset(fail=k)
+        status = c.batch([5000, 300, 5000])
+        reached = ctx.L.fake_mallocs() >= k
+        if status == OK:
+            ran.append(c.state())
+        ctx.reset()
+        assert c.batch([5000, 300, 5000]) == OK and c.batch([4000] * 2) == OK
+        c.state()
+        assert ctx.L.sg_destroy(c.h) == OK
+        if not reached:
+            break
+    assert ran == [["ordered_batch"]] * 5 + [["sym"]]

@@ -267,10 +267,11 @@ int sg_psi_host(sg_context *ctx, int n, int ibeg, int ni,
  * Device pointers, asynchronous on the context stream like
  * sg_compute_device (sg_synchronize reports validation, including
  * non-finite cotangents as SG_ERR_NONFINITE); sg_last_timings covers it.
- * SG_PREC_FP32C runs one wave per 64 particles and partition for sets below
- * 32,768 particles and each unordered far pair once from there on to 2^22
- * (where the device holds the partial sums); otherwise, and in FP64, the
- * workgroup size is that of the forward kernel for the precision. */
+ * The workgroup size is that set for the precision (sg_set_config; one i per
+ * lane).  Where none is set SG_PREC_FP32C runs one wave per 64 particles and
+ * partition for sets below 32,768 particles and each unordered far pair once
+ * from there on to 2^22 (where the device holds the partial sums), else and in
+ * FP64 it is 256. */
 int sg_vjp_device(sg_context *ctx, int n,
                   const double *x, const double *y, const double *z,
                   const double *m, const double *range2, int nkernel, int precision,

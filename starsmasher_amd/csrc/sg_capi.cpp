@@ -1294,9 +1294,11 @@ int sg_vjp_device(sg_context *c, int n, const double *x, const double *y, const 
     a.gm = gm;
     a.gH = gH;
     a.stats = c->stats;
-    // the FP32C pass: sets of ADJ_SYM_MIN_N particles on take each unordered far
-    // pair once, where the device holds its slabs; smaller ones one wave per 64 i
-    if (precision == SG_PREC_FP32C && n >= sg::ADJ_SYM_MIN_N && n <= sg::SYM_MAX_N) {
+    // the FP32C pass, unless a workgroup size is set: sets of ADJ_SYM_MIN_N
+    // particles on take each unordered far pair once, where the device holds its
+    // slabs; smaller ones one wave per 64 i
+    const bool automatic = precision == SG_PREC_FP32C && c->wg[precision] == 0;
+    if (automatic && n >= sg::ADJ_SYM_MIN_N && n <= sg::SYM_MAX_N) {
         sg::EvalPlan p{};
         p.padded = padded;
         sg::plan_sym(p, n, false, false);
@@ -1330,7 +1332,7 @@ int sg_vjp_device(sg_context *c, int n, const double *x, const double *y, const 
             return SG_OK;
         }
     }
-    const bool wave = precision == SG_PREC_FP32C && n < sg::ADJ_SYM_MIN_N;
+    const bool wave = automatic && n < sg::ADJ_SYM_MIN_N;
     const int wg = sg::adj_config_supported(c->wg[precision]) ? c->wg[precision] : 256;
     a.niblocks = (int)((n + (int64_t)wg - 1) / wg);
     a.ngroups = (int64_t)a.niblocks * (wg / 64);

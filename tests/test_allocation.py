@@ -199,3 +199,13 @@ def test_a_batch_without_its_optional_tables(ctx):
         if not reached:
             break
     assert ran == [["ordered_batch"]] * 5 + [["sym"]]
+
+
+@pytest.mark.parametrize("n,automatic", [(4096, "adj_wave"), (40000, "adj_sym")])
+def test_the_gradient_runs_at_the_workgroup_size_asked_for(ctx, n, automatic):
+    for wg in (64, 128, 256):
+        assert ctx.L.sg_set_config(ctx.h, 0, wg, 1, 0) == OK
+        assert ctx.vjp(n) == OK and ctx.state() == [f"adj_ordered{wg}"]
+        ctx.reset()
+    assert ctx.L.sg_set_config(ctx.h, 0, 0, 1, 0) == OK
+    assert ctx.vjp(n) == OK and ctx.state() == [automatic]

@@ -1069,11 +1069,12 @@ __device__ __forceinline__ void soft_pair(double dx, double dy, double dz, doubl
 // collects the sums of its own.  A quarter of the visit's `npairs` pairs is dealt at
 // most: beyond it the busiest lane is near the mean and every lane walks its own
 // (4,096 particles with supports three times the usual, visits of 16 columns: 0.31
-// -> 0.15 ms).  DENSE, for FP64 and psi: `dense` tells whether more than half were
+// -> 0.15 ms).  DENSE, for FP64: `dense` tells whether more than half were
 // softened; the next near visit then lists all its pairs, without the body for the
-// others, a quarter of a softened pair's time.  65,537 particles in FP64 with
-// supports of ten and a hundred times the usual: 19.0 -> 14.6 and 19.8 -> 13.9 ms
-// (tile kernels 12.9 and 13.7).  Returns the lane's softened pairs, of particles.
+// others, a quarter of a softened pair's time.  65,537 particles with supports of
+// ten and a hundred times the usual: 19.0 -> 14.6 and 19.8 -> 13.9 ms (tile kernels
+// 12.9 and 13.7).  In FP32C that body costs as little as looking out for such
+// visits.  Returns the lane's softened pairs, of particles.
 template <int NK, bool PSI, bool FAST, bool DENSE>
 __device__ __forceinline__ unsigned visit_soft(WaveLds &lds, uint64_t mine, uint64_t real,
                                                const SortedSet &J, int64_t j0c, double xr, double yr,
@@ -1158,14 +1159,13 @@ __device__ __forceinline__ void visit_near(WaveLds &lds, uint64_t real, const So
                                            int64_t j0c, int jb, int je, double xr, double yr, double zr, double Hi,
                                            double invHi, double hi2, int idi,
                                            double (&acc)[PSI ? 5 : 4],
-                                           unsigned &nfp64, bool &dense)
+                                           unsigned &nfp64)
 {
     const NearSlice &sl = lds.sl;
     const float hi2f = (float)hi2;
     uint64_t mine = 0;   // bit 63 - jj: the lane's pair with jj is softened
-    if (PSI && dense) mine = (~0ull >> jb) & ~(je < TC ? ~0ull >> je : 0ull);
 #pragma unroll 1
-    for (int f = PSI && dense ? je : jb; f < je; f += FOLD) {
+    for (int f = jb; f < je; f += FOLD) {
         const int fe = min(f + FOLD, je);
         Fold4 sum;
         uint32_t list = 0;
@@ -1192,9 +1192,9 @@ __device__ __forceinline__ void visit_near(WaveLds &lds, uint64_t real, const So
         sum.to(acc);
         mine |= (uint64_t)list << (TC - fe);
     }
-    // without psi the FP32 body costs less than looking out for dense visits
-    nfp64 += visit_soft<NK, PSI, true, PSI>(lds, mine, real, J, j0c, xr, yr, zr, Hi, invHi, hi2, idi,
-                                            acc, 64 * (je - jb), dense);
+    bool dense = false;
+    nfp64 += visit_soft<NK, PSI, true, false>(lds, mine, real, J, j0c, xr, yr, zr, Hi, invHi, hi2, idi,
+                                              acc, 64 * (je - jb), dense);
 }
 
 // Near and far chunks of an FP64 pass.
@@ -1313,7 +1313,6 @@ __global__ __launch_bounds__(64) void k_pair_wave(PairArgs a)
     const float rho2 = fmaf(px, px, fmaf(py, py, pz * pz));
     double acc[PSI ? 5 : 4] = {};
     unsigned nfp64 = 0, visits = 0, nearv = 0, widev = 0;
-    bool dense = false;   // of the last near visit
     // partition jp: part jp % jsub of every (jsplit / jsub)-th chunk
     const int stride = a.jsplit / a.jsub, first = jp / a.jsub;
     const int jb = jp % a.jsub * (TC / a.jsub), je = jb + TC / a.jsub;
@@ -1343,7 +1342,7 @@ __global__ __launch_bounds__(64) void k_pair_wave(PairArgs a)
         ++visits;
         if (v == VISIT_NEAR) {
             ++nearv;
-            visit_near<NK, PSI>(lds, real, a.j, j0c, jb, je, xr, yr, zr, Hi[0], invHi[0], hi2[0], idi[0], acc, nfp64, dense);
+            visit_near<NK, PSI>(lds, real, a.j, j0c, jb, je, xr, yr, zr, Hi[0], invHi[0], hi2[0], idi[0], acc, nfp64);
         } else if (v == VISIT_WIDE) {
             ++widev;
             visit_wide(sl, jb, je, xr, yr, zr, acc);
@@ -1460,7 +1459,7 @@ __global__ __launch_bounds__(64) void k_sym_rest(SymArgs a)
                 visit64<NK, false, PSI>(lds, real, P, j0c, xr, yr, zr, Hi[0], invHi[0], hi2[0], idi[0], acc, dense);
         } else if (v == VISIT_NEAR) {
             visit_near<NK, PSI>(lds, real, P, j0c, 0, TC, xr, yr, zr, Hi[0], invHi[0], hi2[0],
-                                idi[0], acc, nfp64, dense);
+                                idi[0], acc, nfp64);
         } else if (v == VISIT_WIDE) {
             ++widev;
             visit_wide(sl, 0, TC, xr, yr, zr, acc);

@@ -157,6 +157,14 @@ int sg_compute_host(sg_context *ctx, int n, int ibeg, int ni,
  * each).  Every other call runs the ordered tile kernel of the given shape. */
 int sg_set_config(sg_context *ctx, int precision, int wg, int ipl, int jsplit);
 int sg_get_config(sg_context *ctx, int precision, int *wg, int *ipl, int *jsplit);
+/* The device memory, in bytes, that the context may hold for the passes that
+ * evaluate each unordered far pair once (sg_set_config, sg_compute_batch_device,
+ * sg_vjp_device): 4.5 GB at 2^20 particles, 17 GB at 2^22.  Calls that need more
+ * run the ordered kernels; what is held above the limit is given back.  Without a
+ * limit (bytes < 0, the default) that memory is taken where at least as much stays
+ * free, and a size that was not to be had is not asked for again until this is
+ * called. */
+int sg_set_scratch_limit(sg_context *ctx, long long bytes);
 /* The tile shape the last single-set evaluation on the context ran with
  * (sg_compute_device and the calls built on it, the automatic choices
  * resolved; jsplit counts the partial-sum slabs of the pass that ran);

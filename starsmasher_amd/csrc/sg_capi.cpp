@@ -53,6 +53,7 @@ struct sg_context {
     unsigned char *sym = nullptr;
     int64_t cap_sym = 0;
     int64_t sym_refused = INT64_MAX;    // the smallest size not to be had
+    int64_t sym_limit = INT64_MAX;      // sg_set_scratch_limit
     // [4]: chunk visits, near chunk visits, wide chunk visits (FP64-formed
     // differences in the far loop), pairs evaluated in FP64 (FP32C pass)
     unsigned long long *stats = nullptr;
@@ -181,12 +182,23 @@ int grow(sg_context *c, T **p, int64_t *cap, int64_t need)
 // Memory of the passes that evaluate each unordered far pair once: tables,
 // slabs and segment sums in one allocation, taken when the call has all else it
 // needs.  False where it is not to be had; the call then runs the ordered pass.
-// A refused size is not asked for again, which would wait for the device in every
-// call.
+// It is up to 17 GB and stays with the context, so it is taken only where as much
+// stays free for others.  A refused size is not asked for again (until the limit is
+// set), which would wait for the device in every call.
 bool sym_scratch(sg_context *c, int64_t bytes)
 {
+    if (bytes > c->sym_limit) return false;
     if (bytes <= c->cap_sym) return true;
     if (bytes >= c->sym_refused) return false;
+    size_t free = 0, total = 0;
+    if (hipMemGetInfo(&free, &total) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    if (bytes > ((int64_t)free + c->cap_sym) / 2) {
+        c->sym_refused = bytes;
+        return false;
+    }
     if (c->sym && hipFree(c->sym) != hipSuccess) (void)hipGetLastError();
     c->sym = nullptr;
     c->cap_sym = 0;
@@ -643,6 +655,19 @@ int sg_set_config(sg_context *c, int precision, int wg, int ipl, int jsplit)
     c->wg[precision] = wg;
     c->ipl[precision] = ipl;
     c->jsplit[precision] = jsplit;
+    return SG_OK;
+}
+
+int sg_set_scratch_limit(sg_context *c, long long bytes)
+{
+    if (!c) return SG_ERR_ARG;
+    HIP_TRY(hipSetDevice(c->device));
+    c->sym_limit = bytes < 0 ? INT64_MAX : bytes;
+    if (c->cap_sym > c->sym_limit) {
+        const int rc = drop_sym(c);
+        if (rc != SG_OK) return rc;
+    }
+    c->sym_refused = INT64_MAX;
     return SG_OK;
 }
 

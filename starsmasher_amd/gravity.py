@@ -247,6 +247,14 @@ class Gravity:
               "sg_get_config")
         return wg.value, ipl.value, js.value
 
+    def set_scratch_limit(self, limit=None):
+        """Bytes of device memory the context may hold for the passes that
+        evaluate each unordered far pair once (None: as much as stays free);
+        above it their calls run the ordered kernels, and what is held is given
+        back."""
+        check(self._L.sg_set_scratch_limit(self._h, -1 if limit is None else int(limit)),
+              "sg_set_scratch_limit")
+
     def last_config(self):
         """(wg, ipl, jsplit) the last single-set evaluation ran with; raises
         SphgravError (SG_ERR_STATE) before one or after a call of another

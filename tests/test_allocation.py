@@ -156,7 +156,7 @@ def test_whatever_fits_the_ordered_pass_runs(ctx, call):
     assert f(ctx) == OK
     full = ctx.used()
     seen = []
-    for percent in range(1, 111):
+    for percent in range(1, 221):
         c = Context(ctx.L)
         c.reset(budget=ctx.L.fake_used() + full * percent // 100)
         seen.append((f(c), c.state()))
@@ -209,3 +209,49 @@ def test_the_gradient_runs_at_the_workgroup_size_asked_for(ctx, n, automatic):
         ctx.reset()
     assert ctx.L.sg_set_config(ctx.h, 0, 0, 1, 0) == OK
     assert ctx.vjp(n) == OK and ctx.state() == [automatic]
+
+
+@pytest.mark.parametrize("call", sorted(UNORDERED))
+def test_scratch_limit(ctx, call):
+    """A limit holds for the memory of the unordered passes only, gives back what
+    is held above it, and a new one lets a refused size be asked for again."""
+    f, unordered, ordered = UNORDERED[call]
+    replay = [[]] if call.startswith("batch") else []   # of a graph: nothing is launched anew
+    limit = lambda b: ctx.L.sg_set_scratch_limit(ctx.h, C.c_longlong(b))
+    assert ctx.L.sg_set_scratch_limit(None, C.c_longlong(0)) == 1
+    assert f(ctx) == OK and ctx.state() == [unordered]
+    full = ctx.used()
+    assert limit(0) == OK and ctx.used() < full
+    ctx.reset()
+    assert f(ctx) == OK and ctx.state() == [ordered]
+    assert limit(1 << 30) == OK
+    ctx.reset()
+    assert f(ctx) == OK and ctx.state() in [[ordered]] + replay
+    assert ctx.compute(100000) == OK and ctx.state()[-1] == "sym"
+    assert limit(-1) == OK
+    ctx.reset(budget=ctx.L.fake_used() + (1 << 20))
+    assert f(ctx) == OK and ctx.state() in [[ordered]] + replay
+    ctx.reset()
+    assert f(ctx) == OK and ctx.state() in [[ordered]] + replay   # remembered
+    assert limit(-1) == OK
+    ctx.reset()
+    assert f(ctx) == OK and ctx.state() == [unordered]
+
+
+def test_slabs_leave_as_much_free_as_they_take(ctx):
+    """A program that shares the device (torch's allocator) finds at least as much
+    memory free as the unordered pass took."""
+    assert ctx.compute(BIG) == OK
+    held = ctx.used()
+    seen = set()
+    for percent in range(60, 260, 5):
+        c = Context(ctx.L)
+        budget = ctx.L.fake_used() + held * percent // 100
+        c.reset(budget=budget)
+        assert c.compute(BIG) == OK
+        pass_, free = c.state()[0], budget - ctx.L.fake_used()
+        seen.add(pass_)
+        assert pass_ == "ordered" or free >= 0.9 * held
+        c.reset()
+        assert ctx.L.sg_destroy(c.h) == OK
+    assert seen == {"ordered", "sym"}

@@ -336,8 +336,9 @@ __global__ __launch_bounds__(256) void k_adj_sym_reduce(AdjSymArgs a)
     }
     // back to the caller's units: positions' gradients m w / r^3, masses' w / r^2
     const double len = y.bbox[6], unit = 1.0 / y.bbox[7];
-    for (int k = 0; k < 3; ++k) s[k] *= len * len * len * unit;
-    s[3] *= len * len;
+    // (factor by factor: their product may leave the range)
+    for (int k = 0; k < 3; ++k) s[k] = s[k] * unit * len * len * len;
+    s[3] = s[3] * len * len;
     const int c = (int)(i / TC);
     const int e = y.seg[c + 1];
     for (int g = y.seg[c]; g < e; ++g) {

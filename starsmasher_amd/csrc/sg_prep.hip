@@ -96,10 +96,11 @@ __global__ __launch_bounds__(RB) void k_validate_bbox(const double *__restrict__
     }
 }
 
-// The power of two that brings v to [1, 2) (1 where v has none).
+// The power of two that brings v to [1, 2) (1 where v has none; at most 2^1000,
+// so that it and its inverse are finite for denormal v).
 __device__ inline double unit_scale(double v)
 {
-    return v > 0.0 && isfinite(v) ? ldexp(1.0, -ilogb(v)) : 1.0;
+    return v > 0.0 && isfinite(v) ? ldexp(1.0, min(-ilogb(v), 1000)) : 1.0;
 }
 
 // bbox: lo xyz, hi xyz, and the scales that bring the set's extent and its

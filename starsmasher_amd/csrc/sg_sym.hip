@@ -7,9 +7,10 @@
 // and one v_rsq_f32 against 26 and 2 for the two ordered pairs.
 //
 //   * k_sym_classify marks the pairs of 64-particle chunks that qualify: all
-//     pairs Newtonian by the box test, and far enough from the row chunk,
-//     relative to its own half-diagonal, for FP32 differences of positions
-//     rounded relative to its centre.  Every other (chunk, chunk) visit is
+//     pairs Newtonian by the box test, far enough from the row chunk, relative
+//     to its own half-diagonal, for FP32 differences of positions rounded
+//     relative to its centre, and not closer than SCALED_MIN of the set's
+//     extent, which bounds the powers of 1/r below.  Every other (chunk, chunk) visit is
 //     left to the ordered rest kernel (sg_direct.hip).
 //   * k_sym evaluates the marked pairs.  A wave holds a 64-particle row chunk
 //     (the i side) and meets 64-particle column chunks (the j side); its lanes
@@ -20,7 +21,8 @@
 //     four chunk pairs over q.
 //   * Positions and masses are scaled by powers of two (the set's extent and
 //     largest mass become order one; the reduce kernel undoes it), so that r^-3
-//     stays in the FP32 range in any units.
+//     stays in the FP32 range in any units: at most 2^60 (SCALED_MIN), and the
+//     gradient's terms in r^-4 2^84 times the cotangents.
 //   * Sums go to FP64 after at most 16 sequential FP32 additions and a tree
 //     over the lanes.
 //   * Work items are pairs of superblocks.  Every (superblock, superblock)
@@ -38,6 +40,7 @@ constexpr int NP = 4, NQ = 16;         // lane grid: i groups x j groups
 constexpr int IA = TC / NP;            // i per lane
 constexpr int JB = TC / NQ;            // j per lane
 constexpr int JC = 4;                  // column chunks a wave owns at a time
+constexpr double SCALED_MIN = 0x1p-20; // about a cell of the curve: rarely the nearer bound
 static_assert(NP * NQ == 64 && IA == 16 && JB == 4, "lane grid");
 
 // ------------------------------------------------------------ chunk pairs
@@ -89,6 +92,9 @@ __global__ __launch_bounds__(256) void k_sym_classify(SymArgs a)
         rest[r] = a.nchunks;
     }
     const float wide = a.fp64 ? 0.0f : WIDE_K * WIDE_K;
+    // least squared distance (FP32 overflow: the largest, which an infinite d2 passes)
+    const double least = a.fp64 ? 0.0 : SCALED_MIN / a.bbox[6];
+    const float least2 = (float)fmin(least * least, 3.0e38);
     for (int w = 0; w < a.words; ++w) {
         const int cj = w * 64 + lane;
         const int cc = min(cj, a.nchunks - 1);
@@ -103,7 +109,7 @@ __global__ __launch_bounds__(256) void k_sym_classify(SymArgs a)
             const float hm = fmaxf(cl.w, rl[r].w);
             const float rho2 = cj < ci ? ch.w : rh[r].w;
             const bool ok = cj < a.nchunks && cj != ci &&
-                            d2 > fmaxf(hm * hm, wide * rho2) * (1.0f + FAR_MARGIN);
+                            d2 > fmaxf(fmaxf(hm * hm, wide * rho2), least2) * (1.0f + FAR_MARGIN);
             const uint64_t bits = __ballot(ok);
             rest[r] -= __builtin_popcountll(bits);
             if (ci < a.nchunks && lane == 0) a.sym[(int64_t)ci * a.words + w] = bits;
@@ -437,10 +443,9 @@ __global__ __launch_bounds__(256) void k_sym_reduce(SymArgs a)
     }
     // back to the caller's units: a has m / r^2, the potential m / r
     const double len = a.fp64 ? 1.0 : a.bbox[6], unit = a.fp64 ? 1.0 : 1.0 / a.bbox[7];
-    s[0] *= len * len * unit;
-    s[1] *= len * len * unit;
-    s[2] *= len * len * unit;
-    s[3] *= len * unit;
+    // (factor by factor: len^2 alone may leave the range)
+    for (int k = 0; k < 3; ++k) s[k] = s[k] * unit * len * len;
+    s[3] = s[3] * unit * len;
     const int c = (int)(i / TC), ns = a.psi ? 5 : 4;
     const int e = a.seg[c + 1];
     double psi = 0.0;

@@ -1587,18 +1587,17 @@ __global__ __launch_bounds__(64) void k_psi_only(PairArgs a)
         bl[c] = wave_min(bl[c]);
         bh[c] = wave_max(bh[c]);
     }
-    // only side i matters for psi: a chunk farther than the wave's largest
-    // H_i (with the far test's margin) holds no contributing pair
-    const float hmax = wave_max((float)Hi);
-    const float lim2 = hmax * hmax * (1.0f + FAR_MARGIN);
+    // only side i matters for psi: a chunk farther from the group's box than the
+    // wave's largest H_i, or from a lane's particle than its own, holds no pair of
+    // theirs.  A distance r <= H_i, of a pair or of a point of a box, as FP32 sees it
+    // is off by at most sqrt(3) (2^-24 (2 p + r) + the subtraction's 2^-24 r) + 3
+    // 2^-24 r < 2^-22 (p + 2 r), p = |x - O| on the largest axis: the reach below
     const float px = (float)xr, py = (float)yr, pz = (float)zr;
-    const float reach2 = (float)hi2 * (1.0f + FAR_MARGIN);
-    // |x - O| of the lane's particle and of all j within its reach, largest axis
     const float pmax = fmaxf(fabsf(px), fmaxf(fabsf(py), fabsf(pz)));
-    // r as FP32 sees it is off by at most sqrt(3) (2^-24 (2 pmax + r) + the
-    // subtraction's 2^-24 r) + 3 2^-24 r < 2^-22 (pmax + 2 r) for r <= H_i
     const float cand = (float)Hi * (1.0f + 2.0e-6f) + 4.8e-7f * pmax;
     const float cand2 = cand * cand;
+    const float lim = wave_max((float)Hi) * (1.0f + 2.0e-6f) + 4.8e-7f * wave_max(pmax);
+    const float lim2 = lim * lim;
     double ps = 0.0;
     // part p has every jsplit-th chunk (jsplit a power of two), of the tiles
     // that hold one of them
@@ -1620,7 +1619,7 @@ __global__ __launch_bounds__(64) void k_psi_only(PairArgs a)
                 const float gx = fmaxf(0.0f, fmaxf((float)(cm.lo[0] - Ox) - px, px - (float)(cm.hi[0] - Ox)));
                 const float gy = fmaxf(0.0f, fmaxf((float)(cm.lo[1] - Oy) - py, py - (float)(cm.hi[1] - Oy)));
                 const float gz = fmaxf(0.0f, fmaxf((float)(cm.lo[2] - Oz) - pz, pz - (float)(cm.hi[2] - Oz)));
-                if (!__ballot(fmaf(gx, gx, fmaf(gy, gy, gz * gz)) <= reach2)) continue;
+                if (!__ballot(fmaf(gx, gx, fmaf(gy, gy, gz * gz)) <= cand2)) continue;
                 const int64_t j = (c0 + __builtin_ctz(bits)) * TC + lane;
                 wave_lds_sync();
                 const double jx = a.j.x[j] - Ox, jy = a.j.y[j] - Oy, jz = a.j.z[j] - Oz;

@@ -43,3 +43,24 @@ def test_against_oracle(grav, kind, n, ibeg, ni, nk, length):
     assert np.all(psi[rows][~gas] == 0.0)
     got = psi[rows][gas] * length ** 2
     assert np.max(np.abs(got - ref[gas]) / np.abs(ref[gas])) <= 1e-11
+
+
+@pytest.mark.parametrize("nk", [0, 2])
+@pytest.mark.parametrize("H", [1e-5, 1e-7, 1e-8])
+def test_supports_of_the_size_of_fp32_rounding(grav, H, nk):
+    """Tight clumps of 64 + 32 particles, 0.6 H apart, all over a set 1e5 to 1e8
+    times larger than H: chunks that straddle two clumps test boxes whose FP32
+    corners, relative to the group's origin, are off by more than H."""
+    rng = np.random.default_rng(0)
+    pos = []
+    for c in rng.uniform(-1.0, 1.0, (60, 3)):
+        d = rng.normal(size=3)
+        d *= 0.6 * H / np.linalg.norm(d)
+        pos += [c + 0.01 * H * rng.normal(size=(64, 3)), c + d + 0.01 * H * rng.normal(size=(32, 3))]
+    pos = np.concatenate(pos)
+    n = len(pos)
+    args = [*(p.copy() for p in pos.T), rng.uniform(0.5, 1.5, n) / n, np.full(n, H * H)]
+    want = oracle.psi(*args, nkernel=nk)
+    # positions relative to the group's origin are off by 2^-53 of the distance to it
+    tol = 1e-11 + 8.0 * 2.0 ** -53 / H
+    np.testing.assert_allclose(grav.psi(*args, nkernel=nk), want, rtol=tol, atol=0)

@@ -625,7 +625,7 @@ struct AdjLane {
     bool gas;
     int id;
     Lane32 q;      // FP32 (positions unused)
-    float px, py, pz, ph;
+    float px, py, pz, ph, slack;
 };
 
 __device__ __forceinline__ void adj_lane(const SortedSet &P, const double *wx, const double *wy,
@@ -656,6 +656,7 @@ __device__ __forceinline__ void adj_lane(const SortedSet &P, const double *wx, c
     l.py = (float)l.y;
     l.pz = (float)l.z;
     l.ph = (float)l.H;
+    l.slack = box_slack(l.px, l.py, l.pz);
 }
 
 // Whether some lane's pairs with the chunk of box and largest H cm may be
@@ -666,7 +667,7 @@ __device__ __forceinline__ bool adj_chunk_near(const TileMeta &cm, double Ox, do
     const float gx = fmaxf(0.0f, fmaxf((float)(cm.lo[0] - Ox) - l.px, l.px - (float)(cm.hi[0] - Ox)));
     const float gy = fmaxf(0.0f, fmaxf((float)(cm.lo[1] - Oy) - l.py, l.py - (float)(cm.hi[1] - Oy)));
     const float gz = fmaxf(0.0f, fmaxf((float)(cm.lo[2] - Oz) - l.pz, l.pz - (float)(cm.hi[2] - Oz)));
-    const float hm = fmaxf(l.ph, (float)cm.maxH);
+    const float hm = fmaxf(l.ph, (float)cm.maxH) + l.slack;
     return __ballot(!(fmaf(gx, gx, fmaf(gy, gy, gz * gz)) > hm * hm * (1.0f + FAR_MARGIN))) != 0;
 }
 

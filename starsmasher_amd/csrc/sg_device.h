@@ -10,6 +10,14 @@
 namespace sg {
 
 constexpr float FAR_MARGIN = 1.0e-3f;   // relative guard on the box-distance test
+// How far a distance r from a point p to a box, all relative to an origin, is off in
+// FP32 beyond that: at most sqrt(3) (2^-24 (2 P + r) + 2^-24 r) + 3 2^-24 r < 2^-22 (P
+// + 2 r), P the largest coordinate of p.  This times P; r is in the guard.
+constexpr float BOX_ROUND = 4.8e-7f;
+__device__ __forceinline__ float box_slack(float px, float py, float pz)
+{
+    return BOX_ROUND * fmaxf(fabsf(px), fmaxf(fabsf(py), fabsf(pz)));
+}
 // Hi-only differences x_j,hi - x_i,hi carry a relative error of about
 // 2^-24 (|x_i - O| + |x_j - O| + r) / r <= 2^-24 (2 + 2 |x_i - O| / r).
 // Chunks whose box is nearer to the wave's box than WIDE_K rho (rho = the

@@ -1003,18 +1003,19 @@ struct Fold4 {
 enum Visit { VISIT_FAR, VISIT_WIDE, VISIT_NEAR };
 
 // How the chunk with box and largest H cm is evaluated by a wave with one
-// particle per lane at (px, py, pz) relative to O (distance^2 rho2 from it)
-// and support ph: near when some lane's pairs may be softened, else wide when
+// particle per lane at (px, py, pz) relative to O (distance^2 rho2 from it),
+// support ph and box_slack slack: near when some lane's pairs may be softened, else wide when
 // a lane is too close, relative to its distance from O, for differences of
 // positions rounded relative to O.
 __device__ __forceinline__ Visit classify_visit(const TileMeta &cm, double Ox, double Oy, double Oz,
-                                                float px, float py, float pz, float ph, float rho2)
+                                                float px, float py, float pz, float ph, float slack,
+                                                float rho2)
 {
     const float gx = fmaxf(0.0f, fmaxf((float)(cm.lo[0] - Ox) - px, px - (float)(cm.hi[0] - Ox)));
     const float gy = fmaxf(0.0f, fmaxf((float)(cm.lo[1] - Oy) - py, py - (float)(cm.hi[1] - Oy)));
     const float gz = fmaxf(0.0f, fmaxf((float)(cm.lo[2] - Oz) - pz, pz - (float)(cm.hi[2] - Oz)));
     const float d2 = fmaf(gx, gx, fmaf(gy, gy, gz * gz));
-    const float hm = fmaxf(ph, (float)cm.maxH);
+    const float hm = fmaxf(ph, (float)cm.maxH) + slack;
     if (__ballot(!(d2 > hm * hm * (1.0f + FAR_MARGIN)))) return VISIT_NEAR;
     if (__ballot(!(d2 > WIDE_K * WIDE_K * rho2 * (1.0f + FAR_MARGIN)))) return VISIT_WIDE;
     return VISIT_FAR;
@@ -1310,7 +1311,7 @@ __global__ __launch_bounds__(64) void k_pair_wave(PairArgs a)
     int idi[1];
     near_i_state<1>(a.i, ii, Hi, invHi, hi2, idi);
     const float px = (float)xr, py = (float)yr, pz = (float)zr, ph = (float)Hi[0];
-    const float rho2 = fmaf(px, px, fmaf(py, py, pz * pz));
+    const float rho2 = fmaf(px, px, fmaf(py, py, pz * pz)), slack = box_slack(px, py, pz);
     double acc[PSI ? 5 : 4] = {};
     unsigned nfp64 = 0, visits = 0, nearv = 0, widev = 0;
     // partition jp: part jp % jsub of every (jsplit / jsub)-th chunk
@@ -1319,7 +1320,7 @@ __global__ __launch_bounds__(64) void k_pair_wave(PairArgs a)
     int64_t j = (int64_t)first * TC + lane;
     double jx = a.j.x[j], jy = a.j.y[j], jz = a.j.z[j], jm = a.j.m[j], jh = a.j.Hs[j];
     for (int cj = first; cj < nchunks; cj += stride) {
-        const Visit v = classify_visit(a.chunks[cj], Ox, Oy, Oz, px, py, pz, ph, rho2);
+        const Visit v = classify_visit(a.chunks[cj], Ox, Oy, Oz, px, py, pz, ph, slack, rho2);
         const double rx = jx - Ox, ry = jy - Oy, rz = jz - Oz;
         uint64_t real = 0;
         if (v == VISIT_FAR) {
@@ -1410,7 +1411,7 @@ __global__ __launch_bounds__(64) void k_sym_rest(SymArgs a)
     int idi[1];
     near_i_state<1>(P, ii, Hi, invHi, hi2, idi);
     const float px = (float)xr, py = (float)yr, pz = (float)zr, ph = (float)Hi[0];
-    const float rho2 = fmaf(px, px, fmaf(py, py, pz * pz));
+    const float rho2 = fmaf(px, px, fmaf(py, py, pz * pz)), slack = box_slack(px, py, pz);
     constexpr int NS = PSI ? 5 : 4;
     double acc[NS] = {};
     unsigned nfp64 = 0, visits = 0, nearv = 0, widev = 0;
@@ -1429,7 +1430,7 @@ __global__ __launch_bounds__(64) void k_sym_rest(SymArgs a)
            jh = P.Hs[(int64_t)cj * TC + lane];
     for (;;) {
         const Visit v =
-            classify_visit(a.chunks[cj], Ox, Oy, Oz, px, py, pz, ph, FP64 ? 0.0f : rho2);
+            classify_visit(a.chunks[cj], Ox, Oy, Oz, px, py, pz, ph, slack, FP64 ? 0.0f : rho2);
         const double rx = jx - Ox, ry = jy - Oy, rz = jz - Oz;
         uint64_t real = 0;
         if (!FP64 && v == VISIT_FAR) {
@@ -1589,14 +1590,12 @@ __global__ __launch_bounds__(64) void k_psi_only(PairArgs a)
     }
     // only side i matters for psi: a chunk farther from the group's box than the
     // wave's largest H_i, or from a lane's particle than its own, holds no pair of
-    // theirs.  A distance r <= H_i, of a pair or of a point of a box, as FP32 sees it
-    // is off by at most sqrt(3) (2^-24 (2 p + r) + the subtraction's 2^-24 r) + 3
-    // 2^-24 r < 2^-22 (p + 2 r), p = |x - O| on the largest axis: the reach below
+    // theirs.  That of a pair is off in FP32 like that to a box (box_slack).
     const float px = (float)xr, py = (float)yr, pz = (float)zr;
-    const float pmax = fmaxf(fabsf(px), fmaxf(fabsf(py), fabsf(pz)));
-    const float cand = (float)Hi * (1.0f + 2.0e-6f) + 4.8e-7f * pmax;
+    const float slack = box_slack(px, py, pz);
+    const float cand = (float)Hi * (1.0f + 2.0e-6f) + slack;
     const float cand2 = cand * cand;
-    const float lim = wave_max((float)Hi) * (1.0f + 2.0e-6f) + 4.8e-7f * wave_max(pmax);
+    const float lim = wave_max((float)Hi) * (1.0f + 2.0e-6f) + wave_max(slack);
     const float lim2 = lim * lim;
     double ps = 0.0;
     // part p has every jsplit-th chunk (jsplit a power of two), of the tiles

@@ -12,7 +12,7 @@ import pytest
 
 import oracle
 from conftest import rel_errors
-from starsmasher_amd import SG_PREC_FP32C, Gravity
+from starsmasher_amd import SG_PREC_FP32C, SG_PREC_FP64, Gravity
 
 pytestmark = pytest.mark.gpu
 
@@ -85,3 +85,35 @@ def test_masses_and_extents_at_the_ends_of_the_range(grav):
                       (rng.normal(size=(n, 3)), 1e-310, 0.1)):
         res = grav.compute(*(c.copy() for c in pos.T), z + m, z + h * h)
         assert all(np.isfinite(r).all() for r in res)
+
+
+def _clumps(k, H):
+    """Tight clumps of 64 + 32 particles 0.6 H apart: FP32 positions relative to an
+    origin in another clump are off by up to 1e-7, more than H."""
+    rng = np.random.default_rng(0)
+    pos = []
+    for c in rng.uniform(-1.0, 1.0, (k, 3)):
+        d = rng.normal(size=3)
+        d *= 0.6 * H / np.linalg.norm(d)
+        pos += [c + 0.01 * H * rng.normal(size=(64, 3)), c + d + 0.01 * H * rng.normal(size=(32, 3))]
+    pos = np.concatenate(pos)
+    n = len(pos)
+    return [*(p.copy() for p in pos.T), rng.uniform(0.5, 1.5, n) / n, np.full(n, H * H)]
+
+
+# small sets run one wave per 64 particles, the larger ones the rest kernels
+@pytest.mark.parametrize("k,prec", [(60, SG_PREC_FP32C), (560, SG_PREC_FP32C), (560, SG_PREC_FP64)])
+@pytest.mark.parametrize("H", [1e-5, 1e-7, 1e-8])
+def test_supports_of_the_size_of_fp32_rounding(grav, k, prec, H):
+    args = _clumps(k, H)
+    rows = np.arange(0, args[0].size, k // 20)
+    ref = oracle.direct(*args, rows=rows)
+    res = grav.compute(*args, precision=prec)
+    ea, ep = rel_errors(np.stack(res[:3], -1)[rows], res[3][rows], np.stack(ref[:3], -1), ref[3])
+    assert ea.max() <= 1e-5 and ep.max() <= 1e-6
+    if prec == SG_PREC_FP32C:
+        rng = np.random.default_rng(1)
+        cot = [rng.normal(size=args[0].size).astype(np.float32).astype(np.float64) for _ in range(4)]
+        ref = oracle.vjp(*args, np.stack(cot[:3], 1), cot[3], rows=rows)
+        for a, b in zip(grav.vjp(*args, *cot), ref):
+            assert np.abs(a[rows] - b).max() <= 1e-5 * np.sqrt(np.mean(b ** 2))

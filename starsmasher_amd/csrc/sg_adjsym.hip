@@ -26,7 +26,7 @@ constexpr int HC = TC / 2;     // columns per block
 constexpr int JC = 2;          // column chunks a wave owns at a time
 constexpr int NW = 4;          // waves per workgroup
 constexpr int NS = 8;          // sums: G1 (3), G2, G3 (3), GM'
-static_assert(RA * 8 == TC && CB * 8 == HC, "8 x 8 lane grid");
+static_assert(RA * 8 == TC && CB * 8 == HC && NW * JC == ADJ_SYM_STEP, "8 x 8 lane grid");
 
 #define ADJ_DIFF(k, dx, dy, dz, r)                                             \
     "v_sub_f32_e32 v" dx ", %[xj" k "], %[xi]\n\t"                             \

@@ -327,26 +327,21 @@ static SymLayout sym_layout(int nchunks, int64_t words, int64_t slabs, int sums)
 }
 static int64_t sym_words(int nchunks) { return (int64_t)nchunks * ((nchunks + 63) / 64); }
 
-// The whole-set pass evaluates each unordered far pair once.  Up to
+// The whole-set passes that evaluate each unordered far pair once.  Up to
 // SYM_MAX_SB superblocks make the work items (8,256 pairs of them at 128, 16
 // rounds of the workgroups that fit at once) and the partial-sum slabs (32 B
-// per particle each).  A workgroup has as many waves as its superblock has
-// column groups of four chunks, up to four; in FP64 always four, of two chunks
-// each.
-static void plan_sym(EvalPlan &p, int n, bool fp64, bool psi)
+// per particle each).  A superblock is whole column groups of `step` chunks.
+static void plan_sym(EvalPlan &p, int n, int step, int sums)
 {
     const int nchunks = (int)(p.padded / TC);
     const int want = (nchunks + SYM_MAX_SB - 1) / SYM_MAX_SB;
-    p.waves = fp64 || want > 8 ? 4 : (want > 4 ? 2 : 1);
-    const int step = fp64 ? SYM64_STEP : 4 * p.waves;   // a column group
     p.sb = (want + step - 1) / step * step;
     p.nsb = (nchunks + p.sb - 1) / p.sb;
     p.jsplit = p.nsb + 1;
     p.part_elems = p.psipart_elems = p.flag_elems = 0;
-    p.sums = psi ? 5 : 4;
+    p.sums = sums;
     p.sym_bytes = sym_layout(nchunks, sym_words(nchunks), (int64_t)p.jsplit * 4 * n, p.sums).bytes;
     p.sym = true;
-    p.fp64 = fp64;
 }
 
 static SymArgs sym_args(const EvalPlan &p, int n, int nchunks, const PrepBuffers &b,
@@ -418,8 +413,13 @@ EvalPlan plan_eval(int n, int ni, int wg, int ipl, int jsplit_cfg, int precision
         p.psipart_elems = psi ? (int64_t)p.jsplit * ni : 0;
     }
     if (allow_sym && automatic && ni == n && n >= (fp64 ? SYM64_MIN_N : SYM_MIN_N) &&
-        n <= SYM_MAX_N)
-        plan_sym(p, n, fp64, psi);
+        n <= SYM_MAX_N) {
+        // k_sym: two waves of four chunks up to 65,536 particles, whose superblocks
+        // hold no more column groups than that, then four
+        p.fp64 = fp64;
+        p.waves = !fp64 && p.ntiles * CHUNKS <= 8 * SYM_MAX_SB ? 2 : 4;
+        plan_sym(p, n, fp64 ? SYM64_STEP : 4 * p.waves, psi ? 5 : 4);
+    }
     return p;
 }
 
@@ -1326,14 +1326,9 @@ int sg_vjp_device(sg_context *c, int n, const double *x, const double *y, const 
     if (automatic && n >= sg::ADJ_SYM_MIN_N && n <= sg::SYM_MAX_N) {
         sg::EvalPlan p{};
         p.padded = padded;
-        sg::plan_sym(p, n, false, false);
-        p.waves = 4;
-        p.sb = (p.sb + 7) / 8 * 8;   // whole column groups of k_adj_sym
         const int nchunks = (int)(padded / sg::TC);
-        p.nsb = (nchunks + p.sb - 1) / p.sb;
-        p.jsplit = p.nsb + 1;
-        p.sums = 5;
-        p.sym_bytes = sg::sym_layout(nchunks, sg::sym_words(nchunks), (int64_t)p.jsplit * 4 * n, p.sums).bytes;
+        // superblocks as k_sym's, of one or two of its own column groups
+        sg::plan_sym(p, n, (nchunks <= 8 * sg::SYM_MAX_SB ? 1 : 2) * sg::ADJ_SYM_STEP, 5);
         if (sym_scratch(c, p.sym_bytes)) {
             sg::AdjSymArgs q{};
             q.y = sg::sym_args(p, n, nchunks, b, c->sym, nkernel, c->stats);

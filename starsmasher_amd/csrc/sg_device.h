@@ -55,7 +55,7 @@ __device__ __forceinline__ unsigned long long *stat_copy(unsigned long long *sta
 __device__ __forceinline__ unsigned long long wave_sum_count(unsigned v)
 {
     unsigned long long s = 0;
-    for (int bit = 0; __ballot(v >> bit) != 0 && bit < 32; ++bit)
+    for (int bit = 0; bit < 32 && __ballot(v >> bit) != 0; ++bit)
         s += (unsigned long long)__builtin_popcountll(__ballot((v >> bit) & 1u)) << bit;
     return s;
 }

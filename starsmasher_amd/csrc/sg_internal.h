@@ -78,7 +78,8 @@ struct PairArgs {
 // chunk is cut into segments with partial sums of their own: at most SYM_SEGS
 // + nchunks of them, of SYM_SEG_MIN chunk visits or more.
 constexpr int SYM_SEGS = 32768, SYM_SEG_MIN = 8;
-constexpr int SYM64_STEP = 8;   // superblocks of k_sym64 are multiples of this
+// superblocks of k_sym64 and k_adj_sym are multiples of these
+constexpr int SYM64_STEP = 8, ADJ_SYM_STEP = 8;
 // A set of a batch: where its particles, chunks, bits and slabs begin in the
 // batch's arrays.  Segments are numbered over the whole batch.
 struct SymSet {
@@ -96,7 +97,7 @@ struct SymArgs {
     int64_t n;               // real particles
     int nchunks, words;      // padded / TC, (nchunks + 63) / 64
     int sb, nsb;             // chunks per superblock, superblocks
-    int waves;               // waves per workgroup of k_sym (1, 2, 4)
+    int waves;               // waves per workgroup of k_sym (2, 4)
     int nkernel;
     double *partial;         // [nsb + 1][4][n], sorted order
     double *segsum;          // [SYM_SEGS + nchunks][4 (5 with psi)][TC]

@@ -491,7 +491,6 @@ hipError_t launch_sym(const SymArgs &a, hipStream_t s)
 {
     const dim3 grid((unsigned)(a.sets ? a.nitems : a.nsb * (a.nsb + 1) / 2));
     switch (a.waves) {
-    case 1: hipLaunchKernelGGL((k_sym<1>), grid, dim3(64), 0, s, a); break;
     case 2: hipLaunchKernelGGL((k_sym<2>), grid, dim3(128), 0, s, a); break;
     case 4: hipLaunchKernelGGL((k_sym<4>), grid, dim3(256), 0, s, a); break;
     default: return hipErrorInvalidConfiguration;

@@ -22,6 +22,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <mutex>
+#include <new>
 #include <vector>
 
 using sg::TJ;
@@ -1009,7 +1010,13 @@ int sg_compute_batch_device(sg_context *c, int nsets, const long long *offsets, 
     int rc;
     if (!same_plan) {
         HIP_TRY(hipStreamSynchronize(c->stream));
-        if ((rc = build_plan(c, nsets, offsets, wg, ipl)) != SG_OK) {
+        try {
+            rc = build_plan(c, nsets, offsets, wg, ipl);
+        } catch (const std::bad_alloc &) {   // of the host's tables
+            last_hip_error() = hipErrorOutOfMemory;
+            rc = SG_ERR_HIP;
+        }
+        if (rc != SG_OK) {
             P.offsets.clear();   // half built: the next call starts over
             return rc;
         }

@@ -4,6 +4,7 @@ launches are checked for the buffers they would work in."""
 import ctypes as C
 import os
 import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -20,8 +21,12 @@ def built(tmp_path_factory):
                     "-I/opt/rocm/include", f"-I{ROOT}/include", f"-I{csrc}",
                     os.path.join(csrc, "sg_capi.cpp"),
                     os.path.join(ROOT, "tests", "fake_device.cpp"), "-o", str(so)], check=True)
+    return load(str(so))
+
+
+def load(path):
     # RTLD_DEEPBIND: its own hipMalloc and not that of a runtime loaded before
-    L = C.CDLL(str(so), mode=os.RTLD_LOCAL | os.RTLD_DEEPBIND)
+    L = C.CDLL(path, mode=os.RTLD_LOCAL | os.RTLD_DEEPBIND)
     L.fake_used.restype = C.c_longlong
     L.fake_ran.restype = L.fake_fault.restype = C.c_char_p
     return L
@@ -255,3 +260,24 @@ def test_slabs_leave_as_much_free_as_they_take(ctx):
         c.reset()
         assert ctx.L.sg_destroy(c.h) == OK
     assert seen == {"ordered", "sym"}
+
+
+_NO_MEMORY = r"""
+import resource, sys
+sys.path.insert(0, {tests!r})
+import test_allocation as t
+L = t.load({lib!r})
+c = t.Context(L)
+used = int(open("/proc/self/statm").read().split()[0]) * 4096
+resource.setrlimit(resource.RLIMIT_AS, (used + (60 << 20),) * 2)
+print(c.batch([1 << 30, 1 << 29, 300]))
+print(c.batch([5000, 300]), c.state())
+"""
+
+
+def test_a_plan_that_host_memory_does_not_hold(built):
+    """An exception never leaves a C entry point: the call reports the error."""
+    code = _NO_MEMORY.format(tests=os.path.join(ROOT, "tests"), lib=built._name)
+    r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0, (r.returncode, r.stderr[-500:])
+    assert r.stdout.split("\n")[:2] == ["6", "0 ['sym']"]

@@ -3,8 +3,8 @@ both precisions), against the oracle and against the ordered batch kernel, which
 shapes still run.
 
 Bounds: the library's stated FP32C errors (1e-5 on the acceleration, 1e-6 on
-the potential); both passes round each pair to FP32 and sum at most 32 pairs in
-FP32, so they differ by no more than twice that.  FP64: 1e-11 and 1e-12, as in the
+the potential); both passes round each pair to FP32 and sum pairs in FP32 (32 in
+sequence, or 16 and a tree over the lanes), so they differ by no more than twice that.  FP64: 1e-11 and 1e-12, as in the
 other parity tests.
 """
 import numpy as np

@@ -5,8 +5,9 @@ is chosen per precision with sg_set_config / sg_set_batch_config, the
 softening kernel per call, and the legacy entry points' precision by the
 SPHGRAV_PRECISION environment variable.  Each combination instantiates its
 own kernels (k_far_fp32c<wg, ipl, nk>, k_far_fp64<wg, ipl> + k_near<ipl, nk>,
-k_far_batch<wg, ipl, fp64, nk>, k_adj_far<wg, fp64, nk>,
-k_far_fp32c_split<wg> + k_near_psi<fast, nk>), so each is run here on a set
+k_far_batch<wg, ipl, fp64, nk>, k_adj_far<wg, fp64, nk> + k_adj_near<fast, nk>,
+k_far_fp32c_split<wg> + k_near_psi<fast, nk>; the size the automatic one stands for runs
+what the automatic size runs: k_pair_wave, k_sym), so each is run here on a set
 with point particles and a distinct coincident pair.
 
 Reference semantics: grav_force_direct.cu:55-396 (the three softening
@@ -147,8 +148,8 @@ def adj_set():
 @pytest.mark.parametrize("nk", [0, 1, 2])
 @pytest.mark.parametrize("prec", PREC)
 def test_adjoint_workgroup_sizes(grav, adj_set, prec, nk, wg):
-    """The adjoint's far kernel takes the forward workgroup size of its
-    precision: k_adj_far<64|128, fp64, nk> against the oracle's full FP64
+    """The adjoint's far kernel takes the workgroup size set for its precision:
+    k_adj_far<64|128, fp64, nk> and k_adj_near against the oracle's full FP64
     gradient (median and rms-normalised maximum as in test_gpu_adjoint)."""
     x, m, r2, w, cu, refs = adj_set
     old = grav.get_config(prec)
@@ -171,17 +172,18 @@ def test_adjoint_workgroup_sizes(grav, adj_set, prec, nk, wg):
         assert med <= lim and rms <= lim, (key, med, rms)
 
 
-@pytest.mark.parametrize("wg", [64, 128])
+@pytest.mark.parametrize("wg,jsplit", [(64, 0), (128, 0), (128, 3), (256, 3)])
 @pytest.mark.parametrize("nk", [0, 1, 2])
 @pytest.mark.parametrize("prec", PREC)
-def test_grad_h_pass_workgroup_sizes(grav, mixed_set, prec, nk, wg):
+def test_grad_h_pass_workgroup_sizes(grav, mixed_set, prec, nk, wg, jsplit):
     """The pass that forms the grad-h term runs the far kernel at the
-    forward workgroup size with one i per lane (k_far_fp32c_split<64|128> or
-    k_far_fp64<64|128, 1>) and the psi near kernel: a, phi against the
-    oracle and psi against the oracle's exact sum."""
+    forward workgroup size with one i per lane (k_far_fp32c_split<64|128|256> or
+    k_far_fp64<64|128|256, 1>) and the psi near kernel: a, phi against the
+    oracle and psi against the oracle's exact sum.  128 is what the automatic size
+    stands for here: in FP32C without a j-split it runs k_pair_wave<nk, true>."""
     d, refs = mixed_set
     old = grav.get_config(prec)
-    grav.set_config(prec, wg, 1, 0)
+    grav.set_config(prec, wg, 1, jsplit)
     try:
         ax, ay, az, pot, psi = grav.compute_psi(*_args(d), nkernel=nk, precision=prec)
     finally:

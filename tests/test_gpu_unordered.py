@@ -4,8 +4,9 @@
 A context takes it at its automatic configuration from 49,152 particles on;
 an explicit j-split asks for the ordered pass.  Bounds: the library's stated
 FP32C errors (1e-5 on the acceleration, 1e-6 on the potential, as in the other
-parity tests); both passes round each pair to FP32 and sum at most 32 pairs in
-FP32, so they differ from each other by no more than twice that.
+parity tests); both passes round each pair to FP32 and sum pairs in FP32 (the
+ordered one 32 in sequence; this one 16 and a tree over 16 lanes for a row, 16 and a tree
+over four for a column), so they differ from each other by no more than twice that.
 """
 import numpy as np
 import pytest

@@ -48,6 +48,8 @@ FLOPS_PER_UNORDERED_PAIR = 29
 PEAK_FP32_TFLOPS = 157.3      # MI355X FP32 vector (AMD spec)
 PEAK_FP64_TFLOPS = 78.6
 TC = 64                       # j per chunk (the unit of the near / wide decisions)
+# which pass a whole set takes at the automatic shape (csrc/sg_internal.h)
+WAVE_MAX_NI, SYM_MIN_N, SYM64_MIN_N, SYM_MAX_N, AUTO_SMALL_NI = 49151, 49152, 32769, 1 << 22, 65536
 
 # The FP64 steps of the precision specification (FP32 pair arithmetic with
 # hi/lo positions and compensated sums, FP64 only for these), and the FP64
@@ -57,11 +59,11 @@ PRECISION_POLICY = {
                        "total-energy diagnostic"],
     "added_fp64": [
         "wide chunks: pair differences formed in FP64 and rounded once (chunks close to a wave "
-        "relative to its spread about the workgroup origin)",
+        "relative to its spread about its origin)",
         "near chunks: pair differences formed in FP64 and rounded once, FP32 body",
         "softened and self pairs (r < max(H_i, H_j)): whole pair in FP64",
-        "FP32 partial sums folded into FP64 accumulators every 32 j (in place of per-term "
-        "compensated FP32 sums)",
+        "FP32 partial sums added to FP64 accumulators after 16 pairs in sequence and a tree over "
+        "the lanes, or 32 in sequence (in place of per-term compensated FP32 sums)",
     ],
 }
 
@@ -488,6 +490,19 @@ def time_adjoint(g, n_adj, steps, log_fn):
     return res
 
 
+def whole_set_pass(prec, n, config):
+    """The pass a whole set of n runs at this configuration (sg_set_config; where
+    the device holds the memory of the unordered one): "unordered", "waves" or
+    "tiles"."""
+    wg, ipl, jsplit = config
+    if ipl == 1 and jsplit == 0 and wg in (0, 128 if n <= AUTO_SMALL_NI else 256):
+        if (SYM64_MIN_N if prec == 1 else SYM_MIN_N) <= n <= SYM_MAX_N:
+            return "unordered"
+        if prec == 0 and n <= WAVE_MAX_NI:
+            return "waves"
+    return "tiles"
+
+
 def profiled_traffic(wg, ipl):
     """HBM bytes per launch of the far-pair kernel at the default shape, from
     the committed rocprofv3 FETCH_SIZE + WRITE_SIZE summary (None if absent)."""
@@ -619,11 +634,12 @@ def main():
     kernel_pairs = float(n) * padded
 
     def executed_flops(prec):
-        w, i, js = g.get_config(prec)
-        once = i == 1 and js == 0 and w in (0, 256) and 65536 < n <= 1 << 22
-        return once, kernel_pairs * (FLOPS_PER_UNORDERED_PAIR / 2 if once else FLOPS_PER_PAIR)
+        once = whole_set_pass(prec, n, g.get_config(prec)) == "unordered"
+        return kernel_pairs * (FLOPS_PER_UNORDERED_PAIR / 2 if once else FLOPS_PER_PAIR)
 
-    once, flops = executed_flops(SG_PREC_FP32C)
+    kernel = {"unordered": "k_sym + k_sym_rest", "waves": "k_pair_wave",
+              "tiles": "k_far_fp32c"}[whole_set_pass(SG_PREC_FP32C, n, g.get_config(SG_PREC_FP32C))]
+    flops = executed_flops(SG_PREC_FP32C)
     achieved = flops / (r32["far_ms"] * 1e-3) / 1e12
 
     acc = {}
@@ -662,7 +678,7 @@ def main():
         "roofline": {"bound": "valu", "achieved": round(achieved, 3), "peak": PEAK_FP32_TFLOPS,
                      "unit": "TFLOP/s", "frac": round(achieved / PEAK_FP32_TFLOPS, 4),
                      "traffic": (profiled_traffic(wg, ipl) if args.workload == "giant1m" else None),
-                     "kernel": "k_sym + k_sym_rest" if once else "k_far_fp32c",
+                     "kernel": kernel,
                      "flops_per_pair": flops / kernel_pairs,
                      "pairs_per_launch": kernel_pairs, "kernel_ms": round(r32["far_ms"], 3)},
         "phases_ms": {"prep": round(r32["prep_ms"], 3), "pair_kernel": round(r32["far_ms"], 3),
@@ -682,7 +698,7 @@ def main():
     if r64 is not None:
         v64 = pairs / (r64["ms_per_step"] * 1e-3) / 1e9
         # far and near kernels together
-        a64 = executed_flops(SG_PREC_FP64)[1] / ((r64["far_ms"] + r64["near_ms"]) * 1e-3) / 1e12
+        a64 = executed_flops(SG_PREC_FP64) / ((r64["far_ms"] + r64["near_ms"]) * 1e-3) / 1e12
         line["fp64_kernel"] = {"value": round(v64, 3), "unit": "Gpairs/s",
                                "ms_per_step": round(r64["ms_per_step"], 3),
                                "far_kernel_ms": round(r64["far_ms"], 3),

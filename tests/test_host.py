@@ -30,6 +30,23 @@ def test_profiled_traffic_reads_committed_profile():
     assert b.profiled_traffic(64, 4) is None
 
 
+def test_bench_names_the_pass_that_runs():
+    """The bench's rule and limits are those the library is compiled with."""
+    import re
+    b = _bench()
+    src = open(os.path.join(ROOT, "starsmasher_amd", "csrc", "sg_internal.h")).read()
+    for name in ("WAVE_MAX_NI", "SYM_MIN_N", "SYM64_MIN_N", "SYM_MAX_N", "AUTO_SMALL_NI"):
+        value = re.search(rf"\b{name} = ([0-9< ]+)[,;]", src).group(1)
+        assert eval(value) == getattr(b, name), name
+    auto = (0, 1, 0)
+    assert [b.whole_set_pass(0, n, auto) for n in (16384, 49151, 49152, 65536, 1 << 20, (1 << 22) + 1)] == [
+        "waves", "waves", "unordered", "unordered", "unordered", "tiles"]
+    assert [b.whole_set_pass(1, n, auto) for n in (32768, 32769)] == ["tiles", "unordered"]
+    assert b.whole_set_pass(0, 60000, (128, 1, 0)) == "unordered"
+    for config in ((256, 1, 0), (128, 2, 0), (128, 1, 4)):
+        assert b.whole_set_pass(0, 60000, config) == "tiles"
+
+
 def test_bench_refuses_several_gpus():
     import subprocess
     import sys
